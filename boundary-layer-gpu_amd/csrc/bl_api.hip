@@ -417,8 +417,8 @@ void build(Handle &h, const bl_config *c) {
     h.phi = falloc();
     h.nu_t = falloc();
     if (h.les >= 2) {
-        h.dsm = dmalloc(nf * kDsmArrays);
-        BL_HIP(hipMemsetAsync(h.dsm, 0, nf * kDsmArrays * sizeof(double), h.stream));
+        h.dsm = dmalloc(dsm_doubles(h));
+        BL_HIP(hipMemsetAsync(h.dsm, 0, dsm_doubles(h) * sizeof(double), h.stream));
     }
     if (h.les == 1) {
         // sgs_Smagorinsky (subgrid.f90:609-662): Cs = 0.11, Delta_j =

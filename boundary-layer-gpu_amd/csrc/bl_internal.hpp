@@ -198,7 +198,7 @@ struct Handle {
     int icur;       // index of the current (most recent) buffer
     Field3 F1;      // first-stage RHS (RK3); FP64 RK3: G = Uo + dt a21 F1 instead (a21 = a31)
     double *P, *phi, *nu_t;  // float in mixed precision
-    double *dsm;  // dynamic Smagorinsky work arrays (LES = 2, 3 and 4), kDsmArrays field-sized slots
+    double *dsm;  // dynamic Smagorinsky work arrays (LES = 2, 3 and 4), dsm_doubles
     double *smag_c;  // LES = 1: (Cs Delta_j f_j)^2 per y row (nyg)
     // learned closure (LES = 4): BF16 weights, FP32 biases, input range
     unsigned short *cl_w;
@@ -397,7 +397,7 @@ struct IncSrc {
 void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const IncSrc *inc = nullptr);
 // eddy viscosity of f into h.nu_t (bl_dsm.hip): LES = 1 constant-coefficient
 // Smagorinsky, 2 and 4 dynamic Smagorinsky z-averaged, 3 per cell
-constexpr int kDsmArrays = 15;
+size_t dsm_doubles(const Handle &h);  // size of Handle::dsm
 void launch_dsm(Handle &h, const Field3 &f);
 // learned closure over the DSM values in h.nu_t (bl_closure.hip)
 void launch_closure(Handle &h, const Field3 &f);
