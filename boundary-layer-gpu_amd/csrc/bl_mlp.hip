@@ -3,19 +3,21 @@
 //
 // Network: 10 -> 64 -> 64 -> 64 -> 1 with SiLU, predicting the dimensionless
 // eddy viscosity c = nu_t / (Delta^2 |S|) from the normalised velocity-
-// gradient tensor and the wall distance.  FP32 master parameters, Adam; the
-// training forward/backward passes run in FP32 (one sample per lane, weights
-// broadcast from LDS), the weight gradients are per-block partial sums over a
-// batch slice reduced in a fixed order (deterministic).  A BF16 copy of the
+// gradient tensor and the wall distance.  FP32 master parameters, Adam; one
+// kernel does the forward and backward passes and the weight gradients of a
+// batch in FP32 on the matrix cores, with per-block partial gradients that the
+// update kernel adds in a fixed order (deterministic).  A BF16 copy of the
 // weights feeds the MFMA inference kernel (bl_closure.hip).
 //
 // Dataset rows (kRow floats): 10 features, target c, weight, Delta^2 |S|,
 // then S_ij and tau_ij (6 + 6, the a-priori checks).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/blgpu.h"
@@ -31,33 +33,11 @@ constexpr int oW1 = 0, ob1 = oW1 + kH * kIn, oW2 = ob1 + kH, ob2 = oW2 + kH * kH
               ob3 = oW3 + kH * kH, oW4 = ob3 + kH, ob4 = oW4 + kH;
 static_assert(ob4 + 1 == kMlpParams, "parameter layout");
 
-__device__ __forceinline__ float silu(float z) { return z / (1.f + expf(-z)); }
-__device__ __forceinline__ float dsilu(float z) {
-    const float s = 1.f / (1.f + expf(-z));
-    return s * (1.f + z * (1.f - s));
-}
-
 __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
     z += 0x9E3779B97F4A7C15ull;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     return z ^ (z >> 31);
-}
-
-// batch gather: sample b of step s is row hash(seed, s, b) mod n
-__global__ __launch_bounds__(256) void k_gather(const float *__restrict__ rows, long long n, int B,
-                                                unsigned long long seed, long long step, float wscale,
-                                                float *__restrict__ Xb, float *__restrict__ tb,
-                                                float *__restrict__ wb) {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= B) return;
-    const unsigned long long h = mix64(seed ^ mix64((unsigned long long)step * 0x100000001B3ull + (unsigned long long)b));
-    const long long r = (long long)(h % (unsigned long long)n);
-    const float *row = rows + r * kMlpRow;
-#pragma unroll
-    for (int f = 0; f < kIn; ++f) Xb[(long long)f * B + b] = row[f];
-    tb[b] = row[kIn];
-    wb[b] = row[kIn + 1] * wscale;
 }
 
 // sum and count of the positive row weights, per block (fixed order)
@@ -86,205 +66,355 @@ __global__ __launch_bounds__(256) void k_wsum(const float *__restrict__ rows, lo
     }
 }
 
-// stage the parameters in LDS
-__device__ __forceinline__ void load_params(float *sp, const float *__restrict__ theta) {
-    for (int q = threadIdx.x; q < kMlpParams; q += blockDim.x) sp[q] = theta[q];
+// ------------------------------------------------------------------------
+// Forward, backward and weight gradients of a batch, loss = (1/B) sum w (y-t)^2.
+// A block of eight waves takes tiles of kTs = 128 samples, 16 per wave, and
+// keeps everything of a tile on the chip.  Every product runs on
+// v_mfma_f32_16x16x4_f32 (lane l holds A[l%16][l/16], B[l/16][l%16] and
+// D[4 (l/16) + r][l%16], r < 4):
+//   layers   D = W h, columns = the wave's samples.  Accumulator register
+//            (t, r) of a lane is feature 16 t + 4 (l/16) + r of sample l%16;
+//            taking the features in that order along K, it is the next layer's
+//            B operand as it stands, and A is four consecutive weights of a
+//            row, so activations never leave the registers
+//   backward the same with A = W^T, read from the same copy of W
+//   dW       = dz h^T over the 128 samples: dz and h pass through LDS
+//            ([feature][sample]), each wave owns two 16 x 16 tiles of dW2 and
+//            dW3 and half of one of dW1
+// Bias and output-layer gradients are sums over lanes, kept per lane until
+// the end.  The row strides (68, 132) put the 16 rows of an operand read on
+// different banks.  Bound: 3.5 GFLOP at batch 65536 are 22 us of FP32 matrix
+// time, plus the SiLU evaluations between the products; measured 65 us, and
+// 11 us for the update.  The form before it (one sample per lane on the vector
+// units, activations and deltas through memory, seven launches) took 0.99 ms a
+// step.
+// ------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kTs = 128, kTWaves = 8;          // samples and waves per block
+constexpr int kWs = 68, kW1s = 13, kSs = 132;  // LDS row strides: W2 and W3, W1, sample rows
+
+__device__ __forceinline__ f32x4 mfma32(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// where the batch comes from: rows drawn by the counter hash of (seed, step,
+// slot) from the dataset (rows set), or the arrays X[f][b], t, w
+struct BatchSrc {
+    const float *rows;
+    long long n;
+    unsigned long long seed;
+    long long step;
+    float wscale;
+    const float *X, *t, *w;
+};
+
+struct TrainLds {
+    float w2[kH * kWs], w3[kH * kWs], w1[kH * kW1s];
+    float b1[kH], b2[kH], b3[kH], w4[kH];
+};
+struct GradLds {
+    float x[16 * kSs], h1[kH * kSs], h2[kH * kSs], d[kH * kSs];
+};
+
+// GRAD: write the block's partial gradients (part[block][kMlpParams]) and loss
+// sum; otherwise only y[b]
+template <bool GRAD>
+__global__ __launch_bounds__(64 * kTWaves) void k_batch(const float *__restrict__ theta, BatchSrc src, int B,
+                                                        float *__restrict__ y, float *__restrict__ part,
+                                                        double *__restrict__ loss) {
+    __shared__ TrainLds L;
+    __shared__ typename std::conditional<GRAD, GradLds, int>::type G_;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, q4 = lane >> 4;
+    for (int q = tid; q < kH * kH; q += 64 * kTWaves) {
+        L.w2[(q >> 6) * kWs + (q & 63)] = theta[oW2 + q];
+        L.w3[(q >> 6) * kWs + (q & 63)] = theta[oW3 + q];
+    }
+    for (int q = tid; q < kH * 12; q += 64 * kTWaves) {
+        const int o = q / 12, i = q - o * 12;
+        L.w1[o * kW1s + i] = i < kIn ? theta[oW1 + o * kIn + i] : 0.f;
+    }
+    if (tid < kH) {
+        L.b1[tid] = theta[ob1 + tid];
+        L.b2[tid] = theta[ob2 + tid];
+        L.b3[tid] = theta[ob3 + tid];
+        L.w4[tid] = theta[oW4 + tid];
+    }
+    if constexpr (GRAD)
+        for (int q = tid; q < 4 * kSs; q += 64 * kTWaves) G_.x[12 * kSs + q] = 0.f;  // features 12..15 do not exist
+    const float b4 = theta[ob4];
     __syncthreads();
-}
-
-// forward, one sample per lane: Z[l][f][b] pre-activations, y[b]
-__global__ __launch_bounds__(256) void k_fwd(const float *__restrict__ theta, const float *__restrict__ Xb, int B,
-                                             float *__restrict__ Z, float *__restrict__ y) {
-    __shared__ float sp[kMlpParams];
-    load_params(sp, theta);
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= B) return;
-    float x[kIn], h[kH], z[kH];
+    // per lane: bias and output-layer gradients of its features and samples
+    f32x4 g4[4], gb1[4], gb2[4], gb3[4], gw2[2], gw3[2], gw1;
+    float gb4 = 0.f;
+    double sq = 0.0;
 #pragma unroll
-    for (int f = 0; f < kIn; ++f) x[f] = Xb[(long long)f * B + b];
+    for (int t = 0; t < 4; ++t) g4[t] = gb1[t] = gb2[t] = gb3[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    gw2[0] = gw2[1] = gw3[0] = gw3[1] = gw1 = f32x4{0.f, 0.f, 0.f, 0.f};
+    // dW tiles of this wave: rows 16 rt.., columns 16 (ct + c)..; dW1: rows
+    // 16 (wave % 4).. over half of the samples
+    const int rt = wave >> 1, ct = 2 * (wave & 1);
+    auto layer = [&](const float *W, const float *bias, const f32x4 h[4], f32x4 z[4]) {
 #pragma unroll
-    for (int o = 0; o < kH; ++o) {
-        float a = sp[ob1 + o];
+        for (int o = 0; o < 4; ++o) z[o] = *reinterpret_cast<const f32x4 *>(bias + 16 * o + 4 * q4);
 #pragma unroll
-        for (int i = 0; i < kIn; ++i) a += sp[oW1 + o * kIn + i] * x[i];
-        z[o] = a;
-    }
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int o = 0; o < kH; ++o) {
-        Z[(long long)o * B + b] = z[o];
-        h[o] = silu(z[o]);
-    }
-    for (int l = 1; l < 3; ++l) {
-        const int oW = l == 1 ? oW2 : oW3, ob = l == 1 ? ob2 : ob3;
+            for (int o = 0; o < 4; ++o) {
+                const f32x4 w = *reinterpret_cast<const f32x4 *>(W + (16 * o + l16) * kWs + 16 * t + 4 * q4);
 #pragma unroll
-        for (int o = 0; o < kH; ++o) {
-            float a = sp[ob + o];
-#pragma unroll
-            for (int i = 0; i < kH; ++i) a += sp[oW + o * kH + i] * h[i];
-            z[o] = a;
-        }
-#pragma unroll
-        for (int o = 0; o < kH; ++o) {
-            Z[((long long)l * kH + o) * B + b] = z[o];
-            h[o] = silu(z[o]);
-        }
-    }
-    float a = sp[ob4];
-#pragma unroll
-    for (int i = 0; i < kH; ++i) a += sp[oW4 + i] * h[i];
-    y[b] = a;
-}
-
-// backward, one sample per lane: loss = (1/B) sum w (y - t)^2;
-// D[l][f][b] = dloss/dz, dy[b] = dloss/dy, sq[b] = w (y - t)^2
-__global__ __launch_bounds__(256) void k_bwd(const float *__restrict__ theta, const float *__restrict__ Z,
-                                             const float *__restrict__ y, const float *__restrict__ tb,
-                                             const float *__restrict__ wb, int B, float *__restrict__ D,
-                                             float *__restrict__ dyo, float *__restrict__ sq) {
-    __shared__ float sp[kMlpParams];
-    load_params(sp, theta);
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= B) return;
-    const float e = y[b] - tb[b];
-    const float w = wb[b];
-    sq[b] = w * e * e;
-    const float dy = 2.f * w * e / (float)B;
-    dyo[b] = dy;
-    float d[kH], a[kH];
-#pragma unroll
-    for (int o = 0; o < kH; ++o) d[o] = dy * sp[oW4 + o] * dsilu(Z[(2LL * kH + o) * B + b]);
-#pragma unroll
-    for (int o = 0; o < kH; ++o) D[(2LL * kH + o) * B + b] = d[o];
-    for (int l = 2; l >= 1; --l) {
-        const int oW = l == 2 ? oW3 : oW2;
-#pragma unroll
-        for (int i = 0; i < kH; ++i) a[i] = 0.f;
-#pragma unroll
-        for (int o = 0; o < kH; ++o)
-#pragma unroll
-            for (int i = 0; i < kH; ++i) a[i] += sp[oW + o * kH + i] * d[o];
-#pragma unroll
-        for (int i = 0; i < kH; ++i) {
-            d[i] = a[i] * dsilu(Z[((long long)(l - 1) * kH + i) * B + b]);
-            D[((long long)(l - 1) * kH + i) * B + b] = d[i];
-        }
-    }
-}
-
-// per-block partial parameter gradients over a slice of kSlice samples
-constexpr int kSub = 16;  // samples staged in LDS per sub-step
-constexpr int kSlice = 512;
-__global__ __launch_bounds__(256) void k_wgrad(const float *__restrict__ Xb, const float *__restrict__ Z,
-                                               const float *__restrict__ D, const float *__restrict__ dy, int B,
-                                               float *__restrict__ part) {
-    __shared__ float sx[kIn][kSub], sh[3][kH][kSub], sd[3][kH][kSub], sdy[kSub];
-    const int t = threadIdx.x;
-    const int s0 = blockIdx.x * kSlice, s1 = min(s0 + kSlice, B);
-    // thread t owns: W2/W3 rows o = t/4, columns 16*(t%4) .. +16 (32 accumulators)
-    const int o = t >> 2, i0 = (t & 3) * 16;
-    float a2[16], a3[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) a2[q] = a3[q] = 0.f;
-    // and W1 entries t, t+256, t+512 (< 640), one bias or W4 entry each, b4 on thread 0
-    float a1[3] = {0.f, 0.f, 0.f}, ab = 0.f, ab4 = 0.f;
-    for (int s = s0; s < s1; s += kSub) {
-        const int ns = min(kSub, s1 - s);
-        for (int q = t; q < kSub * (kIn + 6 * kH + 1); q += 256) {
-            const int c = q % kSub, r = q / kSub;
-            const int b = s + c;
-            const bool ok = c < ns;
-            if (r < kIn) {
-                sx[r][c] = ok ? Xb[(long long)r * B + b] : 0.f;
-            } else if (r < kIn + 3 * kH) {
-                const int l = (r - kIn) / kH, f = (r - kIn) % kH;
-                sh[l][f][c] = ok ? silu(Z[((long long)l * kH + f) * B + b]) : 0.f;
-            } else if (r < kIn + 6 * kH) {
-                const int l = (r - kIn - 3 * kH) / kH, f = (r - kIn - 3 * kH) % kH;
-                sd[l][f][c] = ok ? D[((long long)l * kH + f) * B + b] : 0.f;
-            } else {
-                sdy[c] = ok ? dy[b] : 0.f;
+                for (int r = 0; r < 4; ++r) z[o] = mfma32(w[r], h[t][r], z[o]);
             }
+    };
+    // z -> SiLU(z) in place, and its derivative
+    auto act = [&](f32x4 z[4], f32x4 ds[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = z[t][r], s = 1.f / (1.f + expf(-v));
+                if constexpr (GRAD) ds[t][r] = s * (1.f + v * (1.f - s));
+                z[t][r] = v / (1.f + expf(-v));
+            }
+    };
+    const int ntile = (B + kTs - 1) / kTs;
+    for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        const int col = 16 * wave + l16, b = tile * kTs + col;
+        const bool live = b < B;
+        const int bc = live ? b : B - 1;
+        float x[3], tgt, w;
+        if (src.rows) {
+            const unsigned long long h =
+                mix64(src.seed ^ mix64((unsigned long long)src.step * 0x100000001B3ull + (unsigned long long)bc));
+            const float *row = src.rows + (long long)(h % (unsigned long long)src.n) * kMlpRow;
+#pragma unroll
+            for (int ks = 0; ks < 3; ++ks) x[ks] = 4 * ks + q4 < kIn ? row[4 * ks + q4] : 0.f;
+            tgt = row[kIn];
+            w = row[kIn + 1] * src.wscale;
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < 3; ++ks) x[ks] = 4 * ks + q4 < kIn ? src.X[(long long)(4 * ks + q4) * B + bc] : 0.f;
+            tgt = GRAD ? src.t[bc] : 0.f;
+            w = GRAD ? src.w[bc] : 0.f;
         }
+        if (!live) w = 0.f;
+        f32x4 h[4], z[4], ds1[4], ds2[4], ds3[4];
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            z[o] = *reinterpret_cast<const f32x4 *>(L.b1 + 16 * o + 4 * q4);
+#pragma unroll
+            for (int ks = 0; ks < 3; ++ks) z[o] = mfma32(L.w1[(16 * o + l16) * kW1s + 4 * ks + q4], x[ks], z[o]);
+        }
+        act(z, ds1);
+        auto put = [&](float *dst, const f32x4 v[4]) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) dst[(16 * t + 4 * q4 + r) * kSs + col] = v[t][r];
+        };
+        if constexpr (GRAD) {
+#pragma unroll
+            for (int ks = 0; ks < 3; ++ks) G_.x[(4 * ks + q4) * kSs + col] = x[ks];
+            put(G_.h1, z);
+        }
+        layer(L.w2, L.b2, z, h);
+        act(h, ds2);
+        if constexpr (GRAD) put(G_.h2, h);
+        layer(L.w3, L.b3, h, z);
+        act(z, ds3);
+        float yv = 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const f32x4 w4 = *reinterpret_cast<const f32x4 *>(L.w4 + 16 * t + 4 * q4);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) yv += w4[r] * z[t][r];
+        }
+        yv += __shfl_xor(yv, 16);
+        yv += __shfl_xor(yv, 32);
+        yv += b4;
+        if constexpr (!GRAD) {
+            if (live && q4 == 0) y[b] = yv;
+        } else {
+            const float e = yv - tgt;
+            const float dy = 2.f * w * e / (float)B;
+            if (q4 == 0) {
+                sq += (double)(w * e * e);
+                gb4 += dy;
+            }
+            f32x4 dz[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const f32x4 w4 = *reinterpret_cast<const f32x4 *>(L.w4 + 16 * t + 4 * q4);
+                g4[t] += dy * z[t];
+                dz[t] = dy * w4 * ds3[t];
+                gb3[t] += dz[t];
+            }
+            // dz of a layer from that of the layer above: W^T dz, times the derivative
+            auto back = [&](const float *W, const f32x4 ds[4]) {
+                f32x4 a[4];
+#pragma unroll
+                for (int o = 0; o < 4; ++o) a[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int o = 0; o < 4; ++o)
+                            a[o] = mfma32(W[(16 * t + 4 * q4 + r) * kWs + 16 * o + l16], dz[t][r], a[o]);
+#pragma unroll
+                for (int o = 0; o < 4; ++o) dz[o] = a[o] * ds[o];
+            };
+            // dW tiles of this wave over the block's samples
+            auto wgrad = [&](const float *hs, f32x4 g[2]) {
+#pragma unroll
+                for (int k = 0; k < kTs / 16; ++k) {
+                    const f32x4 a = *reinterpret_cast<const f32x4 *>(G_.d + (16 * rt + l16) * kSs + 16 * k + 4 * q4);
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const f32x4 v =
+                            *reinterpret_cast<const f32x4 *>(hs + (16 * (ct + c) + l16) * kSs + 16 * k + 4 * q4);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) g[c] = mfma32(a[r], v[r], g[c]);
+                    }
+                }
+            };
+            put(G_.d, dz);
+            __syncthreads();
+            wgrad(G_.h2, gw3);
+            back(L.w3, ds2);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) gb2[t] += dz[t];
+            __syncthreads();  // the deltas of layer 3 are read
+            put(G_.d, dz);
+            __syncthreads();
+            wgrad(G_.h1, gw2);
+            back(L.w2, ds1);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) gb1[t] += dz[t];
+            __syncthreads();
+            put(G_.d, dz);
+            __syncthreads();
+            {
+                const int k0 = (wave >> 2) * (kTs / 32);
+#pragma unroll
+                for (int k = k0; k < k0 + kTs / 32; ++k) {
+                    const f32x4 a =
+                        *reinterpret_cast<const f32x4 *>(G_.d + (16 * (wave & 3) + l16) * kSs + 16 * k + 4 * q4);
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(G_.x + l16 * kSs + 16 * k + 4 * q4);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) gw1 = mfma32(a[r], v[r], gw1);
+                }
+            }
+            __syncthreads();  // before the next tile's x, h and deltas
+        }
+    }
+    if constexpr (GRAD) {
+        float *P = part + (long long)blockIdx.x * kMlpParams;
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = (16 * rt + 4 * q4 + r) * kH + 16 * (ct + c) + l16;
+                P[oW2 + e] = gw2[c][r];
+                P[oW3 + e] = gw3[c][r];
+            }
+        // sums over the 16 lanes of a feature, then over the waves
+        auto sum16 = [&](float v) {
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o);
+            return v;
+        };
+        float *sr = G_.h1;                                 // [wave][4][kH], then gb4
+        float *s1 = G_.h2;                                 // the second half of dW1
+        double *sd = reinterpret_cast<double *>(G_.d);     // [wave]
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int f = 16 * t + 4 * q4 + r;
+                const float a = sum16(gb1[t][r]), c = sum16(gb2[t][r]), e = sum16(gb3[t][r]), g = sum16(g4[t][r]);
+                if (l16 == 0) {
+                    sr[(wave * 4 + 0) * kH + f] = a;
+                    sr[(wave * 4 + 1) * kH + f] = c;
+                    sr[(wave * 4 + 2) * kH + f] = e;
+                    sr[(wave * 4 + 3) * kH + f] = g;
+                }
+            }
+        gb4 = sum16(gb4);  // lanes 0..15 hold the samples
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o);
+        if (lane == 0) {
+            sr[kTWaves * 4 * kH + wave] = gb4;
+            sd[wave] = sq;
+        }
+        if (wave >= 4)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s1[((wave - 4) * 4 + r) * 64 + lane] = gw1[r];
         __syncthreads();
-        for (int c = 0; c < kSub; ++c) {
-            const float d2 = sd[1][o][c], d3 = sd[2][o][c];
+        if (wave < 4 && l16 < kIn)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                a2[q] += d2 * sh[0][i0 + q][c];
-                a3[q] += d3 * sh[1][i0 + q][c];
-            }
+            for (int r = 0; r < 4; ++r)
+                P[oW1 + (16 * wave + 4 * q4 + r) * kIn + l16] = gw1[r] + s1[(wave * 4 + r) * 64 + lane];
+        if (tid < 4 * kH) {
+            const int c = tid >> 6, f = tid & 63;
+            float a = 0.f;
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                const int p = t + 256 * r;
-                if (p < kH * kIn) a1[r] += sd[0][p / kIn][c] * sx[p % kIn][c];
-            }
-            if (t < kH)
-                ab += sd[0][t][c];  // b1
-            else if (t < 2 * kH)
-                ab += sd[1][t - kH][c];  // b2
-            else if (t < 3 * kH)
-                ab += sd[2][t - 2 * kH][c];  // b3
-            else
-                ab += sdy[c] * sh[2][t - 3 * kH][c];  // W4
-            if (t == 0) ab4 += sdy[c];            // b4
+            for (int v = 0; v < kTWaves; ++v) a += sr[(v * 4 + c) * kH + f];
+            P[(c == 0 ? ob1 : (c == 1 ? ob2 : (c == 2 ? ob3 : oW4))) + f] = a;
         }
+        if (tid == 4 * kH) {
+            float a = 0.f;
+            double l = 0.0;
+            for (int v = 0; v < kTWaves; ++v) {
+                a += sr[kTWaves * 4 * kH + v];
+                l += sd[v];
+            }
+            P[ob4] = a;
+            loss[blockIdx.x] = l;
+        }
+    }
+}
+
+// g = the sum of the nb block partials, added in double in a fixed order:
+// eight groups of blocks, then the groups.  32 parameters per block, so that
+// the rows are read as 128-byte segments; one more block adds the loss sums
+// into lossf[0].  adam: also the update.
+__global__ __launch_bounds__(256) void k_update(const float *__restrict__ part, const double *__restrict__ loss, int nb,
+                                                float *__restrict__ g, float *__restrict__ theta,
+                                                float *__restrict__ m, float *__restrict__ v, int adam, float lr,
+                                                float c1, float c2, float *__restrict__ lossf) {
+    __shared__ double sh[8][32];
+    if (blockIdx.x == gridDim.x - 1) {
+        double *t = &sh[0][0], l = 0.0;
+        for (int q = threadIdx.x; q < nb; q += 256) l += loss[q];
+        t[threadIdx.x] = l;
         __syncthreads();
+        for (int st = 128; st > 0; st >>= 1) {
+            if ((int)threadIdx.x < st) t[threadIdx.x] += t[threadIdx.x + st];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) lossf[0] = (float)t[0];
+        return;
     }
-    float *P = part + (long long)blockIdx.x * kMlpParams;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        P[oW2 + o * kH + i0 + q] = a2[q];
-        P[oW3 + o * kH + i0 + q] = a3[q];
-    }
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-        const int p = t + 256 * r;
-        if (p < kH * kIn) P[oW1 + p] = a1[r];
-    }
-    if (t < kH)
-        P[ob1 + t] = ab;
-    else if (t < 2 * kH)
-        P[ob2 + t - kH] = ab;
-    else if (t < 3 * kH)
-        P[ob3 + t - 2 * kH] = ab;
-    else
-        P[oW4 + t - 3 * kH] = ab;
-    if (t == 0) P[ob4] = ab4;
-}
-
-// g[p] = sum over blocks of part[blk][p], fixed order
-__global__ __launch_bounds__(256) void k_gsum(const float *__restrict__ part, int nblk, float *__restrict__ g) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= kMlpParams) return;
-    float a = 0.f;
-    for (int q = 0; q < nblk; ++q) a += part[(long long)q * kMlpParams + p];
-    g[p] = a;
-}
-
-__global__ __launch_bounds__(256) void k_adam(float *__restrict__ theta, float *__restrict__ m, float *__restrict__ v,
-                                              const float *__restrict__ g, float lr, float c1, float c2) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= kMlpParams) return;
-    const float gp = g[p];
-    const float mp = 0.9f * m[p] + 0.1f * gp;
-    const float vp = 0.999f * v[p] + 0.001f * gp * gp;
-    m[p] = mp;
-    v[p] = vp;
-    theta[p] -= lr * (mp / c1) / (sqrtf(vp / c2) + 1e-8f);
-}
-
-// sum of n values into out[0], one block, fixed order
-__global__ __launch_bounds__(256) void k_sum(const float *__restrict__ a, int n, float *__restrict__ out) {
-    __shared__ double sh[256];
-    double s = 0.0;
-    for (int q = threadIdx.x; q < n; q += 256) s += a[q];
-    sh[threadIdx.x] = s;
+    const int f = threadIdx.x & 31, s = threadIdx.x >> 5, p = blockIdx.x * 32 + f;
+    double a = 0.0;
+    if (p < kMlpParams)
+        for (int q = s; q < nb; q += 8) a += (double)part[(long long)q * kMlpParams + p];
+    sh[s][f] = a;
     __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-        __syncthreads();
+    if (s == 0 && p < kMlpParams) {
+        double t = 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t += sh[q][f];
+        const float gp = (float)t;
+        g[p] = gp;
+        if (adam) {
+            const float mp = 0.9f * m[p] + 0.1f * gp;
+            const float vp = 0.999f * v[p] + 0.001f * gp * gp;
+            m[p] = mp;
+            v[p] = vp;
+            theta[p] -= lr * (mp / c1) / (sqrtf(vp / c2) + 1e-8f);
+        }
     }
-    if (threadIdx.x == 0) out[0] = (float)sh[0];
 }
 
 void check() {
@@ -317,16 +447,17 @@ void mlp_init(Mlp &m, long long capacity, int batch_max) {
     m.adam_m = alloc<float>(kMlpParams);
     m.adam_v = alloc<float>(kMlpParams);
     m.g = alloc<float>(kMlpParams);
-    m.nslice = (batch_max + kSlice - 1) / kSlice;
-    m.part = alloc<float>((size_t)m.nslice * kMlpParams);
+    int dev = 0, ncu = 0;
+    BL_HIP(hipGetDevice(&dev));
+    BL_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    // one resident block per compute unit (its LDS), each looping over tiles
+    m.nblk = std::max(1, std::min(ncu, (batch_max + kTs - 1) / kTs));
+    m.part = alloc<float>((size_t)m.nblk * kMlpParams);
+    m.loss = alloc<double>(m.nblk);
     m.Xb = alloc<float>((size_t)kIn * batch_max);
     m.tb = alloc<float>(batch_max);
     m.wb = alloc<float>(batch_max);
-    m.Z = alloc<float>((size_t)3 * kH * batch_max);
-    m.D = alloc<float>((size_t)3 * kH * batch_max);
     m.y = alloc<float>(batch_max);
-    m.dy = alloc<float>(batch_max);
-    m.sq = alloc<float>(batch_max);
     m.scal = alloc<float>(16);
     BL_HIP(hipMemsetAsync(m.theta, 0, kMlpParams * sizeof(float), m.stream));
     BL_HIP(hipMemsetAsync(m.adam_m, 0, kMlpParams * sizeof(float), m.stream));
@@ -336,8 +467,8 @@ void mlp_init(Mlp &m, long long capacity, int batch_max) {
 
 void mlp_free(Mlp &m) {
     for (void *p : {(void *)m.rows, (void *)m.theta, (void *)m.adam_m, (void *)m.adam_v, (void *)m.g, (void *)m.part,
-                    (void *)m.Xb, (void *)m.tb, (void *)m.wb, (void *)m.Z, (void *)m.D, (void *)m.y, (void *)m.dy,
-                    (void *)m.sq, (void *)m.scal})
+                    (void *)m.loss, (void *)m.Xb, (void *)m.tb, (void *)m.wb, (void *)m.y, (void *)m.scal,
+                    (void *)m.hist})
         if (p) (void)hipFree(p);
     if (m.stream) {
         (void)hipStreamSynchronize(m.stream);
@@ -345,21 +476,31 @@ void mlp_free(Mlp &m) {
     }
 }
 
-// forward + backward + weight gradient of the batch already in Xb/tb/wb;
-// leaves g and the batch loss sum in scal[0]
+namespace {
+void launch_grad(Mlp &m, const BatchSrc &src, int B, bool adam, float lr, float c1, float c2, float *loss) {
+    const int nb = std::min(m.nblk, (B + kTs - 1) / kTs);
+    hipLaunchKernelGGL(k_batch<true>, dim3(nb), dim3(64 * kTWaves), 0, m.stream, m.theta, src, B, (float *)nullptr,
+                       m.part, m.loss);
+    check();
+    hipLaunchKernelGGL(k_update, dim3((kMlpParams + 31) / 32 + 1), dim3(256), 0, m.stream, m.part, m.loss, nb, m.g, m.theta,
+                       m.adam_m, m.adam_v, adam ? 1 : 0, lr, c1, c2, loss);
+    check();
+}
+}  // namespace
+
+// the batch in Xb/tb/wb: forward into y, or the gradient into g and the batch
+// loss sum into scal[0]
 void mlp_fwd_bwd(Mlp &m, int B, bool backward) {
-    const dim3 gb((B + 255) / 256), blk(256);
-    hipLaunchKernelGGL(k_fwd, gb, blk, 0, m.stream, m.theta, m.Xb, B, m.Z, m.y);
-    check();
-    if (!backward) return;
-    hipLaunchKernelGGL(k_bwd, gb, blk, 0, m.stream, m.theta, m.Z, m.y, m.tb, m.wb, B, m.D, m.dy, m.sq);
-    check();
-    const int ns = (B + kSlice - 1) / kSlice;
-    hipLaunchKernelGGL(k_wgrad, dim3(ns), blk, 0, m.stream, m.Xb, m.Z, m.D, m.dy, B, m.part);
-    check();
-    hipLaunchKernelGGL(k_gsum, dim3((kMlpParams + 255) / 256), blk, 0, m.stream, m.part, ns, m.g);
-    check();
-    hipLaunchKernelGGL(k_sum, dim3(1), blk, 0, m.stream, m.sq, B, m.scal);
+    BatchSrc src{};
+    src.X = m.Xb;
+    src.t = m.tb;
+    src.w = m.wb;
+    if (backward) {
+        launch_grad(m, src, B, false, 0.f, 1.f, 1.f, m.scal);
+        return;
+    }
+    hipLaunchKernelGGL(k_batch<false>, dim3((B + kTs - 1) / kTs), dim3(64 * kTWaves), 0, m.stream, m.theta, src, B, m.y,
+                       (float *)nullptr, (double *)nullptr);
     check();
 }
 
@@ -405,24 +546,30 @@ void mlp_train(Mlp &m, int steps, int B, float lr, unsigned long long seed, floa
         throw ArgError();
     }
     const float wscale = (float)(wcnt / wsum);
+    // the steps' loss sums stay on the device and cross to the host once
+    if (loss_hist && m.nhist < steps) {
+        if (m.hist) BL_HIP(hipFree(m.hist));
+        m.hist = nullptr;
+        m.nhist = 0;
+        m.hist = alloc<float>(steps);
+        m.nhist = steps;
+    }
+    BatchSrc src{};
+    src.rows = m.rows;
+    src.n = m.n;
+    src.seed = seed;
+    src.wscale = wscale;
     for (int s = 0; s < steps; ++s) {
-        hipLaunchKernelGGL(k_gather, dim3((B + 255) / 256), blk, 0, m.stream, m.rows, m.n, B, seed, m.step, wscale,
-                           m.Xb, m.tb, m.wb);
-        check();
-        mlp_fwd_bwd(m, B, true);
+        src.step = m.step;
         m.step += 1;
         const float c1 = 1.f - powf(0.9f, (float)m.step), c2 = 1.f - powf(0.999f, (float)m.step);
-        hipLaunchKernelGGL(k_adam, dim3((kMlpParams + 255) / 256), blk, 0, m.stream, m.theta, m.adam_m, m.adam_v,
-                           m.g, lr, c1, c2);
-        check();
-        if (loss_hist) {
-            float l = 0.f;
-            BL_HIP(hipMemcpyAsync(&l, m.scal, sizeof(float), hipMemcpyDeviceToHost, m.stream));
-            BL_HIP(hipStreamSynchronize(m.stream));
-            loss_hist[s] = l / (float)B;
-        }
+        launch_grad(m, src, B, true, lr, c1, c2, loss_hist ? m.hist + s : m.scal);
     }
+    if (loss_hist && steps > 0)
+        BL_HIP(hipMemcpyAsync(loss_hist, m.hist, sizeof(float) * steps, hipMemcpyDeviceToHost, m.stream));
     BL_HIP(hipStreamSynchronize(m.stream));
+    if (loss_hist)
+        for (int s = 0; s < steps; ++s) loss_hist[s] /= (float)B;
 }
 
 }  // namespace blgpu

@@ -19,12 +19,15 @@ constexpr int kRowTarget = kMlpIn, kRowWeight = kMlpIn + 1, kRowScale = kMlpIn +
 struct Mlp {
     long long cap, n;   // dataset capacity and fill (rows)
     int bmax;           // largest training batch
-    int nslice;         // partial-gradient slices of bmax
+    int nblk;           // blocks of the gradient kernel at bmax (partial gradients)
     long long step;     // Adam steps taken
     hipStream_t stream;
     float *rows;        // dataset [cap][kMlpRow]
     float *theta, *adam_m, *adam_v, *g, *part;
-    float *Xb, *tb, *wb, *Z, *D, *y, *dy, *sq, *scal;
+    double *loss;       // loss sums per block
+    float *Xb, *tb, *wb, *y, *scal;
+    float *hist;        // loss sums of one training call's steps [nhist]
+    int nhist;
 };
 
 void mlp_init(Mlp &m, long long capacity, int batch_max);

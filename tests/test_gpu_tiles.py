@@ -6,7 +6,7 @@ import sys
 import numpy as np
 import pytest
 
-from . import cases, orc
+from . import cases, mlp_ref as M, orc
 from .blgpu_import import blgpu
 from .test_oracle_dsm import random_case
 
@@ -47,3 +47,42 @@ def test_dsm_tile_edges(shape, les):
     err = np.abs(s.download(4) - ref).max() / np.abs(ref).max()
     say("nu_t err", err)
     assert err < 1e-11
+
+
+# the gradient kernel takes tiles of 128 samples, one block per compute unit
+# (256) looping over them: a part of a wave, one tile and its neighbours, and
+# more tiles than blocks; FP32 sums to 1e-4 as in the closure's gradient tests
+@pytest.mark.parametrize("n", [15, 127, 128, 129, 128 * 256 + 17, 128 * 300])
+def test_mlp_gradient_tiles(n):
+    say("mlp gradient", n)
+    rng = np.random.default_rng(n)
+    X = rng.uniform(-1, 1, (n, 10)).astype(np.float32)
+    t = (0.05 * np.tanh(X[:, 0] * X[:, 1])).astype(np.float32)
+    c = blgpu.Closure(capacity=16, batch_max=n)
+    theta = M.init_params(3).astype(np.float32)
+    c.params = theta
+    g, loss = c.gradient(X, t)
+    gr = M.grad(theta.astype(np.float64), X.astype(np.float64), t.astype(np.float64))
+    y, _ = M.forward(theta.astype(np.float64), X.astype(np.float64))
+    assert np.linalg.norm(g - gr) / np.linalg.norm(gr) < 1e-4
+    assert np.abs(c.forward(X) - y).max() / np.abs(y).max() < 1e-5
+    assert loss == pytest.approx(np.mean((y - t) ** 2), rel=1e-5)
+    c.close()
+
+
+@pytest.mark.parametrize("steps", [0, 1, 3])
+def test_mlp_history_of_repeated_training(steps):
+    """Every call returns its own steps' losses, longer or shorter than the last call's."""
+    rng = np.random.default_rng(1)
+    rows = np.zeros((500, 28), dtype=np.float32)
+    rows[:, :10] = rng.uniform(-1, 1, (500, 10))
+    rows[:, 10] = 0.1 * rows[:, 0]
+    rows[:, 11] = 1.0
+    one, two = (blgpu.Closure(capacity=500, batch_max=300) for _ in range(2))
+    for c in (one, two):
+        c.add_rows(rows)
+        c.params = M.init_params(3).astype(np.float32)
+    a = np.concatenate([one.train(4, 300, seed=5), one.train(steps, 300, seed=5)])
+    b = two.train(4 + steps, 300, seed=5)
+    np.testing.assert_array_equal(a, b)
+    np.testing.assert_array_equal(one.params, two.params)
