@@ -634,7 +634,7 @@ void build(Handle &h, const bl_config *c) {
         // reduction scratch: 3 partials per interior block, flux partials, Cf, monitor planes
         const size_t nb = (size_t)((d.nxg - 2 + 63) / 64) * ((d.nyg - 2 + 3) / 4) * (d.nzg - 2);
         const size_t nq = (size_t)(((d.nyg + 255) / 256) + ((d.nxg + 255) / 256)) * d.nzg;
-        h.red = dmalloc(std::max({3 * nb, nq, (size_t)d.nxg, (size_t)8 * d.nzg, (size_t)1024}));
+        h.red = dmalloc(std::max({3 * nb, nq, (size_t)d.nxg, (size_t)monitor_partials(d), (size_t)1024}));
     }
     BL_HIP(hipStreamSynchronize(h.stream));
 }

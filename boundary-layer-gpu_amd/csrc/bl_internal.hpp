@@ -329,6 +329,7 @@ template <class T>
 void wall_stats(Handle &h, const Fld3<T> &f, double *cf_host);
 template <class T>
 void monitor(Handle &h, const Fld3<T> &f, double *out_host);
+long long monitor_partials(const Dims &d);  // doubles that monitor() needs in Handle::red
 template <class T>
 double dt_convective(Handle &h, const Fld3<T> &f);
 // the z DFT tables cos/sin(2 pi k m / M), [m][k] with leading dimension lda,

@@ -1887,74 +1887,128 @@ __global__ __launch_bounds__(1024) void k_reduce_max(const double *part, long lo
     }
 }
 
-// Cf(x) (statistics.f90:137-160): one thread per x face
+// Cf(x) (statistics.f90:137-160).  64 x faces by 16 groups of z planes per
+// block, whose seven sums meet in LDS in a fixed order; one thread per face
+// walking every plane was a serial chain of 191 loads in four blocks at
+// 814x257x193 (0.116 -> 0.022 ms).
+constexpr int kWsZ = 16;
 template <class T>
-__global__ __launch_bounds__(256) void k_wallstats(Dims d, Metrics m, double nu, const T *U, const T *V,
-                                                   const T *nu_t, double *cf) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= d.nx) return;
+__global__ __launch_bounds__(64 * kWsZ) void k_wallstats(Dims d, Metrics m, double nu, const T *U, const T *V,
+                                                         const T *nu_t, double *cf) {
+    __shared__ double sh[7][kWsZ][64];
+    const int tx = threadIdx.x & 63, g = threadIdx.x >> 6, i = blockIdx.x * 64 + tx;
     const double nz2 = (double)(d.nzg - 2);
     // the x neighbour of the last station is column nxg of nu_t_mean, which
     // compute_statistics never fills (statistics.f90:77 runs ii = 1..nx): 0
-    const bool last = i == d.nx - 1;
-    double u1 = 0.0, u2 = 0.0, uv = 0.0, n1a = 0.0, n2a = 0.0, n1b = 0.0, n2b = 0.0;
-    for (int k = 1; k <= d.nzg - 2; ++k) {
-        const long long p = fidx(d, i, 0, k);
-        const double a = (double)U[p], b = (double)U[p + d.sx];
-        u1 += a;
-        u2 += b;
-        uv += (m.wy0[0] * a + m.wy1[0] * b) * (0.5 * ((double)V[p] + (double)V[p + 1]));
-        n1a += (double)nu_t[p];
-        n2a += (double)nu_t[p + d.sx];
-        if (!last) {
-            n1b += (double)nu_t[p + 1];
-            n2b += (double)nu_t[p + 1 + d.sx];
+    const bool last = i >= d.nx - 1;
+    double s[7] = {0, 0, 0, 0, 0, 0, 0};  // u1, u2, uv, n1a, n2a, n1b, n2b
+    if (i < d.nx)
+        for (int k = 1 + g; k <= d.nzg - 2; k += kWsZ) {
+            const long long p = fidx(d, i, 0, k);
+            const double a = (double)U[p], b = (double)U[p + d.sx];
+            s[0] += a;
+            s[1] += b;
+            s[2] += (m.wy0[0] * a + m.wy1[0] * b) * (0.5 * ((double)V[p] + (double)V[p + 1]));
+            s[3] += (double)nu_t[p];
+            s[4] += (double)nu_t[p + d.sx];
+            if (!last) {
+                s[5] += (double)nu_t[p + 1];
+                s[6] += (double)nu_t[p + 1 + d.sx];
+            }
         }
+#pragma unroll
+    for (int q = 0; q < 7; ++q) sh[q][g][tx] = s[q];
+    __syncthreads();
+    if (g != 0 || i >= d.nx) return;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+        s[q] = 0.0;
+        for (int r = 0; r < kWsZ; ++r) s[q] += sh[q][r][tx];
     }
-    const double dudy = (u2 / nz2 - u1 / nz2) / (m.yg[1] - m.yg[0]);
-    const double tau = 0.25 * (n1a / nz2 + n2a / nz2 + n1b / nz2 + n2b / nz2) * dudy;
-    cf[i] = 2.0 * (-(uv / nz2) + nu * dudy + tau) / 1.0;
+    const double dudy = (s[1] / nz2 - s[0] / nz2) / (m.yg[1] - m.yg[0]);
+    const double tau = 0.25 * (s[3] / nz2 + s[4] / nz2 + s[5] / nz2 + s[6] / nz2) * dudy;
+    cf[i] = 2.0 * (-(s[2] / nz2) + nu * dudy + tau) / 1.0;
 }
 
-// per-plane sums and maxima of the four monitored interiors (monitor.f90:29-52)
+// sums and maxima of the four monitored interiors (monitor.f90:29-52): eight
+// partials per block of kMonJ rows of one plane, then k_monitor_reduce.  Bound
+// by the read of the four fields (1.3 GB, 0.25 ms of HBM time at 814x257x193);
+// one block per plane left the chip idle and took 1.71 ms, this form 0.23.
+constexpr int kMonJ = 8;
 template <class T>
-__global__ __launch_bounds__(256) void k_monitor(Dims d, const T *U, const T *V, const T *W, const T *nu_t,
-                                                 double *part) {
-    const int k = blockIdx.x + 1;  // plane
-    __shared__ double sh[8][256];
+__global__ __launch_bounds__(256) void k_monitor(Dims d, const T *__restrict__ U, const T *__restrict__ V,
+                                                 const T *__restrict__ W, const T *__restrict__ nu_t,
+                                                 double *__restrict__ part) {
+    const int k = blockIdx.y + 1;  // plane
+    __shared__ double sh[8][4];
     double s[4] = {0, 0, 0, 0}, mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int j = 1; j <= d.nyg - 2; ++j)
-        for (int i = threadIdx.x + 1; i <= d.nxg - 2; i += 256) {
-            const long long p = fidx(d, i, j, k);
+    const int j0 = 1 + blockIdx.x * kMonJ;
+    for (int i = threadIdx.x; i <= d.nxg - 2; i += 256) {  // from 0, so that a wave's row starts on a 128-byte line
+        T u[kMonJ], v[kMonJ], w[kMonJ], n[kMonJ];
+#pragma unroll
+        for (int r = 0; r < kMonJ; ++r) {
+            const long long p = fidx(d, i, min(j0 + r, d.nyg - 2), k);
+            u[r] = U[p];
+            v[r] = V[p];
+            w[r] = W[p];
+            n[r] = nu_t[p];
+        }
+#pragma unroll
+        for (int r = 0; r < kMonJ; ++r) {
+            const int j = j0 + r;
+            if (i < 1 || j > d.nyg - 2) continue;
             if (i <= d.nx - 2) {
-                s[0] += (double)U[p];
-                mx[0] = fmax(mx[0], (double)U[p]);
+                s[0] += (double)u[r];
+                mx[0] = fmax(mx[0], (double)u[r]);
             }
             if (j <= d.ny - 2) {
-                s[1] += (double)V[p];
-                mx[1] = fmax(mx[1], (double)V[p]);
+                s[1] += (double)v[r];
+                mx[1] = fmax(mx[1], (double)v[r]);
             }
             if (k <= d.nz - 2) {
-                s[2] += (double)W[p];
-                mx[2] = fmax(mx[2], (double)W[p]);
+                s[2] += (double)w[r];
+                mx[2] = fmax(mx[2], (double)w[r]);
             }
-            s[3] += (double)nu_t[p];
-            mx[3] = fmax(mx[3], (double)nu_t[p]);
+            s[3] += (double)n[r];
+            mx[3] = fmax(mx[3], (double)n[r]);
         }
-    for (int q = 0; q < 4; ++q) {
-        sh[q][threadIdx.x] = s[q];
-        sh[4 + q][threadIdx.x] = mx[q];
     }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        for (int o = 32; o > 0; o >>= 1) {
+            s[q] += __shfl_down(s[q], o);
+            mx[q] = fmax(mx[q], __shfl_down(mx[q], o));
+        }
+    if ((threadIdx.x & 63) == 0)
+        for (int q = 0; q < 4; ++q) {
+            sh[q][threadIdx.x >> 6] = s[q];
+            sh[4 + q][threadIdx.x >> 6] = mx[q];
+        }
+    __syncthreads();
+    if (threadIdx.x < 8) {
+        const double *v = sh[threadIdx.x];
+        const double r = threadIdx.x < 4 ? (v[0] + v[1]) + (v[2] + v[3]) : fmax(fmax(v[0], v[1]), fmax(v[2], v[3]));
+        part[8 * ((long long)blockIdx.x + (long long)gridDim.x * blockIdx.y) + threadIdx.x] = r;
+    }
+}
+
+// block q reduces quantity q (0-3 sums, 4-7 maxima) of the n partials
+__global__ __launch_bounds__(256) void k_monitor_reduce(const double *__restrict__ part, long long n,
+                                                        double *__restrict__ out) {
+    __shared__ double sh[256];
+    const int q = blockIdx.x;
+    double v = q < 4 ? 0.0 : -INFINITY;
+    for (long long t = threadIdx.x; t < n; t += 256) v = q < 4 ? v + part[8 * t + q] : fmax(v, part[8 * t + q]);
+    sh[threadIdx.x] = v;
     __syncthreads();
     for (int st = 128; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st)
-            for (int q = 0; q < 4; ++q) {
-                sh[q][threadIdx.x] += sh[q][threadIdx.x + st];
-                sh[4 + q][threadIdx.x] = fmax(sh[4 + q][threadIdx.x], sh[4 + q][threadIdx.x + st]);
-            }
+        if ((int)threadIdx.x < st) {
+            const double b = sh[threadIdx.x + st];
+            sh[threadIdx.x] = q < 4 ? sh[threadIdx.x] + b : fmax(sh[threadIdx.x], b);
+        }
         __syncthreads();
     }
-    if (threadIdx.x < 8) part[(long long)(k - 1) * 8 + threadIdx.x] = sh[threadIdx.x][0];
+    if (threadIdx.x == 0) out[q] = sh[0];
 }
 
 // reductions: each thread walks z planes with stride kRedZ, so the partials
@@ -2397,7 +2451,7 @@ double dt_convective(Handle &h, const Fld3<T> &f) {
 template <class T>
 void wall_stats(Handle &h, const Fld3<T> &f, double *cf_host) {
     const Dims &d = h.d;
-    hipLaunchKernelGGL(k_wallstats<T>, dim3((d.nx + 255) / 256), dim3(256), 0, h.stream, d, h.m, h.nu, f.u, f.v,
+    hipLaunchKernelGGL(k_wallstats<T>, dim3((d.nx + 63) / 64), dim3(64 * kWsZ), 0, h.stream, d, h.m, h.nu, f.u, f.v,
                        reinterpret_cast<const T *>(h.nu_t), h.red);
     check_launch();
     BL_HIP(hipMemcpyAsync(cf_host, h.red, sizeof(double) * d.nx, hipMemcpyDeviceToHost, h.stream));
@@ -2407,23 +2461,17 @@ void wall_stats(Handle &h, const Fld3<T> &f, double *cf_host) {
 template <class T>
 void monitor(Handle &h, const Fld3<T> &f, double *out) {
     const Dims &d = h.d;
-    const int np = d.nzg - 2;
-    hipLaunchKernelGGL(k_monitor<T>, dim3(np), dim3(256), 0, h.stream, d, f.u, f.v, f.w,
-                       reinterpret_cast<const T *>(h.nu_t), h.red);
+    const dim3 g((d.nyg - 2 + kMonJ - 1) / kMonJ, d.nzg - 2);
+    hipLaunchKernelGGL(k_monitor<T>, g, dim3(256), 0, h.stream, d, f.u, f.v, f.w, reinterpret_cast<const T *>(h.nu_t),
+                       h.red);
     check_launch();
-    std::vector<double> part((size_t)np * 8);
-    BL_HIP(hipMemcpyAsync(part.data(), h.red, sizeof(double) * part.size(), hipMemcpyDeviceToHost, h.stream));
+    hipLaunchKernelGGL(k_monitor_reduce, dim3(8), dim3(256), 0, h.stream, h.red, (long long)g.x * g.y, h.scal);
+    check_launch();
+    BL_HIP(hipMemcpyAsync(out, h.scal, 8 * sizeof(double), hipMemcpyDeviceToHost, h.stream));
     BL_HIP(hipStreamSynchronize(h.stream));
-    for (int q = 0; q < 4; ++q) {
-        out[q] = 0.0;
-        out[4 + q] = -INFINITY;
-    }
-    for (int k = 0; k < np; ++k)
-        for (int q = 0; q < 4; ++q) {
-            out[q] += part[(size_t)k * 8 + q];
-            out[4 + q] = std::fmax(out[4 + q], part[(size_t)k * 8 + 4 + q]);
-        }
 }
+
+long long monitor_partials(const Dims &d) { return 8LL * ((d.nyg - 2 + kMonJ - 1) / kMonJ) * (d.nzg - 2); }
 
 #define BL_INSTANTIATE(T)                                                                                   \
     template void launch_rk_stage<T>(Handle &, const Fld3<T> &, const Fld3<T> &, Fld3<T> &, int, double); \

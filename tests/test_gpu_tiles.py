@@ -86,3 +86,47 @@ def test_mlp_history_of_repeated_training(steps):
     b = two.train(4 + steps, 300, seed=5)
     np.testing.assert_array_equal(a, b)
     np.testing.assert_array_equal(one.params, two.params)
+
+
+# statistics blocks: 64 columns by 4 plane groups, wall stress 64 by 16, monitor
+# 8 rows of 256 columns: one column less and more than a block, fewer planes
+# than groups, the smallest grid.  FP64 sums in another order: a few roundings
+# of at most a few hundred terms, 1e-12 relative to the largest value.
+@pytest.mark.parametrize("shape", [(64, 8, 18), (65, 9, 17), (5, 4, 5), (257, 18, 6), (258, 17, 40)])
+def test_statistics_block_edges(shape):
+    say("statistics", shape)
+    x, y, z, U, V, W = random_case(sum(shape), *shape)
+    rng = np.random.default_rng(2)
+    n = (shape[0] + 1, shape[1] + 1, shape[2] + 1)
+    P, N = (np.asfortranarray(rng.standard_normal(n)) for _ in range(2))
+    s = solver(x, y, z)
+    s.set_fields(U, V, W)
+    s.upload(3, P)
+    s.upload(4, N)
+    st = s.statistics()
+    _, yg = orc.centers(y)
+    w0 = ((yg[1:] - y) / np.diff(yg))[None, :, None]
+    u = w0 * U[:, :-1, 1:-1] + (1 - w0) * U[:, 1:, 1:-1]
+    v = 0.5 * (V[:-1, :, 1:-1] + V[1:, :, 1:-1])
+    w = 0.5 * (W[:-1, :, :-2] + W[1:, :, :-2])
+    w = w0 * w[:, :-1] + (1 - w0) * w[:, 1:]
+    p = P[:-1, :-1, 1:-1]
+    nz = shape[2] - 2
+    ref = dict(Umean=u.mean(2), Vmean=v.mean(2), Wmean=w.sum(2) / nz, U2mean=(u * u).mean(2), V2mean=(v * v).mean(2),
+               W2mean=(w * w).sum(2) / nz, UVmean=(u * v).mean(2), Pmean=p.mean(2), P2mean=(p * p).mean(2))
+    for k, r in ref.items():
+        assert np.abs(st[k] - r).max() < 1e-12 * np.abs(r).max(), k
+    nm = N[:-1, :-1, 1:-1].mean(2)
+    assert np.abs(st["nu_t_mean"][:-1, :-1] - nm).max() < 1e-12 * np.abs(nm).max()
+    dudy = (U[:, 1, 1:-1] - U[:, 0, 1:-1]).mean(1) / (yg[1] - yg[0])
+    nm2 = np.zeros(n[:2])
+    nm2[:-1, :-1] = nm
+    tau = 0.25 * (nm2[:-1, 0] + nm2[:-1, 1] + nm2[1:, 0] + nm2[1:, 1]) * dudy
+    cf = 2 * (1e-5 * dudy + tau - (u[:, 0] * v[:, 0]).mean(1))
+    assert np.abs(st["Cf"] - cf).max() < 1e-12 * np.abs(cf).max()
+    I = slice(1, -1)
+    parts = [a[I, I, I] for a in (U, V, W, N)]
+    scale = np.array([np.abs(a).sum() for a in parts])
+    got = s.monitor()
+    assert np.all(np.abs(got[:4] - [a.sum() for a in parts]) < 1e-13 * scale)
+    np.testing.assert_array_equal(got[4:], [a.max() for a in parts])
