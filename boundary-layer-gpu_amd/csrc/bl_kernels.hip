@@ -2160,22 +2160,40 @@ const MetricsT<float> &metrics<float>(const Handle &h) {
 
 
 template <class T>
-dim3 march_grid(const Dims &d, int chunk) {
+int march_tiles(const Dims &d) {
     constexpr int kTX = MarchTile<T>::TX, kTY = MarchTile<T>::TY;
-    return dim3(xcd_blocks((d.nxg - 1 + kTX - 1) / kTX * ((d.nyg - 2 + kTY - 1) / kTY) *
-                           ((d.nzg - 2 + chunk - 1) / chunk)));
+    return (d.nxg - 1 + kTX - 1) / kTX * ((d.nyg - 2 + kTY - 1) / kTY);
 }
 
-// z-chunk length of the march.  The tiles run in XCD-contiguous order with
-// the z chunk slowest, so with a multiple of 8 chunks each XCD holds whole
-// chunk layers and a tile's x and y neighbours (whose halos it shares) sit in
-// the same L2; the count is the multiple of 8 that gives chunks of about 24
-// planes.  At 814x257x193 (8 chunks of 24 planes) this measured 1 % (FP64)
-// and 2.4 % (FP32) faster than 12 chunks of 16, and 20-plane chunks (10
-// chunks) 4-5 % slower.  Below 128 planes, chunks of up to 16 planes (the
-// two re-read halo planes stay a small share).
-inline int march_chunk(const Dims &d) {
-    const int nz = d.nzg - 2;
+// z-chunk length of the march.
+// While the launch fits in two rounds of resident blocks (three per compute
+// unit, `slots`), the chip is not filled by bytes but by plane steps in
+// sequence, and the chunk is the one with the fewest of them, rounds times
+// (chunk + 2): a block also loads the planes before and behind its chunk.  RK
+// stage, chunks of 16 or 24 planes -> this rule: 192x32x8 21 -> 9 us,
+// 129x49x34 LES FP32 54 -> 12, 257x97x64 LES FP32 76 -> 34, 131x75x53 36 -> 20,
+// 262x66x230 FP32 103 -> 52, 513x97x130 139 -> 109.
+// Larger launches are bound by HBM.  The tiles run in XCD-contiguous order
+// with the z chunk slowest, so with a multiple of 8 chunks each XCD holds
+// whole chunk layers and a tile's x and y neighbours (whose halos it shares)
+// sit in the same L2; the count is the multiple of 8 that gives chunks of
+// about 24 planes.  At 814x257x193 (8 chunks of 24 planes) this measured 1 %
+// (FP64) and 2.4 % (FP32) faster than 12 chunks of 16, and 3 % and 9 % faster
+// than the 28 planes that the first rule would take.  Below 128 planes, chunks
+// of up to 16 planes (the two re-read halo planes stay a small share).
+inline int march_chunk(int nz, int tiles, int slots) {
+    int best = nz;
+    long long cost = -1, nblk = 0;
+    for (int chunk = nz; chunk >= 1; --chunk) {
+        const long long blocks = (long long)tiles * ((nz + chunk - 1) / chunk);
+        const long long c = (blocks + slots - 1) / slots * (chunk + 2);
+        if (cost < 0 || c < cost) {
+            cost = c;
+            best = chunk;
+            nblk = blocks;
+        }
+    }
+    if (nblk <= 2LL * slots) return best;
     const int nch = nz >= 8 * 16 ? 8 * std::max(1, (nz + 8 * 12) / (8 * 24))  // multiple of 8 nearest nz / 24
                                  : (nz + 15) / 16;
     return std::max(1, (nz + nch - 1) / nch);
@@ -2185,8 +2203,8 @@ template <int MODE, int FOUT, class T>
 void march(Handle &h, const Fld3<T> &cur, const Fld3<T> *old, const Fld3<T> *f1, Fld3<T> *nxt, Fld3<T> *fo,
            double c0, double c1, double dt, double g2 = 0.0) {
     const Dims &d = h.d;
-    const int chunk = march_chunk(d);
-    const dim3 grid = march_grid<T>(d, chunk), block(256);
+    const int tiles = march_tiles<T>(d), chunk = march_chunk(d.nzg - 2, tiles, 3 * h.n_cu);
+    const dim3 grid(xcd_blocks(tiles * ((d.nzg - 2 + chunk - 1) / chunk))), block(256);
     const T *o[3] = {old ? old->u : nullptr, old ? old->v : nullptr, old ? old->w : nullptr};
     const T *f[3] = {f1 ? f1->u : nullptr, f1 ? f1->v : nullptr, f1 ? f1->w : nullptr};
     T *n[3] = {nxt ? nxt->u : nullptr, nxt ? nxt->v : nullptr, nxt ? nxt->w : nullptr};

@@ -130,3 +130,25 @@ def test_statistics_block_edges(shape):
     got = s.monitor()
     assert np.all(np.abs(got[:4] - [a.sum() for a in parts]) < 1e-13 * scale)
     np.testing.assert_array_equal(got[4:], [a.max() for a in parts])
+
+
+# the z chunk of the stage march changes with the grid: one plane per block,
+# two, a remainder, and (nz = 193 with one tile row) the many-plane rule
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(70, 9, 5), (131, 20, 13), (66, 25, 101), (300, 60, 40)])
+def test_rhs_march_chunks(shape, precision):
+    say("rhs march", shape, precision)
+    x, y, z, U, V, W = random_case(sum(shape), *shape)
+    if precision:
+        U, V, W = (np.asfortranarray(a.astype(np.float32).astype(np.float64)) for a in (U, V, W))
+    o = orc.Oracle(x, y, z, 1e-5)
+    o.set_fields(U, V, W)
+    ref = o.rhs()
+    s = solver(x, y, z, precision=precision)
+    s.set_fields(U, V, W)
+    # FP64: the reference's rounding order differs in the last digits (1e-12 as
+    # the parity tests); FP32 arithmetic: a few roundings of terms that cancel
+    # against each other by less than a factor of ten on random fields
+    tol = 1e-5 if precision else 1e-12
+    for a, b in zip(s.rhs(), ref):
+        assert np.linalg.norm(a - b) < tol * np.linalg.norm(b)
