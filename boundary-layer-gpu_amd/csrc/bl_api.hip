@@ -630,11 +630,11 @@ void build(Handle &h, const bl_config *c) {
     upload_vec(h.lu_du, dup, h.stream);
 
     h.scal = dmalloc(64);
+    h.bc_mem = dmalloc(bc_doubles(d));
     {
-        // reduction scratch: 3 partials per interior block, flux partials, Cf, monitor planes
+        // reduction scratch: 3 partials per interior block, Cf, monitor planes
         const size_t nb = (size_t)((d.nxg - 2 + 63) / 64) * ((d.nyg - 2 + 3) / 4) * (d.nzg - 2);
-        const size_t nq = (size_t)(((d.nyg + 255) / 256) + ((d.nxg + 255) / 256)) * d.nzg;
-        h.red = dmalloc(std::max({3 * nb, nq, (size_t)d.nxg, (size_t)monitor_partials(d), (size_t)1024}));
+        h.red = dmalloc(std::max({3 * nb, (size_t)d.nxg, (size_t)monitor_partials(d), (size_t)1024}));
     }
     BL_HIP(hipStreamSynchronize(h.stream));
 }
@@ -653,7 +653,7 @@ void free_all(Handle &h) {
     }
     for (void *p : {(void *)h.F1.u, (void *)h.F1.v, (void *)h.F1.w, (void *)h.P, (void *)h.phi,
                     (void *)h.nu_t, (void *)h.T1, (void *)h.S, (void *)h.dct_w1, (void *)h.dct_w2,
-                    (void *)h.dct_wN, (void *)h.dct_rot, (void *)h.dct_mf, h.mx2, (void *)h.zc, (void *)h.zs, (void *)h.zf, (void *)h.bc_extra, (void *)h.lund_mem, (void *)h.wm_mem, (void *)h.lu_dl, (void *)h.lu_dp, (void *)h.lu_du,
+                    (void *)h.dct_wN, (void *)h.dct_rot, (void *)h.dct_mf, h.mx2, (void *)h.zc, (void *)h.zs, (void *)h.zf, (void *)h.bc_extra, (void *)h.bc_mem, (void *)h.lund_mem, (void *)h.wm_mem, (void *)h.lu_dl, (void *)h.lu_dp, (void *)h.lu_du,
                     (void *)h.lu00, (void *)h.th_co,
                     (void *)h.scal, (void *)h.red, (void *)h.dsm, (void *)h.smag_c, h.mem_grid, h.mem_gridf, (void *)h.mx_tab, (void *)h.zmf,
                     (void *)h.p00, (void *)h.inc1, (void *)h.stats, (void *)h.cl_w, (void *)h.cl_b, (void *)h.cl_cnt})
@@ -664,23 +664,20 @@ void free_all(Handle &h) {
 }
 
 // one projection sub-step on the current buffer (projection.f90:21-87);
-// inc: the mixed path's first-stage source (see IncSrc)
-void projection_on(Handle &h, Field3 &f, int rk_step, double dt, const IncSrc *inc = nullptr) {
-    if (h.precision == BL_PREC_MIXED) {
-        Fld3<float> ff = as<float>(f);
-        float *phi = reinterpret_cast<float *>(h.phi);
-        launch_poisson_mixed(h, phi, ff, inc);
-        launch_project(h, ff, (const float *)phi, rk_step == 1 ? reinterpret_cast<float *>(h.P) : nullptr, dt);
-        return;
-    }
-    launch_poisson(h, h.phi, &f);
-    launch_project(h, f, (const double *)h.phi, rk_step == 1 ? h.P : nullptr, dt);
+// bc: the stage's boundary values (null: those in the field); inc: the mixed
+// path's first-stage source (see IncSrc)
+void projection_on(Handle &h, const Field3 &f, int rk_step, double dt, const BcPlanes<float> *bc, const IncSrc *inc) {
+    Fld3<float> ff = as<float>(f);
+    float *phi = reinterpret_cast<float *>(h.phi);
+    launch_poisson_mixed(h, phi, ff, bc, inc);
+    launch_project(h, ff, (const float *)phi, rk_step == 1 ? reinterpret_cast<float *>(h.P) : nullptr, dt);
 }
 
-template <class T>
-void bc_on(Handle &h, Field3 &f, const Field3 &old, int rk_step, double dt, double t) {
-    Fld3<T> ff = as<T>(f);
-    launch_bc(h, ff, as<T>(old), rk_step, dt, t);
+void projection_on(Handle &h, const Field3 &f, int rk_step, double dt, const BcPlanes<double> *bc,
+                   const IncSrc * = nullptr) {
+    Fld3<double> ff = f;
+    launch_poisson(h, h.phi, &f, bc);
+    launch_project(h, ff, (const double *)h.phi, rk_step == 1 ? h.P : nullptr, dt);
 }
 
 template <class T>
@@ -697,6 +694,18 @@ void do_step_t(Handle &h) {
     // Lund rescaling: the step's inflow plane from the step-start field
     if (h.bc.inflow_flag == 3 || h.bc.inflow_flag == 5) launch_lund<T>(h, old, dt);
     h.lund_pending = false;
+    double ts[3];
+    for (int s = 1; s <= nst; ++s) ts[s - 1] = to + (nst == 3 ? h.rk_t[s] : h.rk2_t[s]) * dt;
+    // FP32 fields that a previous step projected: the first stage's
+    // pressure comes from the divergence of the stage increment, not of
+    // U* (see IncSrc); fields set from outside may carry a divergence of
+    // their own, which the first stage projects as the reference does
+    const bool inc = sizeof(T) == 4 && h.inc_ok;
+    // boundary values of all stages, unless a stage changes what they depend
+    // on: the pseudo-Robin wall V takes the stage's slip lengths, and the
+    // outflow speed changes after the first boundary call under Falkner-Skan
+    const bool robin = wall_model_robin(h.bc.iwall), per_stage = robin || h.fs_uc_pending;
+    if (!per_stage) launch_bc_planes(h, old, 1, nst, dt, ts, inc ? h.inc1 : nullptr, to);
     for (int s = 1; s <= nst; ++s) {
         const int nxt = order3[s - 1];
         // eddy viscosity of the stage's input fields (time_integration.f90:341-346)
@@ -706,25 +715,22 @@ void do_step_t(Handle &h) {
         // the stage, and the pseudo-Robin V's wall mean
         if (h.wm_mem && (h.wm_model != 0 || (h.les != 0 && h.wm_istress == 1)))
             launch_wall_model<T>(h, as<T>(h.buf[cur]), old, false);
+        if (per_stage) launch_bc_planes(h, old, s, 1, dt, ts + s - 1, inc && s == 1 ? h.inc1 : nullptr, to);
         Fld3<T> next = as<T>(h.buf[nxt]);
         launch_rk_stage(h, as<T>(h.buf[cur]), old, next, s, dt);
-        const double ts = to + (nst == 3 ? h.rk_t[s] : h.rk2_t[s]) * dt;
-        // FP32 fields that a previous step projected: the first stage's
-        // pressure comes from the divergence of the stage increment, not of
-        // U* (see IncSrc); fields set from outside may carry a divergence of
-        // their own, which the first stage projects as the reference does
-        const bool inc = sizeof(T) == 4 && s == 1 && h.inc_ok;
-        launch_bc(h, next, old, s, dt, ts, inc ? h.inc1 : nullptr, to);
-        if (inc) {
-            const Fld3<float> f1 = as<float>(h.F1), vn = as<float>(h.buf[X]), vs = as<float>(h.buf[nxt]);
-            const IncSrc src{f1.u, f1.v, f1.w, vs.v, vn.v, h.inc1,
-                             dt * (nst == 3 ? h.rk_coef[1][1] : h.rk2_coef[1][1])};
-            projection_on(h, h.buf[nxt], s, dt, &src);
+        // the boundary conditions before the projection change only the faces
+        // that its divergence reads, and those it takes from the stage's values
+        const BcPlanes<T> bc = bc_planes<T>(h, s);
+        if (inc && s == 1) {
+            const Fld3<float> f1 = as<float>(h.F1), vn = as<float>(h.buf[X]);
+            const IncSrc src{f1.u, f1.v, f1.w, vn.v, h.inc1, dt * (nst == 3 ? h.rk_coef[1][1] : h.rk2_coef[1][1])};
+            projection_on(h, h.buf[nxt], s, dt, &bc, &src);
         } else {
-            projection_on(h, h.buf[nxt], s, dt);
+            projection_on(h, h.buf[nxt], s, dt, &bc, nullptr);
         }
-        launch_bc(h, next, old, s, dt, ts);
-        h.t = ts;
+        if (bc_called(h)) launch_bc_planes(h, old, s, 1, dt, ts + s - 1);
+        launch_bc(h, next, s);
+        h.t = ts[s - 1];
         cur = nxt;
     }
     h.icur = h.iold = cur;
@@ -1190,13 +1196,16 @@ int bl_apply_bc(bl_handle *hh, int rk_step, double dt) {
         }
         // the pseudo-Robin V's wall mean from the old fields and the current
         // slip lengths, as apply_pseudo_Robin_bc_y_bottom forms it at every call
-        if (h.precision == BL_PREC_MIXED) {
-            launch_wall_model<float>(h, as<float>(h.buf[h.icur]), as<float>(h.buf[h.iold]), true);
-            bc_on<float>(h, h.buf[h.icur], h.buf[h.iold], rk_step, dt, h.t);
-        } else {
-            launch_wall_model<double>(h, as<double>(h.buf[h.icur]), as<double>(h.buf[h.iold]), true);
-            bc_on<double>(h, h.buf[h.icur], h.buf[h.iold], rk_step, dt, h.t);
-        }
+        auto apply = [&](auto &&f, auto &&old) {
+            launch_wall_model(h, f, old, true);
+            launch_bc_planes(h, old, rk_step, 1, dt, &h.t);
+            launch_bc(h, f, rk_step);
+        };
+        if (h.precision == BL_PREC_MIXED)
+            apply(as<float>(h.buf[h.icur]), as<float>(h.buf[h.iold]));
+        else
+            apply(as<double>(h.buf[h.icur]), as<double>(h.buf[h.iold]));
+        bc_called(h);
         BL_HIP(hipStreamSynchronize(h.stream));
     });
 }
@@ -1236,7 +1245,10 @@ int bl_projection(bl_handle *hh, int rk_step, double dt) {
     return guarded([&] {
         Handle &h = H(hh);
         h.inc_ok = false;
-        projection_on(h, h.buf[h.icur], rk_step, dt);
+        if (h.precision == BL_PREC_MIXED)
+            projection_on(h, h.buf[h.icur], rk_step, dt, (const BcPlanes<float> *)nullptr, nullptr);
+        else
+            projection_on(h, h.buf[h.icur], rk_step, dt, (const BcPlanes<double> *)nullptr, nullptr);
         BL_HIP(hipStreamSynchronize(h.stream));
     });
 }

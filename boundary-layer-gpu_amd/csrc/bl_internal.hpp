@@ -133,6 +133,68 @@ inline Fld3<T> as(const Field3 &f) {
     return {reinterpret_cast<T *>(f.u), reinterpret_cast<T *>(f.v), reinterpret_cast<T *>(f.w)};
 }
 
+// A stage's boundary values, which depend on the step-start field, the time and
+// the tables only (boundary_conditions.f90:137-202, 246-260): the inflow and
+// outflow planes [k][j] (nyg rows; the outflow before the mass-flux shift) as
+// stored, V on the top row, V on the wall (row stride wld: 0 when the wall
+// value does not vary in z), and the shift of the outflow U.
+template <class T>
+struct BcPlanes {
+    T *uin, *vin, *win, *uo, *vo, *wo;
+    T *vtop, *vwall;
+    long long wld;
+    double *du;
+};
+
+// The divergence on the line of cells (i = n + 1, j = c1 + 1, k = c2 + 1).  With
+// bc.du set, the faces on the boundary come from the stage's boundary values
+// instead of from the field: the inflow and the shifted outflow U at the ends of
+// the line, the top and wall V of the first and last rows, and, for the W face
+// below plane 1, its periodic image of plane nz-2 (the pressure solve needs no
+// boundary update of the field before it).  Pointers and ends are fixed per line.
+template <class T>
+struct DivLine {
+    const T *u, *vt, *vb, *wt, *wb;
+    const double *rdx;
+    double ry, rz, ul, ur;
+    int last;  // index of the outflow cell, or -1: read the ends from the field
+    __device__ __forceinline__ DivLine(const Dims &d, const Metrics &m, const BcPlanes<T> &bc, const T *U, const T *V,
+                                       const T *W, int c1, int c2) {
+        const long long p = fidx(d, 1, c1 + 1, c2 + 1);
+        u = U + p;
+        vt = V + p;
+        vb = vt - d.sx;
+        wt = W + p;
+        wb = wt - d.sxy;
+        rdx = m.rdx + 1;
+        ry = m.rdy[c1 + 1];
+        rz = m.rdz[c2 + 1];
+        ul = ur = 0.0;
+        last = -1;
+        if (bc.du) {
+            const long long pl = c1 + 1 + (long long)d.nyg * (c2 + 1);
+            ul = (double)bc.uin[pl];
+            ur = (double)(T)((double)bc.uo[pl] + bc.du[0]);
+            last = d.N - 1;
+            if (c1 == d.NM - 1) vt = bc.vtop + 1;
+            if (c1 == 0) vb = bc.vwall + bc.wld * (c2 + 1) + 1;
+            if (c2 == 0) wb = wt + d.sxy * (d.nz - 3);
+        }
+    }
+    // the six face values and the metric of cell n, and their divergence: apart,
+    // so that the loads of several cells can be issued before the first use
+    struct Raw {
+        T u, l, vt, vb, wt, wb;
+        double rdx;
+    };
+    __device__ __forceinline__ Raw load(int n) const { return {u[n], u[n - 1], vt[n], vb[n], wt[n], wb[n], rdx[n]}; }
+    __device__ __forceinline__ double div(const Raw &a, int n) const {
+        const double r = n == last ? ur : (double)a.u, l = last >= 0 && n == 0 ? ul : (double)a.l;
+        return (r - l) * a.rdx + ((double)a.vt - (double)a.vb) * ry + ((double)a.wt - (double)a.wb) * rz;
+    }
+    __device__ __forceinline__ double at(int n) const { return div(load(n), n); }
+};
+
 // Kernel classes timed by the optional HIP-event profiler.
 enum KernelId {
     KID_RK_STAGE = 0,
@@ -169,6 +231,7 @@ struct Handle {
     double bc_uc;      // U_top(nx): outflow convection speed
     // the general dispatcher (bl_set_boundary)
     long long bc_step = 0;          // steps since the flags were set (inflow_flag 4 stream)
+    double *bc_mem = nullptr;       // three stages' BcPlanes, then their shifts and flux partials
     double *bc_extra = nullptr;     // device V(i, ny) blowing/suction (nxg) + Falkner-Skan U(i, nyg) (nx)
     bool fs_uc_pending = false;     // top_flag 3: U_top(nx) changes after the next BC call
     double fs_uc = 0.0;
@@ -275,14 +338,26 @@ template <class T>
 const MetricsT<T> &metrics(const Handle &h);
 template <class T>
 void launch_rk_stage(Handle &h, const Fld3<T> &cur, const Fld3<T> &old, Fld3<T> &nxt, int stage, double dt);
-// inc1 != null: also write the FP64 increments of the inflow and outflow U
-// planes over the step-start field (t_old its time) and the mass-flux shift
-// into inc1 (layout of Handle::inc1)
+// The boundary values of stages first .. first + nst - 1 (1-based RK steps) at
+// times t[0..nst), from the step-start field.  inc1 != null: also write the
+// FP64 increments of the inflow and outflow U planes over that field (t_old its
+// time) and the mass-flux shift of the first of them into inc1 (layout of
+// Handle::inc1).
+size_t bc_doubles(const Dims &d);
 template <class T>
-void launch_bc(Handle &h, Fld3<T> &f, const Fld3<T> &old, int rk_step, double dt, double t,
-               double *inc1 = nullptr, double t_old = 0.0);
+BcPlanes<T> bc_planes(const Handle &h, int stage);
+template <class T>
+void launch_bc_planes(Handle &h, const Fld3<T> &old, int first, int nst, double dt, const double *t,
+                      double *inc1 = nullptr, double t_old = 0.0);
+// every boundary and ghost entry of f from its interior and the stage's boundary values
+template <class T>
+void launch_bc(Handle &h, Fld3<T> &f, int stage);
+// Falkner-Skan top: the outflow speed changes after the first boundary call; true if it did
+bool bc_called(Handle &h);
 // div != null: the rhs is the divergence of *div (computed inside the x transform)
-void launch_poisson(Handle &h, double *phi_inout, const Field3 *div = nullptr);
+// bc != null: with the boundary faces of *div taken from the stage's boundary
+// values instead of from the field
+void launch_poisson(Handle &h, double *phi_inout, const Field3 *div = nullptr, const BcPlanes<double> *bc = nullptr);
 // u -= grad phi (project_velocity, projection.f90:355-386); with P set, also
 // P = phi / (dt a11) on every cell (projection.f90:75-85)
 template <class T>
@@ -391,11 +466,12 @@ void build_mixed(Handle &h);
 // projection would divide by dt a11 into the recorded pressure.
 struct IncSrc {
     const float *fu, *fv, *fw;     // F1 of the stage
-    const float *vs, *vn;          // V after the stage's boundary update, and at the step start
+    const float *vn;               // V at the step start
     const double *inc1;            // Handle::inc1
     double c0;                     // dt a11
 };
-void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const IncSrc *inc = nullptr);
+void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const BcPlanes<float> *bc = nullptr,
+                          const IncSrc *inc = nullptr);
 // eddy viscosity of f into h.nu_t (bl_dsm.hip): LES = 1 constant-coefficient
 // Smagorinsky, 2 and 4 dynamic Smagorinsky z-averaged, 3 per cell
 size_t dsm_doubles(const Handle &h);  // size of Handle::dsm

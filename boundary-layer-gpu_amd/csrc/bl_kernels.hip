@@ -383,11 +383,9 @@ __global__ __launch_bounds__(256) void k_rk_march(
 }
 
 // ------------------------------------------------------------------------
-// Boundary conditions, in the reference's order (boundary_conditions.f90:
-// 135-260).  Each kernel covers one phase over the planes it writes.
+// Boundary conditions (boundary_conditions.f90:135-260)
 // ------------------------------------------------------------------------
 
-// inflow (:137-190) and outflow (:193-202); one thread per (j,k)
 // deterministic block sum of 256 values; returns the sum in thread 0
 __device__ __forceinline__ double block_sum_256(double v, double *sh) {
     sh[threadIdx.x] = v;
@@ -456,207 +454,269 @@ __device__ __forceinline__ void inflow_values(const Dims &d, const Metrics &m, c
     v = (j < d.ny) ? b.V_inlet[j] + vt : 0.0;
 }
 
+// The boundary values depend on the step-start field, the time and the tables,
+// not on the stage's interior: one launch computes them for the stages of a
+// step (blockIdx.z), with the two parts of the mass flux.  The inflow
+// (boundary_conditions.f90:137-190) and the outflow (:193-202) are one thread per
+// (j, k), blockIdx.x < nb_in; the wall and top V one thread per (i, k).
+struct BcStages {
+    double coef[3], t[3];  // rk_t(stage) dt Uc, and the stage's time
+};
 template <class T>
-__global__ __launch_bounds__(256) void k_bc_inout(Dims d, Metrics m, BCTables b, T *U, T *V, T *W,
-                                                  const T *Uo, const T *Vo, const T *Wo, double coef,
-                                                  double t, double *qpart, double *inc1, double t_old) {
+__global__ __launch_bounds__(256) void k_bc_planes(Dims d, Metrics m, BCTables b, BcPlanes<T> p0, long long stride,
+                                                   const T *__restrict__ Uo, const T *__restrict__ Vo,
+                                                   const T *__restrict__ Wo, BcStages st, int nb_in,
+                                                   double *__restrict__ qpart, double *inc1, double t_old) {
     __shared__ double sh[256];
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    // mass flux through the x boundaries (boundary_conditions.f90:246-249):
-    // (U(1,j,k) - U(nx-1,j,k))*(y(j)-y(j-1)) for j in [1,nyg-2], k in [1,nzg-3]
+    const int k = blockIdx.y, z = blockIdx.z;
+    const long long o = z * stride;
     double q = 0.0;
-    if (j < d.nyg) {
-    const int nx = d.nx, nxg = d.nxg;
-    double ui, vi, wi;
-    const bool lund = b.inflow_flag == 3 || b.inflow_flag == 5;
-    if (lund) {
-        // the step's rescaled plane (:569-597); flag 5 adds it to the inlet
-        // means, with W's planes shifted by 16 (:512-559)
-        const bool f5 = b.inflow_flag == 5;
-        ui = (f5 ? b.U_inlet[j] : 0.0) + b.lund_u[j + (long long)d.nyg * k];
-        wi = 0.0;
-        if (k < d.nz) {
-            const int ks = f5 ? (k + 17) % d.nz : k;
-            wi = (f5 ? b.W_inlet[j] : 0.0) + b.lund_w[j + (long long)d.nyg * ks];
-        }
-        vi = (j < d.ny) ? (f5 ? b.V_inlet[j] : 0.0) + b.lund_v[j + (long long)d.ny * k] : 0.0;
-    } else {
-        inflow_values(d, m, b, j, k, t, b.istep, ui, vi, wi);
-    }
-    const long long p0 = fidx(d, 0, j, k);
-    // U (all j < nyg, k < nzg)
-    const double uin = (double)(T)ui;  // the value stored
-    const long long pl = j + (long long)d.nyg * k;
-    if (inc1) {
-        // FP64 increment of the inflow face over the step-start value: that
-        // value is taken unrounded when it is the stored boundary value of
-        // t_old (the previous step), as it is after any step
-        double uo = 0.0, vo, wo;
-        if (!lund) inflow_values(d, m, b, j, k, t_old, b.istep - 1, uo, vo, wo);
-        const double so = (double)Uo[p0];
-        // (the previous step's rescaled plane is gone: the stored value)
-        inc1[pl] = ui - (!lund && (double)(T)uo == so ? uo : so);
-    }
-    U[p0] = (T)uin;
-    {
-        const long long pa = fidx(d, nx - 2, j, k);
-        const double o1 = Uo[pa], o0 = Uo[pa - 1];
-        const double du = coef * (o1 - o0) / (m.x[nx - 2] - m.x[nx - 3]);
-        const double v = (double)(T)(o1 - du);
-        U[pa] = (T)v;
-        U[pa + 1] = (T)v;
-        // FP64 increment of the outflow face before the mass-flux shift
-        if (inc1) inc1[(long long)d.nyg * d.nzg + pl] = -du;
-        if (j >= 1 && j <= d.nyg - 2 && k >= 1 && k <= d.nzg - 3) q = (uin - v) * (m.y[j] - m.y[j - 1]);
-    }
-    if (k < d.nz) {
-        W[p0] = (T)wi;
-        const long long pa = fidx(d, nxg - 2, j, k);
-        const double o1 = Wo[pa], o0 = Wo[pa - 1];
-        const double v = o1 - coef * (o1 - o0) / (m.xg[nxg - 2] - m.xg[nxg - 3]);
-        W[pa] = (T)v;
-        W[pa + 1] = (T)v;
-    }
-    if (j < d.ny) {
-        V[p0] = (T)vi;
-        const long long pa = fidx(d, nxg - 2, j, k);
-        const double o1 = Vo[pa], o0 = Vo[pa - 1];
-        const double v = o1 - coef * (o1 - o0) / (m.xg[nxg - 2] - m.xg[nxg - 3]);
-        V[pa] = (T)v;
-        V[pa + 1] = (T)v;
-    }
-    }
-    q = block_sum_256(q, sh);
-    if (threadIdx.x == 0) qpart[blockIdx.x + gridDim.x * blockIdx.y] = q;
-}
-
-// periodic z (:205-217); one thread per (i,j)
-template <class T>
-__global__ __launch_bounds__(256) void k_bc_periodic(Dims d, T *U, T *V, T *W) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    if (i >= d.nxg) return;
-    const long long base = fidx(d, i, j, 0), sxy = d.sxy;
-    const int nzg = d.nzg, nz = d.nz;
-    if (i < d.nx) {
-        U[base] = U[base + sxy * (nzg - 3)];
-        U[base + sxy * (nzg - 2)] = U[base + sxy * 1];
-        U[base + sxy * (nzg - 1)] = U[base + sxy * 2];
-    }
-    if (j < d.ny) {
-        V[base] = V[base + sxy * (nzg - 3)];
-        V[base + sxy * (nzg - 2)] = V[base + sxy * 1];
-        V[base + sxy * (nzg - 1)] = V[base + sxy * 2];
-    }
-    W[base] = W[base + sxy * (nz - 2)];
-    W[base + sxy * (nz - 1)] = W[base + sxy * 1];
-}
-
-// top Dirichlet (:220-228) then wall (:231-238); one thread per (i,k)
-template <class T>
-__global__ __launch_bounds__(256) void k_bc_topwall(Dims d, Metrics m, BCTables b, T *U, T *V, T *W,
-                                                    const T *__restrict__ Vo, double *qpart) {
-    __shared__ double sh[256];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    // mass flux through the y boundaries (boundary_conditions.f90:251-253) from
-    // the values written here: (V(i,1,k) - V(i,ny,k))*(x(i)-x(i-1))
-    // V(i, ny) as stored at the top: V_top (top_flag 0), blowing/suction
-    // (1, 2: :648-673; columns below i_rescale keep it, because the
-    // reference's V_top copy of zero_wz_top, :279, writes V(i, nyg), one row
-    // past the top face, which the wall condition then overwrites), or 0
-    // (Falkner-Skan, :1001)
-    const int ii = min(i, d.nxg - 1);
-    const double vtop = b.top_flag == 0 ? (double)(T)b.V_top[ii]
-                                        : (b.top_flag == 3 ? 0.0 : (double)(T)b.vtop_bs[ii]);
-    // V(i, 1) as the wall condition below stores it: 0, or with a Robin wall
-    // model the pseudo-Robin alpha_y dVo/dy less its wall mean beta_y
-    // (apply_pseudo_Robin_bc_y_bottom :1152-1180, id 2)
-    const bool robin = b.iwall != 0 && b.iwall != 11 && b.iwall != 15;
-    double vwall = 0.0;
-    if (robin) {
-        const long long pw = fidx(d, ii, 0, k);
-        vwall = (double)(T)(b.wm_ay[ii] * ((double)Vo[pw + d.sx] - (double)Vo[pw]) / (m.y[1] - m.y[0]) - b.wm_beta[0]);
-    }
-    double q = 0.0;
-    if (i >= 1 && i <= d.nxg - 3 && k >= 1 && k <= d.nzg - 3) q = (vwall - vtop) * (m.x[i] - m.x[i - 1]);
-    q = block_sum_256(q, sh);
-    if (threadIdx.x == 0) qpart[blockIdx.x + gridDim.x * blockIdx.y] = q;
-    if (i >= d.nxg) return;
-    const long long sx = d.sx;
-    const long long p0 = fidx(d, i, 0, k);
-    const long long ut_ = p0 + sx * (d.nyg - 1), vt_ = p0 + sx * (d.ny - 1), wt_ = p0 + sx * (d.nyg - 1);
-    if (b.top_flag == 0) {
-        // Dirichlet (:220-228, :947-964)
-        if (i < d.nx) U[ut_] = (T)b.U_top[i];
-        V[vt_] = (T)b.V_top[i];
-        if (k < d.nz) W[wt_] = (T)b.W_top[i];
-    } else if (b.top_flag == 3) {
-        // Falkner-Skan (:979-1007)
-        if (i < d.nx) U[ut_] = (T)b.utop_fs[i];
-        V[vt_] = (T)0;
-        if (k < d.nz) W[wt_] = W[wt_ - sx];
-    } else {
-        // blowing/suction, then zero_wz_top (:264-283)
-        V[vt_] = (T)b.vtop_bs[i];
-        if (i < d.nx) {
-            const double vp = (double)(T)b.vtop_bs[i + 1], vm = (double)(T)b.vtop_bs[i];
-            U[ut_] = (T)(b.dy_dx * (vp - vm) + (double)U[ut_ - sx]);
-        }
-        if (k < d.nz) W[wt_] = W[wt_ - sx];
-        if (i < b.i_rescale) {
-            if (i < d.nx) U[ut_] = (T)b.U_top[i];
-            if (k < d.nz) W[wt_] = (T)b.W_top[i];
-        }
-    }
-    // walls: no-slip (:231-238), or the wall model's conditions (:73-108):
-    // Neumann U (iwall_model 11, 15: apply_Nozero_Neumann_bc_y :359-372)
-    // with V = W = 0, else Robin U, W (apply_Robin_bc_y_bottom :1107-1132,
-    // id 2) and the pseudo-Robin V
-    if (b.iwall == 0) {
-        if (i < d.nx) U[p0] = -U[p0 + sx];
-        V[p0] = (T)0;
-        if (k < d.nz) W[p0] = -W[p0 + sx];
-    } else {
-        const double dyg = m.yg[1] - m.yg[0];
-        if (!robin) {
-            if (i < d.nx) U[p0] = (T)((double)U[p0 + sx] - b.wm_ax[i] * dyg);
-            V[p0] = (T)0;
-            if (k < d.nz) W[p0] = -W[p0 + sx];
-        } else {
-            if (i < d.nx) {
-                const double r = 2.0 * b.wm_ax[i] / dyg;
-                U[p0] = (T)((r - 1.0) * (double)U[p0 + sx] / (r + 1.0));
+    if ((int)blockIdx.x < nb_in) {
+        // mass flux through the x boundaries (:246-249):
+        // (U(1,j,k) - U(nx-1,j,k))*(y(j)-y(j-1)) for j in [1,nyg-2], k in [1,nzg-3]
+        const int j = blockIdx.x * 256 + threadIdx.x;
+        if (j < d.nyg) {
+            const int nx = d.nx, nxg = d.nxg;
+            const double coef = st.coef[z], t = st.t[z];
+            double ui, vi, wi;
+            const bool lund = b.inflow_flag == 3 || b.inflow_flag == 5;
+            if (lund) {
+                // the step's rescaled plane (:569-597); flag 5 adds it to the inlet
+                // means, with W's planes shifted by 16 (:512-559)
+                const bool f5 = b.inflow_flag == 5;
+                ui = (f5 ? b.U_inlet[j] : 0.0) + b.lund_u[j + (long long)d.nyg * k];
+                wi = 0.0;
+                if (k < d.nz) {
+                    const int ks = f5 ? (k + 17) % d.nz : k;
+                    wi = (f5 ? b.W_inlet[j] : 0.0) + b.lund_w[j + (long long)d.nyg * ks];
+                }
+                vi = (j < d.ny) ? (f5 ? b.V_inlet[j] : 0.0) + b.lund_v[j + (long long)d.ny * k] : 0.0;
+            } else {
+                inflow_values(d, m, b, j, k, t, b.istep, ui, vi, wi);
             }
-            V[p0] = (T)vwall;
+            const double uin = (double)(T)ui;  // the value stored
+            const long long pl = j + (long long)d.nyg * k;
+            if (inc1 && z == 0) {
+                // FP64 increment of the inflow face over the step-start value: that
+                // value is taken unrounded when it is the stored boundary value of
+                // t_old (the previous step), as it is after any step
+                double uo = 0.0, vo, wo;
+                if (!lund) inflow_values(d, m, b, j, k, t_old, b.istep - 1, uo, vo, wo);
+                const double so = (double)Uo[fidx(d, 0, j, k)];
+                // (the previous step's rescaled plane is gone: the stored value)
+                inc1[pl] = ui - (!lund && (double)(T)uo == so ? uo : so);
+            }
+            p0.uin[o + pl] = (T)uin;
+            {
+                const long long pa = fidx(d, nx - 2, j, k);
+                const double o1 = Uo[pa], o0 = Uo[pa - 1];
+                const double du = coef * (o1 - o0) / (m.x[nx - 2] - m.x[nx - 3]);
+                const double v = (double)(T)(o1 - du);
+                p0.uo[o + pl] = (T)v;
+                // FP64 increment of the outflow face before the mass-flux shift
+                if (inc1 && z == 0) inc1[(long long)d.nyg * d.nzg + pl] = -du;
+                if (j >= 1 && j <= d.nyg - 2 && k >= 1 && k <= d.nzg - 3) q = (uin - v) * (m.y[j] - m.y[j - 1]);
+            }
+            const long long pa = fidx(d, nxg - 2, j, k);
+            const double dxo = m.xg[nxg - 2] - m.xg[nxg - 3];
             if (k < d.nz) {
-                const double r = 2.0 * b.wm_az[i] / dyg;
-                W[p0] = (T)((r - 1.0) * (double)W[p0 + sx] / (r + 1.0));
+                const double o1 = Wo[pa], o0 = Wo[pa - 1];
+                p0.win[o + pl] = (T)wi;
+                p0.wo[o + pl] = (T)(o1 - coef * (o1 - o0) / dxo);
+            }
+            if (j < d.ny) {
+                const double o1 = Vo[pa], o0 = Vo[pa - 1];
+                p0.vin[o + pl] = (T)vi;
+                p0.vo[o + pl] = (T)(o1 - coef * (o1 - o0) / dxo);
             }
         }
+    } else {
+        // mass flux through the y boundaries (:251-253):
+        // (V(i,1,k) - V(i,ny,k))*(x(i)-x(i-1))
+        const int i = (blockIdx.x - nb_in) * 256 + threadIdx.x;
+        if (i < d.nxg) {
+            // V(i, ny) as stored at the top: V_top (top_flag 0), blowing/suction
+            // (1, 2: :648-673; columns below i_rescale keep it, because the
+            // reference's V_top copy of zero_wz_top, :279, writes V(i, nyg), one row
+            // past the top face, which the wall condition then overwrites), or 0
+            // (Falkner-Skan, :1001)
+            const double vtop = b.top_flag == 0 ? (double)(T)b.V_top[i]
+                                                : (b.top_flag == 3 ? 0.0 : (double)(T)b.vtop_bs[i]);
+            // V(i, 1) as the wall condition stores it: 0, or with a Robin wall
+            // model the pseudo-Robin alpha_y dVo/dy less its wall mean beta_y
+            // (apply_pseudo_Robin_bc_y_bottom :1152-1180, id 2)
+            double vwall = 0.0;
+            if (p0.wld) {
+                const long long pw = fidx(d, i, 0, k);
+                vwall = (double)(T)(b.wm_ay[i] * ((double)Vo[pw + d.sx] - (double)Vo[pw]) / (m.y[1] - m.y[0]) -
+                                    b.wm_beta[0]);
+            }
+            if (k == 0) p0.vtop[o + i] = (T)vtop;
+            if (p0.wld || k == 0) p0.vwall[o + p0.wld * k + i] = (T)vwall;
+            if (i >= 1 && i <= d.nxg - 3 && k >= 1 && k <= d.nzg - 3) q = (vwall - vtop) * (m.x[i] - m.x[i - 1]);
+        }
+    }
+    q = block_sum_256(q, sh);
+    if (threadIdx.x == 0) {
+        // the x parts first, then the y parts
+        const long long nq_in = (long long)nb_in * gridDim.y;
+        const long long e = (int)blockIdx.x < nb_in
+                                ? blockIdx.x + (long long)nb_in * k
+                                : nq_in + (blockIdx.x - nb_in) + (long long)(gridDim.x - nb_in) * k;
+        qpart[e + (long long)gridDim.x * gridDim.y * z] = q;
     }
 }
 
-// global mass conservation (:241-260): every block re-sums the flux partials
-// in the same order (so all agree bit for bit) and corrects its part of the
-// outflow planes.  One thread per (j,k).
-template <class T>
-__global__ __launch_bounds__(256) void k_bc_massflux(Dims d, double length_y, const double *qpart,
-                                                     int nq, T *U, double *du_out) {
+// global mass conservation (:241-260): the shift of the outflow U of stage
+// blockIdx.x from its nq flux partials
+__global__ __launch_bounds__(256) void k_bc_shift(Dims d, double length_y, const double *__restrict__ qpart, int nq,
+                                                  double *__restrict__ du, double *inc_du) {
     __shared__ double sh[256];
     double acc = 0.0;
-    for (int t = threadIdx.x; t < nq; t += 256) acc += qpart[t];
+    for (int t = threadIdx.x; t < nq; t += 256) acc += qpart[(long long)nq * blockIdx.x + t];
     const double Q = block_sum_256(acc, sh);
-    const double du = Q / length_y / (double)(d.nzg - 3);
-    if (du_out && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) du_out[0] = du;
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (j >= d.nyg) return;
-    const long long pa = fidx(d, d.nx - 2, j, k);
-    const double v = (double)U[pa] + du;
-    U[pa] = (T)v;
-    U[pa + 1] = (T)v;
+    if (threadIdx.x == 0) {
+        const double v = Q / length_y / (double)(d.nzg - 3);
+        du[blockIdx.x] = v;
+        if (inc_du && blockIdx.x == 0) inc_du[0] = v;
+    }
+}
+
+// Every boundary and ghost entry, in one launch: the reference applies inflow and
+// outflow, the periodic planes (:205-217), the top (:220-228, 947-1007), the
+// wall (:231-238, 73-108) and the mass-flux shift one after the other; here
+// each entry is computed from what those leave of the interior entries and
+// the stage's boundary values it derives from, and no entry that another
+// thread reads is written.  Three ranges of one thread index: the ghost z
+// planes (entries (i, j) of three planes), the wall and top rows of planes
+// 1..nzg-3 (entries (i, k)), and the x faces of those planes (entries (j, k)).
+// Eight dependent launches per stage (this, and the same before the pressure
+// solve, which now takes the boundary values directly) were the larger part of
+// the time on small grids: a step of 192x32x8 took 45 launches of 4 to 10 us.
+template <class T>
+struct BcField {
+    Dims d;
+    const Metrics &m;
+    const BCTables &b;
+    const BcPlanes<T> &p;
+    const T *U, *V, *W;
+    double dyg;
+    bool robin;
+
+    __device__ int zc(int k) const { return k == 0 ? d.nzg - 3 : (k == d.nzg - 2 ? 1 : (k == d.nzg - 1 ? 2 : k)); }
+    __device__ int zf(int k) const { return k == 0 ? d.nz - 2 : (k == d.nz - 1 ? 1 : k); }
+    // interior rows and planes, any i, before the shift
+    __device__ T ubase(int i, int j, int k) const {
+        const long long pl = j + (long long)d.nyg * k;
+        return i == 0 ? p.uin[pl] : (i >= d.nx - 2 ? p.uo[pl] : U[fidx(d, i, j, k)]);
+    }
+    __device__ T wbase(int i, int j, int k) const {
+        const long long pl = j + (long long)d.nyg * k;
+        return i == 0 ? p.win[pl] : (i >= d.nxg - 2 ? p.wo[pl] : W[fidx(d, i, j, k)]);
+    }
+    __device__ T u(int i, int j, int k) const {
+        const int kc = zc(k), ib = min(i, d.nx - 2);
+        T v;
+        if (j == 0) {
+            const T x = ubase(ib, 1, kc);
+            if (b.iwall == 0) {
+                v = -x;  // no-slip
+            } else if (!robin) {
+                // Neumann (iwall_model 11, 15: apply_Nozero_Neumann_bc_y :359-372)
+                v = (T)((double)x - b.wm_ax[ib] * dyg);
+            } else {
+                // Robin (apply_Robin_bc_y_bottom :1107-1132, id 2)
+                const double r = 2.0 * b.wm_ax[ib] / dyg;
+                v = (T)((r - 1.0) * (double)x / (r + 1.0));
+            }
+        } else if (j == d.nyg - 1) {
+            if (b.top_flag == 0 || (b.top_flag != 3 && ib < b.i_rescale)) {
+                v = (T)b.U_top[ib];
+            } else if (b.top_flag == 3) {
+                v = (T)b.utop_fs[ib];
+            } else {
+                // zero spanwise vorticity under blowing/suction (zero_wz_top :264-283)
+                const double vp = (double)(T)b.vtop_bs[ib + 1], vm = (double)(T)b.vtop_bs[ib];
+                v = (T)(b.dy_dx * (vp - vm) + (double)ubase(ib, j - 1, kc));
+            }
+        } else {
+            v = ubase(ib, j, kc);
+        }
+        return i >= d.nx - 2 ? (T)((double)v + p.du[0]) : v;
+    }
+    __device__ T v(int i, int j, int k) const {
+        if (j == 0) return p.vwall[p.wld * k + i];
+        if (j == d.ny - 1) return p.vtop[i];
+        const int kc = zc(k);
+        const long long pl = j + (long long)d.nyg * kc;
+        return i == 0 ? p.vin[pl] : (i >= d.nxg - 2 ? p.vo[pl] : V[fidx(d, i, j, kc)]);
+    }
+    __device__ T w(int i, int j, int k) const {
+        const int kc = zf(k);
+        if (j == 0) {
+            const T x = wbase(i, 1, kc);
+            if (!robin) return -x;
+            const double r = 2.0 * b.wm_az[i] / dyg;
+            return (T)((r - 1.0) * (double)x / (r + 1.0));
+        }
+        if (j == d.nyg - 1) {
+            if (b.top_flag == 0 || (b.top_flag != 3 && i < b.i_rescale)) return (T)b.W_top[i];
+            return wbase(i, j - 1, kc);
+        }
+        return wbase(i, j, kc);
+    }
+};
+
+template <class T>
+__global__ __launch_bounds__(256) void k_bc_apply(Dims d, Metrics m, BCTables b, BcPlanes<T> p, T *U, T *V, T *W) {
+    const long long nA = 3LL * d.nxg * d.nyg, nB = (long long)d.nxg * (d.nzg - 3), nC = (long long)(d.nyg - 2) * (d.nzg - 3);
+    long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    const BcField<T> f{d, m, b, p, U, V, W, m.yg[1] - m.yg[0], p.wld != 0};
+    if (e < nA) {
+        const int r = (int)(e % (3 * d.nxg)), j = (int)(e / (3 * d.nxg));
+        const int q = r / d.nxg, i = r - q * d.nxg;
+        const int k = q == 0 ? 0 : d.nzg - 3 + q;  // U, V: planes 0, nzg-2, nzg-1; W: 0 and nz-1 = nzg-2
+        const long long o = fidx(d, i, j, k);
+        if (i < d.nx) U[o] = f.u(i, j, k);
+        if (j < d.ny) V[o] = f.v(i, j, k);
+        if (k < d.nz) W[o] = f.w(i, j, k);
+        return;
+    }
+    e -= nA;
+    if (e < nB) {
+        const int k = 1 + (int)(e / d.nxg), i = (int)(e % d.nxg);
+        const long long o = fidx(d, i, 0, k), top = (long long)d.sx * (d.nyg - 1);
+        if (i < d.nx) {
+            const T lo = f.u(i, 0, k), hi = f.u(i, d.nyg - 1, k);
+            U[o] = lo;
+            U[o + top] = hi;
+        }
+        V[o] = f.v(i, 0, k);
+        V[o + top - d.sx] = f.v(i, d.ny - 1, k);
+        const T lo = f.w(i, 0, k), hi = f.w(i, d.nyg - 1, k);
+        W[o] = lo;
+        W[o + top] = hi;
+        return;
+    }
+    e -= nB;
+    if (e < nC) {
+        const int k = 1 + (int)(e / (d.nyg - 2)), j = 1 + (int)(e % (d.nyg - 2));
+        const long long o = fidx(d, 0, j, k), pl = j + (long long)d.nyg * k;
+        U[o] = p.uin[pl];
+        const T u = (T)((double)p.uo[pl] + p.du[0]);
+        U[o + d.nx - 2] = u;
+        U[o + d.nx - 1] = u;
+        if (j < d.ny - 1) {
+            V[o] = p.vin[pl];
+            const T v = p.vo[pl];
+            V[o + d.nxg - 2] = v;
+            V[o + d.nxg - 1] = v;
+        }
+        W[o] = p.win[pl];
+        const T w = p.wo[pl];
+        W[o + d.nxg - 2] = w;
+        W[o + d.nxg - 1] = w;
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -928,9 +988,10 @@ __device__ __forceinline__ double2 cmulc(double2 a, double2 b) {  // a * conj(b)
 
 // DIV: the line is the pseudo-pressure rhs (projection.f90:38-47) evaluated
 // on the fly from U, V, W (in = U, in2 = V, in3 = W, lines over cells
-// i = 1..N, j = 1..NM, k = 1..M) instead of being read from memory.
+// i = 1..N, j = 1..NM, k = 1..M) instead of being read from memory; with
+// bc.du set the boundary faces come from the stage's boundary values (DivLine).
 template <int LB, bool DIV>
-__global__ __launch_bounds__(256) void k_dct_fwd(DctArgs a, Dims d, Metrics mt,
+__global__ __launch_bounds__(256) void k_dct_fwd(DctArgs a, Dims d, Metrics mt, BcPlanes<double> bc,
                                                  const double *__restrict__ in,
                                                  const double *__restrict__ in2,
                                                  const double *__restrict__ in3,
@@ -953,8 +1014,7 @@ __global__ __launch_bounds__(256) void k_dct_fwd(DctArgs a, Dims d, Metrics mt,
         const long long p = a.in_base + c1 * a.in_c1 + c2 * a.in_c2 + n;
         double f;
         if (DIV) {
-            f = (in[p] - in[p - 1]) * mt.rdx[n + 1] + (in2[p] - in2[p - d.sx]) * mt.rdy[c1 + 1] +
-                (in3[p] - in3[p - d.sxy]) * mt.rdz[c2 + 1];
+            f = DivLine<double>(d, mt, bc, in, in2, in3, c1, c2).at(n);
         } else {
             f = in[p];
         }
@@ -1227,7 +1287,7 @@ __global__ __launch_bounds__(64 * kZmW) void k_zdft_mf(int M, int C, long long p
 }
 
 template <bool DIV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_dct_fwd_m(DctArgs a, Dims d, Metrics mt, const double *__restrict__ in,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_dct_fwd_m(DctArgs a, Dims d, Metrics mt, BcPlanes<double> bc, const double *__restrict__ in,
                                                    const double *__restrict__ in2, const double *__restrict__ in3,
                                                    double *__restrict__ out) {
     extern __shared__ double smem[];
@@ -1242,37 +1302,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     const int line0 = blockIdx.x * kMfL;
     // load and reorder: v[n/2] = f[n] (n even), v[N-1-(n-1)/2] = f[n] (n odd);
     // kLd elements per thread are loaded before the first one is used
-    static_assert(kMfL == 2, "line index below assumes two lines per block");
-    long long lb[kMfL];
-    double ry[kMfL], rz[kMfL];
 #pragma unroll
     for (int l = 0; l < kMfL; ++l) {
         const int c = min(line0 + l, a.C - 1);
         const int c1 = c % a.C1, c2 = c / a.C1;
-        lb[l] = a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
-        ry[l] = DIV ? mt.rdy[c1 + 1] : 0.0;
-        rz[l] = DIV ? mt.rdz[c2 + 1] : 0.0;
-    }
-    for (int i0 = tid; i0 < kMfL * N; i0 += 256 * kLd) {
-        double f[kLd];
+        const double *src = in + a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
+        const DivLine<double> dl(d, mt, bc, in, in2, in3, c1, c2);
+        for (int n0 = tid; n0 < N; n0 += 256 * kLd) {
+            typename DivLine<double>::Raw r[DIV ? kLd : 1];
+            double f[DIV ? 1 : kLd];
 #pragma unroll
-        for (int u = 0; u < kLd; ++u) {
-            const int idx = min(i0 + 256 * u, kMfL * N - 1);
-            const int l = idx >= N ? 1 : 0, n = idx - l * N;
-            const long long p = lb[l] + n;
-            if (DIV) {
-                f[u] = (in[p] - in[p - 1]) * mt.rdx[n + 1] + (in2[p] - in2[p - d.sx]) * ry[l] +
-                       (in3[p] - in3[p - d.sxy]) * rz[l];
-            } else {
-                f[u] = in[p];
+            for (int u = 0; u < kLd; ++u) {
+                const int n = min(n0 + 256 * u, N - 1);
+                if constexpr (DIV)
+                    r[u] = dl.load(n);
+                else
+                    f[u] = src[n];
             }
-        }
 #pragma unroll
-        for (int u = 0; u < kLd; ++u) {
-            const int idx = i0 + 256 * u;
-            if (idx < kMfL * N) {
-                const int l = idx >= N ? 1 : 0, n = idx - l * N;
-                v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = f[u];
+            for (int u = 0; u < kLd; ++u) {
+                const int n = n0 + 256 * u;
+                double x;
+                if constexpr (DIV)
+                    x = dl.div(r[u], n);
+                else
+                    x = f[u];
+                if (n < N) v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = x;
             }
         }
     }
@@ -2089,8 +2144,9 @@ void zdft_launch(Handle &h, int kid, bool forward, const double *in, double *out
 }
 
 void dct_launch(Handle &h, int kid, const DctArgs &a, bool forward, const double *in, double *out,
-                const Field3 *div = nullptr) {
+                const Field3 *div = nullptr, const BcPlanes<double> *bcp = nullptr) {
     ProfScope ps(h, kid);
+    const BcPlanes<double> bc = bcp ? *bcp : BcPlanes<double>{};
     const int K1 = a.K1h + 1;
     if (a.fA) {
         // matrix-core kernels (the shape was checked with the tables)
@@ -2103,10 +2159,10 @@ void dct_launch(Handle &h, int kid, const DctArgs &a, bool forward, const double
         }
         const dim3 grid((a.C + kMfL - 1) / kMfL);
         if (forward && div)
-            hipLaunchKernelGGL(k_dct_fwd_m<true>, grid, dim3(256), lds, h.stream, a, h.d, h.m, div->u, div->v,
+            hipLaunchKernelGGL(k_dct_fwd_m<true>, grid, dim3(256), lds, h.stream, a, h.d, h.m, bc, div->u, div->v,
                                div->w, out);
         else if (forward)
-            hipLaunchKernelGGL(k_dct_fwd_m<false>, grid, dim3(256), lds, h.stream, a, h.d, h.m, in, nullptr,
+            hipLaunchKernelGGL(k_dct_fwd_m<false>, grid, dim3(256), lds, h.stream, a, h.d, h.m, bc, in, nullptr,
                                nullptr, out);
         else
             hipLaunchKernelGGL(k_dct_inv_m, grid, dim3(256), lds, h.stream, a, in, out);
@@ -2122,9 +2178,9 @@ void dct_launch(Handle &h, int kid, const DctArgs &a, bool forward, const double
     const dim3 grid((a.C + kDctLines - 1) / kDctLines);
     if (forward && div)
         hipLaunchKernelGGL((k_dct_fwd<kDctLines, true>), grid, dim3(256), lds, h.stream, a, h.d, h.m,
-                           div->u, div->v, div->w, out);
+                           bc, div->u, div->v, div->w, out);
     else if (forward)
-        hipLaunchKernelGGL((k_dct_fwd<kDctLines, false>), grid, dim3(256), lds, h.stream, a, h.d, h.m, in,
+        hipLaunchKernelGGL((k_dct_fwd<kDctLines, false>), grid, dim3(256), lds, h.stream, a, h.d, h.m, bc, in,
                            nullptr, nullptr, out);
     else
         hipLaunchKernelGGL(k_dct_inv<kDctLines>, grid, dim3(256), lds, h.stream, a, in, out);
@@ -2261,43 +2317,75 @@ void launch_rhs_only(Handle &h, const Fld3<T> &cur, Fld3<T> &rhs) {
                 0.0);
 }
 
+namespace {
+// elements of one stage's BcPlanes
+long long bc_stride(const Dims &d) {
+    return ((6LL * d.nyg + d.nxg) * d.nzg + d.nxg + 31) / 32 * 32;
+}
+int bc_partials(const Dims &d) { return ((d.nyg + 255) / 256 + (d.nxg + 255) / 256) * d.nzg; }
+}  // namespace
+
+size_t bc_doubles(const Dims &d) { return 3 * ((size_t)bc_stride(d) + bc_partials(d)) + 8; }
+
 template <class T>
-void launch_bc(Handle &h, Fld3<T> &f, const Fld3<T> &old, int rk_step, double dt, double t, double *inc1,
-               double t_old) {
+BcPlanes<T> bc_planes(const Handle &h, int stage) {
     const Dims &d = h.d;
-    const double coef = h.rk_t[rk_step] * dt * h.bc_uc;
-    prof_begin(h, KID_BC_INOUT);
-    const dim3 g_in((d.nyg + 255) / 256, d.nzg), g_tw((d.nxg + 255) / 256, d.nzg);
-    const int nq_in = g_in.x * g_in.y, nq_tw = g_tw.x * g_tw.y;
-    double *qpart = h.red;
-    hipLaunchKernelGGL(k_bc_inout<T>, g_in, dim3(256), 0, h.stream, d, h.m, h.bc, f.u, f.v, f.w, old.u, old.v,
-                       old.w, coef, t, qpart, inc1, t_old);
-    check_launch();
-    prof_end(h, KID_BC_INOUT);
-    prof_begin(h, KID_BC_PERIODIC);
-    hipLaunchKernelGGL(k_bc_periodic<T>, dim3((d.nxg + 255) / 256, d.nyg), dim3(256), 0, h.stream, d, f.u, f.v,
-                       f.w);
-    check_launch();
-    prof_end(h, KID_BC_PERIODIC);
-    prof_begin(h, KID_BC_TOPWALL);
-    hipLaunchKernelGGL(k_bc_topwall<T>, g_tw, dim3(256), 0, h.stream, d, h.m, h.bc, f.u, f.v, f.w, old.v,
-                       qpart + nq_in);
-    check_launch();
-    prof_end(h, KID_BC_TOPWALL);
-    prof_begin(h, KID_BC_MASSFLUX);
-    hipLaunchKernelGGL(k_bc_massflux<T>, g_in, dim3(256), 0, h.stream, d, h.length_y, qpart, nq_in + nq_tw, f.u,
-                       inc1 ? inc1 + 2 * (long long)d.nyg * d.nzg : nullptr);
-    check_launch();
-    prof_end(h, KID_BC_MASSFLUX);
-    // Falkner-Skan top: U_top is the Falkner-Skan profile from the first call
-    // on, and with it the outflow's convective velocity U_top(nx)
-    if (h.fs_uc_pending) {
-        h.bc_uc = h.fs_uc;
-        h.fs_uc_pending = false;
-    }
+    const long long npl = (long long)d.nyg * d.nzg;
+    T *p = reinterpret_cast<T *>(h.bc_mem) + (stage - 1) * bc_stride(d);
+    BcPlanes<T> b;
+    T **f[6] = {&b.uin, &b.vin, &b.win, &b.uo, &b.vo, &b.wo};
+    for (int q = 0; q < 6; ++q) *f[q] = p + q * npl;
+    b.vtop = p + 6 * npl;
+    b.vwall = b.vtop + d.nxg;
+    b.wld = wall_model_robin(h.bc.iwall) ? d.nxg : 0;
+    b.du = h.bc_mem + 3 * bc_stride(d) + (stage - 1);
+    return b;
 }
 
-void launch_poisson(Handle &h, double *phi, const Field3 *div) {
+template <class T>
+void launch_bc_planes(Handle &h, const Fld3<T> &old, int first, int nst, double dt, const double *t, double *inc1,
+                      double t_old) {
+    const Dims &d = h.d;
+    BcStages st{};
+    for (int s = 0; s < nst; ++s) {
+        st.coef[s] = h.rk_t[first + s] * dt * h.bc_uc;
+        st.t[s] = t[s];
+    }
+    const BcPlanes<T> p = bc_planes<T>(h, first);
+    const int nb_in = (d.nyg + 255) / 256, nb = nb_in + (d.nxg + 255) / 256, nq = bc_partials(d);
+    double *qpart = h.bc_mem + 3 * bc_stride(d) + 8;
+    {
+        ProfScope ps(h, KID_BC_INOUT);
+        hipLaunchKernelGGL(k_bc_planes<T>, dim3(nb, d.nzg, nst), dim3(256), 0, h.stream, d, h.m, h.bc, p, bc_stride(d),
+                           old.u, old.v, old.w, st, nb_in, qpart, inc1, t_old);
+        check_launch();
+    }
+    ProfScope ps(h, KID_BC_MASSFLUX);
+    hipLaunchKernelGGL(k_bc_shift, dim3(nst), dim3(256), 0, h.stream, d, h.length_y, qpart, nq, p.du,
+                       inc1 ? inc1 + 2 * (long long)d.nyg * d.nzg : nullptr);
+    check_launch();
+}
+
+template <class T>
+void launch_bc(Handle &h, Fld3<T> &f, int stage) {
+    const Dims &d = h.d;
+    ProfScope ps(h, KID_BC_TOPWALL);
+    const long long n = 3LL * d.nxg * d.nyg + (long long)d.nxg * (d.nzg - 3) + (long long)(d.nyg - 2) * (d.nzg - 3);
+    hipLaunchKernelGGL(k_bc_apply<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h.stream, d, h.m, h.bc,
+                       bc_planes<T>(h, stage), f.u, f.v, f.w);
+    check_launch();
+}
+
+bool bc_called(Handle &h) {
+    // U_top is the Falkner-Skan profile from the first call on, and with it
+    // the outflow's convective velocity U_top(nx)
+    if (!h.fs_uc_pending) return false;
+    h.bc_uc = h.fs_uc;
+    h.fs_uc_pending = false;
+    return true;
+}
+
+void launch_poisson(Handle &h, double *phi, const Field3 *div, const BcPlanes<double> *bc) {
     const Dims &d = h.d;
     const int N = d.N, M = d.M, NM = d.NM;
     const long long plane = (long long)N * NM;
@@ -2326,7 +2414,7 @@ void launch_poisson(Handle &h, double *phi, const Field3 *div) {
     da.out_c1 = N;
     da.out_c2 = plane;
     da.scale = 1.0;
-    dct_launch(h, KID_XFORM_X_FWD, da, true, phi, h.T1, div);
+    dct_launch(h, KID_XFORM_X_FWD, da, true, phi, h.T1, div, bc);
     // forward z: columns (kx, j) of T1 -> S[q][j][kx]
     zdft_launch(h, KID_XFORM_Z_FWD, true, h.T1, h.S);
     {
@@ -2494,7 +2582,10 @@ long long monitor_partials(const Dims &d) { return 8LL * ((d.nyg - 2 + kMonJ - 1
 #define BL_INSTANTIATE(T)                                                                                   \
     template void launch_rk_stage<T>(Handle &, const Fld3<T> &, const Fld3<T> &, Fld3<T> &, int, double); \
     template void launch_rhs_only<T>(Handle &, const Fld3<T> &, Fld3<T> &);                                \
-    template void launch_bc<T>(Handle &, Fld3<T> &, const Fld3<T> &, int, double, double, double *, double); \
+    template BcPlanes<T> bc_planes<T>(const Handle &, int);                                                \
+    template void launch_bc_planes<T>(Handle &, const Fld3<T> &, int, int, double, const double *, double *, \
+                                      double);                                                             \
+    template void launch_bc<T>(Handle &, Fld3<T> &, int);                                                  \
     template void launch_project<T>(Handle &, Fld3<T> &, const T *, T *, double);                         \
     template bool launch_thomas_seg<T>(Handle &, T *, int, long long, const Solve00 &);                   \
     template double max_divergence<T>(Handle &, const Fld3<T> &);                                         \

@@ -23,6 +23,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "bl_internal.hpp"
@@ -539,27 +540,62 @@ __device__ __forceinline__ f32x4 mfma_split(const u16x8 *A, bf16x8 bh, bf16x8 bl
 // (plus the mass-flux shift on the outflow), the difference of the stored
 // values on the wall and top V faces; the W face below plane 1 is the
 // periodic image of plane nz-2
-__device__ __forceinline__ double inc_div(const Dims &d, const Metrics &mt, const IncSrc &s, long long p, int i,
-                                          int j, int k) {
-    const long long pl = j + (long long)d.nyg * k, npl = (long long)d.nyg * d.nzg;
-    const double ur = (i == d.nx - 2) ? s.inc1[npl + pl] + s.inc1[2 * npl] : s.c0 * (double)s.fu[p];
-    const double ul = (i == 1) ? s.inc1[pl] : s.c0 * (double)s.fu[p - 1];
-    const double vt = (j == d.ny - 1) ? (double)s.vs[p] - (double)s.vn[p] : s.c0 * (double)s.fv[p];
-    const long long pb = p - d.sx;
-    const double vb = (j == 1) ? (double)s.vs[pb] - (double)s.vn[pb] : s.c0 * (double)s.fv[pb];
-    const long long pw = (k == 1) ? p + d.sxy * (long long)(d.nz - 3) : p - d.sxy;
-    const double wt = s.c0 * (double)s.fw[p], wb = s.c0 * (double)s.fw[pw];
-    return (ur - ul) * mt.rdx[i] + (vt - vb) * mt.rdy[j] + (wt - wb) * mt.rdz[k];
-}
+// (pointers, scales and ends fixed per line, as DivLine)
+struct IncLine {
+    const float *u, *vt, *vb, *wt, *wb;  // F1, or V of the stage on the top and wall faces
+    const float *nt, *nb;                // there: V at the step start (else null)
+    const double *rdx;
+    double c0, ry, rz, ul, ur;
+    int last;
+    __device__ __forceinline__ IncLine(const Dims &d, const Metrics &m, const IncSrc &s, const BcPlanes<float> &bc,
+                                       int c1, int c2) {
+        const long long p = fidx(d, 1, c1 + 1, c2 + 1), npl = (long long)d.nyg * d.nzg;
+        const long long pl = c1 + 1 + (long long)d.nyg * (c2 + 1);
+        u = s.fu + p;
+        vt = s.fv + p;
+        vb = vt - d.sx;
+        wt = s.fw + p;
+        wb = c2 == 0 ? wt + d.sxy * (d.nz - 3) : wt - d.sxy;
+        nt = nb = nullptr;
+        if (c1 == d.NM - 1) {
+            vt = bc.vtop + 1;
+            nt = s.vn + p;
+        }
+        if (c1 == 0) {
+            vb = bc.vwall + bc.wld * (c2 + 1) + 1;
+            nb = s.vn + p - d.sx;
+        }
+        rdx = m.rdx + 1;
+        ry = m.rdy[c1 + 1];
+        rz = m.rdz[c2 + 1];
+        c0 = s.c0;
+        ul = s.inc1[pl];
+        ur = s.inc1[npl + pl] + s.inc1[2 * npl];
+        last = d.N - 1;
+    }
+    struct Raw {
+        float u, l, vt, vb, wt, wb;
+        double rdx;
+    };
+    __device__ __forceinline__ Raw load(int n) const { return {u[n], u[n - 1], vt[n], vb[n], wt[n], wb[n], rdx[n]}; }
+    __device__ __forceinline__ double div(const Raw &a, int n) const {
+        const double r = n == last ? ur : c0 * (double)a.u, l = n == 0 ? ul : c0 * (double)a.l;
+        const double t = nt ? (double)a.vt - (double)nt[n] : c0 * (double)a.vt;
+        const double b = nb ? (double)a.vb - (double)nb[n] : c0 * (double)a.vb;
+        return (r - l) * a.rdx + (t - b) * ry + (c0 * (double)a.wt - c0 * (double)a.wb) * rz;
+    }
+    __device__ __forceinline__ double at(int n) const { return div(load(n), n); }
+};
 
 // forward: the pseudo-pressure rhs (projection.f90:38-47) of kXL lines
 // (cells i = 1..N of row j, plane m; line c = j-1 + NM (m-1)) formed in FP64
 // (from the increment when use_inc), its FP64 line sums for the (0,0) mode
 // (part[(j-1) M + m-1]), then the transform into T1[c NP + kx]
+constexpr int kXLd = 4;  // cells per thread whose loads are in flight together
 __global__ __launch_bounds__(256) void k_xfwd_mx(Dims d, Metrics mt, XArgs a, const float *__restrict__ U,
                                                  const float *__restrict__ V, const float *__restrict__ W,
-                                                 float *__restrict__ out, double *__restrict__ part, IncSrc inc,
-                                                 int use_inc) {
+                                                 float *__restrict__ out, double *__restrict__ part, BcPlanes<float> bc,
+                                                 IncSrc inc, int use_inc) {
     extern __shared__ float smx[];
     const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1;
     // twiddle indices n2 k1 stay below N (n2 < N2, k1 <= N1/2): no reduction
@@ -576,17 +612,26 @@ __global__ __launch_bounds__(256) void k_xfwd_mx(Dims d, Metrics mt, XArgs a, co
     for (int l = 0; l < kXL; ++l) {
         const int c = min(line0 + l, a.C - 1);
         const int c1 = c % a.C1, c2 = c / a.C1;
-        const long long base = fidx(d, 1, c1 + 1, c2 + 1);
-        const double ry = mt.rdy[c1 + 1], rz = mt.rdz[c2 + 1];
-        for (int n = tid; n < N; n += 256) {
-            const long long p = base + n;
-            const double dv = use_inc ? inc_div(d, mt, inc, p, n + 1, c1 + 1, c2 + 1)
-                                      : ((double)U[p] - (double)U[p - 1]) * mt.rdx[n + 1] +
-                                            ((double)V[p] - (double)V[p - d.sx]) * ry +
-                                            ((double)W[p] - (double)W[p - d.sxy]) * rz;
+        auto put = [&](int n, double dv) {
             ps[l] += dv;
             v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = (float)dv;
-        }
+        };
+        auto line = [&](const auto &dl) {
+            for (int n0 = tid; n0 < N; n0 += 256 * kXLd) {
+                typename std::decay<decltype(dl)>::type::Raw r[kXLd];
+#pragma unroll
+                for (int u = 0; u < kXLd; ++u) r[u] = dl.load(min(n0 + 256 * u, N - 1));
+#pragma unroll
+                for (int u = 0; u < kXLd; ++u) {
+                    const int n = n0 + 256 * u;
+                    if (n < N) put(n, dl.div(r[u], n));
+                }
+            }
+        };
+        if (use_inc)
+            line(IncLine(d, mt, inc, bc, c1, c2));
+        else
+            line(DivLine<float>(d, mt, bc, U, V, W, c1, c2));
     }
 #pragma unroll
     for (int l = 0; l < kXL; ++l) {
@@ -797,17 +842,13 @@ __global__ __launch_bounds__(256) void k_xinv_mx(Dims d, XArgs a, const float *_
 __global__ __launch_bounds__(256) void k_div_mixed(Dims d, Metrics m, const float *__restrict__ U,
                                                    const float *__restrict__ V, const float *__restrict__ W,
                                                    int NP, float *__restrict__ div, double *__restrict__ part,
-                                                   IncSrc inc, int use_inc) {
+                                                   BcPlanes<float> bc, IncSrc inc, int use_inc) {
     const int ii = blockIdx.x * 64 + (threadIdx.x & 63);
     const int jj = blockIdx.y * 4 + (threadIdx.x >> 6);
     const int mm = blockIdx.z;
     double v = 0.0;
     if (ii < d.N && jj < d.NM) {
-        const int i = ii + 1, j = jj + 1, k = mm + 1;
-        const long long p = fidx(d, i, j, k);
-        v = use_inc ? inc_div(d, m, inc, p, i, j, k)
-                    : ((double)U[p] - (double)U[p - 1]) * m.rdx[i] + ((double)V[p] - (double)V[p - d.sx]) * m.rdy[j] +
-                          ((double)W[p] - (double)W[p - d.sxy]) * m.rdz[k];
+        v = use_inc ? IncLine(d, m, inc, bc, jj, mm).at(ii) : DivLine<float>(d, m, bc, U, V, W, jj, mm).at(ii);
         div[((long long)mm * d.NM + jj) * NP + ii] = (float)v;
     }
     for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
@@ -1119,8 +1160,9 @@ void build_mixed(Handle &h) {
     BL_HIP(hipStreamSynchronize(h.stream));
 }
 
-void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const IncSrc *inc) {
+void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const BcPlanes<float> *bcp, const IncSrc *inc) {
     const Dims &d = h.d;
+    const BcPlanes<float> bc = bcp ? *bcp : BcPlanes<float>{};
     const IncSrc src = inc ? *inc : IncSrc{};
     const int use_inc = inc ? 1 : 0;
     const int N = d.N, M = d.M, NM = d.NM, NP = h.NP;
@@ -1150,15 +1192,15 @@ void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const Inc
         // divergence, FP64 line sums and forward x transform in one kernel
         ProfScope ps(h, KID_XFORM_X_FWD);
         const size_t lds = sizeof(float) * (size_t)kXL * N + sizeof(float2) * (size_t)kXL * K1 * N2;
-        hipLaunchKernelGGL(k_xfwd_mx, xgrid, dim3(256), lds, h.stream, d, h.m, xa, f.u, f.v, f.w, T1, h.p00, src,
-                           use_inc);
+        hipLaunchKernelGGL(k_xfwd_mx, xgrid, dim3(256), lds, h.stream, d, h.m, xa, f.u, f.v, f.w, T1, h.p00, bc,
+                           src, use_inc);
         check();
     }
     // rhs: divergence lines into S (as scratch), FP64 plane partials
     if (!h.mx_two) {
         ProfScope ps(h, KID_DIVERGENCE);
         hipLaunchKernelGGL(k_div_mixed, dim3((N + 63) / 64, (NM + 3) / 4, M), dim3(256), 0, h.stream, d, h.m,
-                           f.u, f.v, f.w, NP, S, h.p00, src, use_inc);
+                           f.u, f.v, f.w, NP, S, h.p00, bc, src, use_inc);
         check();
     }
     // forward x: T1[(m*NM + j)*NP + kx] = sum_n Dxf[kx][n] div[(m*NM + j)*NP + n]
