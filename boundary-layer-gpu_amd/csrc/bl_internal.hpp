@@ -28,6 +28,13 @@ __host__ __device__ inline long long fidx(const Dims &d, int i, int j, int k) {
     return (long long)i + (long long)d.sx * ((long long)j + (long long)d.sy * k);
 }
 
+// (cos, sin) pairs of the fragment table of a folded DFT of length L: row tiles
+// x k steps x 64 lanes over rows and columns 0..L/2
+inline int dct_frag(int L) {
+    const int H = L / 2 + 1;
+    return (H + 15) / 16 * ((H + 3) / 4) * 64;
+}
+
 // a / b for 0 <= a < 16384 and 1 <= b <= 128, with rb = 1.0f / b: exact on
 // that range (checked exhaustively), and a few instructions instead of the
 // integer division sequence
@@ -275,10 +282,7 @@ struct Handle {
     int lda_zt;                      // leading dimension of the z cos/sin tables
     double *zc, *zs;                 // z tables cos/sin(2 pi k m / M), [m][k]
     double *zf = nullptr;            // their matrix-core fragments (M/2 + 1 <= 96)
-    double *dct_w1, *dct_w2, *dct_wN, *dct_rot;  // x-DCT twiddle tables (complex)
-    bool dct_mfma = false;                       // x-DCT on the FP64 matrix cores (shape fits)
-    double *dct_mf = nullptr;                    // their operand tables: fA, fC, iC, iA
-    size_t dct_mf_off[4] = {0, 0, 0, 0};
+    double *dct_tab = nullptr;       // x-DCT tables as double2: rot[N], twA, twC [K1 N2], t1, t1i, t2 (dct_frag)
     double *lu_dl, *lu_dp, *lu_du;  // Thomas factors [k][j][kx], [k][j][kx], [j] (table kernel only)
     double *lu00;                   // the pinned (0,0) system: multipliers [NM], reciprocal pivots [NM]
     int th_p = 0;                   // segments of the partitioned Thomas kernel (0: table kernel)
@@ -297,7 +301,7 @@ struct Handle {
     bool mx_two = false;            // x transform as two short DFTs (k_xfwd_mx / k_xinv_mx)
     void *mx2 = nullptr;            // their operand and twiddle tables (one allocation)
     const void *x2_fA = nullptr, *x2_fC = nullptr, *x2_iC = nullptr, *x2_iA = nullptr;
-    const float *x2_tw = nullptr;   // wN[N], rot[N] as float2
+    const float *x2_tw = nullptr;   // float2 twiddles: W_N^{n2 k1} as [k1][n2] and [n2][k1], then rot[N]
     unsigned short *mx_tab;         // one allocation for the eight matrices below
     unsigned short *zmf = nullptr;  // folded z transform fragments (k_zdft_mx), M/2 + 1 <= 96
     int zmf_rt = 0;

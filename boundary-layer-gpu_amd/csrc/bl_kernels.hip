@@ -964,19 +964,33 @@ __global__ __launch_bounds__(256) void k_zdft_inv(int M, int C, long long plane,
 // twiddle, projection.f90:110-134).  Inverse: f[n] = (1/(N M)) (g[0]/2 +
 // sum_k g[k] cos(pi k (2n+1)/(2N))) (projection.f90:160-202 with the
 // 1/(2 nxp nzp) factor).
-// Tables (cos, sin interleaved): w1[q] = e^{-2 pi i q/N1}, w2[q] = e^{-2 pi i q/N2},
-// wN[q] = e^{-2 pi i q/N}, rot[k] = e^{-i pi k/(2N)}.
+//
+// Both short DFTs run on the FP64 matrix cores (v_mfma_f64_16x16x4_f64; lane l
+// holds A[l%16][l/16], B[l/16][l%16] and D[l/16 + 4r][l%16], r < 4), folded by
+// the symmetry of cosine and sine: the sums over n of a length L take the pairs
+// x[n] + x[L-n] and x[n] - x[L-n], and the outputs k and L-k come from the same
+// two sums, so a product has (L/2)^2 terms instead of L^2.  At 814x257x193
+// (28 x 29) that is 64 matrix instructions per two lines where the unfolded
+// products took 176.
+// Forward, step A (N1 points, real): B[k1][n2] = W_N^{n2 k1} sum_n1 v[N2 n1 + n2]
+//   W_N1^{n1 k1}; columns (line, n2), rows k1.
+// Forward, step C (N2 points, complex): V[k1 + N1 k2] = sum_n2 B W_N2^{n2 k2};
+//   columns (line, k1), rows k2; X[k] = 2 Re(rot_k V), X[N-k] = -2 Im(rot_k V).
+// Inverse, step C': the conjugate of C on V[k] = conj(rot_k) (g[k] - i g[N-k])/2;
+//   step A': v[N2 n1 + n2] = sum_k1 c_k1 Re(C~ conj(W_N1^{n1 k1})) with the
+//   Hermitian weights (1, 2, .., 1) in the table.
+// Tables: rot[k] = e^{-i pi k/(2N)}; twA, twC = W_N^{n2 k1} as [k1][n2] and [n2][k1]
+// (16 lanes read consecutive entries); t1, t1i, t2: (cos, sin)(2 pi a b/L) for
+// row a and column b in lane order per (row tile, k step), b weighted in t1i.
 // ------------------------------------------------------------------------
 struct DctArgs {
     int N, N1, N2, K1h;
-    int C1, C;  // lines c = c1 + C1*c2
+    int LB;        // lines per block
+    int C1, C;     // lines c = c1 + C1*c2
     long long in_base, in_c1, in_c2;
     long long out_base, out_c1, out_c2;
     double scale;  // inverse only: 1/(N*M)
-    const double2 *w1, *w2, *wN, *rot;
-    // FP64 MFMA operand tables of the two short DFTs, in lane order (see
-    // k_dct_fwd_m); null when the shape does not fit those kernels
-    const double *fA, *fC, *iC, *iA;
+    const double2 *twA, *twC, *rot, *t1, *t1i, *t2;
 };
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
@@ -986,184 +1000,351 @@ __device__ __forceinline__ double2 cmulc(double2 a, double2 b) {  // a * conj(b)
     return make_double2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
 }
 
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+constexpr int kLd = 4;  // loads per thread in flight in the line load phases
+
+__device__ __forceinline__ dbl4 mfma64(double a, double b, dbl4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// row stride of the complex intermediate: odd, so that 16 lanes reading one
+// entry of 16 rows use different banks
+__host__ __device__ inline int dct_ld(int N2) { return N2 | 1; }
+// LDS doubles of the line area (even: the complex area behind it is 16-byte aligned)
+__host__ __device__ inline int dct_lines(int LB, int N) { return (LB * N + 1) / 2 * 2; }
+
+// the folded length-N2 DFT of the complex rows Bl (one per column): the four
+// real sums of row tile rt
+struct DctSums {
+    dbl4 cr, ci, sr, si;  // sum E cos, sum O sin (real and imaginary parts)
+};
+__device__ __forceinline__ DctSums dct_sums(const DctArgs &a, const double2 *Bl, bool cok, int rt, int q, int lane) {
+    const int H = a.N2 / 2 + 1, KS = (H + 3) / 4;
+    const dbl4 z = {0.0, 0.0, 0.0, 0.0};
+    DctSums s{z, z, z, z};
+    const double2 *t = a.t2 + (long long)rt * KS * 64 + lane;
+    // four k steps at a time, their operands read before the first product, from the last to the first: a smooth
+    // field's spectrum falls with k, and adding its large end last rounds the
+    // large partial sums least often
+    for (int k0 = (KS - 1) / 4 * 4; k0 >= 0; k0 -= 4) {
+        double2 w[4], x[4], y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int n = 4 * (k0 + u) + q;
+            w[u] = t[min(k0 + u, KS - 1) * 64];
+            x[u] = y[u] = make_double2(0.0, 0.0);
+            if (cok && n < H) {
+                x[u] = Bl[n];
+                y[u] = Bl[n == 0 ? 0 : a.N2 - n];
+            }
+        }
+#pragma unroll
+        for (int u = 3; u >= 0; --u) {
+            const int n = 4 * (k0 + u) + q;
+            const bool single = n == 0 || 2 * n == a.N2;  // x = y there
+            if (k0 + u >= KS) continue;
+            s.cr = mfma64(w[u].x, single ? x[u].x : x[u].x + y[u].x, s.cr);
+            s.ci = mfma64(w[u].x, single ? x[u].y : x[u].y + y[u].y, s.ci);
+            s.sr = mfma64(w[u].y, x[u].x - y[u].x, s.sr);
+            s.si = mfma64(w[u].y, x[u].y - y[u].y, s.si);
+        }
+    }
+    return s;
+}
+
+// SMALL (N1, N2 <= 31): two lines and two waves per block; step A has two
+// column tiles per wave, step C one, so every product stays in registers until
+// its inputs are read and the lines and the spectra share one LDS area (13.9 KB
+// at N = 812: the blocks' load, product and store phases overlap across ten
+// blocks per CU).  Otherwise four or eight waves, and LB lines in an area of their
+// own.  At 814x257x193 the forward (inverse) transform takes 0.345 (0.203) ms, bound
+// by the latency of its loads (HBM time 0.25 (0.125)); the unfolded products in
+// four waves took 0.42 (0.30).  511 points (7 x 73): 0.086 (0.060) ms per 12288
+// lines, on the vector units 0.15 (0.15).
 // DIV: the line is the pseudo-pressure rhs (projection.f90:38-47) evaluated
 // on the fly from U, V, W (in = U, in2 = V, in3 = W, lines over cells
 // i = 1..N, j = 1..NM, k = 1..M) instead of being read from memory; with
 // bc.du set the boundary faces come from the stage's boundary values (DivLine).
-template <int LB, bool DIV>
-__global__ __launch_bounds__(256) void k_dct_fwd(DctArgs a, Dims d, Metrics mt, BcPlanes<double> bc,
-                                                 const double *__restrict__ in,
-                                                 const double *__restrict__ in2,
-                                                 const double *__restrict__ in3,
-                                                 double *__restrict__ out) {
-    extern __shared__ double smem[];
-    const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1;
-    double *v = smem;                                    // LB*N
-    double2 *B = reinterpret_cast<double2 *>(v + LB * N);  // LB*K1*N2
-    double2 *w1 = B + LB * K1 * N2;                      // N1
-    double2 *w2 = w1 + N1;                               // N2
-    const int tid = threadIdx.x;
-    for (int q = tid; q < N1; q += 256) w1[q] = a.w1[q];
-    for (int q = tid; q < N2; q += 256) w2[q] = a.w2[q];
+template <bool DIV, bool SMALL>
+__global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_fwd_m(DctArgs a, Dims d, Metrics mt, BcPlanes<double> bc,
+                                                                 const double *__restrict__ in,
+                                                                 const double *__restrict__ in2,
+                                                                 const double *__restrict__ in3,
+                                                                 double *__restrict__ out) {
+    extern __shared__ double2 smem2[];
+    const int NW = SMALL ? 2 : blockDim.x >> 6;
+    const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1, LB = SMALL ? 2 : a.LB, ld = dct_ld(N2);
+    double *v = reinterpret_cast<double *>(smem2);
+    double2 *Bc = SMALL ? smem2 : smem2 + dct_lines(LB, N) / 2;  // [line][k1][ld]
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int line0 = blockIdx.x * LB;
-    // load and reorder: v[n/2] = f[n] (n even), v[N-1-(n-1)/2] = f[n] (n odd)
-    for (int idx = tid; idx < LB * N; idx += 256) {
-        const int l = idx / N, n = idx - l * N;
+    // load and reorder: v[n/2] = f[n] (n even), v[N-1-(n-1)/2] = f[n] (n odd);
+    // a line per wave, kLd elements per lane loaded before the first is used
+    for (int l = wave; l < LB; l += NW) {
         const int c = min(line0 + l, a.C - 1);
         const int c1 = c % a.C1, c2 = c / a.C1;
-        const long long p = a.in_base + c1 * a.in_c1 + c2 * a.in_c2 + n;
-        double f;
-        if (DIV) {
-            f = DivLine<double>(d, mt, bc, in, in2, in3, c1, c2).at(n);
-        } else {
-            f = in[p];
+        const double *src = in + a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
+        const DivLine<double> dl(d, mt, bc, in, in2, in3, c1, c2);
+        for (int n0 = lane; n0 < N; n0 += 64 * kLd) {
+            typename DivLine<double>::Raw r[DIV ? kLd : 1];
+            double f[DIV ? 1 : kLd];
+#pragma unroll
+            for (int u = 0; u < kLd; ++u) {
+                const int n = min(n0 + 64 * u, N - 1);
+                if constexpr (DIV)
+                    r[u] = dl.load(n);
+                else
+                    f[u] = src[n];
+            }
+#pragma unroll
+            for (int u = 0; u < kLd; ++u) {
+                const int n = n0 + 64 * u;
+                double x;
+                if constexpr (DIV)
+                    x = dl.div(r[u], n);
+                else
+                    x = f[u];
+                if (n < N) v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = x;
+            }
         }
-        v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = f;
     }
     __syncthreads();
-    // step A: B[k1][n2] = W_N^{n2 k1} sum_n1 v[N2 n1 + n2] W_N1^{n1 k1}
-    for (int idx = tid; idx < LB * K1 * N2; idx += 256) {
-        const int l = idx / (K1 * N2), r = idx - l * K1 * N2;
-        const int k1 = r / N2, n2 = r - k1 * N2;
-        const double *vl = v + l * N + n2;
-        double re = 0.0, im = 0.0;
-        int q = 0;
-        for (int n1 = 0; n1 < N1; ++n1) {
-            const double x = vl[n1 * N2];
-            const double2 w = w1[q];
-            re = fma(x, w.x, re);
-            im = fma(x, w.y, im);
-            q += k1;
-            if (q >= N1) q -= N1;
+    // ---- step A
+    const int H1 = K1, KS1 = (H1 + 3) / 4, RT1 = (H1 + 15) / 16, CA = (LB * N2 + 15) / 16;
+    auto sums_a = [&](int ct, int rt, dbl4 &re, dbl4 &im) {
+        const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
+        const bool cok = col < LB * N2;
+        const double *vl = v + ln * N + n2;
+        const double2 *t = a.t1 + rt * KS1 * 64 + lane;
+        re = im = dbl4{0.0, 0.0, 0.0, 0.0};
+        for (int k0 = 0; k0 < KS1; k0 += 4) {
+            double2 w[4];
+            double x[4], y[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int n = 4 * (k0 + u) + q;
+                w[u] = t[min(k0 + u, KS1 - 1) * 64];
+                x[u] = y[u] = 0.0;
+                if (cok && n < H1) {
+                    x[u] = vl[N2 * n];
+                    y[u] = vl[n == 0 ? 0 : N2 * (N1 - n)];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int n = 4 * (k0 + u) + q;
+                const bool single = n == 0 || 2 * n == N1;  // x = y there
+                if (k0 + u >= KS1) continue;
+                re = mfma64(w[u].x, single ? x[u] : x[u] + y[u], re);
+                im = mfma64(w[u].y, x[u] - y[u], im);
+            }
         }
-        B[idx] = cmul(make_double2(re, im), a.wN[(n2 * k1) % N]);
+    };
+    auto put_a = [&](int ct, int rt, const dbl4 &re, const dbl4 &im) {
+        const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
+        if (col >= LB * N2) return;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int k1 = 16 * rt + q + 4 * r;
+            if (k1 < K1) Bc[(ln * K1 + k1) * ld + n2] = cmul(make_double2(re[r], -im[r]), a.twA[k1 * N2 + n2]);
+        }
+    };
+    if constexpr (SMALL) {
+        dbl4 re[2], im[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) sums_a(2 * wave + h, 0, re[h], im[h]);
+        __syncthreads();  // v is read; Bc overwrites it
+#pragma unroll
+        for (int h = 0; h < 2; ++h) put_a(2 * wave + h, 0, re[h], im[h]);
+    } else {
+        for (int e = wave; e < CA * RT1; e += NW) {
+            const int ct = e / RT1, rt = e - ct * RT1;
+            dbl4 re, im;
+            sums_a(ct, rt, re, im);
+            put_a(ct, rt, re, im);
+        }
     }
     __syncthreads();
-    // step C: V[k1 + N1 k2] = sum_n2 B[k1][n2] W_N2^{n2 k2}; X[k] = 2 Re(rot_k V),
-    // X[N-k] = -2 Im(rot_k V)
-    for (int idx = tid; idx < LB * K1 * N2; idx += 256) {
-        const int l = idx / (K1 * N2), r = idx - l * K1 * N2;
-        const int k1 = r / N2, k2 = r - k1 * N2;
-        const double2 *Bl = B + l * K1 * N2 + k1 * N2;
-        double re = 0.0, im = 0.0;
-        int q = 0;
-        for (int n2 = 0; n2 < N2; ++n2) {
-            const double2 b = Bl[n2], w = w2[q];
-            re = fma(b.x, w.x, fma(-b.y, w.y, re));
-            im = fma(b.x, w.y, fma(b.y, w.x, im));
-            q += k2;
-            if (q >= N2) q -= N2;
+    // ---- step C
+    const int H2 = N2 / 2 + 1, RT2 = (H2 + 15) / 16, CC = (LB * K1 + 15) / 16;
+    auto put_c = [&](int ct, int rt, const DctSums &s) {
+        const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
+        if (col >= LB * K1) return;
+        auto put = [&](int k2, double re, double im) {
+            const int k = k1 + N1 * k2;
+            const double2 wv = cmul(a.rot[k], make_double2(re, im));
+            v[ln * N + k] = 2.0 * wv.x;
+            // the mirror N - k of k1 = 0 and k1 = N1/2 is one of their own outputs
+            if (k1 != 0 && 2 * k1 != N1) v[ln * N + N - k] = -2.0 * wv.y;
+        };
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int k2 = 16 * rt + q + 4 * r;
+            if (k2 >= H2) continue;
+            put(k2, s.cr[r] + s.si[r], s.ci[r] - s.sr[r]);
+            if (k2 != 0 && 2 * k2 != N2) put(N2 - k2, s.cr[r] - s.si[r], s.ci[r] + s.sr[r]);
         }
-        const int k = k1 + N1 * k2;
-        const double2 wv = cmul(a.rot[k], make_double2(re, im));
-        v[l * N + k] = 2.0 * wv.x;
-        // the mirror N - k of k1 = 0 and k1 = N1/2 is written directly (k1' = k1)
-        if (k1 != 0 && 2 * k1 != N1) v[l * N + N - k] = -2.0 * wv.y;
+    };
+    auto sums_c = [&](int ct, int rt) {
+        const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
+        return dct_sums(a, Bc + (ln * K1 + k1) * ld, col < LB * K1, rt, q, lane);
+    };
+    if constexpr (SMALL) {
+        const DctSums s = sums_c(wave, 0);
+        __syncthreads();  // Bc is read; v overwrites it
+        put_c(wave, 0, s);
+    } else {
+        for (int e = wave; e < CC * RT2; e += NW) {
+            const int ct = e / RT2, rt = e - ct * RT2;
+            put_c(ct, rt, sums_c(ct, rt));
+        }
     }
     __syncthreads();
-    for (int idx = tid; idx < LB * N; idx += 256) {
-        const int l = idx / N, kx = idx - l * N;
+    for (int l = wave; l < LB; l += NW) {
         const int c = line0 + l;
-        if (c >= a.C) continue;
-        const int c1 = c % a.C1, c2 = c / a.C1;
-        out[a.out_base + c1 * a.out_c1 + c2 * a.out_c2 + kx] = v[l * N + kx];
+        if (c >= a.C) break;
+        double *dst = out + a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
+        for (int kx = lane; kx < N; kx += 64) dst[kx] = v[l * N + kx];
     }
 }
 
-template <int LB>
-__global__ __launch_bounds__(256) void k_dct_inv(DctArgs a, const double *__restrict__ in,
-                                                 double *__restrict__ out) {
-    extern __shared__ double smem[];
-    const int N = a.N, N1 = a.N1, N2 = a.N2, K1h = a.K1h, K1 = K1h + 1;
-    double2 *Vs = reinterpret_cast<double2 *>(smem);  // LB*N, later the output lines (as doubles)
-    double2 *C = Vs + LB * N;                         // LB*K1*N2
-    double2 *w1 = C + LB * K1 * N2;
-    double2 *w2 = w1 + N1;
-    const int tid = threadIdx.x;
-    for (int q = tid; q < N1; q += 256) w1[q] = a.w1[q];
-    for (int q = tid; q < N2; q += 256) w2[q] = a.w2[q];
+template <bool SMALL>
+__global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_inv_m(DctArgs a, const double *__restrict__ in,
+                                                                 double *__restrict__ out) {
+    extern __shared__ double2 smem2[];
+    const int NW = SMALL ? 2 : blockDim.x >> 6;
+    const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1, LB = SMALL ? 2 : a.LB, ld = dct_ld(N2);
+    const float rK1 = 1.0f / (float)K1;
+    // SMALL: one area for V, C~ and the output lines in turn; otherwise V (later
+    // the lines, which are no longer) and C~ apart
+    double2 *Vs = smem2, *Cs = SMALL ? smem2 : smem2 + LB * K1 * ld;
+    double *o = reinterpret_cast<double *>(smem2);
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int line0 = blockIdx.x * LB;
-    // V[k] = conj(rot_k) (g[k] - i g[N-k]) / 2, g read straight from the spectrum line
-    for (int idx = tid; idx < LB * N; idx += 256) {
-        const int l = idx / N, k = idx - l * N;
+    // V[k1 + N1 k2] = conj(rot_k) (g[k] - i g[N-k]) / 2 for k1 <= N1/2: Vs[l][k1][k2],
+    // a line per wave, k1 fastest over the lanes (runs of K1 consecutive entries of
+    // the line), kLd elements per lane loaded before the first is used
+    const int nv = K1 * N2;
+    for (int l = wave; l < LB; l += NW) {
         const int c = min(line0 + l, a.C - 1);
-        const int c1 = c % a.C1, c2 = c / a.C1;
-        const double *gl = in + a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
-        const double gk = gl[k], gm = (k == 0) ? 0.0 : gl[N - k];
-        Vs[idx] = cmulc(make_double2(0.5 * gk, -0.5 * gm), a.rot[k]);
-    }
-    __syncthreads();
-    // step C': C~[k1][n2] = W_N^{-n2 k1} sum_k2 V[k1 + N1 k2] W_N2^{-n2 k2}
-    for (int idx = tid; idx < LB * K1 * N2; idx += 256) {
-        const int l = idx / (K1 * N2), r = idx - l * K1 * N2;
-        const int k1 = r / N2, n2 = r - k1 * N2;
-        const double2 *Vl = Vs + l * N + k1;
-        double re = 0.0, im = 0.0;
-        int q = 0;
-        for (int k2 = 0; k2 < N2; ++k2) {
-            const double2 V = Vl[N1 * k2];
-            const double2 w = w2[q];  // use conj(w)
-            re = fma(V.x, w.x, fma(V.y, w.y, re));
-            im = fma(V.y, w.x, fma(-V.x, w.y, im));
-            q += n2;
-            if (q >= N2) q -= N2;
+        const double *g = in + a.in_base + (long long)(c % a.C1) * a.in_c1 + (long long)(c / a.C1) * a.in_c2;
+        for (int i0 = lane; i0 < nv; i0 += 64 * kLd) {
+            double gk[kLd], gm[kLd];
+            double2 rt[kLd];
+#pragma unroll
+            for (int u = 0; u < kLd; ++u) {
+                const int r = min(i0 + 64 * u, nv - 1), k2 = small_div(r, rK1), k1 = r - k2 * K1;
+                const int k = k1 + N1 * k2;
+                gk[u] = g[k];
+                gm[u] = g[k == 0 ? 0 : N - k];
+                rt[u] = a.rot[k];
+                if (k == 0) gm[u] = 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < kLd; ++u) {
+                const int r = i0 + 64 * u, k2 = small_div(r, rK1), k1 = r - k2 * K1;
+                if (r < nv)
+                    Vs[(l * K1 + k1) * ld + k2] = cmulc(make_double2(0.5 * gk[u], -0.5 * gm[u]), rt[u]);
+            }
         }
-        C[idx] = cmulc(make_double2(re, im), a.wN[(n2 * k1) % N]);
     }
     __syncthreads();
-    // step A': v[N2 n1 + n2] = (1/N) (Re C~[0] + sum_{k1>=1} c_k1 Re(C~[k1] W_N1^{-n1 k1}))
-    double *o = smem;  // LB*N doubles inside the V area, which is no longer read
-    for (int idx = tid; idx < LB * N; idx += 256) {
-        const int l = idx / N, n = idx - l * N;
-        const int n1 = n / N2, n2 = n - n1 * N2;
-        const double2 *Cl = C + l * K1 * N2 + n2;
-        double acc = Cl[0].x;
-        int q = 0;
-        for (int k1 = 1; k1 <= K1h; ++k1) {
-            q += n1;
-            if (q >= N1) q -= N1;
-            const double2 c = Cl[k1 * N2], w = w1[q];
-            const double t = c.x * w.x + c.y * w.y;  // Re(c * conj(w))
-            acc += ((N1 % 2 == 0) && k1 == K1h) ? t : 2.0 * t;
+    // ---- step C': C~[k1][n2] = W_N^{-n2 k1} sum_k2 V W_N2^{-n2 k2}
+    const int H2 = N2 / 2 + 1, RT2 = (H2 + 15) / 16, CC = (LB * K1 + 15) / 16;
+    auto sums_c = [&](int ct, int rt) {
+        const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
+        return dct_sums(a, Vs + (ln * K1 + k1) * ld, col < LB * K1, rt, q, lane);
+    };
+    auto put_c = [&](int ct, int rt, const DctSums &s) {
+        const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
+        if (col >= LB * K1) return;
+        auto put = [&](int n2, double re, double im) {
+            Cs[(ln * K1 + k1) * ld + n2] = cmulc(make_double2(re, im), a.twC[n2 * K1 + k1]);
+        };
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int n2 = 16 * rt + q + 4 * r;
+            if (n2 >= H2) continue;
+            put(n2, s.cr[r] - s.si[r], s.ci[r] + s.sr[r]);
+            if (n2 != 0 && 2 * n2 != N2) put(N2 - n2, s.cr[r] + s.si[r], s.ci[r] - s.sr[r]);
         }
-        const int pos = (n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1;
-        o[l * N + pos] = acc * a.scale;
+    };
+    if constexpr (SMALL) {
+        const DctSums s = sums_c(wave, 0);
+        __syncthreads();  // Vs is read; Cs overwrites it
+        put_c(wave, 0, s);
+    } else {
+        for (int e = wave; e < CC * RT2; e += NW) {
+            const int ct = e / RT2, rt = e - ct * RT2;
+            put_c(ct, rt, sums_c(ct, rt));
+        }
     }
     __syncthreads();
-    for (int idx = tid; idx < LB * N; idx += 256) {
-        const int l = idx / N, n = idx - l * N;
+    // ---- step A'
+    const int KS1 = (K1 + 3) / 4, RT1 = (K1 + 15) / 16, CA = (LB * N2 + 15) / 16;
+    auto sums_a = [&](int ct, int rt, dbl4 &p, dbl4 &s) {
+        const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
+        const bool cok = col < LB * N2;
+        const double2 *cl = Cs + ln * K1 * ld + n2;
+        const double2 *t = a.t1i + rt * KS1 * 64 + lane;
+        p = s = dbl4{0.0, 0.0, 0.0, 0.0};
+        for (int k0 = (KS1 - 1) / 4 * 4; k0 >= 0; k0 -= 4) {  // the large end last, as in dct_sums
+            double2 w[4], x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k1 = 4 * (k0 + u) + q;
+                w[u] = t[min(k0 + u, KS1 - 1) * 64];
+                x[u] = make_double2(0.0, 0.0);
+                if (cok && k1 < K1) x[u] = cl[k1 * ld];
+            }
+#pragma unroll
+            for (int u = 3; u >= 0; --u) {
+                if (k0 + u >= KS1) continue;
+                p = mfma64(w[u].x, x[u].x, p);
+                s = mfma64(w[u].y, x[u].y, s);
+            }
+        }
+    };
+    auto put_a = [&](int ct, int rt, const dbl4 &p, const dbl4 &s) {
+        const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
+        if (col >= LB * N2) return;
+        auto put = [&](int n1, double x) {
+            const int n = N2 * n1 + n2;
+            const int pos = (n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1;
+            o[ln * N + pos] = x * a.scale;
+        };
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int n1 = 16 * rt + q + 4 * r;
+            if (n1 >= K1) continue;
+            put(n1, p[r] - s[r]);
+            if (n1 != 0 && 2 * n1 != N1) put(N1 - n1, p[r] + s[r]);
+        }
+    };
+    if constexpr (SMALL) {
+        dbl4 p[2], s[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) sums_a(2 * wave + h, 0, p[h], s[h]);
+        __syncthreads();  // Cs is read; o overwrites it
+#pragma unroll
+        for (int h = 0; h < 2; ++h) put_a(2 * wave + h, 0, p[h], s[h]);
+    } else {
+        for (int e = wave; e < CA * RT1; e += NW) {
+            const int ct = e / RT1, rt = e - ct * RT1;
+            dbl4 p, s;
+            sums_a(ct, rt, p, s);
+            put_a(ct, rt, p, s);
+        }
+    }
+    __syncthreads();
+    for (int l = wave; l < LB; l += NW) {
         const int c = line0 + l;
-        if (c >= a.C) continue;
-        const int c1 = c % a.C1, c2 = c / a.C1;
-        out[a.out_base + c1 * a.out_c1 + c2 * a.out_c2 + n] = o[idx];
+        if (c >= a.C) break;
+        double *dst = out + a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
+        for (int n = lane; n < N; n += 64) dst[n] = o[l * N + n];
     }
-}
-
-// ------------------------------------------------------------------------
-// The same transforms with both short DFTs on the FP64 matrix cores
-// (v_mfma_f64_16x16x4_f64; lane l holds A[l%16][l/16], B[l/16][l%16] and
-// D[l/16 + 4r][l%16], r < 4).  kMfL lines per block, four waves.
-// Step A / A' use 2 kMfL column tiles (kMfL / 2 per wave), step C / C' kMfL.
-// Forward, step A: [Re, Im of B[k1][n2]] = WA [N1 x (line, n2)] with the
-//   rows of WA ordered so that a lane's D rows r = 0, 1 are Re, Im of one k1
-//   and r = 2, 3 those of k1 + 4; the twiddle W_N^{n2 k1} is applied in
-//   registers and B' goes to LDS as complex.
-// Forward, step C: [Re, Im of V[k1 + N1 k2]] = WC [(n2, re/im) x (line, k1)],
-//   rows paired the same way over k2; the post-rotation and the Makhoul
-//   placement write the output line into LDS.
-// Inverse, step C': the conjugate DFT over k2, rows paired over n2, then the
-//   conjugate twiddle; step A': the real output v[N2 n1 + n2] as one
-//   real matrix WA' [n1 x (k1, re/im)] with the Hermitian weights (1, 2, .., 1).
-// The operand tables are built on the host in lane order (one double per
-// lane per (row tile, k step)); shapes: N1 <= 32, N1/2 + 1 <= 16, N2 <= 32.
-// ------------------------------------------------------------------------
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-constexpr int kMfL = 2;                   // lines per block
-constexpr int kLd = 4;                    // loads per thread in flight in the line load phases
-constexpr int kMfKA = 8, kMfKC = 16;      // k steps: step A (N1 <= 32), step C (2 N2 <= 64)
-
-__device__ __forceinline__ dbl4 mfma64(double a, double b, dbl4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
 // ------------------------------------------------------------------------
@@ -1283,296 +1464,6 @@ __global__ __launch_bounds__(64 * kZmW) void k_zdft_mf(int M, int C, long long p
                 }
             }
         }
-    }
-}
-
-template <bool DIV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_dct_fwd_m(DctArgs a, Dims d, Metrics mt, BcPlanes<double> bc, const double *__restrict__ in,
-                                                   const double *__restrict__ in2, const double *__restrict__ in3,
-                                                   double *__restrict__ out) {
-    extern __shared__ double smem[];
-    const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1;
-    // twiddle indices n2 k1 stay below N (n2 < N2, k1 <= N1/2): no reduction
-    const float rN2 = 1.0f / (float)N2, rK1 = 1.0f / (float)K1;
-    // v (kMfL*N doubles) and Bc (kMfL*K1*N2 complex) share one LDS area: each
-    // step finishes reading its input before a barrier and then writes its output
-    double *v = smem;
-    double2 *Bc = reinterpret_cast<double2 *>(smem);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
-    const int line0 = blockIdx.x * kMfL;
-    // load and reorder: v[n/2] = f[n] (n even), v[N-1-(n-1)/2] = f[n] (n odd);
-    // kLd elements per thread are loaded before the first one is used
-#pragma unroll
-    for (int l = 0; l < kMfL; ++l) {
-        const int c = min(line0 + l, a.C - 1);
-        const int c1 = c % a.C1, c2 = c / a.C1;
-        const double *src = in + a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
-        const DivLine<double> dl(d, mt, bc, in, in2, in3, c1, c2);
-        for (int n0 = tid; n0 < N; n0 += 256 * kLd) {
-            typename DivLine<double>::Raw r[DIV ? kLd : 1];
-            double f[DIV ? 1 : kLd];
-#pragma unroll
-            for (int u = 0; u < kLd; ++u) {
-                const int n = min(n0 + 256 * u, N - 1);
-                if constexpr (DIV)
-                    r[u] = dl.load(n);
-                else
-                    f[u] = src[n];
-            }
-#pragma unroll
-            for (int u = 0; u < kLd; ++u) {
-                const int n = n0 + 256 * u;
-                double x;
-                if constexpr (DIV)
-                    x = dl.div(r[u], n);
-                else
-                    x = f[u];
-                if (n < N) v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = x;
-            }
-        }
-    }
-    const int KSA = (N1 + 3) / 4, KSC = (2 * N2 + 3) / 4;
-    double fa[2][kMfKA];
-#pragma unroll
-    for (int ks = 0; ks < kMfKA; ++ks) {
-        fa[0][ks] = ks < KSA ? a.fA[(0 * KSA + ks) * 64 + lane] : 0.0;
-        fa[1][ks] = ks < KSA ? a.fA[(1 * KSA + ks) * 64 + lane] : 0.0;
-    }
-    __syncthreads();
-    // ---- step A: wave w owns kMfL / 2 column tiles (columns (line, n2))
-    for (int ct = wave * (kMfL / 2); ct < (wave + 1) * (kMfL / 2); ++ct) {
-        const int col = ct * 16 + c16;
-        const int ln = small_div(col, rN2), n2 = col - ln * N2;
-        const bool cok = col < kMfL * N2;
-        dbl4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int ks = 0; ks < kMfKA; ++ks) {
-            if (ks < KSA) {
-                const int n1 = 4 * ks + q;
-                const double b = (cok && n1 < N1) ? v[ln * N + N2 * n1 + n2] : 0.0;
-                acc0 = mfma64(fa[0][ks], b, acc0);
-                acc1 = mfma64(fa[1][ks], b, acc1);
-            }
-        }
-        static_assert(kMfL == 2, "one step-A column tile per wave");
-        __syncthreads();  // v is read; Bc overwrites it
-        if (cok) {
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {  // (row tile, pair): k1 = 8 (h/2) + q + 4 (h%2)
-                const dbl4 &acc = (h < 2) ? acc0 : acc1;
-                const int k1 = 8 * (h / 2) + q + 4 * (h % 2);
-                if (k1 < K1) {
-                    const double re = acc[2 * (h % 2)], im = acc[2 * (h % 2) + 1];
-                    Bc[(ln * K1 + k1) * N2 + n2] = cmul(make_double2(re, im), a.wN[n2 * k1]);
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // ---- step C: wave w owns row tile w (k2 = 8w + q, 8w + q + 4), all
-    // kMfL column tiles (columns (line, k1))
-    {
-        double fc[kMfKC];
-#pragma unroll
-        for (int ks = 0; ks < kMfKC; ++ks) fc[ks] = ks < KSC ? a.fC[(wave * KSC + ks) * 64 + lane] : 0.0;
-        dbl4 accs[kMfL];
-#pragma unroll
-        for (int ct = 0; ct < kMfL; ++ct) {
-            const int col = ct * 16 + c16;
-            const int ln = small_div(col, rK1), k1 = col - ln * K1;
-            const bool cok = col < kMfL * K1;
-            const double *Bl = reinterpret_cast<const double *>(Bc + (ln * K1 + k1) * N2);
-            dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int ks = 0; ks < kMfKC; ++ks) {
-                if (ks < KSC) {
-                    const int kk = 4 * ks + q;  // (n2, re/im) = (kk / 2, kk % 2)
-                    const double b = (cok && (kk >> 1) < N2) ? Bl[kk] : 0.0;
-                    acc = mfma64(fc[ks], b, acc);
-                }
-            }
-            accs[ct] = acc;
-        }
-        __syncthreads();  // Bc is read; v overwrites it
-#pragma unroll
-        for (int ct = 0; ct < kMfL; ++ct) {
-            const int col = ct * 16 + c16;
-            const int ln = small_div(col, rK1), k1 = col - ln * K1;
-            const bool cok = col < kMfL * K1;
-            const dbl4 acc = accs[ct];
-            if (cok) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int k2 = 8 * wave + q + 4 * h;
-                    if (k2 < N2) {
-                        const int k = k1 + N1 * k2;
-                        const double2 wv = cmul(a.rot[k], make_double2(acc[2 * h], acc[2 * h + 1]));
-                        v[ln * N + k] = 2.0 * wv.x;
-                        // the mirror N - k of k1 = 0 and k1 = N1/2 is written
-                        // directly by another lane (k1' = k1): one writer each
-                        if (k1 != 0 && 2 * k1 != N1) v[ln * N + N - k] = -2.0 * wv.y;
-                    }
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // per-line output bases, then one element per thread and step (kMfL = 2)
-    long long ob[kMfL];
-#pragma unroll
-    for (int l = 0; l < kMfL; ++l) {
-        const int c = min(line0 + l, a.C - 1);
-        ob[l] = a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
-    }
-    for (int idx = tid; idx < kMfL * N; idx += 256) {
-        const int l = idx >= N ? 1 : 0, kx = idx - l * N;
-        if (line0 + l >= a.C) continue;
-        out[ob[l] + kx] = v[idx];
-    }
-}
-
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_dct_inv_m(DctArgs a, const double *__restrict__ in, double *__restrict__ out) {
-    extern __shared__ double smem[];
-    const int N = a.N, N1 = a.N1, N2 = a.N2, K1h = a.K1h, K1 = K1h + 1;
-    // twiddle indices n2 k1 stay below N (n2 < N2, k1 <= N1/2): no reduction
-    const float rN2 = 1.0f / (float)N2, rK1 = 1.0f / (float)K1;
-    // Vs, Cs (kMfL*K1*N2 complex each) and the output lines o (kMfL*N doubles)
-    // share one LDS area: each step finishes reading its input before a
-    // barrier and then writes its output
-    double2 *Vs = reinterpret_cast<double2 *>(smem);
-    double2 *Cs = Vs;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
-    const int line0 = blockIdx.x * kMfL;
-    // V[k1 + N1 k2] = conj(rot_k) (g[k] - i g[N-k]) / 2 for k1 <= N1/2: Vs[l][k1][k2];
-    // kLd elements per thread are loaded before the first one is used
-    static_assert(kMfL == 2, "line index below assumes two lines per block");
-    const double *gls[kMfL];
-#pragma unroll
-    for (int l = 0; l < kMfL; ++l) {
-        const int c = min(line0 + l, a.C - 1);
-        const int c1 = c % a.C1, c2 = c / a.C1;
-        gls[l] = in + a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
-    }
-    const int nv = kMfL * K1 * N2;
-    for (int i0 = tid; i0 < nv; i0 += 256 * kLd) {
-        double gk[kLd], gm[kLd];
-        double2 rt[kLd];
-#pragma unroll
-        for (int u = 0; u < kLd; ++u) {
-            const int idx = min(i0 + 256 * u, nv - 1);
-            const int l = idx >= K1 * N2 ? 1 : 0, r = idx - l * K1 * N2;
-            const int k1 = small_div(r, rN2), k2 = r - k1 * N2;
-            const int k = k1 + N1 * k2;
-            gk[u] = gls[l][k];
-            gm[u] = gls[l][k == 0 ? 0 : N - k];
-            rt[u] = a.rot[k];
-            if (k == 0) gm[u] = 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < kLd; ++u) {
-            const int idx = i0 + 256 * u;
-            if (idx < nv) Vs[idx] = cmulc(make_double2(0.5 * gk[u], -0.5 * gm[u]), rt[u]);
-        }
-    }
-    const int KSC = (2 * N2 + 3) / 4, KSA = (2 * K1 + 3) / 4;
-    __syncthreads();
-    // ---- step C': wave w owns row tile w (n2 = 8w + q, 8w + q + 4), all
-    // kMfL column tiles (columns (line, k1))
-    {
-        double fc[kMfKC];
-#pragma unroll
-        for (int ks = 0; ks < kMfKC; ++ks) fc[ks] = ks < KSC ? a.iC[(wave * KSC + ks) * 64 + lane] : 0.0;
-        dbl4 accs[kMfL];
-#pragma unroll
-        for (int ct = 0; ct < kMfL; ++ct) {
-            const int col = ct * 16 + c16;
-            const int ln = small_div(col, rK1), k1 = col - ln * K1;
-            const bool cok = col < kMfL * K1;
-            const double *Vl = reinterpret_cast<const double *>(Vs + (ln * K1 + k1) * N2);
-            dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int ks = 0; ks < kMfKC; ++ks) {
-                if (ks < KSC) {
-                    const int kk = 4 * ks + q;  // (k2, re/im) = (kk / 2, kk % 2)
-                    const double b = (cok && (kk >> 1) < N2) ? Vl[kk] : 0.0;
-                    acc = mfma64(fc[ks], b, acc);
-                }
-            }
-            accs[ct] = acc;
-        }
-        __syncthreads();  // Vs is read; Cs overwrites it
-#pragma unroll
-        for (int ct = 0; ct < kMfL; ++ct) {
-            const int col = ct * 16 + c16;
-            const int ln = small_div(col, rK1), k1 = col - ln * K1;
-            const bool cok = col < kMfL * K1;
-            const dbl4 acc = accs[ct];
-            if (cok) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int n2 = 8 * wave + q + 4 * h;
-                    if (n2 < N2)
-                        Cs[(ln * K1 + k1) * N2 + n2] =
-                            cmulc(make_double2(acc[2 * h], acc[2 * h + 1]), a.wN[n2 * k1]);
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // ---- step A': v[N2 n1 + n2] = sum over (k1, re/im) of WA'[n1][.] C~;
-    // wave w owns kMfL / 2 column tiles (columns (line, n2)), both row tiles
-    double *o = smem;  // kMfL*N doubles over Cs, written after Cs is read
-    {
-        double fa[2][kMfKA];
-#pragma unroll
-        for (int ks = 0; ks < kMfKA; ++ks) {
-            fa[0][ks] = ks < KSA ? a.iA[(0 * KSA + ks) * 64 + lane] : 0.0;
-            fa[1][ks] = ks < KSA ? a.iA[(1 * KSA + ks) * 64 + lane] : 0.0;
-        }
-        for (int ct = wave * (kMfL / 2); ct < (wave + 1) * (kMfL / 2); ++ct) {
-            const int col = ct * 16 + c16;
-            const int ln = small_div(col, rN2), n2 = col - ln * N2;
-            const bool cok = col < kMfL * N2;
-            dbl4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int ks = 0; ks < kMfKA; ++ks) {
-                if (ks < KSA) {
-                    const int kk = 4 * ks + q;  // (k1, re/im)
-                    const int k1 = kk >> 1;
-                    const double b =
-                        (cok && k1 < K1) ? reinterpret_cast<const double *>(Cs + (ln * K1 + k1) * N2 + n2)[kk & 1]
-                                         : 0.0;
-                    acc0 = mfma64(fa[0][ks], b, acc0);
-                    acc1 = mfma64(fa[1][ks], b, acc1);
-                }
-            }
-            static_assert(kMfL == 2, "one step-A' column tile per wave");
-            __syncthreads();  // Cs is read; o overwrites it
-            if (cok) {
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {  // n1 = 16 (r / 4) + q + 4 (r % 4)
-                    const int n1 = 16 * (r / 4) + q + 4 * (r % 4);
-                    if (n1 < N1) {
-                        const int n = N2 * n1 + n2;
-                        const int pos = (n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1;
-                        o[ln * N + pos] = (r < 4 ? acc0[r % 4] : acc1[r % 4]) * a.scale;
-                    }
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // per-line output bases, then one element per thread and step (kMfL = 2)
-    long long ob[kMfL];
-#pragma unroll
-    for (int l = 0; l < kMfL; ++l) {
-        const int c = min(line0 + l, a.C - 1);
-        ob[l] = a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
-    }
-    for (int idx = tid; idx < kMfL * N; idx += 256) {
-        const int l = idx >= N ? 1 : 0, n = idx - l * N;
-        if (line0 + l >= a.C) continue;
-        out[ob[l] + n] = o[idx];
     }
 }
 
@@ -2082,7 +1973,6 @@ void check_launch() {
     }
 }
 
-constexpr int kDctLines = 2;
 constexpr int kZRows = 16, kZPre = 4;
 
 // the matrix-core z DFT with RT row tiles (RT = rt, one instantiation per
@@ -2143,47 +2033,51 @@ void zdft_launch(Handle &h, int kid, bool forward, const double *in, double *out
     zdft_raw(h.stream, z, C, (long long)C, forward, in, out);
 }
 
-void dct_launch(Handle &h, int kid, const DctArgs &a, bool forward, const double *in, double *out,
+// lines per block of the x transform past the SMALL shapes: 16 columns of step
+// C (line, k1), as far as 80 KB of LDS (two blocks per CU) hold them; fewer lines
+// leave columns empty and read the tables more often (at N = 129, 3774 lines, 8,
+// 3 and 1 lines per block took 22, 25 and 40 us)
+int dct_block_lines(const DctArgs &a) {
+    const int K1 = a.K1h + 1;
+    const size_t line = sizeof(double) * a.N + sizeof(double2) * K1 * dct_ld(a.N2);
+    return std::max(1, std::min(std::max(2, (15 + K1) / K1), (int)(81920 / line)));
+}
+
+void dct_launch(Handle &h, int kid, DctArgs a, bool forward, const double *in, double *out,
                 const Field3 *div = nullptr, const BcPlanes<double> *bcp = nullptr) {
     ProfScope ps(h, kid);
     const BcPlanes<double> bc = bcp ? *bcp : BcPlanes<double>{};
-    const int K1 = a.K1h + 1;
-    if (a.fA) {
-        // matrix-core kernels (the shape was checked with the tables)
-        // one shared area per block: the lines (kMfL*N doubles) and the
-        // intermediate spectra (kMfL*K1*N2 complex) in turn
-        const size_t lds = std::max(sizeof(double) * (size_t)kMfL * a.N, sizeof(double2) * (size_t)kMfL * K1 * a.N2);
-        if (lds > 163840) {
-            last_error() = "x transform length too large for the LDS-resident DCT (N = " + std::to_string(a.N) + ")";
-            throw ArgError();
-        }
-        const dim3 grid((a.C + kMfL - 1) / kMfL);
-        if (forward && div)
-            hipLaunchKernelGGL(k_dct_fwd_m<true>, grid, dim3(256), lds, h.stream, a, h.d, h.m, bc, div->u, div->v,
-                               div->w, out);
-        else if (forward)
-            hipLaunchKernelGGL(k_dct_fwd_m<false>, grid, dim3(256), lds, h.stream, a, h.d, h.m, bc, in, nullptr,
-                               nullptr, out);
-        else
-            hipLaunchKernelGGL(k_dct_inv_m, grid, dim3(256), lds, h.stream, a, in, out);
-        check_launch();
-        return;
-    }
-    const size_t lds = (forward ? sizeof(double) : sizeof(double2)) * (size_t)kDctLines * a.N +
-                       sizeof(double2) * ((size_t)kDctLines * K1 * a.N2 + a.N1 + a.N2);
-    if (lds > 65536) {
+    const int K1 = a.K1h + 1, ld = dct_ld(a.N2);
+    const bool small = a.N1 <= 31 && a.N2 <= 31;
+    a.LB = small ? 2 : dct_block_lines(a);
+    const size_t lines = sizeof(double) * dct_lines(a.LB, a.N), spec = sizeof(double2) * (size_t)a.LB * K1 * ld;
+    // the inverse past the SMALL shapes: V (an area that also holds the lines) and C~
+    const size_t lds = small ? std::max(lines, spec) : (forward ? lines + spec : 2 * std::max(lines, spec));
+    if (lds > 163840) {
         last_error() = "x transform length too large for the LDS-resident DCT (N = " + std::to_string(a.N) + ")";
         throw ArgError();
     }
-    const dim3 grid((a.C + kDctLines - 1) / kDctLines);
-    if (forward && div)
-        hipLaunchKernelGGL((k_dct_fwd<kDctLines, true>), grid, dim3(256), lds, h.stream, a, h.d, h.m,
-                           bc, div->u, div->v, div->w, out);
-    else if (forward)
-        hipLaunchKernelGGL((k_dct_fwd<kDctLines, false>), grid, dim3(256), lds, h.stream, a, h.d, h.m, bc, in,
-                           nullptr, nullptr, out);
-    else
-        hipLaunchKernelGGL(k_dct_inv<kDctLines>, grid, dim3(256), lds, h.stream, a, in, out);
+    const dim3 grid((a.C + a.LB - 1) / a.LB);
+    // four waves per block, or eight where the blocks do not fill the chip (at 511
+    // points and 12288 lines four take 86 us and eight 103, at 129 points and
+    // 3774 lines 19 and 17)
+    const dim3 block(small ? 128 : ((int)grid.x < 4 * h.n_cu ? 512 : 256));
+    auto fwd = [&](auto kern) {
+        if (div)
+            hipLaunchKernelGGL(kern, grid, block, lds, h.stream, a, h.d, h.m, bc, div->u, div->v, div->w, out);
+        else
+            hipLaunchKernelGGL(kern, grid, block, lds, h.stream, a, h.d, h.m, bc, in, nullptr, nullptr, out);
+    };
+    if (forward) {
+        if (small)
+            div ? fwd(k_dct_fwd_m<true, true>) : fwd(k_dct_fwd_m<false, true>);
+        else
+            div ? fwd(k_dct_fwd_m<true, false>) : fwd(k_dct_fwd_m<false, false>);
+    } else if (small) {
+        hipLaunchKernelGGL(k_dct_inv_m<true>, grid, block, lds, h.stream, a, in, out);
+    } else {
+        hipLaunchKernelGGL(k_dct_inv_m<false>, grid, block, lds, h.stream, a, in, out);
+    }
     check_launch();
 }
 
@@ -2397,15 +2291,15 @@ void launch_poisson(Handle &h, double *phi, const Field3 *div, const BcPlanes<do
     da.K1h = h.dct_n1 / 2;
     da.C1 = NM;
     da.C = NM * M;
-    da.w1 = reinterpret_cast<const double2 *>(h.dct_w1);
-    da.w2 = reinterpret_cast<const double2 *>(h.dct_w2);
-    da.wN = reinterpret_cast<const double2 *>(h.dct_wN);
-    da.rot = reinterpret_cast<const double2 *>(h.dct_rot);
-    if (h.dct_mfma) {
-        da.fA = h.dct_mf + h.dct_mf_off[0];
-        da.fC = h.dct_mf + h.dct_mf_off[1];
-        da.iC = h.dct_mf + h.dct_mf_off[2];
-        da.iA = h.dct_mf + h.dct_mf_off[3];
+    {
+        const int K1 = da.K1h + 1;
+        const double2 *t = reinterpret_cast<const double2 *>(h.dct_tab);
+        da.rot = t;
+        da.twA = da.rot + N;
+        da.twC = da.twA + K1 * da.N2;
+        da.t1 = da.twC + K1 * da.N2;
+        da.t1i = da.t1 + dct_frag(da.N1);
+        da.t2 = da.t1i + dct_frag(da.N1);
     }
     da.in_base = fidx(d, 1, 1, 1);
     da.in_c1 = d.sx;

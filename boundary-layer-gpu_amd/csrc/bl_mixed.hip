@@ -498,7 +498,7 @@ void zdft_mx_launch(Handle &h, int kid, int rt, int M, int C, long long plane, b
 struct XArgs {
     int N, N1, N2, K1h, NP, C1, C, M;
     const u16x8 *fA, *fC, *iC, *iA;  // [(rt * KS + ks) * 64 + lane][hi, lo]
-    const float2 *wN, *rot;          // e^{-2 pi i q/N}, e^{-i pi k/(2N)}
+    const float2 *twA, *twC, *rot;   // W_N^{n2 k1} as [k1][n2] and [n2][k1], e^{-i pi k/(2N)}
     float scale;                     // inverse: 1/(N M)
 };
 
@@ -667,7 +667,7 @@ __global__ __launch_bounds__(256) void k_xfwd_mx(Dims d, Metrics mt, XArgs a, co
                 const int k1 = 8 * (h / 2) + 2 * q + (h % 2);
                 if (k1 < K1)
                     Bc[(ln * K1 + k1) * N2 + n2] =
-                        cmulf(make_float2(acc[2 * (h % 2)], acc[2 * (h % 2) + 1]), a.wN[n2 * k1]);
+                        cmulf(make_float2(acc[2 * (h % 2)], acc[2 * (h % 2) + 1]), a.twA[k1 * N2 + n2]);
             }
         }
     }
@@ -739,8 +739,9 @@ __global__ __launch_bounds__(256) void k_xinv_mx(Dims d, XArgs a, const float *_
 #pragma unroll
         for (int u = 0; u < kLdx; ++u) {
             const int idx = min(i0 + 256 * u, nv - 1);
+            // k1 fastest: runs of K1 consecutive entries of the line per wave
             const int l = idx >= K1 * N2 ? 1 : 0, r = idx - l * K1 * N2;
-            const int k1 = small_div(r, rN2), k2 = r - k1 * N2;
+            const int k2 = small_div(r, rK1), k1 = r - k2 * K1;
             const int k = k1 + N1 * k2;
             gk[u] = gls[l][k];
             gm[u] = gls[l][k == 0 ? 0 : N - k];
@@ -750,7 +751,10 @@ __global__ __launch_bounds__(256) void k_xinv_mx(Dims d, XArgs a, const float *_
 #pragma unroll
         for (int u = 0; u < kLdx; ++u) {
             const int idx = i0 + 256 * u;
-            if (idx < nv) Vs[idx] = cmulcf(make_float2(0.5f * gk[u], -0.5f * gm[u]), rt[u]);
+            const int l = idx >= K1 * N2 ? 1 : 0, r = idx - l * K1 * N2;
+            const int k2 = small_div(r, rK1), k1 = r - k2 * K1;
+            if (idx < nv)
+                Vs[(l * K1 + k1) * N2 + k2] = cmulcf(make_float2(0.5f * gk[u], -0.5f * gm[u]), rt[u]);
         }
     }
     __syncthreads();
@@ -780,7 +784,7 @@ __global__ __launch_bounds__(256) void k_xinv_mx(Dims d, XArgs a, const float *_
                 const int n2 = 8 * wave + 2 * q + h;
                 if (n2 < N2)
                     Cs[(ln * K1 + k1) * N2 + n2] =
-                        cmulcf(make_float2(acc[2 * h], acc[2 * h + 1]), a.wN[n2 * k1]);
+                        cmulcf(make_float2(acc[2 * h], acc[2 * h + 1]), a.twC[n2 * K1 + k1]);
             }
         }
     }
@@ -1123,14 +1127,17 @@ void build_mixed(Handle &h) {
                 const auto w = cis((long long)nn1 * k1, n1);
                 return c * (pin == 0 ? w.first : w.second);
             });
-            std::vector<float> tw(4 * (size_t)N);
-            for (int q = 0; q < N; ++q) {
-                const auto w = cis(q, N), r = cis(q, 4LL * N);
-                tw[2 * q] = (float)w.first;
-                tw[2 * q + 1] = (float)w.second;
-                tw[2 * N + 2 * q] = (float)r.first;
-                tw[2 * N + 2 * q + 1] = (float)r.second;
-            }
+            // twA [k1][n2], twC [n2][k1] (n2 k1 < N), rot
+            std::vector<float> tw;
+            auto push = [&](std::pair<long double, long double> w) {
+                tw.push_back((float)w.first);
+                tw.push_back((float)w.second);
+            };
+            for (int k1 = 0; k1 < k1n; ++k1)
+                for (int nn = 0; nn < n2; ++nn) push(cis((long long)nn * k1, N));
+            for (int nn = 0; nn < n2; ++nn)
+                for (int k1 = 0; k1 < k1n; ++k1) push(cis((long long)nn * k1, N));
+            for (int q = 0; q < N; ++q) push(cis(q, 4LL * N));
             const size_t nb = (fA.size() + fC.size() + iC.size() + iA.size()) * sizeof(uint16_t) + tw.size() * 4;
             BL_HIP(hipMalloc(&h.mx2, nb));
             char *base = reinterpret_cast<char *>(h.mx2);
@@ -1182,8 +1189,9 @@ void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const BcP
         xa.fC = reinterpret_cast<const u16x8 *>(h.x2_fC);
         xa.iC = reinterpret_cast<const u16x8 *>(h.x2_iC);
         xa.iA = reinterpret_cast<const u16x8 *>(h.x2_iA);
-        xa.wN = reinterpret_cast<const float2 *>(h.x2_tw);
-        xa.rot = reinterpret_cast<const float2 *>(h.x2_tw) + N;
+        xa.twA = reinterpret_cast<const float2 *>(h.x2_tw);
+        xa.twC = xa.twA + (xa.K1h + 1) * xa.N2;
+        xa.rot = xa.twC + (xa.K1h + 1) * xa.N2;
         xa.scale = (float)(1.0 / ((double)N * (double)M));
     }
     const int K1 = h.dct_n1 / 2 + 1, N2 = N / h.dct_n1;

@@ -152,3 +152,28 @@ def test_rhs_march_chunks(shape, precision):
     tol = 1e-5 if precision else 1e-12
     for a, b in zip(s.rhs(), ref):
         assert np.linalg.norm(a - b) < tol * np.linalg.norm(b)
+
+
+# the x transform: lengths of one factor pair each side of the 31 x 31 limit of
+# the shared-area kernel, primes (one column per line), even factors (a pair
+# index that is its own mirror), 32 x 32, and line counts that leave a part of a
+# block; with many and with few lines (four or eight waves).  Solution against
+# the oracle to the Poisson parity tests' 2e-11.
+@pytest.mark.parametrize("n,ny,nz", [(4, 5, 6), (7, 4, 5), (22, 24, 10), (31, 9, 7), (127, 6, 8), (129, 75, 53), (197, 5, 6),
+                                     (511, 12, 9), (961, 7, 6), (992, 6, 8), (1024, 5, 7), (146, 60, 66)])
+def test_x_transform_lengths(n, ny, nz):
+    say("x transform", n, ny, nz)
+    rng = np.random.default_rng(n)
+    nx = n + 2
+    x = 1.0 + 0.001 * np.arange(nx)
+    y = np.cumsum(np.r_[0, 0.002 + 0.0005 * rng.random(ny - 1)])
+    z = 0.0015 * np.arange(nz)
+    o = orc.Oracle(x, y, z, 1e-5)
+    s = solver(x, y, z)
+    r = np.asfortranarray(rng.standard_normal((nx + 1, ny + 1, nz + 1)))
+    ref, got = o.poisson(r), s.poisson(r)
+    I = (slice(1, n + 1), slice(1, ny), slice(1, nz - 1))
+    err = np.linalg.norm((got - ref)[I]) / np.linalg.norm(ref[I])
+    say("err", err)
+    assert err < 2e-11
+    s.close()
