@@ -118,50 +118,38 @@ double *field_dev(Handle &h, int field) {
     }
 }
 
-// strided copies between a host array of extent (n1, n2, n3) and the padded
-// device layout; element type E on the device
-template <class E>
-void copy_in(Handle &h, E *dev, const E *host, int n1, int n2, int n3) {
-    const Dims &d = h.d;
-    for (int k = 0; k < n3; ++k)
-        BL_HIP(hipMemcpy2DAsync(dev + (size_t)k * d.sxy, (size_t)d.sx * sizeof(E), host + (size_t)k * n1 * n2,
-                                (size_t)n1 * sizeof(E), (size_t)n1 * sizeof(E), n2, hipMemcpyHostToDevice,
-                                h.stream));
-    BL_HIP(hipStreamSynchronize(h.stream));
-}
-
-template <class E>
-void copy_out(Handle &h, E *host, const E *dev, int n1, int n2, int n3) {
-    const Dims &d = h.d;
-    BL_HIP(hipStreamSynchronize(h.stream));
-    for (int k = 0; k < n3; ++k)
-        BL_HIP(hipMemcpy2DAsync(host + (size_t)k * n1 * n2, (size_t)n1 * sizeof(E), dev + (size_t)k * d.sxy,
-                                (size_t)d.sx * sizeof(E), (size_t)n1 * sizeof(E), n2, hipMemcpyDeviceToHost,
-                                h.stream));
-    BL_HIP(hipStreamSynchronize(h.stream));
-}
-
-// host FP64 arrays <-> device fields (rounded to float in mixed precision)
 size_t elem_size(const Handle &h) { return h.precision == BL_PREC_MIXED ? sizeof(float) : sizeof(double); }
 
+// host FP64 arrays of extent (n1, n2, n3) <-> padded device fields (rounded to
+// float in mixed precision).  The planes pass through the x transform's work
+// array, which no call leaves data in, unpadded and in FP64, as many at a time as
+// it holds, so that one contiguous copy crosses to the host: a 2-D copy per
+// plane costs about 100 us each whatever its size, and the fields of a 24x16x8
+// grid took 3 ms to read.
+int stage_planes(const Handle &h, int n1, int n2, int n3) {
+    return (int)std::max(1LL, std::min((long long)n3, h.n_stage / ((long long)n1 * n2)));
+}
+
 void copy_to_device(Handle &h, double *dev, const double *host, int n1, int n2, int n3) {
-    if (h.precision != BL_PREC_MIXED) {
-        copy_in(h, dev, host, n1, n2, n3);
-        return;
+    const int np = stage_planes(h, n1, n2, n3);
+    for (int k = 0; k < n3; k += np) {
+        const int n = std::min(np, n3 - k);
+        BL_HIP(hipMemcpyAsync(h.T1, host + (size_t)k * n1 * n2, sizeof(double) * n1 * n2 * n, hipMemcpyHostToDevice,
+                              h.stream));
+        launch_unpack(h, h.T1, dev, n1, n2, k, n);
     }
-    std::vector<float> tmp((size_t)n1 * n2 * n3);
-    for (size_t q = 0; q < tmp.size(); ++q) tmp[q] = (float)host[q];
-    copy_in(h, reinterpret_cast<float *>(dev), tmp.data(), n1, n2, n3);
+    BL_HIP(hipStreamSynchronize(h.stream));
 }
 
 void copy_to_host(Handle &h, double *host, const double *dev, int n1, int n2, int n3) {
-    if (h.precision != BL_PREC_MIXED) {
-        copy_out(h, host, dev, n1, n2, n3);
-        return;
+    const int np = stage_planes(h, n1, n2, n3);
+    for (int k = 0; k < n3; k += np) {
+        const int n = std::min(np, n3 - k);
+        launch_pack(h, dev, h.T1, n1, n2, k, n);
+        BL_HIP(hipMemcpyAsync(host + (size_t)k * n1 * n2, h.T1, sizeof(double) * n1 * n2 * n, hipMemcpyDeviceToHost,
+                              h.stream));
     }
-    std::vector<float> tmp((size_t)n1 * n2 * n3);
-    copy_out(h, tmp.data(), reinterpret_cast<const float *>(dev), n1, n2, n3);
-    for (size_t q = 0; q < tmp.size(); ++q) host[q] = (double)tmp[q];
+    BL_HIP(hipStreamSynchronize(h.stream));
 }
 
 void check_config(const bl_config *c) {
@@ -438,18 +426,21 @@ void build(Handle &h, const bl_config *c) {
         h.smag_c = dmalloc(cj.size());
         upload_vec(h.smag_c, cj, h.stream);
     }
-    const size_t nspec = (size_t)d.N * d.NM * d.M;
+    // one plane at least: T1 also stages the transfers of fields
+    const size_t nspec = std::max((size_t)d.N * d.NM * d.M, (size_t)d.nxg * d.nyg);
     if (h.precision == BL_PREC_MIXED) {
         // FP32 spectra with kx stride NP; T1 doubles as the FP64 Thomas scratch
         build_mixed(h);
         const size_t nsf = (size_t)h.NP * d.NM * d.M;
         const size_t t1 = std::max(nspec, (nsf + 1) / 2), s1 = (nsf + 1) / 2;
         h.T1 = dmalloc(t1);
+        h.n_stage = (long long)t1;
         h.S = dmalloc(s1);
         BL_HIP(hipMemsetAsync(h.T1, 0, t1 * sizeof(double), h.stream));
         BL_HIP(hipMemsetAsync(h.S, 0, s1 * sizeof(double), h.stream));
     } else {
         h.T1 = dmalloc(nspec);
+        h.n_stage = (long long)nspec;
         h.S = dmalloc(nspec);
     }
 

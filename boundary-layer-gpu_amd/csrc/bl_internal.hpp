@@ -278,6 +278,7 @@ struct Handle {
     int cl_nblk;
     int cl_ready;
     double *T1, *S;  // transform intermediates: [m][j][kx] and [q][j][kx]
+    long long n_stage = 0;           // doubles of T1, which also stages field transfers
     int dct_n1;                      // x-DCT factorisation N = dct_n1 * (N / dct_n1)
     int lda_zt;                      // leading dimension of the z cos/sin tables
     double *zc, *zs;                 // z tables cos/sin(2 pi k m / M), [m][k]
@@ -453,6 +454,10 @@ long long stats_size(const Dims &d);
 // (device, stats_size doubles): Umean, Vmean, Wmean, U2mean, V2mean, W2mean,
 // UVmean, Pmean, P2mean as (nx, ny), then nu_t_mean (nxg, nyg)
 void launch_statistics(Handle &h, const Field3 &f, double *out);
+// n planes from k0 of a padded device field (double, or float in mixed
+// precision) to or from an unpadded FP64 array of n1 x n2 planes on the device
+void launch_pack(Handle &h, const double *field, double *dst, int n1, int n2, int k0, int n);
+void launch_unpack(Handle &h, const double *src, double *field, int n1, int n2, int k0, int n);
 // pack the current U, V, W, P, nu_t on the solver's stream and copy them to
 // pinned host memory on the copy stream
 void snapshot_begin(Handle &h);

@@ -95,23 +95,44 @@ __global__ __launch_bounds__(256) void k_statistics_edges(Dims d, double *__rest
     if (t < d.nxg) ntm[t + (long long)d.nxg * d.ny] = 0.0;
 }
 
-// padded device field (element T) -> unpadded FP64 array (n1, n2, n3)
+// planes k0.. of a padded device field (element T) -> unpadded FP64 array of
+// n1 x n2 planes, and back
 template <class T>
 __global__ __launch_bounds__(256) void k_pack(Dims d, const T *__restrict__ src, double *__restrict__ dst, int n1,
-                                              int n2, int n3) {
+                                              int n2, int k0) {
     const int i = blockIdx.x * 256 + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
-    if (i >= n1 || j >= n2 || k >= n3) return;
-    dst[i + (long long)n1 * (j + (long long)n2 * k)] = (double)src[fidx(d, i, j, k)];
+    if (i >= n1) return;
+    dst[i + (long long)n1 * (j + (long long)n2 * k)] = (double)src[fidx(d, i, j, k0 + k)];
 }
-
 template <class T>
-void pack(Handle &h, const double *src, double *dst, int n1, int n2, int n3) {
-    hipLaunchKernelGGL(k_pack<T>, dim3((n1 + 255) / 256, n2, n3), dim3(256), 0, h.stream, h.d,
-                       reinterpret_cast<const T *>(src), dst, n1, n2, n3);
-    check_launch();
+__global__ __launch_bounds__(256) void k_unpack(Dims d, const double *__restrict__ src, T *__restrict__ dst, int n1,
+                                                int n2, int k0) {
+    const int i = blockIdx.x * 256 + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
+    if (i >= n1) return;
+    dst[fidx(d, i, j, k0 + k)] = (T)src[i + (long long)n1 * (j + (long long)n2 * k)];
 }
 
 }  // namespace
+
+void launch_pack(Handle &h, const double *field, double *dst, int n1, int n2, int k0, int n) {
+    const dim3 grid((n1 + 255) / 256, n2, n);
+    if (h.precision == BL_PREC_MIXED)
+        hipLaunchKernelGGL(k_pack<float>, grid, dim3(256), 0, h.stream, h.d, reinterpret_cast<const float *>(field),
+                           dst, n1, n2, k0);
+    else
+        hipLaunchKernelGGL(k_pack<double>, grid, dim3(256), 0, h.stream, h.d, field, dst, n1, n2, k0);
+    check_launch();
+}
+
+void launch_unpack(Handle &h, const double *src, double *field, int n1, int n2, int k0, int n) {
+    const dim3 grid((n1 + 255) / 256, n2, n);
+    if (h.precision == BL_PREC_MIXED)
+        hipLaunchKernelGGL(k_unpack<float>, grid, dim3(256), 0, h.stream, h.d, src, reinterpret_cast<float *>(field),
+                           n1, n2, k0);
+    else
+        hipLaunchKernelGGL(k_unpack<double>, grid, dim3(256), 0, h.stream, h.d, src, field, n1, n2, k0);
+    check_launch();
+}
 
 long long stats_size(const Dims &d) { return 9LL * d.nx * d.ny + (long long)d.nxg * d.nyg; }
 
@@ -161,10 +182,7 @@ void snapshot_begin(Handle &h) {
     const Field3 &f = h.buf[h.icur];
     const double *src[5] = {f.u, f.v, f.w, h.P, h.nu_t};
     for (int a = 0; a < 5; ++a) {
-        if (h.precision == BL_PREC_MIXED)
-            pack<float>(h, src[a], h.snap_dev + h.snap_off[a], ext[a][0], ext[a][1], ext[a][2]);
-        else
-            pack<double>(h, src[a], h.snap_dev + h.snap_off[a], ext[a][0], ext[a][1], ext[a][2]);
+        launch_pack(h, src[a], h.snap_dev + h.snap_off[a], ext[a][0], ext[a][1], 0, ext[a][2]);
     }
     BL_HIP(hipEventRecord(h.snap_packed, h.stream));
     BL_HIP(hipStreamWaitEvent(h.copy_stream, h.snap_packed, 0));

@@ -177,3 +177,22 @@ def test_x_transform_lengths(n, ny, nz):
     say("err", err)
     assert err < 2e-11
     s.close()
+
+
+# transfers pass through a work array of (nx-2)(ny-1)(nz-2) values, planes of
+# up to (nx+1)(ny+1): grids where it holds one plane, a part of the planes,
+# and nearly all of them; both directions, exact (FP32 storage: rounded once)
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(5, 4, 5), (6, 5, 40), (24, 16, 8), (300, 30, 20)])
+def test_field_transfers(shape, precision):
+    say("transfers", shape, precision)
+    x, y, z, U, V, W = random_case(1, *shape)
+    s = solver(x, y, z, precision=precision)
+    rng = np.random.default_rng(4)
+    fields = [np.asfortranarray(rng.standard_normal(sh)) for sh in s.shapes]
+    for f, a in enumerate(fields):
+        s.upload(f, a)
+    for f, a in enumerate(fields):
+        want = a.astype(np.float32).astype(np.float64) if precision else a
+        np.testing.assert_array_equal(s.download(f), want)
+    s.close()
