@@ -20,9 +20,9 @@ class is bracketed (the events of every class would add ~0.3 ms to a step),
 and `roofline` is its average launch time there.  `cpu_baseline` is the
 FP64 C oracle timed on this host at the full size (all cores this process may
 use), with a one-core estimate from a z-slab.
-`mixed` is the same workload in mixed precision (FP32 fields, split-BF16x3
-MFMA transforms, FP64 Thomas / mass flux / statistics): its ns/cell/step, the
-MFMA rate of its x-transform GEMM, and the relative L2 difference of u, v, w,
+`mixed` is the same workload in mixed precision (FP32 fields, FP32 x and
+split-BF16x3 z MFMA transforms, FP64 Thomas / mass flux / statistics): its
+ns/cell/step, the MFMA rates of its transforms, and the relative L2 difference of u, v, w,
 p and Cf from the FP64 run after the same warm-up + timed steps.
 `les` is the learned-closure LES against dynamic Smagorinsky (both in the
 mixed-precision form) on an LES grid that a DNS refines by (4, 2, 4): the
@@ -230,31 +230,39 @@ def dct_factor(N):
     return n1, N // n1
 
 
+FP32_MFMA_PEAK_TFLOPS = 157.3
+
+
 def mixed_mfma(prof, nx, ny, nz):
-    """MFMA rates of the mixed path's transform kernels: BF16 flops issued
-    (16x16x32 MFMAs x 16384 flop, three per split product, padded tiles) per
-    launch / launch time.  x: two short DFTs per line pair (k_xfwd_mx, 2 lines
-    per block: step A 4 column tiles x 2 row tiles x 1 K step, step C 4 row
-    tiles x 2 column tiles x 2 K steps; the divergence is fused in); z: the
-    dense 191-point DFT GEMM (256 x 128 tiles, K padded to 64)."""
+    """MFMA rates of the mixed path's transform kernels: flops issued per
+    launch / launch time.  x: two short folded DFTs per line pair in FP32
+    (k_dct_fwd_m<float>, 16x16x4 MFMAs of 2048 flop; per two lines 4 column
+    tiles x 2 products of step A and 2 column tiles x 4 products of step C;
+    the divergence is fused in), for factors up to 31; z: the folded DFT
+    (k_zdft_mx, 16x16x32 BF16 MFMAs of 16384 flop, cos and sin products, three
+    per split product) up to 191 points, the dense split-BF16 GEMM beyond."""
     N, M, NM = nx - 2, nz - 2, ny - 1
     NP = -(-N // 32) * 32
     out = {}
     n1, n2 = dct_factor(N)
-    if n1 <= 32 and n1 // 2 + 1 <= 16 and n2 <= 32:
-        blocks = -(-(NM * M) // 2)
-        mfmas = blocks * (4 * 2 * 1 + 4 * 2 * 2) * 3
-        x_issued = mfmas * 16384.0
+    k1, k2, kz = n1 // 2 + 1, n2 // 2 + 1, M // 2 + 1
+    issued = {}
+    if n1 <= 31 and n2 <= 31:
+        issued["xform_x_fwd"] = ("fp32", -(-(NM * M) // 2) * (8 * -(-k1 // 4) + 8 * -(-k2 // 4)) * 2048.0,
+                                 FP32_MFMA_PEAK_TFLOPS)
+    if kz <= 96:
+        issued["xform_z_fwd"] = ("bf16", -(-(NM * NP) // 16) * -(-kz // 16) * -(-kz // 32) * 6 * 16384.0,
+                                 BF16_PEAK_TFLOPS)
     else:
-        x_issued = 3 * 2.0 * (-(-N // 128) * 128) * NP * (-(-(NM * M) // 128) * 128)
-    z_issued = 3 * 2.0 * 256 * (-(-M // 64) * 64) * (-(-(NM * NP) // 128) * 128)
-    for name, issued in (("xform_x_fwd", x_issued), ("xform_z_fwd", z_issued)):
+        issued["xform_z_fwd"] = ("bf16", 3 * 2.0 * 256 * (-(-M // 64) * 64) * (-(-(NM * NP) // 128) * 128),
+                                 BF16_PEAK_TFLOPS)
+    for name, (kind, flop, peak) in issued.items():
         if name not in prof or prof[name][1] == 0:
             continue
         avg_s = prof[name][0] / prof[name][1] * 1e-3
-        ach = issued / avg_s / 1e12
-        out[name] = dict(bf16_tflops_issued=ach, peak=BF16_PEAK_TFLOPS, frac=ach / BF16_PEAK_TFLOPS,
-                         avg_launch_ms=prof[name][0] / prof[name][1])
+        ach = flop / avg_s / 1e12
+        out[name] = {kind + "_tflops_issued": ach, "peak": peak, "frac": ach / peak,
+                     "avg_launch_ms": prof[name][0] / prof[name][1]}
     return out
 
 

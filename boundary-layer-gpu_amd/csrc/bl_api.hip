@@ -502,11 +502,21 @@ void build(Handle &h, const bl_config *c) {
                         push({c, s});
                     }
         };
-        frag(n1, false);
-        frag(n1, true);
-        frag(n2, false);
-        h.dct_tab = dmalloc(tab.size());
-        upload_vec(h.dct_tab, tab, h.stream);
+        if (h.precision == BL_PREC_FP64 || h.mx_two) {
+            frag(n1, false);
+            frag(n1, true);
+            frag(n2, false);
+        }
+        if (h.precision == BL_PREC_FP64) {
+            double *t = dmalloc(tab.size());
+            h.dct_tab = t;
+            upload_vec(t, tab, h.stream);
+        } else {
+            const std::vector<float> tf(tab.begin(), tab.end());
+            h.dct_tab = dmalloc((tf.size() + 1) / 2);
+            BL_HIP(hipMemcpyAsync(h.dct_tab, tf.data(), tf.size() * sizeof(float), hipMemcpyHostToDevice, h.stream));
+            BL_HIP(hipStreamSynchronize(h.stream));
+        }
     }
     // z cos/sin tables, symmetric in (k, m): lda covers the padded row blocks
     {
@@ -604,7 +614,7 @@ void free_all(Handle &h) {
         f(h.buf[b].w);
     }
     for (void *p : {(void *)h.F1.u, (void *)h.F1.v, (void *)h.F1.w, (void *)h.P, (void *)h.phi,
-                    (void *)h.nu_t, (void *)h.T1, (void *)h.S, (void *)h.dct_tab, h.mx2, (void *)h.zc, (void *)h.zs, (void *)h.zf, (void *)h.bc_extra, (void *)h.bc_mem, (void *)h.lund_mem, (void *)h.wm_mem, (void *)h.lu_dl, (void *)h.lu_dp, (void *)h.lu_du,
+                    (void *)h.nu_t, (void *)h.T1, (void *)h.S, h.dct_tab, (void *)h.zc, (void *)h.zs, (void *)h.zf, (void *)h.bc_extra, (void *)h.bc_mem, (void *)h.lund_mem, (void *)h.wm_mem, (void *)h.lu_dl, (void *)h.lu_dp, (void *)h.lu_du,
                     (void *)h.lu00, (void *)h.th_co,
                     (void *)h.scal, (void *)h.red, (void *)h.dsm, (void *)h.smag_c, h.mem_grid, h.mem_gridf, (void *)h.mx_tab, (void *)h.zmf,
                     (void *)h.p00, (void *)h.inc1, (void *)h.stats, (void *)h.cl_w, (void *)h.cl_b, (void *)h.cl_cnt})

@@ -202,6 +202,73 @@ struct DivLine {
     __device__ __forceinline__ double at(int n) const { return div(load(n), n); }
 };
 
+// The first stage's pressure source in the mixed path: the divergence of the
+// stage's increment U* - Un, taken as c0 F1 on the faces the stage update
+// moves and as the FP64 boundary increments (Handle::inc1) or the difference
+// of the stored values on the boundary faces, instead of div U*.  In exact
+// arithmetic the two agree (div Un is zero after the previous projection);
+// in FP32 storage div Un is rounding noise of order eps |u| / dx, which the
+// projection would divide by dt a11 into the recorded pressure.
+struct IncSrc {
+    const float *fu, *fv, *fw;     // F1 of the stage
+    const float *vn;               // V at the step start
+    const double *inc1;            // Handle::inc1
+    double c0;                     // dt a11
+};
+
+// divergence of the first stage's increment U* - Un at cell (i, j, k), p its
+// index (the IncSrc form of the pseudo-pressure rhs): c0 F1 on the faces the
+// stage update moves, the FP64 increments on the inflow and outflow U faces
+// (plus the mass-flux shift on the outflow), the difference of the stored
+// values on the wall and top V faces; the W face below plane 1 is the
+// periodic image of plane nz-2
+// (pointers, scales and ends fixed per line, as DivLine)
+struct IncLine {
+    const float *u, *vt, *vb, *wt, *wb;  // F1, or V of the stage on the top and wall faces
+    const float *nt, *nb;                // there: V at the step start (else null)
+    const double *rdx;
+    double c0, ry, rz, ul, ur;
+    int last;
+    __device__ __forceinline__ IncLine(const Dims &d, const Metrics &m, const IncSrc &s, const BcPlanes<float> &bc,
+                                       int c1, int c2) {
+        const long long p = fidx(d, 1, c1 + 1, c2 + 1), npl = (long long)d.nyg * d.nzg;
+        const long long pl = c1 + 1 + (long long)d.nyg * (c2 + 1);
+        u = s.fu + p;
+        vt = s.fv + p;
+        vb = vt - d.sx;
+        wt = s.fw + p;
+        wb = c2 == 0 ? wt + d.sxy * (d.nz - 3) : wt - d.sxy;
+        nt = nb = nullptr;
+        if (c1 == d.NM - 1) {
+            vt = bc.vtop + 1;
+            nt = s.vn + p;
+        }
+        if (c1 == 0) {
+            vb = bc.vwall + bc.wld * (c2 + 1) + 1;
+            nb = s.vn + p - d.sx;
+        }
+        rdx = m.rdx + 1;
+        ry = m.rdy[c1 + 1];
+        rz = m.rdz[c2 + 1];
+        c0 = s.c0;
+        ul = s.inc1[pl];
+        ur = s.inc1[npl + pl] + s.inc1[2 * npl];
+        last = d.N - 1;
+    }
+    struct Raw {
+        float u, l, vt, vb, wt, wb;
+        double rdx;
+    };
+    __device__ __forceinline__ Raw load(int n) const { return {u[n], u[n - 1], vt[n], vb[n], wt[n], wb[n], rdx[n]}; }
+    __device__ __forceinline__ double div(const Raw &a, int n) const {
+        const double r = n == last ? ur : c0 * (double)a.u, l = n == 0 ? ul : c0 * (double)a.l;
+        const double t = nt ? (double)a.vt - (double)nt[n] : c0 * (double)a.vt;
+        const double b = nb ? (double)a.vb - (double)nb[n] : c0 * (double)a.vb;
+        return (r - l) * a.rdx + (t - b) * ry + (c0 * (double)a.wt - c0 * (double)a.wb) * rz;
+    }
+    __device__ __forceinline__ double at(int n) const { return div(load(n), n); }
+};
+
 // Kernel classes timed by the optional HIP-event profiler.
 enum KernelId {
     KID_RK_STAGE = 0,
@@ -283,7 +350,7 @@ struct Handle {
     int lda_zt;                      // leading dimension of the z cos/sin tables
     double *zc, *zs;                 // z tables cos/sin(2 pi k m / M), [m][k]
     double *zf = nullptr;            // their matrix-core fragments (M/2 + 1 <= 96)
-    double *dct_tab = nullptr;       // x-DCT tables as double2: rot[N], twA, twC [K1 N2], t1, t1i, t2 (dct_frag)
+    void *dct_tab = nullptr;         // x-DCT tables as double2 (float2 in mixed precision): rot[N], twA, twC [K1 N2], t1, t1i, t2 (dct_frag)
     double *lu_dl, *lu_dp, *lu_du;  // Thomas factors [k][j][kx], [k][j][kx], [j] (table kernel only)
     double *lu00;                   // the pinned (0,0) system: multipliers [NM], reciprocal pivots [NM]
     int th_p = 0;                   // segments of the partitioned Thomas kernel (0: table kernel)
@@ -299,10 +366,7 @@ struct Handle {
     // mixed precision: BF16 hi/lo transform matrices, FP64 (0,0) mode
     int NP;                         // kx stride of the FP32 spectral arrays (N rounded up to 32)
     int kpx, kpz;                   // GEMM depths N and M rounded up to 32
-    bool mx_two = false;            // x transform as two short DFTs (k_xfwd_mx / k_xinv_mx)
-    void *mx2 = nullptr;            // their operand and twiddle tables (one allocation)
-    const void *x2_fA = nullptr, *x2_fC = nullptr, *x2_iC = nullptr, *x2_iA = nullptr;
-    const float *x2_tw = nullptr;   // float2 twiddles: W_N^{n2 k1} as [k1][n2] and [n2][k1], then rot[N]
+    bool mx_two = false;            // x transform as two short FP32 DFTs (dct_fits_mixed), else a dense GEMM
     unsigned short *mx_tab;         // one allocation for the eight matrices below
     unsigned short *zmf = nullptr;  // folded z transform fragments (k_zdft_mx), M/2 + 1 <= 96
     int zmf_rt = 0;
@@ -466,19 +530,12 @@ void snapshot_end(Handle &h, const double **ptr);
 void snapshot_free(Handle &h);
 // ---- mixed precision (bl_mixed.hip) ----
 void build_mixed(Handle &h);
-// The first stage's pressure source in the mixed path: the divergence of the
-// stage's increment U* - Un, taken as c0 F1 on the faces the stage update
-// moves and as the FP64 boundary increments (Handle::inc1) or the difference
-// of the stored values on the boundary faces, instead of div U*.  In exact
-// arithmetic the two agree (div Un is zero after the previous projection);
-// in FP32 storage div Un is rounding noise of order eps |u| / dx, which the
-// projection would divide by dt a11 into the recorded pressure.
-struct IncSrc {
-    const float *fu, *fv, *fw;     // F1 of the stage
-    const float *vn;               // V at the step start
-    const double *inc1;            // Handle::inc1
-    double c0;                     // dt a11
-};
+// the mixed path's x transforms as two short FP32 DFTs (bl_kernels.hip), for
+// lengths N = N1 N2 that they take: divergence, its FP64 line sums (p00[j][m]) and
+// the forward transform into rows of stride NP; the inverse plus add[j]
+bool dct_fits_mixed(int N, int N1);
+void launch_xfwd_mixed(Handle &h, const Fld3<float> &f, float *T1, const BcPlanes<float> *bc, const IncSrc *inc);
+void launch_xinv_mixed(Handle &h, const float *T1, const double *add, float *phi);
 void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const BcPlanes<float> *bc = nullptr,
                           const IncSrc *inc = nullptr);
 // eddy viscosity of f into h.nu_t (bl_dsm.hip): LES = 1 constant-coefficient

@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "bl_internal.hpp"
@@ -983,56 +984,92 @@ __global__ __launch_bounds__(256) void k_zdft_inv(int M, int C, long long plane,
 // (16 lanes read consecutive entries); t1, t1i, t2: (cos, sin)(2 pi a b/L) for
 // row a and column b in lane order per (row tile, k step), b weighted in t1i.
 // ------------------------------------------------------------------------
-struct DctArgs {
-    int N, N1, N2, K1h;
-    int LB;        // lines per block
-    int C1, C;     // lines c = c1 + C1*c2
-    long long in_base, in_c1, in_c2;
-    long long out_base, out_c1, out_c2;
-    double scale;  // inverse only: 1/(N*M)
-    const double2 *twA, *twC, *rot, *t1, *t1i, *t2;
-};
-
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double2 cmulc(double2 a, double2 b) {  // a * conj(b)
-    return make_double2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
-}
-
 typedef double dbl4 __attribute__((ext_vector_type(4)));
+typedef float flt4 __attribute__((ext_vector_type(4)));
 constexpr int kLd = 4;  // loads per thread in flight in the line load phases
 
 __device__ __forceinline__ dbl4 mfma64(double a, double b, dbl4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// the matrix instruction of a storage type: the operands' layout is the same,
+// the rows of the accumulator are 4 apart in FP64 and consecutive in FP32
+template <class T>
+struct Mf;
+template <>
+struct Mf<double> {
+    typedef double2 T2;
+    typedef dbl4 V4;
+    static __device__ __forceinline__ V4 mul(double a, double b, V4 c) { return mfma64(a, b, c); }
+    static __device__ __forceinline__ int row(int q, int r) { return q + 4 * r; }
+    static __device__ __forceinline__ T2 make(double a, double b) { return make_double2(a, b); }
+};
+template <>
+struct Mf<float> {
+    typedef float2 T2;
+    typedef flt4 V4;
+    static __device__ __forceinline__ V4 mul(float a, float b, V4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int q, int r) { return 4 * q + r; }
+    static __device__ __forceinline__ T2 make(float a, float b) { return make_float2(a, b); }
+};
+
+template <class T>
+struct DctArgs {
+    typedef typename Mf<T>::T2 T2;
+    int N, N1, N2, K1h;
+    int LB;        // lines per block
+    int C1, C;     // lines c = c1 + C1*c2
+    long long in_base, in_c1, in_c2;
+    long long out_base, out_c1, out_c2;
+    T scale;       // inverse only: 1/(N*M)
+    const T2 *twA, *twC, *rot, *t1, *t1i, *t2;
+    double *part;       // forward, not null: FP64 line sums of the rhs, part[c1 part_ld + c2]
+    int part_ld;
+    const double *add;  // inverse, not null: a constant per c1 added to the line
+};
+
+template <class T2>
+__device__ __forceinline__ T2 cmul(T2 a, T2 b) {
+    return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+}
+template <class T2>
+__device__ __forceinline__ T2 cmulc(T2 a, T2 b) {  // a * conj(b)
+    return {a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y};
+}
+
 // row stride of the complex intermediate: odd, so that 16 lanes reading one
 // entry of 16 rows use different banks
 __host__ __device__ inline int dct_ld(int N2) { return N2 | 1; }
-// LDS doubles of the line area (even: the complex area behind it is 16-byte aligned)
+// LDS elements of the line area (even: the complex area behind it is aligned)
 __host__ __device__ inline int dct_lines(int LB, int N) { return (LB * N + 1) / 2 * 2; }
 
 // the folded length-N2 DFT of the complex rows Bl (one per column): the four
 // real sums of row tile rt
+template <class T>
 struct DctSums {
-    dbl4 cr, ci, sr, si;  // sum E cos, sum O sin (real and imaginary parts)
+    typename Mf<T>::V4 cr, ci, sr, si;  // sum E cos, sum O sin (real and imaginary parts)
 };
-__device__ __forceinline__ DctSums dct_sums(const DctArgs &a, const double2 *Bl, bool cok, int rt, int q, int lane) {
+// REAL: the rows' imaginary parts are zero (N1 = 1)
+template <bool REAL, class T>
+__device__ __forceinline__ DctSums<T> dct_sums(const DctArgs<T> &a, const typename Mf<T>::T2 *Bl, bool cok, int rt,
+                                               int q, int lane) {
+    typedef typename Mf<T>::T2 T2;
     const int H = a.N2 / 2 + 1, KS = (H + 3) / 4;
-    const dbl4 z = {0.0, 0.0, 0.0, 0.0};
-    DctSums s{z, z, z, z};
-    const double2 *t = a.t2 + (long long)rt * KS * 64 + lane;
+    const typename Mf<T>::V4 z = {0, 0, 0, 0};
+    DctSums<T> s{z, z, z, z};
+    const T2 *t = a.t2 + (long long)rt * KS * 64 + lane;
     // four k steps at a time, their operands read before the first product, from the last to the first: a smooth
     // field's spectrum falls with k, and adding its large end last rounds the
     // large partial sums least often
     for (int k0 = (KS - 1) / 4 * 4; k0 >= 0; k0 -= 4) {
-        double2 w[4], x[4], y[4];
+        T2 w[4], x[4], y[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int n = 4 * (k0 + u) + q;
             w[u] = t[min(k0 + u, KS - 1) * 64];
-            x[u] = y[u] = make_double2(0.0, 0.0);
+            x[u] = y[u] = Mf<T>::make(0, 0);
             if (cok && n < H) {
                 x[u] = Bl[n];
                 y[u] = Bl[n == 0 ? 0 : a.N2 - n];
@@ -1043,10 +1080,10 @@ __device__ __forceinline__ DctSums dct_sums(const DctArgs &a, const double2 *Bl,
             const int n = 4 * (k0 + u) + q;
             const bool single = n == 0 || 2 * n == a.N2;  // x = y there
             if (k0 + u >= KS) continue;
-            s.cr = mfma64(w[u].x, single ? x[u].x : x[u].x + y[u].x, s.cr);
-            s.ci = mfma64(w[u].x, single ? x[u].y : x[u].y + y[u].y, s.ci);
-            s.sr = mfma64(w[u].y, x[u].x - y[u].x, s.sr);
-            s.si = mfma64(w[u].y, x[u].y - y[u].y, s.si);
+            s.cr = Mf<T>::mul(w[u].x, single ? x[u].x : x[u].x + y[u].x, s.cr);
+            if (!REAL) s.ci = Mf<T>::mul(w[u].x, single ? x[u].y : x[u].y + y[u].y, s.ci);
+            s.sr = Mf<T>::mul(w[u].y, x[u].x - y[u].x, s.sr);
+            if (!REAL) s.si = Mf<T>::mul(w[u].y, x[u].y - y[u].y, s.si);
         }
     }
     return s;
@@ -1060,22 +1097,27 @@ __device__ __forceinline__ DctSums dct_sums(const DctArgs &a, const double2 *Bl,
 // own.  At 814x257x193 the forward (inverse) transform takes 0.345 (0.203) ms, bound
 // by the latency of its loads (HBM time 0.25 (0.125)); the unfolded products in
 // four waves took 0.42 (0.30).  511 points (7 x 73): 0.086 (0.060) ms per 12288
-// lines, on the vector units 0.15 (0.15).
+// lines, on the vector units 0.15 (0.15).  FP32 (v_mfma_f32_16x16x4_f32, 814x257x193):
+// 0.218 (0.124) ms; unfolded split-BF16x3 products in four waves 0.25 (0.144).
 // DIV: the line is the pseudo-pressure rhs (projection.f90:38-47) evaluated
 // on the fly from U, V, W (in = U, in2 = V, in3 = W, lines over cells
 // i = 1..N, j = 1..NM, k = 1..M) instead of being read from memory; with
-// bc.du set the boundary faces come from the stage's boundary values (DivLine).
-template <bool DIV, bool SMALL>
-__global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_fwd_m(DctArgs a, Dims d, Metrics mt, BcPlanes<double> bc,
-                                                                 const double *__restrict__ in,
-                                                                 const double *__restrict__ in2,
-                                                                 const double *__restrict__ in3,
-                                                                 double *__restrict__ out) {
-    extern __shared__ double2 smem2[];
+// bc.du set the boundary faces come from the stage's boundary values (DivLine),
+// and with inc.inc1 set from the stage's increment (IncLine, FP32 fields).
+template <bool DIV, bool SMALL, class T>
+__global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? (sizeof(T) == 4 ? 6 : 5) : 4) void k_dct_fwd_m(DctArgs<T> a, Dims d, Metrics mt, BcPlanes<T> bc, IncSrc inc,
+                                                                 const T *__restrict__ in,
+                                                                 const T *__restrict__ in2,
+                                                                 const T *__restrict__ in3,
+                                                                 T *__restrict__ out) {
+    extern __shared__ double2 smem16[];
+    typedef typename Mf<T>::T2 T2;
+    typedef typename Mf<T>::V4 V4;
+    T2 *smem2 = reinterpret_cast<T2 *>(smem16);
     const int NW = SMALL ? 2 : blockDim.x >> 6;
     const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1, LB = SMALL ? 2 : a.LB, ld = dct_ld(N2);
-    double *v = reinterpret_cast<double *>(smem2);
-    double2 *Bc = SMALL ? smem2 : smem2 + dct_lines(LB, N) / 2;  // [line][k1][ld]
+    T *v = reinterpret_cast<T *>(smem2);
+    T2 *Bc = SMALL ? smem2 : smem2 + dct_lines(LB, N) / 2;  // [line][k1][ld]
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int line0 = blockIdx.x * LB;
@@ -1084,48 +1126,64 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_fwd_m(
     for (int l = wave; l < LB; l += NW) {
         const int c = min(line0 + l, a.C - 1);
         const int c1 = c % a.C1, c2 = c / a.C1;
-        const double *src = in + a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
-        const DivLine<double> dl(d, mt, bc, in, in2, in3, c1, c2);
-        for (int n0 = lane; n0 < N; n0 += 64 * kLd) {
-            typename DivLine<double>::Raw r[DIV ? kLd : 1];
-            double f[DIV ? 1 : kLd];
+        T *vl = v + l * N;
+        auto put = [&](int n, T x) { vl[(n & 1) ? N - 1 - (n >> 1) : (n >> 1)] = x; };
+        if constexpr (DIV) {
+            double sum = 0.0;
+            auto line = [&](const auto &dl) {
+                for (int n0 = lane; n0 < N; n0 += 64 * kLd) {
+                    typename std::decay<decltype(dl)>::type::Raw r[kLd];
 #pragma unroll
-            for (int u = 0; u < kLd; ++u) {
-                const int n = min(n0 + 64 * u, N - 1);
-                if constexpr (DIV)
-                    r[u] = dl.load(n);
+                    for (int u = 0; u < kLd; ++u) r[u] = dl.load(min(n0 + 64 * u, N - 1));
+#pragma unroll
+                    for (int u = 0; u < kLd; ++u) {
+                        const int n = n0 + 64 * u;
+                        if (n >= N) continue;
+                        const double x = dl.div(r[u], n);
+                        if constexpr (sizeof(T) == 4) sum += x;
+                        put(n, (T)x);
+                    }
+                }
+            };
+            if constexpr (sizeof(T) == 4) {
+                if (inc.inc1)
+                    line(IncLine(d, mt, inc, bc, c1, c2));
                 else
-                    f[u] = src[n];
+                    line(DivLine<T>(d, mt, bc, in, in2, in3, c1, c2));
+                for (int o = 32; o > 0; o >>= 1) sum += __shfl_down(sum, o);
+                if (lane == 0 && line0 + l < a.C) a.part[(long long)c1 * a.part_ld + c2] = sum;
+            } else {
+                line(DivLine<T>(d, mt, bc, in, in2, in3, c1, c2));
             }
+        } else {
+            const T *src = in + a.in_base + c1 * a.in_c1 + c2 * a.in_c2;
+            for (int n0 = lane; n0 < N; n0 += 64 * kLd) {
+                T f[kLd];
 #pragma unroll
-            for (int u = 0; u < kLd; ++u) {
-                const int n = n0 + 64 * u;
-                double x;
-                if constexpr (DIV)
-                    x = dl.div(r[u], n);
-                else
-                    x = f[u];
-                if (n < N) v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = x;
+                for (int u = 0; u < kLd; ++u) f[u] = src[min(n0 + 64 * u, N - 1)];
+#pragma unroll
+                for (int u = 0; u < kLd; ++u)
+                    if (n0 + 64 * u < N) put(n0 + 64 * u, f[u]);
             }
         }
     }
     __syncthreads();
     // ---- step A
     const int H1 = K1, KS1 = (H1 + 3) / 4, RT1 = (H1 + 15) / 16, CA = (LB * N2 + 15) / 16;
-    auto sums_a = [&](int ct, int rt, dbl4 &re, dbl4 &im) {
+    auto sums_a = [&](int ct, int rt, V4 &re, V4 &im) {
         const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
         const bool cok = col < LB * N2;
-        const double *vl = v + ln * N + n2;
-        const double2 *t = a.t1 + rt * KS1 * 64 + lane;
-        re = im = dbl4{0.0, 0.0, 0.0, 0.0};
+        const T *vl = v + ln * N + n2;
+        const T2 *t = a.t1 + rt * KS1 * 64 + lane;
+        re = im = V4{0, 0, 0, 0};
         for (int k0 = 0; k0 < KS1; k0 += 4) {
-            double2 w[4];
-            double x[4], y[4];
+            T2 w[4];
+            T x[4], y[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int n = 4 * (k0 + u) + q;
                 w[u] = t[min(k0 + u, KS1 - 1) * 64];
-                x[u] = y[u] = 0.0;
+                x[u] = y[u] = 0;
                 if (cok && n < H1) {
                     x[u] = vl[N2 * n];
                     y[u] = vl[n == 0 ? 0 : N2 * (N1 - n)];
@@ -1136,31 +1194,36 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_fwd_m(
                 const int n = 4 * (k0 + u) + q;
                 const bool single = n == 0 || 2 * n == N1;  // x = y there
                 if (k0 + u >= KS1) continue;
-                re = mfma64(w[u].x, single ? x[u] : x[u] + y[u], re);
-                im = mfma64(w[u].y, x[u] - y[u], im);
+                re = Mf<T>::mul(w[u].x, single ? x[u] : x[u] + y[u], re);
+                im = Mf<T>::mul(w[u].y, x[u] - y[u], im);
             }
         }
     };
-    auto put_a = [&](int ct, int rt, const dbl4 &re, const dbl4 &im) {
+    auto put_a = [&](int ct, int rt, const V4 &re, const V4 &im) {
         const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
         if (col >= LB * N2) return;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int k1 = 16 * rt + q + 4 * r;
-            if (k1 < K1) Bc[(ln * K1 + k1) * ld + n2] = cmul(make_double2(re[r], -im[r]), a.twA[k1 * N2 + n2]);
+            const int k1 = 16 * rt + Mf<T>::row(q, r);
+            if (k1 < K1) Bc[(ln * K1 + k1) * ld + n2] = cmul(Mf<T>::make(re[r], -im[r]), a.twA[k1 * N2 + n2]);
         }
     };
     if constexpr (SMALL) {
-        dbl4 re[2], im[2];
+        V4 re[2], im[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) sums_a(2 * wave + h, 0, re[h], im[h]);
         __syncthreads();  // v is read; Bc overwrites it
 #pragma unroll
         for (int h = 0; h < 2; ++h) put_a(2 * wave + h, 0, re[h], im[h]);
+    } else if (N1 == 1) {  // one point: a copy
+        for (int e = tid; e < LB * N; e += blockDim.x) {
+            const int ln = e / N, n2 = e - ln * N;
+            Bc[ln * ld + n2] = Mf<T>::make(v[e], 0);
+        }
     } else {
         for (int e = wave; e < CA * RT1; e += NW) {
             const int ct = e / RT1, rt = e - ct * RT1;
-            dbl4 re, im;
+            V4 re, im;
             sums_a(ct, rt, re, im);
             put_a(ct, rt, re, im);
         }
@@ -1168,19 +1231,19 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_fwd_m(
     __syncthreads();
     // ---- step C
     const int H2 = N2 / 2 + 1, RT2 = (H2 + 15) / 16, CC = (LB * K1 + 15) / 16;
-    auto put_c = [&](int ct, int rt, const DctSums &s) {
+    auto put_c = [&](int ct, int rt, const DctSums<T> &s) {
         const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
         if (col >= LB * K1) return;
-        auto put = [&](int k2, double re, double im) {
+        auto put = [&](int k2, T re, T im) {
             const int k = k1 + N1 * k2;
-            const double2 wv = cmul(a.rot[k], make_double2(re, im));
-            v[ln * N + k] = 2.0 * wv.x;
+            const T2 wv = cmul(a.rot[k], Mf<T>::make(re, im));
+            v[ln * N + k] = 2 * wv.x;
             // the mirror N - k of k1 = 0 and k1 = N1/2 is one of their own outputs
-            if (k1 != 0 && 2 * k1 != N1) v[ln * N + N - k] = -2.0 * wv.y;
+            if (k1 != 0 && 2 * k1 != N1) v[ln * N + N - k] = -2 * wv.y;
         };
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int k2 = 16 * rt + q + 4 * r;
+            const int k2 = 16 * rt + Mf<T>::row(q, r);
             if (k2 >= H2) continue;
             put(k2, s.cr[r] + s.si[r], s.ci[r] - s.sr[r]);
             if (k2 != 0 && 2 * k2 != N2) put(N2 - k2, s.cr[r] - s.si[r], s.ci[r] + s.sr[r]);
@@ -1188,10 +1251,12 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_fwd_m(
     };
     auto sums_c = [&](int ct, int rt) {
         const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
-        return dct_sums(a, Bc + (ln * K1 + k1) * ld, col < LB * K1, rt, q, lane);
+        const T2 *Bl = Bc + (ln * K1 + k1) * ld;
+        return N1 == 1 ? dct_sums<true>(a, Bl, col < LB * K1, rt, q, lane)
+                       : dct_sums<false>(a, Bl, col < LB * K1, rt, q, lane);
     };
     if constexpr (SMALL) {
-        const DctSums s = sums_c(wave, 0);
+        const DctSums<T> s = sums_c(wave, 0);
         __syncthreads();  // Bc is read; v overwrites it
         put_c(wave, 0, s);
     } else {
@@ -1204,22 +1269,25 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_fwd_m(
     for (int l = wave; l < LB; l += NW) {
         const int c = line0 + l;
         if (c >= a.C) break;
-        double *dst = out + a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
+        T *dst = out + a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
         for (int kx = lane; kx < N; kx += 64) dst[kx] = v[l * N + kx];
     }
 }
 
-template <bool SMALL>
-__global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_inv_m(DctArgs a, const double *__restrict__ in,
-                                                                 double *__restrict__ out) {
-    extern __shared__ double2 smem2[];
+template <bool SMALL, class T>
+__global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? (sizeof(T) == 4 ? 6 : 5) : 4) void k_dct_inv_m(DctArgs<T> a, const T *__restrict__ in,
+                                                                 T *__restrict__ out) {
+    extern __shared__ double2 smem16[];
+    typedef typename Mf<T>::T2 T2;
+    typedef typename Mf<T>::V4 V4;
+    T2 *smem2 = reinterpret_cast<T2 *>(smem16);
     const int NW = SMALL ? 2 : blockDim.x >> 6;
     const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1, LB = SMALL ? 2 : a.LB, ld = dct_ld(N2);
     const float rK1 = 1.0f / (float)K1;
     // SMALL: one area for V, C~ and the output lines in turn; otherwise V (later
     // the lines, which are no longer) and C~ apart
-    double2 *Vs = smem2, *Cs = SMALL ? smem2 : smem2 + LB * K1 * ld;
-    double *o = reinterpret_cast<double *>(smem2);
+    T2 *Vs = smem2, *Cs = SMALL ? smem2 : smem2 + LB * K1 * ld;
+    T *o = reinterpret_cast<T *>(smem2);
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int line0 = blockIdx.x * LB;
@@ -1229,10 +1297,10 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_inv_m(
     const int nv = K1 * N2;
     for (int l = wave; l < LB; l += NW) {
         const int c = min(line0 + l, a.C - 1);
-        const double *g = in + a.in_base + (long long)(c % a.C1) * a.in_c1 + (long long)(c / a.C1) * a.in_c2;
+        const T *g = in + a.in_base + (long long)(c % a.C1) * a.in_c1 + (long long)(c / a.C1) * a.in_c2;
         for (int i0 = lane; i0 < nv; i0 += 64 * kLd) {
-            double gk[kLd], gm[kLd];
-            double2 rt[kLd];
+            T gk[kLd], gm[kLd];
+            T2 rt[kLd];
 #pragma unroll
             for (int u = 0; u < kLd; ++u) {
                 const int r = min(i0 + 64 * u, nv - 1), k2 = small_div(r, rK1), k1 = r - k2 * K1;
@@ -1240,13 +1308,13 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_inv_m(
                 gk[u] = g[k];
                 gm[u] = g[k == 0 ? 0 : N - k];
                 rt[u] = a.rot[k];
-                if (k == 0) gm[u] = 0.0;
+                if (k == 0) gm[u] = 0;
             }
 #pragma unroll
             for (int u = 0; u < kLd; ++u) {
                 const int r = i0 + 64 * u, k2 = small_div(r, rK1), k1 = r - k2 * K1;
                 if (r < nv)
-                    Vs[(l * K1 + k1) * ld + k2] = cmulc(make_double2(0.5 * gk[u], -0.5 * gm[u]), rt[u]);
+                    Vs[(l * K1 + k1) * ld + k2] = cmulc(Mf<T>::make((T)0.5 * gk[u], (T)-0.5 * gm[u]), rt[u]);
             }
         }
     }
@@ -1255,24 +1323,24 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_inv_m(
     const int H2 = N2 / 2 + 1, RT2 = (H2 + 15) / 16, CC = (LB * K1 + 15) / 16;
     auto sums_c = [&](int ct, int rt) {
         const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
-        return dct_sums(a, Vs + (ln * K1 + k1) * ld, col < LB * K1, rt, q, lane);
+        return dct_sums<false>(a, Vs + (ln * K1 + k1) * ld, col < LB * K1, rt, q, lane);
     };
-    auto put_c = [&](int ct, int rt, const DctSums &s) {
+    auto put_c = [&](int ct, int rt, const DctSums<T> &s) {
         const int col = ct * 16 + c16, ln = col / K1, k1 = col - ln * K1;
         if (col >= LB * K1) return;
-        auto put = [&](int n2, double re, double im) {
-            Cs[(ln * K1 + k1) * ld + n2] = cmulc(make_double2(re, im), a.twC[n2 * K1 + k1]);
+        auto put = [&](int n2, T re, T im) {
+            Cs[(ln * K1 + k1) * ld + n2] = cmulc(Mf<T>::make(re, im), a.twC[n2 * K1 + k1]);
         };
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int n2 = 16 * rt + q + 4 * r;
+            const int n2 = 16 * rt + Mf<T>::row(q, r);
             if (n2 >= H2) continue;
             put(n2, s.cr[r] - s.si[r], s.ci[r] + s.sr[r]);
             if (n2 != 0 && 2 * n2 != N2) put(N2 - n2, s.cr[r] + s.si[r], s.ci[r] - s.sr[r]);
         }
     };
     if constexpr (SMALL) {
-        const DctSums s = sums_c(wave, 0);
+        const DctSums<T> s = sums_c(wave, 0);
         __syncthreads();  // Vs is read; Cs overwrites it
         put_c(wave, 0, s);
     } else {
@@ -1284,56 +1352,61 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_inv_m(
     __syncthreads();
     // ---- step A'
     const int KS1 = (K1 + 3) / 4, RT1 = (K1 + 15) / 16, CA = (LB * N2 + 15) / 16;
-    auto sums_a = [&](int ct, int rt, dbl4 &p, dbl4 &s) {
+    auto sums_a = [&](int ct, int rt, V4 &p, V4 &s) {
         const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
         const bool cok = col < LB * N2;
-        const double2 *cl = Cs + ln * K1 * ld + n2;
-        const double2 *t = a.t1i + rt * KS1 * 64 + lane;
-        p = s = dbl4{0.0, 0.0, 0.0, 0.0};
+        const T2 *cl = Cs + ln * K1 * ld + n2;
+        const T2 *t = a.t1i + rt * KS1 * 64 + lane;
+        p = s = V4{0, 0, 0, 0};
         for (int k0 = (KS1 - 1) / 4 * 4; k0 >= 0; k0 -= 4) {  // the large end last, as in dct_sums
-            double2 w[4], x[4];
+            T2 w[4], x[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int k1 = 4 * (k0 + u) + q;
                 w[u] = t[min(k0 + u, KS1 - 1) * 64];
-                x[u] = make_double2(0.0, 0.0);
+                x[u] = Mf<T>::make(0, 0);
                 if (cok && k1 < K1) x[u] = cl[k1 * ld];
             }
 #pragma unroll
             for (int u = 3; u >= 0; --u) {
                 if (k0 + u >= KS1) continue;
-                p = mfma64(w[u].x, x[u].x, p);
-                s = mfma64(w[u].y, x[u].y, s);
+                p = Mf<T>::mul(w[u].x, x[u].x, p);
+                s = Mf<T>::mul(w[u].y, x[u].y, s);
             }
         }
     };
-    auto put_a = [&](int ct, int rt, const dbl4 &p, const dbl4 &s) {
+    auto put_a = [&](int ct, int rt, const V4 &p, const V4 &s) {
         const int col = ct * 16 + c16, ln = col / N2, n2 = col - ln * N2;
         if (col >= LB * N2) return;
-        auto put = [&](int n1, double x) {
+        auto put = [&](int n1, T x) {
             const int n = N2 * n1 + n2;
             const int pos = (n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1;
             o[ln * N + pos] = x * a.scale;
         };
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int n1 = 16 * rt + q + 4 * r;
+            const int n1 = 16 * rt + Mf<T>::row(q, r);
             if (n1 >= K1) continue;
             put(n1, p[r] - s[r]);
             if (n1 != 0 && 2 * n1 != N1) put(N1 - n1, p[r] + s[r]);
         }
     };
     if constexpr (SMALL) {
-        dbl4 p[2], s[2];
+        V4 p[2], s[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) sums_a(2 * wave + h, 0, p[h], s[h]);
         __syncthreads();  // Cs is read; o overwrites it
 #pragma unroll
         for (int h = 0; h < 2; ++h) put_a(2 * wave + h, 0, p[h], s[h]);
+    } else if (N1 == 1) {
+        for (int e = tid; e < LB * N; e += blockDim.x) {
+            const int ln = e / N, n = e - ln * N;
+            o[ln * N + ((n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1)] = Cs[ln * ld + n].x * a.scale;
+        }
     } else {
         for (int e = wave; e < CA * RT1; e += NW) {
             const int ct = e / RT1, rt = e - ct * RT1;
-            dbl4 p, s;
+            V4 p, s;
             sums_a(ct, rt, p, s);
             put_a(ct, rt, p, s);
         }
@@ -1342,8 +1415,9 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? 5 : 4) void k_dct_inv_m(
     for (int l = wave; l < LB; l += NW) {
         const int c = line0 + l;
         if (c >= a.C) break;
-        double *dst = out + a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
-        for (int n = lane; n < N; n += 64) dst[n] = o[l * N + n];
+        T *dst = out + a.out_base + (long long)(c % a.C1) * a.out_c1 + (long long)(c / a.C1) * a.out_c2;
+        const T ad = a.add ? (T)a.add[c % a.C1] : (T)0;
+        for (int n = lane; n < N; n += 64) dst[n] = a.add ? o[l * N + n] + ad : o[l * N + n];
     }
 }
 
@@ -2037,22 +2111,41 @@ void zdft_launch(Handle &h, int kid, bool forward, const double *in, double *out
 // C (line, k1), as far as 80 KB of LDS (two blocks per CU) hold them; fewer lines
 // leave columns empty and read the tables more often (at N = 129, 3774 lines, 8,
 // 3 and 1 lines per block took 22, 25 and 40 us)
-int dct_block_lines(const DctArgs &a) {
-    const int K1 = a.K1h + 1;
-    const size_t line = sizeof(double) * a.N + sizeof(double2) * K1 * dct_ld(a.N2);
-    return std::max(1, std::min(std::max(2, (15 + K1) / K1), (int)(81920 / line)));
+size_t dct_line_bytes(int N, int N1, size_t es) {
+    return es * (N + 1 + 2 * (size_t)(N1 / 2 + 1) * dct_ld(N / N1));
 }
 
-void dct_launch(Handle &h, int kid, DctArgs a, bool forward, const double *in, double *out,
-                const Field3 *div = nullptr, const BcPlanes<double> *bcp = nullptr) {
+template <class T>
+void dct_launch(Handle &h, int kid, DctArgs<T> a, bool forward, const T *in, T *out, const Fld3<T> *div = nullptr,
+                const BcPlanes<T> *bcp = nullptr, const IncSrc *incp = nullptr) {
+    typedef typename Mf<T>::T2 T2;
     ProfScope ps(h, kid);
-    const BcPlanes<double> bc = bcp ? *bcp : BcPlanes<double>{};
+    const Dims &d = h.d;
+    const BcPlanes<T> bc = bcp ? *bcp : BcPlanes<T>{};
+    const IncSrc inc = incp ? *incp : IncSrc{};
+    a.N = d.N;
+    a.N1 = h.dct_n1;
+    a.N2 = d.N / h.dct_n1;
+    a.K1h = h.dct_n1 / 2;
+    a.C1 = d.NM;
+    a.C = d.NM * d.M;
     const int K1 = a.K1h + 1, ld = dct_ld(a.N2);
+    a.rot = reinterpret_cast<const T2 *>(h.dct_tab);
+    a.twA = a.rot + a.N;
+    a.twC = a.twA + K1 * a.N2;
+    a.t1 = a.twC + K1 * a.N2;
+    a.t1i = a.t1 + dct_frag(a.N1);
+    a.t2 = a.t1i + dct_frag(a.N1);
     const bool small = a.N1 <= 31 && a.N2 <= 31;
-    a.LB = small ? 2 : dct_block_lines(a);
-    const size_t lines = sizeof(double) * dct_lines(a.LB, a.N), spec = sizeof(double2) * (size_t)a.LB * K1 * ld;
+    a.LB = small ? 2
+                 : std::max(1, std::min(std::max(2, (15 + K1) / K1),
+                                        (int)(81920 / dct_line_bytes(a.N, a.N1, sizeof(T)))));
+    // fewer lines where the blocks would not reach every compute unit (127 points,
+    // 1536 lines: 16 lines 14.9 and 11.8 us, 8 lines 12.6 and 10.5)
+    if (!small && (a.C + a.LB - 1) / a.LB < h.n_cu) a.LB = (a.LB + 1) / 2;
+    const size_t lines = sizeof(T) * dct_lines(a.LB, a.N), spec = sizeof(T2) * (size_t)a.LB * K1 * ld;
     // the inverse past the SMALL shapes: V (an area that also holds the lines) and C~
-    const size_t lds = small ? std::max(lines, spec) : (forward ? lines + spec : 2 * std::max(lines, spec));
+    const size_t lds = small ? std::max(lines, spec) : (forward ? lines + spec : std::max(lines, spec) + spec);
     if (lds > 163840) {
         last_error() = "x transform length too large for the LDS-resident DCT (N = " + std::to_string(a.N) + ")";
         throw ArgError();
@@ -2064,19 +2157,19 @@ void dct_launch(Handle &h, int kid, DctArgs a, bool forward, const double *in, d
     const dim3 block(small ? 128 : ((int)grid.x < 4 * h.n_cu ? 512 : 256));
     auto fwd = [&](auto kern) {
         if (div)
-            hipLaunchKernelGGL(kern, grid, block, lds, h.stream, a, h.d, h.m, bc, div->u, div->v, div->w, out);
+            hipLaunchKernelGGL(kern, grid, block, lds, h.stream, a, d, h.m, bc, inc, div->u, div->v, div->w, out);
         else
-            hipLaunchKernelGGL(kern, grid, block, lds, h.stream, a, h.d, h.m, bc, in, nullptr, nullptr, out);
+            hipLaunchKernelGGL(kern, grid, block, lds, h.stream, a, d, h.m, bc, inc, in, nullptr, nullptr, out);
     };
     if (forward) {
-        if (small)
-            div ? fwd(k_dct_fwd_m<true, true>) : fwd(k_dct_fwd_m<false, true>);
-        else
-            div ? fwd(k_dct_fwd_m<true, false>) : fwd(k_dct_fwd_m<false, false>);
+        if (div)
+            small ? fwd(k_dct_fwd_m<true, true, T>) : fwd(k_dct_fwd_m<true, false, T>);
+        else if constexpr (sizeof(T) == 8)
+            small ? fwd(k_dct_fwd_m<false, true, T>) : fwd(k_dct_fwd_m<false, false, T>);
     } else if (small) {
-        hipLaunchKernelGGL(k_dct_inv_m<true>, grid, block, lds, h.stream, a, in, out);
+        hipLaunchKernelGGL((k_dct_inv_m<true, T>), grid, block, lds, h.stream, a, in, out);
     } else {
-        hipLaunchKernelGGL(k_dct_inv_m<false>, grid, block, lds, h.stream, a, in, out);
+        hipLaunchKernelGGL((k_dct_inv_m<false, T>), grid, block, lds, h.stream, a, in, out);
     }
     check_launch();
 }
@@ -2284,23 +2377,7 @@ void launch_poisson(Handle &h, double *phi, const Field3 *div, const BcPlanes<do
     const int N = d.N, M = d.M, NM = d.NM;
     const long long plane = (long long)N * NM;
     // forward x: lines (j, m) of the padded field -> T1[m][j][kx]
-    DctArgs da{};
-    da.N = N;
-    da.N1 = h.dct_n1;
-    da.N2 = N / h.dct_n1;
-    da.K1h = h.dct_n1 / 2;
-    da.C1 = NM;
-    da.C = NM * M;
-    {
-        const int K1 = da.K1h + 1;
-        const double2 *t = reinterpret_cast<const double2 *>(h.dct_tab);
-        da.rot = t;
-        da.twA = da.rot + N;
-        da.twC = da.twA + K1 * da.N2;
-        da.t1 = da.twC + K1 * da.N2;
-        da.t1i = da.t1 + dct_frag(da.N1);
-        da.t2 = da.t1i + dct_frag(da.N1);
-    }
+    DctArgs<double> da{};
     da.in_base = fidx(d, 1, 1, 1);
     da.in_c1 = d.sx;
     da.in_c2 = d.sxy;
@@ -2308,7 +2385,7 @@ void launch_poisson(Handle &h, double *phi, const Field3 *div, const BcPlanes<do
     da.out_c1 = N;
     da.out_c2 = plane;
     da.scale = 1.0;
-    dct_launch(h, KID_XFORM_X_FWD, da, true, phi, h.T1, div, bc);
+    dct_launch(h, KID_XFORM_X_FWD, da, true, (const double *)phi, h.T1, div, bc);
     // forward z: columns (kx, j) of T1 -> S[q][j][kx]
     zdft_launch(h, KID_XFORM_Z_FWD, true, h.T1, h.S);
     {
@@ -2334,7 +2411,36 @@ void launch_poisson(Handle &h, double *phi, const Field3 *div, const BcPlanes<do
     da.out_c1 = d.sx;
     da.out_c2 = d.sxy;
     da.scale = 1.0 / ((double)N * (double)M);
-    dct_launch(h, KID_XFORM_X_INV, da, false, h.T1, phi);
+    dct_launch(h, KID_XFORM_X_INV, da, false, (const double *)h.T1, phi);
+}
+
+bool dct_fits_mixed(int N, int N1) {
+    const int N2 = N / N1, K1 = N1 / 2 + 1;
+    // small_div's range, and one line in LDS (forward and inverse)
+    return N2 <= 256 && K1 <= 128 && K1 * N2 < 16384 && 2 * dct_line_bytes(N, N1, sizeof(float)) <= 163840;
+}
+
+void launch_xfwd_mixed(Handle &h, const Fld3<float> &f, float *T1, const BcPlanes<float> *bc, const IncSrc *inc) {
+    const Dims &d = h.d;
+    DctArgs<float> a{};
+    a.out_c1 = h.NP;
+    a.out_c2 = (long long)h.NP * d.NM;
+    a.part = h.p00;
+    a.part_ld = d.M;
+    dct_launch(h, KID_XFORM_X_FWD, a, true, (const float *)nullptr, T1, &f, bc, inc);
+}
+
+void launch_xinv_mixed(Handle &h, const float *T1, const double *add, float *phi) {
+    const Dims &d = h.d;
+    DctArgs<float> a{};
+    a.in_c1 = h.NP;
+    a.in_c2 = (long long)h.NP * d.NM;
+    a.out_base = fidx(d, 1, 1, 1);
+    a.out_c1 = d.sx;
+    a.out_c2 = d.sxy;
+    a.scale = (float)(1.0 / ((double)d.N * (double)d.M));
+    a.add = add;
+    dct_launch(h, KID_XFORM_X_INV, a, false, T1, phi);
 }
 
 template <class T>

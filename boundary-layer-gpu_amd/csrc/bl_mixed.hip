@@ -482,362 +482,6 @@ void zdft_mx_launch(Handle &h, int kid, int rt, int M, int C, long long plane, b
 }
 
 // ------------------------------------------------------------------------
-// x transform as two short DFTs on the matrix cores (N = N1 N2, Makhoul's
-// reordering, k1 <= N1/2 only; the same factorisation as the FP64 kernels),
-// each DFT a small GEMM with split-BF16x3 products accumulated in FP32.
-// Forward, step A: [Re, Im of B[k1][n2]] = WA [n1 x (line, n2)], K = N1 <= 32
-//   (one K step); step C: [Re, Im of V[k1 + N1 k2]] = WC [(n2, re/im) x
-//   (line, k1)], K = 2 N2 <= 64 (two K steps).  Inverse: the conjugate DFT
-//   over k2 (step C'), then the real output over (k1, re/im) with the
-//   Hermitian weights (step A').
-// Operand tables (host, lane order): per (row tile, K step) and lane l the
-// BF16 hi and lo of A[l%16][8(l/16) + e], e < 8.  In a paired table a tile
-// row R is (Re, Im) = R % 2 of index 8 rt + 2 (R/4) + (R%4)/2, so that a
-// lane's four accumulator rows 4(l/16) + r hold (Re, Im) of two indices.
-// ------------------------------------------------------------------------
-struct XArgs {
-    int N, N1, N2, K1h, NP, C1, C, M;
-    const u16x8 *fA, *fC, *iC, *iA;  // [(rt * KS + ks) * 64 + lane][hi, lo]
-    const float2 *twA, *twC, *rot;   // W_N^{n2 k1} as [k1][n2] and [n2][k1], e^{-i pi k/(2N)}
-    float scale;                     // inverse: 1/(N M)
-};
-
-constexpr int kXL = 2;   // lines per block (even)
-constexpr int kLdx = 4;  // loads per thread in flight in the inverse's gather
-
-__device__ __forceinline__ float2 cmulf(float2 a, float2 b) {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ float2 cmulcf(float2 a, float2 b) {  // a * conj(b)
-    return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
-}
-
-// split 8 FP32 values into BF16 hi / lo fragments
-__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 &hi, bf16x8 &lo) {
-    u16x8 h, l;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const unsigned short b = bf16_bits(x[e]);
-        h[e] = b;
-        l[e] = bf16_bits(x[e] - bf16_float(b));
-    }
-    hi = __builtin_bit_cast(bf16x8, h);
-    lo = __builtin_bit_cast(bf16x8, l);
-}
-
-// a b with a = a_hi + a_lo, b = b_hi + b_lo as the three split-BF16 products
-// a_lo b_hi + a_hi b_lo + a_hi b_hi (small terms first), FP32 accumulation
-__device__ __forceinline__ f32x4 mfma_split(const u16x8 *A, bf16x8 bh, bf16x8 bl, f32x4 acc) {
-    const bf16x8 ah = __builtin_bit_cast(bf16x8, A[0]), al = __builtin_bit_cast(bf16x8, A[1]);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, acc, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, acc, 0, 0, 0);
-}
-
-// divergence of the first stage's increment U* - Un at cell (i, j, k), p its
-// index (the IncSrc form of the pseudo-pressure rhs): c0 F1 on the faces the
-// stage update moves, the FP64 increments on the inflow and outflow U faces
-// (plus the mass-flux shift on the outflow), the difference of the stored
-// values on the wall and top V faces; the W face below plane 1 is the
-// periodic image of plane nz-2
-// (pointers, scales and ends fixed per line, as DivLine)
-struct IncLine {
-    const float *u, *vt, *vb, *wt, *wb;  // F1, or V of the stage on the top and wall faces
-    const float *nt, *nb;                // there: V at the step start (else null)
-    const double *rdx;
-    double c0, ry, rz, ul, ur;
-    int last;
-    __device__ __forceinline__ IncLine(const Dims &d, const Metrics &m, const IncSrc &s, const BcPlanes<float> &bc,
-                                       int c1, int c2) {
-        const long long p = fidx(d, 1, c1 + 1, c2 + 1), npl = (long long)d.nyg * d.nzg;
-        const long long pl = c1 + 1 + (long long)d.nyg * (c2 + 1);
-        u = s.fu + p;
-        vt = s.fv + p;
-        vb = vt - d.sx;
-        wt = s.fw + p;
-        wb = c2 == 0 ? wt + d.sxy * (d.nz - 3) : wt - d.sxy;
-        nt = nb = nullptr;
-        if (c1 == d.NM - 1) {
-            vt = bc.vtop + 1;
-            nt = s.vn + p;
-        }
-        if (c1 == 0) {
-            vb = bc.vwall + bc.wld * (c2 + 1) + 1;
-            nb = s.vn + p - d.sx;
-        }
-        rdx = m.rdx + 1;
-        ry = m.rdy[c1 + 1];
-        rz = m.rdz[c2 + 1];
-        c0 = s.c0;
-        ul = s.inc1[pl];
-        ur = s.inc1[npl + pl] + s.inc1[2 * npl];
-        last = d.N - 1;
-    }
-    struct Raw {
-        float u, l, vt, vb, wt, wb;
-        double rdx;
-    };
-    __device__ __forceinline__ Raw load(int n) const { return {u[n], u[n - 1], vt[n], vb[n], wt[n], wb[n], rdx[n]}; }
-    __device__ __forceinline__ double div(const Raw &a, int n) const {
-        const double r = n == last ? ur : c0 * (double)a.u, l = n == 0 ? ul : c0 * (double)a.l;
-        const double t = nt ? (double)a.vt - (double)nt[n] : c0 * (double)a.vt;
-        const double b = nb ? (double)a.vb - (double)nb[n] : c0 * (double)a.vb;
-        return (r - l) * a.rdx + (t - b) * ry + (c0 * (double)a.wt - c0 * (double)a.wb) * rz;
-    }
-    __device__ __forceinline__ double at(int n) const { return div(load(n), n); }
-};
-
-// forward: the pseudo-pressure rhs (projection.f90:38-47) of kXL lines
-// (cells i = 1..N of row j, plane m; line c = j-1 + NM (m-1)) formed in FP64
-// (from the increment when use_inc), its FP64 line sums for the (0,0) mode
-// (part[(j-1) M + m-1]), then the transform into T1[c NP + kx]
-constexpr int kXLd = 4;  // cells per thread whose loads are in flight together
-__global__ __launch_bounds__(256) void k_xfwd_mx(Dims d, Metrics mt, XArgs a, const float *__restrict__ U,
-                                                 const float *__restrict__ V, const float *__restrict__ W,
-                                                 float *__restrict__ out, double *__restrict__ part, BcPlanes<float> bc,
-                                                 IncSrc inc, int use_inc) {
-    extern __shared__ float smx[];
-    const int N = a.N, N1 = a.N1, N2 = a.N2, K1 = a.K1h + 1;
-    // twiddle indices n2 k1 stay below N (n2 < N2, k1 <= N1/2): no reduction
-    const float rN2 = 1.0f / (float)N2, rK1 = 1.0f / (float)K1;
-    float *v = smx;                                         // kXL*N
-    float2 *Bc = reinterpret_cast<float2 *>(v + kXL * N);   // kXL*K1*N2 (8-byte aligned: kXL*N even)
-    __shared__ double lsum[kXL][4];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
-    const int line0 = blockIdx.x * kXL;
-    double ps[kXL];
-#pragma unroll
-    for (int l = 0; l < kXL; ++l) ps[l] = 0.0;
-#pragma unroll
-    for (int l = 0; l < kXL; ++l) {
-        const int c = min(line0 + l, a.C - 1);
-        const int c1 = c % a.C1, c2 = c / a.C1;
-        auto put = [&](int n, double dv) {
-            ps[l] += dv;
-            v[l * N + ((n & 1) ? N - 1 - (n >> 1) : (n >> 1))] = (float)dv;
-        };
-        auto line = [&](const auto &dl) {
-            for (int n0 = tid; n0 < N; n0 += 256 * kXLd) {
-                typename std::decay<decltype(dl)>::type::Raw r[kXLd];
-#pragma unroll
-                for (int u = 0; u < kXLd; ++u) r[u] = dl.load(min(n0 + 256 * u, N - 1));
-#pragma unroll
-                for (int u = 0; u < kXLd; ++u) {
-                    const int n = n0 + 256 * u;
-                    if (n < N) put(n, dl.div(r[u], n));
-                }
-            }
-        };
-        if (use_inc)
-            line(IncLine(d, mt, inc, bc, c1, c2));
-        else
-            line(DivLine<float>(d, mt, bc, U, V, W, c1, c2));
-    }
-#pragma unroll
-    for (int l = 0; l < kXL; ++l) {
-        double t = ps[l];
-        for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o);
-        if (lane == 0) lsum[l][wave] = t;
-    }
-    __syncthreads();
-    if (tid < kXL && line0 + tid < a.C) {
-        const int c = line0 + tid, c1 = c % a.C1, c2 = c / a.C1;
-        part[(long long)c1 * a.M + c2] = (lsum[tid][0] + lsum[tid][1]) + (lsum[tid][2] + lsum[tid][3]);
-    }
-    // ---- step A: wave w owns column tiles (line, n2) kXL/2 w .. kXL/2 (w+1)
-    for (int ct = wave * (kXL / 2); ct < (wave + 1) * (kXL / 2); ++ct) {
-        const int col = ct * 16 + c16;
-        const int ln = small_div(col, rN2), n2 = col - ln * N2;
-        const bool cok = col < kXL * N2;
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int n1 = 8 * q + e;
-            x[e] = (cok && n1 < N1) ? v[ln * N + N2 * n1 + n2] : 0.f;
-        }
-        bf16x8 bh, bl;
-        split8(x, bh, bl);
-        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-        const f32x4 acc0 = mfma_split(a.fA + (0 * 64 + lane) * 2, bh, bl, z);
-        const f32x4 acc1 = mfma_split(a.fA + (1 * 64 + lane) * 2, bh, bl, z);
-        if (cok) {
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {  // (row tile, pair): k1 = 8 (h/2) + 2 q + h%2
-                const f32x4 &acc = (h < 2) ? acc0 : acc1;
-                const int k1 = 8 * (h / 2) + 2 * q + (h % 2);
-                if (k1 < K1)
-                    Bc[(ln * K1 + k1) * N2 + n2] =
-                        cmulf(make_float2(acc[2 * (h % 2)], acc[2 * (h % 2) + 1]), a.twA[k1 * N2 + n2]);
-            }
-        }
-    }
-    __syncthreads();
-    // ---- step C: wave w owns row tile w (k2 = 8w + 2q, 8w + 2q + 1), all kXL
-    // column tiles (line, k1)
-    for (int ct = 0; ct < kXL; ++ct) {
-        const int col = ct * 16 + c16;
-        const int ln = small_div(col, rK1), k1 = col - ln * K1;
-        const bool cok = col < kXL * K1;
-        const float *Bl = reinterpret_cast<const float *>(Bc + (ln * K1 + k1) * N2);
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            float x[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int kk = 32 * ks + 8 * q + e;  // (n2, re/im) = (kk/2, kk%2)
-                x[e] = (cok && (kk >> 1) < N2) ? Bl[kk] : 0.f;
-            }
-            bf16x8 bh, bl;
-            split8(x, bh, bl);
-            acc = mfma_split(a.fC + ((wave * 2 + ks) * 64 + lane) * 2, bh, bl, acc);
-        }
-        if (cok) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int k2 = 8 * wave + 2 * q + h;
-                if (k2 < N2) {
-                    const int k = k1 + N1 * k2;
-                    const float2 wv = cmulf(a.rot[k], make_float2(acc[2 * h], acc[2 * h + 1]));
-                    v[ln * N + k] = 2.f * wv.x;
-                    // the mirror N - k of k1 = 0 and k1 = N1/2 is written
-                    // directly by another lane (k1' = k1): one writer each
-                    if (k1 != 0 && 2 * k1 != N1) v[ln * N + N - k] = -2.f * wv.y;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < kXL * N; idx += 256) {
-        const int l = idx >= N ? 1 : 0, kx = idx - l * N;  // kXL = 2
-        const int c = line0 + l;
-        if (c < a.C) out[(long long)c * a.NP + kx] = v[idx];
-    }
-}
-
-// inverse: T1 lines (c NP + kx) -> phi cells (1..N, j, m) plus the (0,0)
-// constant add[j-1] of each y row
-__global__ __launch_bounds__(256) void k_xinv_mx(Dims d, XArgs a, const float *__restrict__ in,
-                                                 const double *__restrict__ add, float *__restrict__ phi) {
-    extern __shared__ float smx[];
-    const int N = a.N, N1 = a.N1, N2 = a.N2, K1h = a.K1h, K1 = K1h + 1;
-    // twiddle indices n2 k1 stay below N (n2 < N2, k1 <= N1/2): no reduction
-    const float rN2 = 1.0f / (float)N2, rK1 = 1.0f / (float)K1;
-    float2 *Vs = reinterpret_cast<float2 *>(smx);  // kXL*K1*N2, later the output lines (kXL*N floats)
-    float2 *Cs = Vs + kXL * K1 * N2;               // kXL*K1*N2
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, c16 = lane & 15;
-    const int line0 = blockIdx.x * kXL;
-    // kLdx elements per thread loaded before the first one is used
-    static_assert(kXL == 2, "line index below assumes two lines per block");
-    const float *gls[kXL];
-#pragma unroll
-    for (int l = 0; l < kXL; ++l) gls[l] = in + (long long)min(line0 + l, a.C - 1) * a.NP;
-    const int nv = kXL * K1 * N2;
-    for (int i0 = tid; i0 < nv; i0 += 256 * kLdx) {
-        float gk[kLdx], gm[kLdx];
-        float2 rt[kLdx];
-#pragma unroll
-        for (int u = 0; u < kLdx; ++u) {
-            const int idx = min(i0 + 256 * u, nv - 1);
-            // k1 fastest: runs of K1 consecutive entries of the line per wave
-            const int l = idx >= K1 * N2 ? 1 : 0, r = idx - l * K1 * N2;
-            const int k2 = small_div(r, rK1), k1 = r - k2 * K1;
-            const int k = k1 + N1 * k2;
-            gk[u] = gls[l][k];
-            gm[u] = gls[l][k == 0 ? 0 : N - k];
-            rt[u] = a.rot[k];
-            if (k == 0) gm[u] = 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < kLdx; ++u) {
-            const int idx = i0 + 256 * u;
-            const int l = idx >= K1 * N2 ? 1 : 0, r = idx - l * K1 * N2;
-            const int k2 = small_div(r, rK1), k1 = r - k2 * K1;
-            if (idx < nv)
-                Vs[(l * K1 + k1) * N2 + k2] = cmulcf(make_float2(0.5f * gk[u], -0.5f * gm[u]), rt[u]);
-        }
-    }
-    __syncthreads();
-    // ---- step C': wave w owns row tile w (n2 = 8w + 2q, +1), all kXL column
-    // tiles (line, k1)
-    for (int ct = 0; ct < kXL; ++ct) {
-        const int col = ct * 16 + c16;
-        const int ln = small_div(col, rK1), k1 = col - ln * K1;
-        const bool cok = col < kXL * K1;
-        const float *Vl = reinterpret_cast<const float *>(Vs + (ln * K1 + k1) * N2);
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            float x[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int kk = 32 * ks + 8 * q + e;  // (k2, re/im)
-                x[e] = (cok && (kk >> 1) < N2) ? Vl[kk] : 0.f;
-            }
-            bf16x8 bh, bl;
-            split8(x, bh, bl);
-            acc = mfma_split(a.iC + ((wave * 2 + ks) * 64 + lane) * 2, bh, bl, acc);
-        }
-        if (cok) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int n2 = 8 * wave + 2 * q + h;
-                if (n2 < N2)
-                    Cs[(ln * K1 + k1) * N2 + n2] =
-                        cmulcf(make_float2(acc[2 * h], acc[2 * h + 1]), a.twC[n2 * K1 + k1]);
-            }
-        }
-    }
-    __syncthreads();
-    // ---- step A': wave w owns column tiles (line, n2) kXL/2 w .. kXL/2 (w+1),
-    // both row tiles (n1 = 16 rt + 4 q + r)
-    float *o = smx;  // kXL*N floats inside the Vs area, which is no longer read
-    for (int ct = wave * (kXL / 2); ct < (wave + 1) * (kXL / 2); ++ct) {
-        const int col = ct * 16 + c16;
-        const int ln = small_div(col, rN2), n2 = col - ln * N2;
-        const bool cok = col < kXL * N2;
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int kk = 8 * q + e, k1 = kk >> 1;  // (k1, re/im)
-            x[e] = (cok && k1 < K1) ? reinterpret_cast<const float *>(Cs + (ln * K1 + k1) * N2 + n2)[kk & 1] : 0.f;
-        }
-        bf16x8 bh, bl;
-        split8(x, bh, bl);
-        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-        const f32x4 acc0 = mfma_split(a.iA + (0 * 64 + lane) * 2, bh, bl, z);
-        const f32x4 acc1 = mfma_split(a.iA + (1 * 64 + lane) * 2, bh, bl, z);
-        if (cok) {
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const int n1 = 16 * (r / 4) + 4 * q + (r % 4);
-                if (n1 < N1) {
-                    const int n = N2 * n1 + n2;
-                    const int pos = (n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1;
-                    o[ln * N + pos] = (r < 4 ? acc0[r % 4] : acc1[r % 4]) * a.scale;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // per-line output bases and (0,0) constants, then one element per thread
-    // and step (kXL = 2)
-    long long ob[kXL];
-    float ad[kXL];
-#pragma unroll
-    for (int l = 0; l < kXL; ++l) {
-        const int c = min(line0 + l, a.C - 1), c1 = c % a.C1, c2 = c / a.C1;
-        ob[l] = fidx(d, 1, c1 + 1, c2 + 1);
-        ad[l] = (float)add[c1];
-    }
-    for (int idx = tid; idx < kXL * N; idx += 256) {
-        const int l = idx >= N ? 1 : 0, n = idx - l * N;
-        if (line0 + l >= a.C) continue;
-        phi[ob[l] + n] = o[idx] + ad[l];
-    }
-}
-
-// ------------------------------------------------------------------------
 // pseudo-pressure rhs (projection.f90:38-47) in compact lines
 // DIV[(m*NM + j)*NP + i] (cells i+1, j+1, m+1), and per x-z plane FP64
 // partial sums of the same divergence for the (0,0) mode: one wave = one y
@@ -1010,9 +654,17 @@ void build_mixed(Handle &h) {
     auto sz = [&](int k, int m) { return sinl(2.0L * pi * (long double)(((long long)k * m) % M) / M); };
     const long double nm = (long double)N * (long double)M;
     std::vector<uint16_t> t[8];
-    split_matrix(N, N, rpx, h.kpx, [&](int k, int n) { return 2.0L * cosx(k, n); }, t[0], t[1]);
-    split_matrix(N, N, rpx, h.kpx,
-                 [&](int n, int k) { return (k == 0 ? 0.5L : 1.0L) * cosx(k, n) / nm; }, t[2], t[3]);
+    // N = N1 N2 with N1 the largest divisor <= sqrt(N); the dense x matrices
+    // only for the lengths that the two short DFTs do not take
+    h.dct_n1 = 1;
+    for (int a = 1; (long long)a * a <= N; ++a)
+        if (N % a == 0) h.dct_n1 = a;
+    h.mx_two = dct_fits_mixed(N, h.dct_n1);
+    if (!h.mx_two) {
+        split_matrix(N, N, rpx, h.kpx, [&](int k, int n) { return 2.0L * cosx(k, n); }, t[0], t[1]);
+        split_matrix(N, N, rpx, h.kpx,
+                     [&](int n, int k) { return (k == 0 ? 0.5L : 1.0L) * cosx(k, n) / nm; }, t[2], t[3]);
+    }
     split_matrix(M, M, rpz, h.kpz,
                  [&](int q, int m) -> long double {
                      if (q == 0) return 1.0L;
@@ -1035,6 +687,7 @@ void build_mixed(Handle &h) {
                                      &h.zf_hi,  &h.zf_lo,  &h.zi_hi,  &h.zi_lo};
     size_t off = 0;
     for (int q = 0; q < 8; ++q) {
+        if (t[q].empty()) continue;
         BL_HIP(hipMemcpyAsync(h.mx_tab + off, t[q].data(), t[q].size() * sizeof(uint16_t), hipMemcpyHostToDevice,
                               h.stream));
         *dst[q] = h.mx_tab + off;
@@ -1064,96 +717,6 @@ void build_mixed(Handle &h) {
         BL_HIP(hipMemcpyAsync(h.zmf, zf.data(), zf.size() * sizeof(uint16_t), hipMemcpyHostToDevice, h.stream));
         h.zmf_rt = RT;
     }
-    // two-factor x transform (k_xfwd_mx / k_xinv_mx) when N = N1 N2 fits it
-    {
-        // N = N1 N2 with N1 the largest divisor <= sqrt(N), as for the FP64 tables
-        int n1 = 1;
-        for (int a = 1; (long long)a * a <= N; ++a)
-            if (N % a == 0) n1 = a;
-        h.dct_n1 = n1;
-        const int n2 = N / n1, k1n = n1 / 2 + 1;
-        h.mx_two = n1 <= 32 && k1n <= 16 && n2 <= 32;
-        if (h.mx_two) {
-            auto cis = [&](long long num, long long den) {  // e^{-2 pi i num/den}, exact reduction
-                const long double ang = -2.0L * pi * (long double)(num % den) / (long double)den;
-                return std::pair<long double, long double>(cosl(ang), sinl(ang));
-            };
-            // one table: tiles x ks x 64 lanes x (hi, lo) x 8 k values
-            auto frag = [&](int tiles, int ks_n, auto f) {
-                std::vector<uint16_t> t((size_t)tiles * ks_n * 64 * 16, 0);
-                for (int rt = 0; rt < tiles; ++rt)
-                    for (int ks = 0; ks < ks_n; ++ks)
-                        for (int l = 0; l < 64; ++l)
-                            for (int e = 0; e < 8; ++e) {
-                                const float v = (float)f(rt, l % 16, 32 * ks + 8 * (l / 16) + e);
-                                const uint16_t hb = host_bf16(v);
-                                const size_t o = (((size_t)rt * ks_n + ks) * 64 + l) * 16;
-                                t[o + e] = hb;
-                                t[o + 8 + e] = host_bf16(v - host_bf16_float(hb));
-                            }
-                return t;
-            };
-            auto pair_row = [](int rt, int R, int &idx, int &part) {
-                idx = 8 * rt + 2 * (R / 4) + (R % 4) / 2;
-                part = R % 2;
-            };
-            std::vector<uint16_t> fA = frag(2, 1, [&](int rt, int R, int k) -> long double {
-                int k1, part;
-                pair_row(rt, R, k1, part);
-                if (k1 >= k1n || k >= n1) return 0.0L;
-                const auto w = cis((long long)k * k1, n1);
-                return part == 0 ? w.first : w.second;
-            });
-            std::vector<uint16_t> fC = frag(4, 2, [&](int rt, int R, int k) -> long double {
-                int k2, part;
-                pair_row(rt, R, k2, part);
-                const int nn = k / 2, pin = k % 2;
-                if (k2 >= n2 || nn >= n2) return 0.0L;
-                const auto w = cis((long long)nn * k2, n2);
-                return part == 0 ? (pin == 0 ? w.first : -w.second) : (pin == 0 ? w.second : w.first);
-            });
-            std::vector<uint16_t> iC = frag(4, 2, [&](int rt, int R, int k) -> long double {
-                int nn, part;
-                pair_row(rt, R, nn, part);
-                const int k2 = k / 2, pin = k % 2;
-                if (nn >= n2 || k2 >= n2) return 0.0L;
-                const auto w = cis((long long)nn * k2, n2);
-                return part == 0 ? (pin == 0 ? w.first : w.second) : (pin == 0 ? -w.second : w.first);
-            });
-            std::vector<uint16_t> iA = frag(2, 1, [&](int rt, int R, int k) -> long double {
-                const int nn1 = 16 * rt + R, k1 = k / 2, pin = k % 2;
-                if (nn1 >= n1 || k1 >= k1n) return 0.0L;
-                const long double c = (k1 == 0 || (n1 % 2 == 0 && k1 == n1 / 2)) ? 1.0L : 2.0L;
-                const auto w = cis((long long)nn1 * k1, n1);
-                return c * (pin == 0 ? w.first : w.second);
-            });
-            // twA [k1][n2], twC [n2][k1] (n2 k1 < N), rot
-            std::vector<float> tw;
-            auto push = [&](std::pair<long double, long double> w) {
-                tw.push_back((float)w.first);
-                tw.push_back((float)w.second);
-            };
-            for (int k1 = 0; k1 < k1n; ++k1)
-                for (int nn = 0; nn < n2; ++nn) push(cis((long long)nn * k1, N));
-            for (int nn = 0; nn < n2; ++nn)
-                for (int k1 = 0; k1 < k1n; ++k1) push(cis((long long)nn * k1, N));
-            for (int q = 0; q < N; ++q) push(cis(q, 4LL * N));
-            const size_t nb = (fA.size() + fC.size() + iC.size() + iA.size()) * sizeof(uint16_t) + tw.size() * 4;
-            BL_HIP(hipMalloc(&h.mx2, nb));
-            char *base = reinterpret_cast<char *>(h.mx2);
-            size_t off = 0;
-            const void **dst[4] = {(const void **)&h.x2_fA, (const void **)&h.x2_fC, (const void **)&h.x2_iC,
-                                   (const void **)&h.x2_iA};
-            std::vector<uint16_t> *src[4] = {&fA, &fC, &iC, &iA};
-            for (int t = 0; t < 4; ++t) {
-                BL_HIP(hipMemcpyAsync(base + off, src[t]->data(), src[t]->size() * 2, hipMemcpyHostToDevice, h.stream));
-                *dst[t] = base + off;
-                off += src[t]->size() * 2;
-            }
-            BL_HIP(hipMemcpyAsync(base + off, tw.data(), tw.size() * 4, hipMemcpyHostToDevice, h.stream));
-            h.x2_tw = reinterpret_cast<const float *>(base + off);
-        }
-    }
     // FP64 (0,0) mode scratch: per-line (two-factor path) or per-block plane
     // partials of the divergence, then phi00/(2NM)
     h.np00 = h.mx_two ? M : ((N + 63) / 64) * M;
@@ -1175,35 +738,8 @@ void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const BcP
     const int N = d.N, M = d.M, NM = d.NM, NP = h.NP;
     float *S = reinterpret_cast<float *>(h.S);
     float *T1 = reinterpret_cast<float *>(h.T1);
-    XArgs xa{};
-    if (h.mx_two) {
-        xa.N = N;
-        xa.N1 = h.dct_n1;
-        xa.N2 = N / h.dct_n1;
-        xa.K1h = h.dct_n1 / 2;
-        xa.NP = NP;
-        xa.C1 = NM;
-        xa.C = NM * M;
-        xa.M = M;
-        xa.fA = reinterpret_cast<const u16x8 *>(h.x2_fA);
-        xa.fC = reinterpret_cast<const u16x8 *>(h.x2_fC);
-        xa.iC = reinterpret_cast<const u16x8 *>(h.x2_iC);
-        xa.iA = reinterpret_cast<const u16x8 *>(h.x2_iA);
-        xa.twA = reinterpret_cast<const float2 *>(h.x2_tw);
-        xa.twC = xa.twA + (xa.K1h + 1) * xa.N2;
-        xa.rot = xa.twC + (xa.K1h + 1) * xa.N2;
-        xa.scale = (float)(1.0 / ((double)N * (double)M));
-    }
-    const int K1 = h.dct_n1 / 2 + 1, N2 = N / h.dct_n1;
-    const dim3 xgrid((NM * M + kXL - 1) / kXL);
-    if (h.mx_two) {
-        // divergence, FP64 line sums and forward x transform in one kernel
-        ProfScope ps(h, KID_XFORM_X_FWD);
-        const size_t lds = sizeof(float) * (size_t)kXL * N + sizeof(float2) * (size_t)kXL * K1 * N2;
-        hipLaunchKernelGGL(k_xfwd_mx, xgrid, dim3(256), lds, h.stream, d, h.m, xa, f.u, f.v, f.w, T1, h.p00, bc,
-                           src, use_inc);
-        check();
-    }
+    // divergence, FP64 line sums and forward x transform in one kernel
+    if (h.mx_two) launch_xfwd_mixed(h, f, T1, bcp, inc);
     // rhs: divergence lines into S (as scratch), FP64 plane partials
     if (!h.mx_two) {
         ProfScope ps(h, KID_DIVERGENCE);
@@ -1278,10 +814,7 @@ void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const BcP
     g.o_c2 = d.sxy;
     g.add = h.c00;
     if (h.mx_two) {
-        ProfScope ps(h, KID_XFORM_X_INV);
-        const size_t lds = 2 * sizeof(float2) * (size_t)kXL * K1 * N2;
-        hipLaunchKernelGGL(k_xinv_mx, xgrid, dim3(256), lds, h.stream, d, xa, T1, h.c00, phi);
-        check();
+        launch_xinv_mixed(h, T1, h.c00, phi);
     } else {
         gemm<kWRx, kWCx, kBKx, true, true>(h, KID_XFORM_X_INV, g);
     }

@@ -196,3 +196,33 @@ def test_field_transfers(shape, precision):
         want = a.astype(np.float32).astype(np.float64) if precision else a
         np.testing.assert_array_equal(s.download(f), want)
     s.close()
+
+
+# the FP32 x transform takes lengths up to 256 points per factor, the dense
+# product the others: both sides of that rule, primes and 31 x 31.  The pressure
+# recorded by one mixed projection against the FP64 one of the same FP32 fields.
+# The largest errors on the way are those of the split-BF16 products along z: the
+# two-term split of either operand and the dropped low x low product are 2^-18
+# of a product each, 1.1e-5 in all if every term had the same sign, twice (forward
+# and inverse); with the FP32 roundings of the x transforms and of what is stored
+# between them (6e-8 each) 5e-5 of the norm is twice that.
+@pytest.mark.parametrize("n,ny,nz", [(4, 5, 6), (127, 6, 8), (251, 7, 6), (257, 6, 7), (514, 5, 6), (961, 7, 6)])
+def test_x_transform_lengths_mixed(n, ny, nz):
+    say("mixed x transform", n, ny, nz)
+    rng = np.random.default_rng(n)
+    nx = n + 2
+    x = 1.0 + 0.001 * np.arange(nx)
+    y = np.cumsum(np.r_[0, 0.002 + 0.0005 * rng.random(ny - 1)])
+    z = 0.0015 * np.arange(nz)
+    shapes = [(nx, ny + 1, nz + 1), (nx + 1, ny, nz + 1), (nx + 1, ny + 1, nz)]
+    f = [np.asfortranarray(rng.standard_normal(sh).astype(np.float32).astype(np.float64)) for sh in shapes]
+    P = []
+    for precision in (0, 1):
+        s = solver(x, y, z, precision=precision)
+        s.set_fields(*f)
+        s.projection(1, 1e-4)
+        P.append(s.download(3)[1:n + 1, 1:ny, 1:nz - 1])
+        s.close()
+    err = np.linalg.norm(P[1] - P[0]) / np.linalg.norm(P[0])
+    say("err", err)
+    assert err < 5e-5
