@@ -25,6 +25,7 @@
 // Delta^2 |S|.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -297,39 +298,28 @@ __global__ __launch_bounds__(256) void k_samples(Coarsen cz, Metrics mc, const d
 }
 
 // ------------------------------------------------------------------------
-// BF16 MFMA inference of the network for 64 cells per wave
+// BF16 MFMA inference of the network for 64 cells per wave, four column tiles of
+// 16 cells: D = W h on v_mfma_f32_16x16x32_bf16 (lane l holds A[l%16][8 (l/16) + e],
+// B[8 (l/16) + e][l%16], e < 8, and D[4 (l/16) + r][l%16], r < 4).  The hidden
+// features are numbered along K so that the eight B values of a lane are the
+// accumulator rows it already holds, feature 32 s + 16 (e/4) + 4 (l/16) + e%4 at
+// K step s, so activations never leave the registers; the weights lie in LDS as
+// ready A fragments, read as 16 consecutive bytes per lane.  Bound by the SiLU
+// evaluations (192 per lane) and the FP64 features: 25 us per stage at 129x49x34.
+// With the activations passing through a 64 x 64 LDS tile (16-way bank conflicts
+// on its reads and the weights') the closure took 52 us there.
 // ------------------------------------------------------------------------
-// LDS weights: BF16 W1 [64][32] (inputs padded to 32), W2, W3 [64][64],
-// W4 as a [16][64] block with row 0 = W4; FP32 biases.
+constexpr int kFrag1 = 0, kFrag2 = 4, kFrag3 = 12, kFrag4 = 20, kFrags = 22;  // first fragment of each layer
 struct InferLds {
-    unsigned short w1[kH * 32], w2[kH * kH], w3[kH * kH], w4[16 * kH];
-    float b1[kH], b2[kH], b3[kH], b4;
+    u16x8 w[kFrags * 64];
+    float b[3 * kH];
+    float b4;
 };
 
 __device__ void load_infer_weights(InferLds &L, const unsigned short *__restrict__ wbf, const float *__restrict__ bias) {
-    constexpr int n1 = kH * 32, n2 = kH * kH, n4 = 16 * kH;
-    for (int q = threadIdx.x; q < n1 + 2 * n2 + n4; q += blockDim.x) {
-        const unsigned short v = wbf[q];
-        if (q < n1)
-            L.w1[q] = v;
-        else if (q < n1 + n2)
-            L.w2[q - n1] = v;
-        else if (q < n1 + 2 * n2)
-            L.w3[q - n1 - n2] = v;
-        else
-            L.w4[q - n1 - 2 * n2] = v;
-    }
-    for (int q = threadIdx.x; q < 3 * kH + 1; q += blockDim.x) {
-        const float v = bias[q];
-        if (q < kH)
-            L.b1[q] = v;
-        else if (q < 2 * kH)
-            L.b2[q - kH] = v;
-        else if (q < 3 * kH)
-            L.b3[q - 2 * kH] = v;
-        else
-            L.b4 = v;
-    }
+    for (int q = threadIdx.x; q < kFrags * 64; q += blockDim.x) L.w[q] = reinterpret_cast<const u16x8 *>(wbf)[q];
+    for (int q = threadIdx.x; q < 3 * kH; q += blockDim.x) L.b[q] = bias[q];
+    if (threadIdx.x == 0) L.b4 = bias[3 * kH];
 }
 
 __device__ __forceinline__ unsigned short to_bf16(float x) { return __builtin_bit_cast(unsigned short, (__bf16)x); }
@@ -337,76 +327,76 @@ __device__ __forceinline__ unsigned short to_bf16(float x) { return __builtin_bi
 // rounded to BF16 next); finite for all finite z: exp(-z) = inf gives z * 0
 __device__ __forceinline__ float silu(float z) { return z * __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
 
-// one hidden layer of a wave's 64 cells: act[cell][0..K) (BF16) times W^T
-// (W stored [64 outputs][K]), bias, SiLU, written back to act[cell][0..64)
-template <int K>
-__device__ __forceinline__ void hidden_layer(const unsigned short *Wt, const float *bias, unsigned short *act) {
-    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
-    constexpr int KS = K / 32;
-    bf16x8 a[4][KS];
+// one hidden layer: KS K steps from fragment f0, inputs h[ks][tile], outputs
+// SiLU(W h + b) as the next layer's inputs
+template <int KS>
+__device__ __forceinline__ void hidden_layer(const InferLds &L, int f0, const float *bias, const bf16x8 (&h)[2][4],
+                                             bf16x8 (&out)[2][4]) {
+    const int lane = threadIdx.x & 63, lq = lane >> 4;
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
+    for (int s = 0; s < 2; ++s) {  // output tiles 2 s and 2 s + 1 make K step s of the next layer
+        f32x4 z[2][4];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-            a[cb][ks] = __builtin_bit_cast(
-                bf16x8, *reinterpret_cast<const u16x8 *>(act + (cb * 16 + l16) * kH + ks * 32 + 8 * lq));
-    __builtin_amdgcn_wave_barrier();
-    // one 16-output block at a time keeps the register count low enough for
-    // two waves per SIMD (the LDS use allows two blocks per CU)
-#pragma unroll 1
-    for (int ob = 0; ob < 4; ++ob) {
-        f32x4 acc[4];
+        for (int t = 0; t < 2; ++t) {
+            const f32x4 b = *reinterpret_cast<const f32x4 *>(bias + 16 * (2 * s + t) + 4 * lq);
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int c = 0; c < 4; ++c) z[t][c] = b;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const bf16x8 b =
-                __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8 *>(Wt + (ob * 16 + l16) * K + ks * 32 + 8 * lq));
+            for (int ks = 0; ks < KS; ++ks) {
+                const bf16x8 a = __builtin_bit_cast(bf16x8, L.w[(f0 + (2 * s + t) * KS + ks) * 64 + lane]);
 #pragma unroll
-            for (int cb = 0; cb < 4; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[cb][ks], b, acc[cb], 0, 0, 0);
+                for (int c = 0; c < 4; ++c) z[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[ks][c], z[t][c], 0, 0, 0);
+            }
         }
-        const int feat = ob * 16 + l16;
-        const float bv = bias[feat];
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
+        for (int c = 0; c < 4; ++c) {
+            u16x8 v;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) act[(cb * 16 + 4 * lq + r) * kH + feat] = to_bf16(silu(acc[cb][r] + bv));
+            for (int e = 0; e < 8; ++e) v[e] = to_bf16(silu(z[e >> 2][c][e & 3]));
+            out[s][c] = __builtin_bit_cast(bf16x8, v);
+        }
     }
-    __builtin_amdgcn_wave_barrier();
 }
 
-// act: this wave's [64 cells][64] BF16 activation buffer; on entry row
-// `lane` holds the lane's 10 features in columns 0..9 (others zero).
-// Returns the network output for the lane's cell.
-__device__ float infer_wave(const InferLds &L, unsigned short *act, float *outb) {
+// the network output for the lane's cell from its features
+__device__ float infer_wave(const InferLds &L, const float (&f)[kMlpIn]) {
     const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
-    hidden_layer<32>(L.w1, L.b1, act);
-    hidden_layer<kH>(L.w2, L.b2, act);
-    hidden_layer<kH>(L.w3, L.b3, act);
-    // output layer: W4 as the first of 16 output columns
-    bf16x8 a[4][2];
+    // B fragments of the first layer: lanes of quarter 0 take features 0..7 of
+    // their column's cell, quarter 1 features 8 and 9, the others none
+    int p[kMlpIn / 2];
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
+    for (int q = 0; q < kMlpIn / 2; ++q) p[q] = (int)to_bf16(f[2 * q]) | ((int)to_bf16(f[2 * q + 1]) << 16);
+    bf16x8 h[2][4], g[2][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        int v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int x = __shfl(p[q], 16 * c + l16);
+            v[q] = lq == 0 ? x : 0;
+        }
+        const int y = __shfl(p[4], 16 * c + l16);
+        if (lq == 1) v[0] = y;
+        typedef int i32x4 __attribute__((ext_vector_type(4)));
+        h[0][c] = __builtin_bit_cast(bf16x8, (i32x4){v[0], v[1], v[2], v[3]});
+    }
+    hidden_layer<1>(L, kFrag1, L.b, h, g);
+    hidden_layer<2>(L, kFrag2, L.b + kH, g, h);
+    hidden_layer<2>(L, kFrag3, L.b + 2 * kH, h, g);
+    // output layer: W4 as row 0 of a 16-row tile, so cell 16 c + l16's output is
+    // the first accumulator row of lane l16 (quarter 0) of tile c
+    float out = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
-            a[cb][ks] =
-                __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8 *>(act + (cb * 16 + l16) * kH + ks * 32 + 8 * lq));
-    f32x4 o[4];
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) o[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        const bf16x8 b = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8 *>(L.w4 + l16 * kH + ks * 32 + 8 * lq));
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) o[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[cb][ks], b, o[cb], 0, 0, 0);
+            o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, L.w[(kFrag4 + ks) * 64 + lane]),
+                                                        g[ks][c], o, 0, 0, 0);
+        const float x = __shfl(o[0], l16);
+        if (lq == c) out = x;
     }
-    if (l16 == 0)
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) outb[cb * 16 + 4 * lq + r] = o[cb][r] + L.b4;
-    __builtin_amdgcn_wave_barrier();
-    return outb[lane];
+    return out + L.b4;
 }
 
 // inference on feature rows (parity checks): x[n][10] -> y[n]
@@ -414,71 +404,63 @@ __global__ __launch_bounds__(256) void k_infer_rows(const unsigned short *__rest
                                                     const float *__restrict__ bias, const float *__restrict__ x,
                                                     long long n, float *__restrict__ y) {
     __shared__ InferLds L;
-    __shared__ unsigned short act[4][64 * kH];
-    __shared__ float outb[4][64];
     load_infer_weights(L, wbf, bias);
     __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long cell = ((long long)blockIdx.x * 4 + wave) * 64 + lane;
-    unsigned short *A = act[wave];
-    for (int q = 0; q < kH; ++q) A[lane * kH + q] = 0;
-    if (cell < n)
-        for (int q = 0; q < kMlpIn; ++q) A[lane * kH + q] = to_bf16(x[cell * kMlpIn + q]);
-    __builtin_amdgcn_wave_barrier();
-    const float c = infer_wave(L, A, outb[wave]);
+    const long long cell = (long long)blockIdx.x * 256 + threadIdx.x;
+    float f[kMlpIn];
+#pragma unroll
+    for (int q = 0; q < kMlpIn; ++q) f[q] = cell < n ? x[cell * kMlpIn + q] : 0.f;
+    const float c = infer_wave(L, f);
     if (cell < n) y[cell] = c;
 }
 
 // LES = 4: per interior cell, the network's eddy viscosity or the DSM value
-// already in nu_t when a feature is out of range; fallback counts per block.
+// already in nu_t when a feature is out of range; fallback counts per 256 cells.
 template <class T>
-__global__ __launch_bounds__(256) void k_closure(Dims d, Metrics m, const T *__restrict__ U, const T *__restrict__ V,
+__global__ __launch_bounds__(256, 4) void k_closure(Dims d, Metrics m, const T *__restrict__ U, const T *__restrict__ V,
                                                  const T *__restrict__ W,
                                                  const unsigned short *__restrict__ wbf, const float *__restrict__ bias,
                                                  const float *__restrict__ lo, const float *__restrict__ hi,
-                                                 double inv_d99, int dirichlet, T *__restrict__ nu_t,
+                                                 double inv_d99, int dirichlet, T *__restrict__ nu_t, int nblk,
                                                  double *__restrict__ cnt) {
     __shared__ InferLds L;
-    __shared__ unsigned short act[4][64 * kH];
-    __shared__ float outb[4][64];
     __shared__ int nfb[4];
     load_infer_weights(L, wbf, bias);
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long long ni = d.nxg - 2, nj = d.nyg - 2, nk = d.nzg - 2;
-    const long long cell = ((long long)blockIdx.x * 4 + wave) * 64 + lane;
-    const bool live = cell < ni * nj * nk;
-    int i = 1, j = 1, k = 1;
-    if (live) {
-        i = 1 + (int)(cell % ni);
-        j = 1 + (int)((cell / ni) % nj);
-        k = 1 + (int)(cell / (ni * nj));
-    }
-    CellFeat cf;
-    cell_features(d, m, U, V, W, i, j, k, inv_d99, cf);
-    bool fb = false;
+    for (int blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
+        const long long cell = (long long)blk * 256 + threadIdx.x;
+        const bool live = cell < ni * nj * nk;
+        int i = 1, j = 1, k = 1;
+        if (live) {
+            i = 1 + (int)(cell % ni);
+            j = 1 + (int)((cell / ni) % nj);
+            k = 1 + (int)(cell / (ni * nj));
+        }
+        CellFeat cf;
+        cell_features(d, m, U, V, W, i, j, k, inv_d99, cf);
+        bool fb = false;
 #pragma unroll
-    for (int q = 0; q < kMlpIn; ++q) fb = fb || (cf.f[q] < lo[q]) || (cf.f[q] > hi[q]);
-    unsigned short *A = act[wave];
-    for (int q = 0; q < kH; ++q) A[lane * kH + q] = 0;
-    for (int q = 0; q < kMlpIn; ++q) A[lane * kH + q] = to_bf16(cf.f[q]);
-    __builtin_amdgcn_wave_barrier();
-    const float c = infer_wave(L, A, outb[wave]);
-    if (live && !fb) {
-        // the cell and, next to a y boundary, its ghost (apply_Neumann_bc_y /
-        // apply_Dirichlet_bc_y on nu_t, subgrid.f90:406-411); DSM cells keep
-        // the ghosts the DSM pass wrote
-        const T v = (T)(fmax((double)c, 0.0) * cf.scale);
-        const T sg = dirichlet == 1 ? (T)-1 : (T)1;
-        nu_t[fidx(d, i, j, k)] = v;
-        if (j == 1) nu_t[fidx(d, i, 0, k)] = sg * v;
-        if (j == d.nyg - 2) nu_t[fidx(d, i, d.nyg - 1, k)] = sg * v;
+        for (int q = 0; q < kMlpIn; ++q) fb = fb || (cf.f[q] < lo[q]) || (cf.f[q] > hi[q]);
+        const float c = infer_wave(L, cf.f);
+        if (live && !fb) {
+            // the cell and, next to a y boundary, its ghost (apply_Neumann_bc_y /
+            // apply_Dirichlet_bc_y on nu_t, subgrid.f90:406-411); DSM cells keep
+            // the ghosts the DSM pass wrote
+            const T v = (T)(fmax((double)c, 0.0) * cf.scale);
+            const T sg = dirichlet == 1 ? (T)-1 : (T)1;
+            nu_t[fidx(d, i, j, k)] = v;
+            if (j == 1) nu_t[fidx(d, i, 0, k)] = sg * v;
+            if (j == d.nyg - 2) nu_t[fidx(d, i, d.nyg - 1, k)] = sg * v;
+        }
+        // fallback count of the 256 cells
+        const unsigned long long bal = __ballot(live && fb);
+        if (lane == 0) nfb[wave] = __popcll(bal);
+        __syncthreads();
+        if (threadIdx.x == 0) cnt[blk] = (double)(nfb[0] + nfb[1] + nfb[2] + nfb[3]);
+        __syncthreads();
     }
-    // fallback count of the block
-    const unsigned long long bal = __ballot(live && fb);
-    if (lane == 0) nfb[wave] = __popcll(bal);
-    __syncthreads();
-    if (threadIdx.x == 0) cnt[blockIdx.x] = (double)(nfb[0] + nfb[1] + nfb[2] + nfb[3]);
 }
 
 // per-feature min / max / sum / sum of squares over weighted rows, per block
@@ -542,8 +524,8 @@ void check() {
 
 }  // namespace
 
-// host: BF16 inference weights from the FP32 master parameters, in the LDS
-// order of load_infer_weights, and the FP32 biases
+// host: BF16 inference weights from the FP32 master parameters as the A fragments
+// of infer_wave, [fragment][lane][8], and the FP32 biases
 void closure_weights(const float *theta, std::vector<unsigned short> &wbf, std::vector<float> &bias) {
     auto bf = [](float x) {
         uint32_t u;
@@ -553,14 +535,23 @@ void closure_weights(const float *theta, std::vector<unsigned short> &wbf, std::
     };
     const float *W1 = theta, *b1 = W1 + kH * kMlpIn, *W2 = b1 + kH, *b2 = W2 + kH * kH, *W3 = b2 + kH,
                 *b3 = W3 + kH * kH, *W4 = b3 + kH, *b4 = W4 + kH;
-    wbf.assign(kH * 32 + 2 * kH * kH + 16 * kH, 0);
-    for (int o = 0; o < kH; ++o)
-        for (int i = 0; i < kMlpIn; ++i) wbf[o * 32 + i] = bf(W1[o * kMlpIn + i]);
-    for (int q = 0; q < kH * kH; ++q) {
-        wbf[kH * 32 + q] = bf(W2[q]);
-        wbf[kH * 32 + kH * kH + q] = bf(W3[q]);
-    }
-    for (int i = 0; i < kH; ++i) wbf[kH * 32 + 2 * kH * kH + i] = bf(W4[i]);
+    wbf.assign((size_t)kFrags * 64 * 8, 0);
+    for (int l = 0; l < 64; ++l)
+        for (int e = 0; e < 8; ++e) {
+            const int row = l % 16, lq = l / 16;
+            auto at = [&](int frag) -> unsigned short & { return wbf[((size_t)frag * 64 + l) * 8 + e]; };
+            const int k = 8 * lq + e;
+            for (int o = 0; o < 4; ++o)
+                if (k < kMlpIn) at(kFrag1 + o) = bf(W1[(16 * o + row) * kMlpIn + k]);
+            for (int s = 0; s < 2; ++s) {
+                const int f = 32 * s + 16 * (e / 4) + 4 * lq + e % 4;
+                for (int o = 0; o < 4; ++o) {
+                    at(kFrag2 + 2 * o + s) = bf(W2[(16 * o + row) * kH + f]);
+                    at(kFrag3 + 2 * o + s) = bf(W3[(16 * o + row) * kH + f]);
+                }
+                if (row == 0) at(kFrag4 + s) = bf(W4[f]);
+            }
+        }
     bias.assign(3 * kH + 1, 0.f);
     for (int q = 0; q < kH; ++q) {
         bias[q] = b1[q];
@@ -603,14 +594,17 @@ void launch_closure(Handle &h, const Field3 &f) {
     }
     const Dims &d = h.d;
     ProfScope ps(h, KID_CLOSURE);
+    // as many blocks as fit at once (128 VGPRs, 23 KB of LDS: four per CU) load the
+    // weights once and loop over the cells
+    const dim3 grid(std::min(h.cl_nblk, 4 * std::max(1, h.n_cu)));
     if (h.precision == BL_PREC_MIXED) {
         const Fld3<float> ff = as<float>(f);
         float *nut = reinterpret_cast<float *>(h.nu_t);
-        hipLaunchKernelGGL(k_closure<float>, dim3(h.cl_nblk), dim3(256), 0, h.stream, d, h.m, ff.u, ff.v, ff.w, h.cl_w,
-                           h.cl_b, h.cl_lo, h.cl_hi, h.cl_inv_d99, h.nut_bc, nut, h.cl_cnt);
+        hipLaunchKernelGGL(k_closure<float>, grid, dim3(256), 0, h.stream, d, h.m, ff.u, ff.v, ff.w, h.cl_w, h.cl_b,
+                           h.cl_lo, h.cl_hi, h.cl_inv_d99, h.nut_bc, nut, h.cl_nblk, h.cl_cnt);
     } else {
-        hipLaunchKernelGGL(k_closure<double>, dim3(h.cl_nblk), dim3(256), 0, h.stream, d, h.m, f.u, f.v, f.w, h.cl_w,
-                           h.cl_b, h.cl_lo, h.cl_hi, h.cl_inv_d99, h.nut_bc, h.nu_t, h.cl_cnt);
+        hipLaunchKernelGGL(k_closure<double>, grid, dim3(256), 0, h.stream, d, h.m, f.u, f.v, f.w, h.cl_w, h.cl_b,
+                           h.cl_lo, h.cl_hi, h.cl_inv_d99, h.nut_bc, h.nu_t, h.cl_nblk, h.cl_cnt);
     }
     check();
 }

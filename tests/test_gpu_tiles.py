@@ -6,7 +6,7 @@ import sys
 import numpy as np
 import pytest
 
-from . import cases, mlp_ref as M, orc
+from . import cases, closure_ref as R, mlp_ref as M, orc
 from .blgpu_import import blgpu
 from .test_oracle_dsm import random_case
 
@@ -226,3 +226,36 @@ def test_x_transform_lengths_mixed(n, ny, nz):
     err = np.linalg.norm(P[1] - P[0]) / np.linalg.norm(P[0])
     say("err", err)
     assert err < 5e-5
+
+
+# the closure's blocks take 256 cells each and loop once there are more than four
+# per CU (262144 cells on 256 CUs); fewer cells than a wave's 64, and a remainder.
+# Every cell against the row inference of the same network, which no loop is in.
+# The features agree to FP64 rounding before the FP32 one, so a BF16 input of the
+# network differs only where that rounding crosses a BF16 midpoint: fewer than 1 %
+# of the cells, and there by no more than BF16 inference itself is off (5e-2).
+@pytest.mark.parametrize("nx,ny,nz", [(5, 4, 5), (33, 12, 9), (162, 62, 40)])
+def test_closure_blocks(nx, ny, nz):
+    say("closure blocks", nx, ny, nz)
+    x, y, z, U, V, W = random_case(nx + ny, nx, ny, nz)
+    s = solver(x, y, z, les=4)
+    s.set_fields(U, V, W)
+    c = blgpu.Closure(capacity=16, batch_max=16)
+    c.params = M.init_params(5).astype(np.float32)
+    rows = np.ones((2, blgpu.MLP_ROW), dtype=np.float32)
+    rows[1, :10] = -1.0
+    c.add_rows(rows)
+    d99 = 0.5 * y[-1]
+    c.install(s, d99, 1e30)
+    s.eddy_viscosity()
+    got = s.download(4)[1:-1, 1:-1, 1:-1]
+    f, _, _, scale = R.features(x, y, z, U, V, W, d99)
+    X = f.reshape(10, -1, order="F").T.astype(np.float32)
+    want = np.maximum(c.infer_bf16(X).reshape(f.shape[1:], order="F"), 0) * scale
+    assert s.closure_fallback() == (got.size, 0)
+    err = np.abs(got - want) / np.abs(want).max()
+    say("cells", got.size, "largest", err.max(), "beyond 1e-6", (err > 1e-6).mean())
+    assert err.max() < 5e-2
+    assert (err > 1e-6).mean() < 1e-2
+    c.close()
+    s.close()
