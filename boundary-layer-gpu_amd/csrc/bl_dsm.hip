@@ -96,48 +96,131 @@ __device__ __forceinline__ double at(PlanePtr<T> base, unsigned o) {
     return (double)*(PlanePtr<T>)((PlanePtr<char>)base + o * (unsigned)sizeof(T));
 }
 
-// compute_Sij at interior cell (i, j, k) with o = i + sx j: diagonal terms at
-// the centre, the off-diagonal terms averaged from the four surrounding edges;
-// returns |S|.
+// A plane as a buffer resource: an element is a scalar base, one register with
+// the byte offset of a cell's south-west neighbour (shared by all arrays of one
+// element size), a scalar row offset and an immediate column offset, and the
+// hardware returns 0 for whatever lies outside the plane.
 template <class T>
-__device__ __forceinline__ double strain(const Dims &d, const Metrics &m, const StrainMet &sm,
-                                         const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
-                                         unsigned o, int k, double s[6]) {
-    const unsigned sx = d.sx;
-    const double rz0 = m.rdzg[k - 1], rz1 = m.rdzg[k];
-    // planes k-1, k, k+1 (of W: k-1 and k)
-    const PlanePtr<T> Uc = plane_ptr(U + k * d.sxy), Vc = plane_ptr(V + k * d.sxy), Wc = plane_ptr(W + k * d.sxy);
-    const PlanePtr<T> Um = plane_ptr(U + (k - 1) * d.sxy), Up = plane_ptr(U + (k + 1) * d.sxy);
-    const PlanePtr<T> Vm = plane_ptr(V + (k - 1) * d.sxy), Vp = plane_ptr(V + (k + 1) * d.sxy);
-    const PlanePtr<T> Wm = plane_ptr(W + (k - 1) * d.sxy);
-    s[0] = (at<T>(Uc, o) - at<T>(Uc, o - 1)) * sm.rdx;
-    s[1] = (at<T>(Vc, o) - at<T>(Vc, o - sx)) * sm.rdy;
-    s[2] = (at<T>(Wc, o) - at<T>(Wm, o)) * m.rdz[k];
-    // edges (i + a, j + b, k), (i + a, j, k + c), (i, j + b, k + c)
-    auto e4 = [&](int a, int b) {
-        const unsigned q = o + a + (b ? sx : 0u);
-        return 0.5 * ((at<T>(Uc, q - 1) - at<T>(Uc, q - 1 - sx)) * (b ? sm.rdyg1 : sm.rdyg0) +
-                      (at<T>(Vc, q - sx) - at<T>(Vc, q - 1 - sx)) * (a ? sm.rdxg1 : sm.rdxg0));
-    };
-    auto e5 = [&](int a, int c) {
-        const unsigned q = o + a;
-        const PlanePtr<T> Wq = c ? Wc : Wm;
-        return 0.5 * ((at<T>(c ? Up : Uc, q - 1) - at<T>(c ? Uc : Um, q - 1)) * (c ? rz1 : rz0) +
-                      (at<T>(Wq, q) - at<T>(Wq, q - 1)) * (a ? sm.rdxg1 : sm.rdxg0));
-    };
-    auto e6 = [&](int b, int c) {
-        const unsigned q = o + (b ? sx : 0u);
-        const PlanePtr<T> Wq = c ? Wc : Wm;
-        return 0.5 * ((at<T>(c ? Vp : Vc, q - sx) - at<T>(c ? Vc : Vm, q - sx)) * (c ? rz1 : rz0) +
-                      (at<T>(Wq, q) - at<T>(Wq, q - sx)) * (b ? sm.rdyg1 : sm.rdyg0));
-    };
-    s[3] = 0.25 * (e4(0, 0) + e4(1, 0) + e4(0, 1) + e4(1, 1));
-    s[4] = 0.25 * (e5(0, 0) + e5(1, 0) + e5(0, 1) + e5(1, 1));
-    s[5] = 0.25 * (e6(0, 0) + e6(1, 0) + e6(0, 1) + e6(1, 1));
-    double a = 0.0;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const Dims &d, const T *p, long long k) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(p + k * d.sxy), 0, (int)(unsigned)(d.sxy * sizeof(T)), 0x00020000);
+}
+template <class T>
+__device__ __forceinline__ T buf_at(__amdgpu_buffer_rsrc_t r, unsigned sw, unsigned row, int col) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, sw + col * 4, row, 0));
+    else
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, sw + col * 8, row, 0));
+}
+
+// compute_Sij along z at one column of cells: diagonal terms at the centre, the
+// off-diagonal terms averaged from the four surrounding edges.  The average of
+// the edges' differences is the sum of the differences of the neighbouring
+// pairs, so a cell needs U at two points of five rows or planes, V likewise and W
+// at five points of two planes; what the next plane uses again stays in
+// registers (17 loads a plane instead of 30).  All loads of a plane are issued
+// together by load(); eval() uses them.
+template <class T>
+struct StrainMarch {
+    T u[2], v[2];          // plane k: U(i-1), U(i); V(j-1), V(j)
+    T um[2], vm[2], wm[5];  // plane k-1; W at the cell, i-1, i+1, j-1, j+1
+    T us[2], un[2], ve[2], vw[2], up[2], vp[2], w[5];
+
+    __device__ __forceinline__ static void load_u(const Dims &d, const T *U, unsigned sw, int k, T o[2]) {
+        const unsigned sxb = (unsigned)(d.sx * sizeof(T));
+        const auto r = plane_rsrc(d, U, k);
+        o[0] = buf_at<T>(r, sw, sxb, 0);
+        o[1] = buf_at<T>(r, sw, sxb, 1);
+    }
+    __device__ __forceinline__ static void load_v(const Dims &d, const T *V, unsigned sw, int k, T o[2]) {
+        const unsigned sxb = (unsigned)(d.sx * sizeof(T));
+        const auto r = plane_rsrc(d, V, k);
+        o[0] = buf_at<T>(r, sw, 0, 1);
+        o[1] = buf_at<T>(r, sw, sxb, 1);
+    }
+    __device__ __forceinline__ static void load_w(const Dims &d, const T *W, unsigned sw, int k, T o[5]) {
+        const unsigned sxb = (unsigned)(d.sx * sizeof(T));
+        const auto r = plane_rsrc(d, W, k);
+        o[0] = buf_at<T>(r, sw, sxb, 1);
+        o[1] = buf_at<T>(r, sw, sxb, 0);
+        o[2] = buf_at<T>(r, sw, sxb, 2);
+        o[3] = buf_at<T>(r, sw, 0, 1);
+        o[4] = buf_at<T>(r, sw, 2 * sxb, 1);
+    }
+    // what plane k takes from planes k-1 and k, at the start and where k jumps
+    __device__ __forceinline__ void begin(const Dims &d, const T *U, const T *V, const T *W, unsigned sw, int k) {
+        load_u(d, U, sw, k, u);
+        load_v(d, V, sw, k, v);
+        load_u(d, U, sw, k - 1, um);
+        load_v(d, V, sw, k - 1, vm);
+        load_w(d, W, sw, k - 1, wm);
+    }
+    __device__ __forceinline__ void load(const Dims &d, const T *U, const T *V, const T *W, unsigned sw, int k) {
+        const unsigned sxb = (unsigned)(d.sx * sizeof(T));
+        const auto ru = plane_rsrc(d, U, k), rv = plane_rsrc(d, V, k);
+        us[0] = buf_at<T>(ru, sw, 0, 0);
+        us[1] = buf_at<T>(ru, sw, 0, 1);
+        un[0] = buf_at<T>(ru, sw, 2 * sxb, 0);
+        un[1] = buf_at<T>(ru, sw, 2 * sxb, 1);
+        vw[0] = buf_at<T>(rv, sw, 0, 0);
+        vw[1] = buf_at<T>(rv, sw, sxb, 0);
+        ve[0] = buf_at<T>(rv, sw, 0, 2);
+        ve[1] = buf_at<T>(rv, sw, sxb, 2);
+        load_w(d, W, sw, k, w);
+        load_u(d, U, sw, k + 1, up);
+        load_v(d, V, sw, k + 1, vp);
+    }
+    // S_ij and |S| of plane k, the centred velocities too where asked for
+    __device__ __forceinline__ double eval(const Metrics &m, const StrainMet &sm, int k, double s[6],
+                                           double *c = nullptr) {
+        const double rz0 = m.rdzg[k - 1], rz1 = m.rdzg[k];
+        // the differences of a pair against the pair before and behind it
+        auto diff = [](const T a[2], const T b[2], double ra, const T e[2], double re) {
+            return (((double)b[0] - (double)a[0]) + ((double)b[1] - (double)a[1])) * ra +
+                   (((double)e[0] - (double)b[0]) + ((double)e[1] - (double)b[1])) * re;
+        };
+        const T wc[2] = {wm[0], w[0]}, ww[2] = {wm[1], w[1]}, we[2] = {wm[2], w[2]}, ws[2] = {wm[3], w[3]},
+                wn[2] = {wm[4], w[4]};
+        s[0] = ((double)u[1] - (double)u[0]) * sm.rdx;
+        s[1] = ((double)v[1] - (double)v[0]) * sm.rdy;
+        s[2] = ((double)w[0] - (double)wm[0]) * m.rdz[k];
+        s[3] = 0.125 * (diff(us, u, sm.rdyg0, un, sm.rdyg1) + diff(vw, v, sm.rdxg0, ve, sm.rdxg1));
+        s[4] = 0.125 * (diff(um, u, rz0, up, rz1) + diff(ww, wc, sm.rdxg0, we, sm.rdxg1));
+        s[5] = 0.125 * (diff(vm, v, rz0, vp, rz1) + diff(ws, wc, sm.rdyg0, wn, sm.rdyg1));
+        if (c) {
+            c[0] = 0.5 * ((double)u[0] + (double)u[1]);
+            c[1] = 0.5 * ((double)v[0] + (double)v[1]);
+            c[2] = 0.5 * ((double)wm[0] + (double)w[0]);
+        }
+        double a = 0.0;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) a = a + (c < 3 ? 2.0 : 4.0) * s[c] * s[c];
-    return sqrt(a);
+        for (int q = 0; q < 6; ++q) a = a + (q < 3 ? 2.0 : 4.0) * s[q] * s[q];
+        return sqrt(a);
+    }
+    __device__ __forceinline__ void next() {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            um[q] = u[q];
+            vm[q] = v[q];
+            u[q] = up[q];
+            v[q] = vp[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 5; ++q) wm[q] = w[q];
+    }
+};
+// byte offset of the south-west neighbour of (i, j), i, j >= 1
+template <class T>
+__device__ __forceinline__ unsigned sw_offset(const Dims &d, int i, int j) {
+    return (unsigned)(i - 1 + (int)d.sx * (j - 1)) * (unsigned)sizeof(T);
+}
+template <class T>
+__device__ __forceinline__ double strain(const Dims &d, const Metrics &m, const StrainMet &sm, const T *U, const T *V,
+                                         const T *W, int i, int j, int k, double s[6]) {
+    StrainMarch<T> q;
+    const unsigned sw = sw_offset<T>(d, i, j);
+    q.begin(d, U, V, W, sw, k);
+    q.load(d, U, V, W, sw, k);
+    return q.eval(m, sm, k, s);
 }
 
 // filter_xzy (subgrid.f90:140-187) is separable: its xz weights (4/9, 1/9,
@@ -230,130 +313,159 @@ __global__ __launch_bounds__(256) void k_dsm_vfilter(Dims d, const T *__restrict
 }
 
 // L:M and M:M.  A block owns 30 x 6 cells and a chunk of z planes and marches
-// in z.  Each of its 256 threads forms, at its cell of the tile with a
-// one-cell halo (32 x 8), the centred velocities, |S| and |S| S_ij of a plane
-// from the fields and leaves nine values in LDS (three more where a ghost
-// index is read unmapped); the threads of the inner cells then filter the
-// three velocities, six products and six |S| S_ij in x and y from LDS and in z
-// through two running values per quantity in registers.  Nothing but |S| and
-// the two sums per column and chunk goes to memory.  The work is FP64
-// arithmetic and LDS reads (81 per cell), two blocks per CU by its registers.
-// At 257x97x64 in FP32 fields the model's three passes take 0.024 + 0.153 +
-// 0.011 ms per stage; the form in which every cell read the 27 neighbours of
-// twelve FP64 arrays written by other passes took 0.04 + 0.07 + 0.53 + 0.05.
+// in z with two kinds of waves.  Four waves form, at each cell of the tile with a
+// one-cell halo (32 x 8), the centred velocities, |S| and |S| S_ij of a plane and
+// the filtered field's 4 |S^| S^_ij of the plane before and leave them in LDS (three
+// more values where a ghost index is read unmapped).  Three waves, one thread
+// per cell of the six inner rows, filter the three velocities, six products and
+// six |S| S_ij of the other buffer in y from LDS, in x between lanes and in z
+// through two running values per quantity in registers, and contract.  Nothing
+// but |S| and the two sums per column and chunk goes to memory.  Bound by
+// issue: FP64 arithmetic with two blocks (14 waves) per CU, 120 registers.
+// At 257x97x64 in FP32 fields the model's three passes take 0.022 + 0.064 +
+// 0.010 ms per stage.  With all steps in four waves, the edge differences one
+// by one, filters of 9 LDS reads and plain loads, which waited one after the
+// other, the middle one took 0.153; the form in which every cell read the 27
+// neighbours of twelve FP64 arrays written by other passes took 0.04 + 0.07 +
+// 0.53 + 0.05.  Tiles of 32 x 16 measured the same (0.063), loads of the
+// filtered field a plane ahead 0.093 (registers).
 constexpr int kDsX = 32, kDsY = 8;  // tile with its halo
 
+constexpr int kDsOwn = kDsX * (kDsY - 2);  // threads of the second role: its inner rows
+
+// the value of the lane one below (-1) or above (+1), its two halves by DPP
+template <int D>
+__device__ __forceinline__ double lane_shift(double x) {
+    const int2 v = __builtin_bit_cast(int2, x);
+    constexpr int ctl = D < 0 ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+    const int2 r = {__builtin_amdgcn_mov_dpp(v.x, ctl, 0xf, 0xf, true), __builtin_amdgcn_mov_dpp(v.y, ctl, 0xf, 0xf, true)};
+    return __builtin_bit_cast(double, r);
+}
+
 template <bool PX, class T>
-__global__ __launch_bounds__(256) void k_dsm_stress(Dims d, Metrics m, const T *__restrict__ U,
-                                                    const T *__restrict__ V, const T *__restrict__ W,
-                                                    const double *__restrict__ Uf, const double *__restrict__ Vf,
-                                                    const double *__restrict__ Wf, double *__restrict__ S,
-                                                    double *__restrict__ part, int chunk) {
-    __shared__ double sq[12][kDsX * kDsY];  // 0-2 centred velocities, 3-8 |S| S_ij (mapped), 9-11 velocities unmapped
-    const int tid = threadIdx.x, tx = tid % kDsX, ty = tid / kDsX;
+__global__ __launch_bounds__(kDsX *kDsY + kDsOwn, 4) void k_dsm_stress(
+    Dims d, Metrics m, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
+    const double *__restrict__ Uf, const double *__restrict__ Vf, const double *__restrict__ Wf, double *__restrict__ S,
+    double *__restrict__ part, int chunk) {
+    // per plane: 0-2 centred velocities, 3-8 |S| S_ij (both mapped), 9-11 velocities
+    // unmapped where that differs; of the plane before: 12-17 4 |S^| S^_ij, 18 |S|
+    __shared__ double sq[2][18 + PX][kDsX * kDsY];
+    const int role = __builtin_amdgcn_readfirstlane(threadIdx.x >= kDsX * kDsY);
     const int nbx = (d.nxg - 2 + kDsX - 3) / (kDsX - 2);
     const int bx = blockIdx.x % nbx, by = blockIdx.x / nbx;
+    // whether some cell of the tile has an x ghost index
+    const bool xghost = bx == 0 || bx * (kDsX - 2) + kDsX - 1 >= d.nxg - 2;
+    const int tid = role == 0 ? threadIdx.x : threadIdx.x - (kDsX * kDsY - kDsX), tx = tid % kDsX, ty = tid / kDsX;
     const int i = min(bx * (kDsX - 2) + tx, d.nxg - 1), j = min(by * (kDsY - 2) + ty, d.nyg - 1);
-    const int im = xmap_c<PX>(d, i);
     const bool row = j >= 1 && j <= d.nyg - 2;  // rows 0 and nyg-1 have weight 0 and no value
     const bool own = tx >= 1 && tx <= kDsX - 2 && ty >= 1 && ty <= kDsY - 2 && row && bx * (kDsX - 2) + tx <= d.nxg - 2 &&
                      by * (kDsY - 2) + ty <= d.nyg - 2;
-    // whether some cell of the tile has an x ghost index
-    const bool xghost = bx == 0 || bx * (kDsX - 2) + kDsX - 1 >= d.nxg - 2;
-    const int jc = max(1, min(j, d.nyg - 2));
-    const StrainMet sm = strain_met(m, im, jc);  // im = i at the cells whose results are used
-    const YWeights w = yweights(jc, 1, d.nyg - 2);
+    const int jc = clampi(j, 1, d.nyg - 2);
     const int kb = 1 + blockIdx.y * chunk, ke = min(kb + chunk, d.nzg - 2);  // planes 1..nzg-3
     const long long sxy = d.sxy;
-    const unsigned sx = d.sx, oi = i + sx * j, om = im + sx * j;
-    double last[15], pend[15], lmsum = 0.0, mmsum = 0.0, magp = 0.0;
+    const unsigned oi = i + (unsigned)d.sx * j;
+    // Both roles make the same steps kk and pass the same barrier in each: behind
+    // it the second reads the buffer that the first has left, the first fills the
+    // other one, which the second has read before it.
+    if (role == 0) {
+        const int im = xmap_c<PX>(d, i), ic = clampi(i, 1, d.nxg - 2);
+        // every lane's cell is inside, so that no load depends on a mask; im = i
+        // at the cells whose results are used
+        const unsigned swm = sw_offset<T>(d, im, jc), swf = sw_offset<double>(d, ic, jc);
+        const unsigned south = (unsigned)(i + (int)d.sx * (jc - 1)) * (unsigned)sizeof(T);  // unmapped, row j-1
+        const StrainMet sm = strain_met(m, im, jc);
+        StrainMarch<T> a;
+        StrainMarch<double> f;
+        double mag1 = 0.0;
+        a.begin(d, U, V, W, swm, zmap_c(d, kb - 1));
+        a.load(d, U, V, W, swm, zmap_c(d, kb - 1));
+        f.begin(d, Uf, Vf, Wf, swf, kb);
+        for (int kk = kb - 1; kk <= ke; ++kk) {
+            double(&o)[18 + PX][kDsX * kDsY] = sq[(kk - kb + 1) & 1];
+            const int km = zmap_c(d, kk);
+            double s[6], c[3];
+            const double mag = a.eval(m, sm, km, s, c);
 #pragma unroll
-    for (int q = 0; q < 15; ++q) last[q] = pend[q] = 0.0;
-    for (int kk = kb - 1; kk <= ke; ++kk) {
-        const int km = zmap_c(d, kk);
-        const bool ghost = xghost || km != kk;
-        double v[12], mag = 0.0;
+            for (int q = 0; q < 3; ++q) o[q][tid] = row ? c[q] : 0.0;
 #pragma unroll
-        for (int q = 0; q < 12; ++q) v[q] = 0.0;
-        if (row) {
-            double s[6];
-            const PlanePtr<T> Uk = plane_ptr(U + km * sxy), Vk = plane_ptr(V + km * sxy), Wk = plane_ptr(W + km * sxy);
-            const PlanePtr<T> Wb = plane_ptr(W + (km - 1) * sxy);
-            v[0] = 0.5 * (at<T>(Uk, om - 1) + at<T>(Uk, om));
-            v[1] = 0.5 * (at<T>(Vk, om - sx) + at<T>(Vk, om));
-            v[2] = 0.5 * (at<T>(Wb, om) + at<T>(Wk, om));
-            mag = strain(d, m, sm, U, V, W, om, km, s);
+            for (int q = 0; q < 6; ++q) o[3 + q][tid] = row ? mag * s[q] : 0.0;
+            if (xghost || km != kk) {  // U at the mapped x index
+                const unsigned sxb = (unsigned)(d.sx * sizeof(T));
+                const auto rv = plane_rsrc(d, V, kk), rw0 = plane_rsrc(d, W, km - 1), rw1 = plane_rsrc(d, W, km);
+                T g[6];
+                StrainMarch<T>::load_u(d, U, swm, kk, g);
+                g[2] = buf_at<T>(rv, south, 0, 0);
+                g[3] = buf_at<T>(rv, south, sxb, 0);
+                g[4] = buf_at<T>(rw0, south, sxb, 0);
+                g[5] = buf_at<T>(rw1, south, sxb, 0);
 #pragma unroll
-            for (int c = 0; c < 6; ++c) v[3 + c] = mag * s[c];
-            if (ghost) {
-                const PlanePtr<T> Ug = plane_ptr(U + kk * sxy), Vg = plane_ptr(V + kk * sxy);
-                v[9] = 0.5 * (at<T>(Ug, om - 1) + at<T>(Ug, om));
-                v[10] = 0.5 * (at<T>(Vg, oi - sx) + at<T>(Vg, oi));
-                v[11] = 0.5 * (at<T>(Wb, oi) + at<T>(Wk, oi));
+                for (int q = 0; q < 3; ++q) o[9 + q][tid] = row ? 0.5 * ((double)g[2 * q] + (double)g[2 * q + 1]) : 0.0;
             }
-            if (own && !PX) {
-                // nu_t reads |S| on planes 1..nzg-2, the duplicated plane's own value among them
-                if (kk >= kb && kk < ke)
-                    S[kk * sxy + oi] = mag;
-                else if (kk == d.nzg - 2)
-                    S[kk * sxy + oi] = strain(d, m, sm, U, V, W, oi, kk, s);
+            // nu_t reads |S| on planes 1..nzg-2
+            if (own && !PX && kk >= kb && kk < ke) S[kk * sxy + oi] = mag;
+            if (kk > kb) f.load(d, Uf, Vf, Wf, swf, kk - 1);
+            if (kk > kb) {
+                const double magh = f.eval(m, sm, kk - 1, s);
+#pragma unroll
+                for (int q = 0; q < 6; ++q) o[12 + q][tid] = 4.0 * magh * s[q];
+                if constexpr (PX) o[18][tid] = mag1;
+                f.next();
             }
+            mag1 = mag;
+            __builtin_amdgcn_sched_barrier(0);
+            a.next();
+            if (kk < ke) {
+                const int kn = zmap_c(d, kk + 1);
+                if (kn != km + 1) a.begin(d, U, V, W, swm, kn);
+                a.load(d, U, V, W, swm, kn);
+            }
+            __syncthreads();
         }
-        __syncthreads();  // the previous plane is read
+        if (!PX && own && ke == d.nzg - 2) {  // the duplicated plane's own value
+            double s[6];
+            S[ke * sxy + oi] = strain(d, m, sm, U, V, W, i, j, ke, s);
+        }
+    } else {
+        const YWeights w = yweights(jc, 1, d.nyg - 2);
+        double last[15], pend[15], lmsum = 0.0, mmsum = 0.0;
 #pragma unroll
-        for (int q = 0; q < 9; ++q) sq[q][tid] = v[q];
-        if (ghost)
-#pragma unroll
-            for (int q = 9; q < 12; ++q) sq[q][tid] = v[q];
-        __syncthreads();
-        if (own) {
-            auto filt_row = [&](double q0, double q1, double q2) { return w.m * q0 + w.c * q1 + w.p * q2; };
-            // the z part: the plane kk - 1 of quantity q is complete with this
-            // plane's value f
-            auto zstep = [&](int q, double f) {
+        for (int q = 0; q < 15; ++q) last[q] = pend[q] = 0.0;
+        for (int kk = kb - 1; kk <= ke; ++kk) {
+            const double(&o)[18 + PX][kDsX * kDsY] = sq[(kk - kb + 1) & 1];
+            const bool ghost = xghost || zmap_c(d, kk) != kk;
+            __syncthreads();
+            auto filt_y = [&](double q0, double q1, double q2) { return w.m * q0 + w.c * q1 + w.p * q2; };
+            auto filt_lds = [&](const double *Q) { return filt_y(Q[tid - kDsX], Q[tid], Q[tid + kDsX]); };
+            // the x part between lanes (a tile row's first and last lane are not
+            // its own), then the z part: the plane kk - 1 of quantity q is complete
+            // with this plane's value
+            auto xzstep = [&](int q, double g) {
+                const double f = kF0 * g + kF1 * (lane_shift<-1>(g) + lane_shift<1>(g));
                 const double h = pend[q] + kF1 * f;
                 pend[q] = kF1 * last[q] + kF0 * f;
                 last[q] = f;
                 return h;
             };
-            auto filt_lds = [&](const double *Q) {
-                double c[3];
-#pragma unroll
-                for (int a = 0; a < 3; ++a) c[a] = filt_row(Q[tid + a - 1 - kDsX], Q[tid + a - 1], Q[tid + a - 1 + kDsX]);
-                return kF1 * c[0] + kF0 * c[1] + kF1 * c[2];
-            };
-            // one group of quantities at a time: with all 81 LDS reads in
-            // flight the kernel took 390 registers
-            double L[6], hs[6];
+            double L[6];
             {
-                double f[6];
+                double x[3], y[3], z[3], h[3];
 #pragma unroll
-                for (int c = 0; c < 6; ++c) f[c] = 0.0;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    double x[3], y[3], z[3];
-#pragma unroll
-                    for (int r = 0; r < 3; ++r) {
-                        const int e = tid + a - 1 + (r - 1) * kDsX;
-                        x[r] = sq[0][e];
-                        y[r] = sq[1][e];
-                        z[r] = sq[2][e];
-                    }
-                    const double wx = a == 1 ? kF0 : kF1;
-                    f[0] += wx * filt_row(x[0] * x[0], x[1] * x[1], x[2] * x[2]);
-                    f[1] += wx * filt_row(y[0] * y[0], y[1] * y[1], y[2] * y[2]);
-                    f[2] += wx * filt_row(z[0] * z[0], z[1] * z[1], z[2] * z[2]);
-                    f[3] += wx * filt_row(x[0] * y[0], x[1] * y[1], x[2] * y[2]);
-                    f[4] += wx * filt_row(x[0] * z[0], x[1] * z[1], x[2] * z[2]);
-                    f[5] += wx * filt_row(y[0] * z[0], y[1] * z[1], y[2] * z[2]);
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int r = 0; r < 3; ++r) {
+                    const int e = tid + (r - 1) * kDsX;
+                    x[r] = o[0][e];
+                    y[r] = o[1][e];
+                    z[r] = o[2][e];
                 }
+                L[0] = xzstep(3, filt_y(x[0] * x[0], x[1] * x[1], x[2] * x[2]));
+                L[1] = xzstep(4, filt_y(y[0] * y[0], y[1] * y[1], y[2] * y[2]));
+                L[2] = xzstep(5, filt_y(z[0] * z[0], z[1] * z[1], z[2] * z[2]));
+                L[3] = xzstep(6, filt_y(x[0] * y[0], x[1] * y[1], x[2] * y[2]));
+                L[4] = xzstep(7, filt_y(x[0] * z[0], x[1] * z[1], x[2] * z[2]));
+                L[5] = xzstep(8, filt_y(y[0] * z[0], y[1] * z[1], y[2] * z[2]));
+                __builtin_amdgcn_sched_barrier(0);
                 const int uo = ghost ? 9 : 0;
-                double h[3];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) h[c] = zstep(c, filt_lds(sq[uo + c]));
-#pragma unroll
-                for (int c = 0; c < 6; ++c) L[c] = zstep(3 + c, f[c]);
+                for (int c = 0; c < 3; ++c) h[c] = xzstep(c, filt_lds(o[uo + c]));
                 L[0] -= h[0] * h[0];
                 L[1] -= h[1] * h[1];
                 L[2] -= h[2] * h[2];
@@ -361,40 +473,28 @@ __global__ __launch_bounds__(256) void k_dsm_stress(Dims d, Metrics m, const T *
                 L[4] -= h[0] * h[2];
                 L[5] -= h[1] * h[2];
             }
+            double lm = 0.0, mm = 0.0;
 #pragma unroll
             for (int c = 0; c < 6; ++c) {
-                __builtin_amdgcn_sched_barrier(0);
-                hs[c] = zstep(9 + c, filt_lds(sq[3 + c]));
+                if (c % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                const double M = o[12 + c][tid] - xzstep(9 + c, filt_lds(o[3 + c]));
+                lm = lm + (c < 3 ? 1.0 : 2.0) * M * L[c];
+                mm = mm + (c < 3 ? 1.0 : 2.0) * M * M;
             }
-            __builtin_amdgcn_sched_barrier(0);
-            if (kk > kb) {  // plane k = kk - 1 has its three planes
-                const int k = kk - 1;
-                double M[6];
-                const double magh = strain(d, m, sm, Uf, Vf, Wf, oi, k, M);
-#pragma unroll
-                for (int e = 0; e < 6; ++e) M[e] = 4.0 * magh * M[e] - hs[e];
-                double lm = M[0] * L[0];
-                lm = lm + M[1] * L[1];
-                lm = lm + M[2] * L[2];
-                lm = lm + 2.0 * M[3] * L[3];
-                lm = lm + 2.0 * M[4] * L[4];
-                lm = lm + 2.0 * M[5] * L[5];
-                const double mm = M[0] * M[0] + M[1] * M[1] + M[2] * M[2] +
-                                  2.0 * (M[3] * M[3] + M[4] * M[4] + M[5] * M[5]);
+            if (own && kk > kb) {  // plane k = kk - 1 has its three planes
                 if constexpr (PX) {
-                    S[k * sxy + oi] = fmax(-0.5 * (lm / mm) * magp, 0.0);
+                    S[(kk - 1) * sxy + oi] = fmax(-0.5 * (lm / mm) * o[18][tid], 0.0);
                 } else {
                     lmsum += lm;
                     mmsum += mm;
                 }
             }
-            magp = mag;
         }
-    }
-    if (!PX && own) {
-        double *o = part + 2 * (long long)blockIdx.y * sxy + oi;
-        o[0] = lmsum;
-        o[sxy] = mmsum;
+        if (!PX && own) {
+            double *o = part + 2 * (long long)blockIdx.y * sxy + oi;
+            o[0] = lmsum;
+            o[sxy] = mmsum;
+        }
     }
 }
 
@@ -456,7 +556,7 @@ __global__ __launch_bounds__(256) void k_smag(Dims d, Metrics m, const T *__rest
     const int k = 1 + blockIdx.z;
     if (i > d.nxg - 2 || j > d.nyg - 2) return;
     double s[6];
-    const double mag = strain(d, m, strain_met(m, i, j), U, V, W, (unsigned)(i + d.sx * j), k, s);
+    const double mag = strain(d, m, strain_met(m, i, j), U, V, W, i, j, k, s);
     nu_t[fidx(d, i, j, k)] = (T)(coef[j] * mag);
 }
 
@@ -486,7 +586,7 @@ int dsm_chunk(int nk, int tiles, int slots) {
     }
     return best;
 }
-// resident blocks per compute unit, by their registers
+// resident blocks per compute unit, by their registers (and the LDS of k_dsm_stress)
 constexpr int kStressPerCU = 2, kVfilterPerCU = 4;
 int stress_tiles(const Dims &d) {
     return ((d.nxg - 2 + kDsX - 3) / (kDsX - 2)) * ((d.nyg - 2 + kDsY - 3) / (kDsY - 2));
@@ -512,7 +612,7 @@ void dsm_t(Handle &h, const Fld3<T> &f, T *nu_t) {
     const int chunk = dsm_chunk(nk, tiles, kStressPerCU * h.n_cu), nch = (nk + chunk - 1) / chunk;
     {
         ProfScope ps(h, KID_DSM_FILTER);
-        hipLaunchKernelGGL((k_dsm_stress<PX, T>), dim3(tiles, nch), block, 0, h.stream, d, h.m, f.u, f.v, f.w, Uf, Vf,
+        hipLaunchKernelGGL((k_dsm_stress<PX, T>), dim3(tiles, nch), dim3(kDsX * kDsY + kDsOwn), 0, h.stream, d, h.m, f.u, f.v, f.w, Uf, Vf,
                            Wf, S, part, chunk);
         check();
     }
