@@ -578,7 +578,7 @@ void build(Handle &h, const bl_config *c) {
         std::vector<double> co(3 * (size_t)L + N + Kz, 0.0);
         for (int j = 0; j < L; ++j) {
             co[j] = (j >= 1 && j < NM) ? dlo[j - 1] : 0.0;
-            co[L + j] = j < NM ? dd[j] : 1.0;
+            co[L + j] = j < NM ? dd[j] : -1.0;
             co[2 * L + j] = j < NM - 1 ? dup[j] : 0.0;
         }
         for (int i = 0; i < N; ++i) co[3 * L + i] = kxx[i];

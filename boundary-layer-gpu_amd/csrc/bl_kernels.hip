@@ -1607,8 +1607,6 @@ __global__ __launch_bounds__(256) void k_thomas(Dims d, const double *__restrict
     }
 }
 
-// a copy of a uniform pointer that the compiler cannot prove equal to the
-// original (loads through it are not merged with loads through the original)
 // 1/x for the normal, finite pivots of the Thomas sweeps: the hardware
 // reciprocal refined by two Newton steps (within an ulp or so of the rounded
 // quotient, without the special-case scaling of a full division)
@@ -1620,12 +1618,7 @@ __device__ __forceinline__ double rcp64(double x) {
     return fma(r, e, r);
 }
 
-// in the constant address space, so that uniform loads through it are scalar
-using cdptr = const double __attribute__((address_space(4))) *;
-__device__ __forceinline__ cdptr opaque(const double *p) {
-    asm volatile("" : "+s"(p));
-    return (cdptr)p;
-}
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 template <int NMAX>
 __device__ void solve00_block(const Solve00 &z, int NM);
@@ -1640,18 +1633,26 @@ __device__ void solve00_block(const Solve00 &z, int NM);
 // with x = y + alpha xL + beta xR on the segment ends, the 2P interface
 // values follow from a two-term recurrence over the segments (every lane
 // runs it for its own system), and the segment is solved again with the
-// neighbour values moved to its right-hand side.  Rows past NM are identity
-// rows (a = c = 0, b = 1).  co = {a[L], b[L], c[L], kxx[N], kzz[Kz]},
+// neighbour values moved to its right-hand side.  Rows past NM stand alone
+// (a = c = 0, b = -1: the pivot b + kxx + kzz <= -1).  co = {a[L], b[L], c[L], kxx[N], kzz[Kz]},
 // L = 32 P: a[j] couples x(j-1), c[j] couples x(j+1), b[j] + kxx + kzz is
 // the diagonal.  The (0,0) system (kx = 0, q = 0, pinned first pivot) is
 // skipped (zero00 = 0) or zeroed (zero00 = 1); block 0 solves it (z) while
-// the other blocks run.  The other blocks (one resident per CU: 8 waves of
-// more than 128 VGPRs each) loop over the nq * ceil(N/64) tiles of 64 systems.
+// the other blocks run.  The other blocks (8 waves of more than 128 VGPRs each
+// reside on a CU) loop over the nq * ceil(N/64) tiles of 64 systems.
+// A tile's time is that of its loads plus that of its arithmetic (the 8 waves of
+// a CU go through both together).  The coefficients come from LDS, a row is a
+// scalar offset into a buffer and no row is masked: with scalar coefficient
+// loads and guarded rows 900 of the 2500 instructions were scalar register
+// spills and selects.  At 511x96x128 45 -> 30 us (with more than one block a CU),
+// 260x65x228 FP32 39 -> 24, 812x256x191 FP32 117 -> 109, FP64 156 -> 152, on
+// 255x96x62 and 127x48x32 FP32 27 -> 13 and 19 -> 10 (with the sums of block 0).
 template <class T>
 __global__ __launch_bounds__(64 * kThMaxP) void k_thomas_seg(int N, int NM, int P, int nq, int ldj, long long ldq,
                                                              const double *__restrict__ co, int zero00,
                                                              T *__restrict__ S, Solve00 z) {
     __shared__ double xs[6][kThMaxP][64];
+    __shared__ double ca[kThSeg * kThMaxP], cb[kThSeg * kThMaxP], cc[kThSeg * kThMaxP];
     if (blockIdx.x == 0) {  // the (0,0) system, alongside the other blocks
         solve00_block<kThSeg * kThMaxP>(z, NM);
         return;
@@ -1660,8 +1661,14 @@ __global__ __launch_bounds__(64 * kThMaxP) void k_thomas_seg(int N, int NM, int 
     const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nkb = (N + 63) / 64, ntiles = nkb * nq, nblk = gridDim.x - 1;
     const int L = P * kThSeg;
-    const double *ca = co, *cb = co + L, *cc = co + 2 * L;
     const int r0 = p * kThSeg;
+    for (int e = threadIdx.x; e < L; e += blockDim.x) {
+        ca[e] = co[e];
+        cb[e] = co[L + e];
+        cc[e] = co[2 * L + e];
+    }
+    __syncthreads();
+    const unsigned rowb = (unsigned)ldj * (unsigned)sizeof(T);  // a plane is below 4 GB
     // tiles (q, 64 kx) bid, bid + nblk, ... (holding the next tile's rows
     // in registers during a solve spills them)
     for (int tile = blockIdx.x - 1; tile < ntiles; tile += nblk) {
@@ -1670,38 +1677,46 @@ __global__ __launch_bounds__(64 * kThMaxP) void k_thomas_seg(int N, int NM, int 
         const bool live = kx < N;
         const int kxc = live ? kx : N - 1;
         const double lam = co[3 * L + kxc] + co[3 * L + N + (q + 1) / 2];
-        T *col = S + q * ldq + kxc;
+        const unsigned vo = (unsigned)kxc * (unsigned)sizeof(T);
+        // rows of the segment left below NM; hidden from the compiler, which would
+        // keep the comparison with each row across the tiles
+        int left = NM - r0;
+        asm volatile("" : "+s"(left));
+        // the q plane as a buffer: a row is a scalar offset
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(S + q * ldq), 0, (int)((unsigned)NM * rowb), 0x00020000);
+        const unsigned row0 = (unsigned)min(r0, NM - 1) * rowb;
         double dv[kThSeg], ip[kThSeg];
         {
-            // unconditional loads (rows past NM clamped, then zeroed), all
-            // issued before the first conversion waits on one
+            // unconditional loads (rows past NM repeat the last one, their
+            // systems are apart), all issued before the first conversion waits
             T raw[kThSeg];
+            unsigned ro = row0;
 #pragma unroll
-            for (int i = 0; i < kThSeg; ++i) raw[i] = col[(long long)min(r0 + i, NM - 1) * ldj];
+            for (int i = 0; i < kThSeg; ++i) {
+                if constexpr (sizeof(T) == 4)
+                    raw[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, ro, 0));
+                else
+                    raw[i] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, vo, ro, 0));
+                ro += i + 1 < left ? rowb : 0u;
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < kThSeg; ++i) dv[i] = (r0 + i < NM) ? (double)raw[i] : 0.0;
+            for (int i = 0; i < kThSeg; ++i) dv[i] = (double)raw[i];
         }
-        // Each sweep reads the coefficients through its own opaque copy of the
-        // pointer, so that a value loaded by one sweep is not kept in registers
-        // for the other sweeps' use of the same row.
-        const cdptr la = opaque(ca), lb = opaque(cb), lc = opaque(cc);
-        const cdptr ua = opaque(ca), ub = opaque(cb), uc = opaque(cc);
         // LU (index i) and UL (index kThSeg-1-i) sweeps, interleaved
         double dp = dv[0], s = 1.0;
-        ip[0] = rcp64(lb[r0] + (r0 < NM ? lam : 0.0));
-        const int rl = r0 + kThSeg - 1;
-        double iu = rcp64(ub[rl] + (rl < NM ? lam : 0.0)), du = dv[kThSeg - 1], t = 1.0;
+        ip[0] = rcp64(cb[r0] + lam);
+        double iu = rcp64(cb[r0 + kThSeg - 1] + lam), du = dv[kThSeg - 1], t = 1.0;
 #pragma unroll
         for (int i = 1; i < kThSeg; ++i) {
             const int j = r0 + i;
-            const double m = la[j] * ip[i - 1];
-            ip[i] = rcp64(lb[j] + (j < NM ? lam : 0.0) - m * lc[j - 1]);
+            const double m = ca[j] * ip[i - 1];
+            ip[i] = rcp64(cb[j] + lam - m * cc[j - 1]);
             dp = dv[i] - m * dp;
             s = -m * s;
             const int iv = kThSeg - 1 - i, jv = r0 + iv;
-            const double mu = uc[jv] * iu;
-            iu = rcp64(ub[jv] + (jv < NM ? lam : 0.0) - mu * ua[jv + 1]);
+            const double mu = cc[jv] * iu;
+            iu = rcp64(cb[jv] + lam - mu * ca[jv + 1]);
             du = dv[iv] - mu * du;
             t = -mu * t;
             if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
@@ -1745,19 +1760,37 @@ __global__ __launch_bounds__(64 * kThMaxP) void k_thomas_seg(int N, int NM, int 
             }
         }
         // the segment with its neighbour values on the right-hand side
-        const cdptr fa = opaque(ca), fc = opaque(cc);
         dv[0] -= aL * xL;
         dv[kThSeg - 1] -= cR * xR;
 #pragma unroll
-        for (int i = 1; i < kThSeg; ++i) dv[i] -= fa[r0 + i] * ip[i - 1] * dv[i - 1];
+        for (int i = 1; i < kThSeg; ++i) {
+            dv[i] -= ca[r0 + i] * ip[i - 1] * dv[i - 1];
+            if (i % 8 == 0) __builtin_amdgcn_sched_barrier(0);
+        }
         dv[kThSeg - 1] *= ip[kThSeg - 1];
 #pragma unroll
-        for (int i = kThSeg - 2; i >= 0; --i) dv[i] = (dv[i] - fc[r0 + i] * dv[i + 1]) * ip[i];
+        for (int i = kThSeg - 2; i >= 0; --i) {
+            dv[i] = (dv[i] - cc[r0 + i] * dv[i + 1]) * ip[i];
+            if (i % 8 == 0) __builtin_amdgcn_sched_barrier(0);
+        }
         const bool is00 = q == 0 && kx == 0;
-        if (live && !(is00 && !zero00)) {
+        if (is00 && zero00)
 #pragma unroll
-            for (int i = 0; i < kThSeg; ++i)
-                if (r0 + i < NM) col[(long long)(r0 + i) * ldj] = is00 ? (T)0 : (T)dv[i];
+            for (int i = 0; i < kThSeg; ++i) dv[i] = 0.0;
+        if (live && !(is00 && !zero00)) {
+            unsigned ro = row0;
+            asm volatile("" : "+s"(left));
+            if (left >= kThSeg) left = kThSeg;
+#pragma unroll
+            for (int i = 0; i < kThSeg; ++i) {
+                if (i < left) {
+                    if constexpr (sizeof(T) == 4)
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (T)dv[i]), rsrc, vo, ro, 0);
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, (T)dv[i]), rsrc, vo, ro, 0);
+                }
+                ro += rowb;
+            }
         }
     }
 }
@@ -1767,7 +1800,7 @@ __global__ __launch_bounds__(64 * kThMaxP) void k_thomas_seg(int N, int NM, int 
 // table kernel, from LDS copies of the stored multipliers L00 and reciprocal
 // pivots D00.  With z.part set, the right-hand side is first formed as
 // r(j) = 2 sum_q part[j][q] (the FP64 plane sums of the mixed path's
-// divergence), one wave per row.  The sweeps read one array and write
+// divergence), 16 lanes per row.  The sweeps read one array and write
 // another, so that the LDS reads of the unrolled iterations are issued ahead
 // of the dependent chain.  Any block size that is a multiple of 64.
 template <int NMAX>
@@ -1775,12 +1808,24 @@ __device__ void solve00_block(const Solve00 &z, int NM) {
     __shared__ double r[NMAX], o[NMAX], L[NMAX], D[NMAX], U[NMAX];
     const int tid = threadIdx.x, nt = blockDim.x;
     if (z.part) {
-        const int lane = tid & 63;
-        for (int j = tid >> 6; j < NM; j += nt >> 6) {
-            double v = 0.0;
-            for (int q = lane; q < z.npart; q += 64) v += z.part[(long long)j * z.npart + q];
-            for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-            if (lane == 0) r[j] = 2.0 * v;
+        // 16 lanes a row, 32 rows of a wave at a time: their loads are in flight
+        // together (one row after the other waited 0.6 us for each, 20 us for 96
+        // rows on three waves, longer than the other blocks take there)
+        const int lane = tid & 63, l16 = lane & 15;
+        for (int j0 = (tid >> 6) * 32; j0 < NM; j0 += (nt >> 6) * 32) {
+            const int j = j0 + (lane >> 4);
+            double v[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = 0.0;
+#pragma unroll 2
+            for (int q = l16; q < z.npart; q += 16)
+#pragma unroll
+                for (int t = 0; t < 8; ++t) v[t] += z.part[(long long)min(j + 4 * t, NM - 1) * z.npart + q];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                for (int off = 8; off > 0; off >>= 1) v[t] += __shfl_xor(v[t], off);
+                if (l16 == 0 && j + 4 * t < NM) r[j + 4 * t] = 2.0 * v[t];
+            }
         }
     } else {
         for (int j = tid; j < NM; j += nt) r[j] = z.x[(long long)j * z.ldx];
@@ -2447,10 +2492,11 @@ template <class T>
 bool launch_thomas_seg(Handle &h, T *S, int ldj, long long ldq, const Solve00 &z) {
     const Dims &d = h.d;
     if (h.th_p == 0) return false;
-    // one resident block per CU (the registers of 8 waves), each looping over
-    // its tiles, plus block 0 for the (0,0) system
+    // the resident blocks (a CU has the registers of 8 waves), each looping over
+    // its tiles, one of them block 0 for the (0,0) system.  With one block per CU
+    // also where a block is 3 waves the solve took 39 us at 260x65x228 (FP32).
     const int ntiles = (d.N + 63) / 64 * d.M;
-    const int nblk = std::max(1, std::min(ntiles, h.n_cu > 1 ? h.n_cu - 1 : ntiles));
+    const int nblk = std::max(1, std::min(ntiles, std::max(2, h.n_cu) * (kThMaxP / h.th_p) - 1));
     hipLaunchKernelGGL(k_thomas_seg<T>, dim3(1 + nblk), dim3(64 * h.th_p), 0, h.stream, d.N, d.NM, h.th_p, d.M,
                        ldj, ldq, (const double *)h.th_co, z.part ? 1 : 0, S, z);
     check_launch();

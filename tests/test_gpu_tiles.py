@@ -179,6 +179,15 @@ def test_x_transform_lengths(n, ny, nz):
     s.close()
 
 
+# the y solves: 32-row segments, with a last one of a single row and a full one,
+# and more tiles of 64 systems than the blocks that reside at a time (8 / segments
+# per CU), so that blocks take several; 1, 2, 3, 5 and 8 segments
+@pytest.mark.parametrize("n,ny,nz", [(65, 5, 1032), (200, 34, 262), (140, 66, 182), (70, 130, 132), (66, 226, 130),
+                                     (30, 33, 12), (30, 65, 12)])
+def test_y_solve_segments(n, ny, nz):
+    test_x_transform_lengths(n, ny, nz)
+
+
 # transfers pass through a work array of (nx-2)(ny-1)(nz-2) values, planes of
 # up to (nx+1)(ny+1): grids where it holds one plane, a part of the planes,
 # and nearly all of them; both directions, exact (FP32 storage: rounded once)
