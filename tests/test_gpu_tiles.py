@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 from . import cases, closure_ref as R, mlp_ref as M, orc
-from .blgpu_import import blgpu
+from .blgpu_import import blgpu, solver_for
+from .test_gpu_mixed import mixed_solver
 from .test_oracle_dsm import random_case
 
 pytestmark = pytest.mark.gpu
@@ -267,4 +268,25 @@ def test_closure_blocks(nx, ny, nz):
     assert err.max() < 5e-2
     assert (err > 1e-6).mean() < 1e-2
     c.close()
+    s.close()
+
+
+# the march accesses its fields past the caches where nine arrays exceed 256 MB:
+# one step of grids just above that line (no model, a model with nu_t, RK2, FP32),
+# to the bounds of the step parity tests (FP64 1e-10, mixed 1e-4 of |U|)
+@pytest.mark.parametrize("nx,scheme,les,precision", [(130, 3, 0, 0), (130, 2, 0, 0), (130, 3, 1, 0), (260, 3, 0, 1),
+                                                     (260, 2, 0, 1), (260, 3, 1, 1)])
+def test_march_streams(nx, scheme, les, precision):
+    say("streaming march", nx, scheme, les, precision)
+    case = cases.laminar_small(nx=nx, ny=130, nz=250, Lz=0.15, noise=0.01, seed=5, scheme=scheme, les=les, cfl=-1e-5)
+    o = case.oracle()
+    s = (mixed_solver(case, o) if precision else solver_for(case, o)[0])
+    o.compute_dt(), s.compute_dt()
+    o.step()
+    s.step()
+    U = np.linalg.norm(o.fields()[0])
+    for a, b in zip(s.fields(), o.fields()):
+        err = np.linalg.norm(a - b) / U
+        say("err", err)
+        assert err < (1e-4 if precision else 1e-10)
     s.close()
