@@ -1474,8 +1474,17 @@ __global__ __launch_bounds__(64 * kZmW) void k_zdft_mf(int M, int C, long long p
     // built on the host in this order (zf)
     for (int e = threadIdx.x; e < RT * KS * 64; e += 64 * kZmW) sA[e] = zf[e];
     __syncthreads();
+    // A wave takes tile after tile; the last, partial round goes to the first waves
+    // of all blocks instead of all waves of the first ones (812x256x191: the
+    // busiest SIMDs do 13 tiles instead of 14; 191 -> 180 and 200 -> 187 us,
+    // 511x96x128 46 -> 38 and 44 -> 37).  A first round that is the only one keeps
+    // neighbouring tiles in one block.
     const int ntile = (C + 15) / 16, stride = gridDim.x * kZmW;
-    int tile = blockIdx.x * kZmW + wave;
+    auto tile_of = [&](int base) {
+        return base == 0 || base + stride <= ntile ? base + (int)blockIdx.x * kZmW + wave
+                                                   : base + wave * (int)gridDim.x + (int)blockIdx.x;
+    };
+    int base = 0, tile = tile_of(0);
     if (tile >= ntile) return;
     // k steps past M/2 multiply zeros
     const int KSr = (KS + kZmPF - 1) / kZmPF * kZmPF;
@@ -1501,7 +1510,10 @@ __global__ __launch_bounds__(64 * kZmW) void k_zdft_mf(int M, int C, long long p
 #pragma unroll
     for (int u = 0; u < kZmPF; ++u) raw(tile, u, pa[u], pb[u]);
 
-    for (; tile < ntile; tile += stride) {
+    for (int next; tile < ntile; tile = next) {
+        base += stride;
+        next = tile_of(base);
+        const int ahead = min(next, ntile - 1);
         dbl4 ac[RT], as[RT];
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
@@ -1518,7 +1530,7 @@ __global__ __launch_bounds__(64 * kZmW) void k_zdft_mf(int M, int C, long long p
                 // ahead: k step ks + kZmPF of this tile, or of the next one
                 const int kn = ks + kZmPF;
                 const bool here = kn < KSr;
-                raw(here ? tile : min(tile + stride, ntile - 1), here ? kn : kn - KSr, pa[u], pb[u]);
+                raw(here ? tile : ahead, here ? kn : kn - KSr, pa[u], pb[u]);
                 double bc, bs;
                 if (FWD) {
                     bc = a + b;                  // b = 0 for the single elements

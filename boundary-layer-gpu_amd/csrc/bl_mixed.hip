@@ -352,8 +352,14 @@ __global__ __launch_bounds__(64 * kZxW) void k_zdft_mx(int M, int C, long long p
     for (int e = threadIdx.x; e < RT * KS * 64 * 4; e += 64 * kZxW) sA[e] = zfr[e];
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, c16 = lane & 15;
+    // tile after tile, the last, partial round by the first waves of all blocks
+    // (as in k_zdft_mf; 812x256x191 81 -> 76 and 83 -> 80 us)
     const int ntile = (C + 15) / 16, stride = gridDim.x * kZxW;
-    int tile = blockIdx.x * kZxW + wave;
+    auto tile_of = [&](int base) {
+        return base == 0 || base + stride <= ntile ? base + (int)blockIdx.x * kZxW + wave
+                                                   : base + wave * (int)gridDim.x + (int)blockIdx.x;
+    };
+    int base = 0, tile = tile_of(0);
     if (tile >= ntile) return;
     // raw inputs of k step s of tile tl: kk = 32 s + 8 q + e (rows clamped
     // to M/2, columns to C - 1; masked where used), one step ahead: the
@@ -379,7 +385,10 @@ __global__ __launch_bounds__(64 * kZxW) void k_zdft_mx(int M, int C, long long p
         }
     };
     load(tile, 0);
-    for (; tile < ntile; tile += stride) {
+    for (int next; tile < ntile; tile = next) {
+        base += stride;
+        next = tile_of(base);
+        const int ahead = min(next, ntile - 1);
         f32x4 ac[RT], as[RT];
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
@@ -410,7 +419,7 @@ __global__ __launch_bounds__(64 * kZxW) void k_zdft_mx(int M, int C, long long p
                 bsl[e] = l1;
             }
             const bool here = s + 1 < KS;
-            load(here ? tile : min(tile + stride, ntile - 1), here ? s + 1 : 0);
+            load(here ? tile : ahead, here ? s + 1 : 0);
             const bf16x8 ch = __builtin_bit_cast(bf16x8, bch), cl = __builtin_bit_cast(bf16x8, bcl);
             const bf16x8 sh = __builtin_bit_cast(bf16x8, bsh), sl = __builtin_bit_cast(bf16x8, bsl);
 #pragma unroll

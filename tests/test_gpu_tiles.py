@@ -189,6 +189,18 @@ def test_y_solve_segments(n, ny, nz):
     test_x_transform_lengths(n, ny, nz)
 
 
+# the z transforms' tiles of 16 columns: one full round of the resident waves
+# (2048 FP64 tiles, 4096 FP32), a part of a second one, and two rounds and a part
+@pytest.mark.parametrize("n,ny,nz", [(128, 257, 8), (129, 257, 8), (268, 257, 7)])
+def test_z_transform_rounds(n, ny, nz):
+    test_x_transform_lengths(n, ny, nz)
+
+
+@pytest.mark.parametrize("n,ny,nz", [(256, 257, 8), (258, 257, 8), (520, 257, 7)])
+def test_z_transform_rounds_mixed(n, ny, nz):
+    test_x_transform_lengths_mixed(n, ny, nz)
+
+
 # transfers pass through a work array of (nx-2)(ny-1)(nz-2) values, planes of
 # up to (nx+1)(ny+1): grids where it holds one plane, a part of the planes,
 # and nearly all of them; both directions, exact (FP32 storage: rounded once)
