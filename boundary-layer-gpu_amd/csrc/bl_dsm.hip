@@ -98,8 +98,7 @@ __device__ __forceinline__ double at(PlanePtr<T> base, unsigned o) {
 
 // A plane as a buffer resource: an element is a scalar base, one register with
 // the byte offset of a cell's south-west neighbour (shared by all arrays of one
-// element size), a scalar row offset and an immediate column offset, and the
-// hardware returns 0 for whatever lies outside the plane.
+// element size), a scalar row offset and an immediate column offset.
 template <class T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const Dims &d, const T *p, long long k) {
     return __builtin_amdgcn_make_buffer_rsrc((void *)(p + k * d.sxy), 0, (int)(unsigned)(d.sxy * sizeof(T)), 0x00020000);
@@ -113,10 +112,9 @@ __device__ __forceinline__ T buf_at(__amdgpu_buffer_rsrc_t r, unsigned sw, unsig
 }
 
 // compute_Sij along z at one column of cells: diagonal terms at the centre, the
-// off-diagonal terms averaged from the four surrounding edges.  The average of
-// the edges' differences is the sum of the differences of the neighbouring
-// pairs, so a cell needs U at two points of five rows or planes, V likewise and W
-// at five points of two planes; what the next plane uses again stays in
+// off-diagonal terms averaged from the four surrounding edges.  A cell needs U at
+// two points of five rows or planes, V likewise and W at five points of two
+// planes; what the next plane uses again stays in
 // registers (17 loads a plane instead of 30).  All loads of a plane are issued
 // together by load(); eval() uses them.
 template <class T>
@@ -173,19 +171,24 @@ struct StrainMarch {
     __device__ __forceinline__ double eval(const Metrics &m, const StrainMet &sm, int k, double s[6],
                                            double *c = nullptr) {
         const double rz0 = m.rdzg[k - 1], rz1 = m.rdzg[k];
-        // the differences of a pair against the pair before and behind it
-        auto diff = [](const T a[2], const T b[2], double ra, const T e[2], double re) {
-            return (((double)b[0] - (double)a[0]) + ((double)b[1] - (double)a[1])) * ra +
-                   (((double)e[0] - (double)b[0]) + ((double)e[1] - (double)b[1])) * re;
+        // the four edges around the cell (twice their value): the pair b of one
+        // component against the pairs before (a) and behind (e) it along one
+        // direction, and the other component's pair along the other, in the
+        // reference's order
+        auto edges = [](const T a[2], const T b[2], const T e[2], double ra, double re, const T f[2], const T g[2],
+                        const T h[2], double rf, double rh) {
+            auto dif = [](T p, T q) { return (double)p - (double)q; };
+            return ((dif(b[0], a[0]) * ra + dif(g[0], f[0]) * rf) + (dif(b[1], a[1]) * ra + dif(h[0], g[0]) * rh)) +
+                   (dif(e[0], b[0]) * re + dif(g[1], f[1]) * rf) + (dif(e[1], b[1]) * re + dif(h[1], g[1]) * rh);
         };
         const T wc[2] = {wm[0], w[0]}, ww[2] = {wm[1], w[1]}, we[2] = {wm[2], w[2]}, ws[2] = {wm[3], w[3]},
                 wn[2] = {wm[4], w[4]};
         s[0] = ((double)u[1] - (double)u[0]) * sm.rdx;
         s[1] = ((double)v[1] - (double)v[0]) * sm.rdy;
         s[2] = ((double)w[0] - (double)wm[0]) * m.rdz[k];
-        s[3] = 0.125 * (diff(us, u, sm.rdyg0, un, sm.rdyg1) + diff(vw, v, sm.rdxg0, ve, sm.rdxg1));
-        s[4] = 0.125 * (diff(um, u, rz0, up, rz1) + diff(ww, wc, sm.rdxg0, we, sm.rdxg1));
-        s[5] = 0.125 * (diff(vm, v, rz0, vp, rz1) + diff(ws, wc, sm.rdyg0, wn, sm.rdyg1));
+        s[3] = 0.125 * edges(us, u, un, sm.rdyg0, sm.rdyg1, vw, v, ve, sm.rdxg0, sm.rdxg1);
+        s[4] = 0.125 * edges(um, u, up, rz0, rz1, ww, wc, we, sm.rdxg0, sm.rdxg1);
+        s[5] = 0.125 * edges(vm, v, vp, rz0, rz1, ws, wc, wn, sm.rdyg0, sm.rdyg1);
         if (c) {
             c[0] = 0.5 * ((double)u[0] + (double)u[1]);
             c[1] = 0.5 * ((double)v[0] + (double)v[1]);
@@ -323,9 +326,8 @@ __global__ __launch_bounds__(256) void k_dsm_vfilter(Dims d, const T *__restrict
 // but |S| and the two sums per column and chunk goes to memory.  Bound by
 // issue: FP64 arithmetic with two blocks (14 waves) per CU, 120 registers.
 // At 257x97x64 in FP32 fields the model's three passes take 0.022 + 0.064 +
-// 0.010 ms per stage.  With all steps in four waves, the edge differences one
-// by one, filters of 9 LDS reads and plain loads, which waited one after the
-// other, the middle one took 0.153; the form in which every cell read the 27
+// 0.010 ms per stage.  With all steps in four waves, filters of 9 LDS reads and
+// plain loads, which waited one after the other, the middle one took 0.153; the form in which every cell read the 27
 // neighbours of twelve FP64 arrays written by other passes took 0.04 + 0.07 +
 // 0.53 + 0.05.  Tiles of 32 x 16 measured the same (0.063), loads of the
 // filtered field a plane ahead 0.093 (registers).
@@ -440,7 +442,7 @@ __global__ __launch_bounds__(kDsX *kDsY + kDsOwn, 4) void k_dsm_stress(
             // its own), then the z part: the plane kk - 1 of quantity q is complete
             // with this plane's value
             auto xzstep = [&](int q, double g) {
-                const double f = kF0 * g + kF1 * (lane_shift<-1>(g) + lane_shift<1>(g));
+                const double f = kF1 * lane_shift<-1>(g) + kF0 * g + kF1 * lane_shift<1>(g);
                 const double h = pend[q] + kF1 * f;
                 pend[q] = kF1 * last[q] + kF0 * f;
                 last[q] = f;
@@ -473,14 +475,15 @@ __global__ __launch_bounds__(kDsX *kDsY + kDsOwn, 4) void k_dsm_stress(
                 L[4] -= h[0] * h[2];
                 L[5] -= h[1] * h[2];
             }
-            double lm = 0.0, mm = 0.0;
+            double lm = 0.0, mm = 0.0, mo = 0.0;
 #pragma unroll
             for (int c = 0; c < 6; ++c) {
                 if (c % 2 == 0) __builtin_amdgcn_sched_barrier(0);
                 const double M = o[12 + c][tid] - xzstep(9 + c, filt_lds(o[3 + c]));
                 lm = lm + (c < 3 ? 1.0 : 2.0) * M * L[c];
-                mm = mm + (c < 3 ? 1.0 : 2.0) * M * M;
+                (c < 3 ? mm : mo) += M * M;
             }
+            mm += 2.0 * mo;
             if (own && kk > kb) {  // plane k = kk - 1 has its three planes
                 if constexpr (PX) {
                     S[(kk - 1) * sxy + oi] = fmax(-0.5 * (lm / mm) * o[18][tid], 0.0);
