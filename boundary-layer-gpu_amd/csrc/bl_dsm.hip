@@ -327,10 +327,11 @@ __global__ __launch_bounds__(256) void k_dsm_vfilter(Dims d, const T *__restrict
 // issue: FP64 arithmetic with two blocks (14 waves) per CU, 120 registers.
 // At 257x97x64 in FP32 fields the model's three passes take 0.022 + 0.064 +
 // 0.010 ms per stage.  With all steps in four waves, filters of 9 LDS reads and
-// plain loads, which waited one after the other, the middle one took 0.153; the form in which every cell read the 27
-// neighbours of twelve FP64 arrays written by other passes took 0.04 + 0.07 +
-// 0.53 + 0.05.  Tiles of 32 x 16 measured the same (0.063), loads of the
-// filtered field a plane ahead 0.093 (registers).
+// plain loads, which waited one after the other, the middle one took 0.153;
+// the form in which every cell read the 27 neighbours of twelve FP64 arrays
+// written by other passes took 0.04 + 0.07 + 0.53 + 0.05.  Tiles of 32 x 16
+// measured the same (0.063), loads of the filtered field a plane ahead 0.093
+// (registers).
 constexpr int kDsX = 32, kDsY = 8;  // tile with its halo
 
 constexpr int kDsOwn = kDsX * (kDsY - 2);  // threads of the second role: its inner rows

@@ -1114,11 +1114,11 @@ __device__ __forceinline__ DctSums<T> dct_sums(const DctArgs<T> &a, const typena
 // its inputs are read and the lines and the spectra share one LDS area (13.9 KB
 // at N = 812: the blocks' load, product and store phases overlap across ten
 // blocks per CU).  Otherwise four or eight waves, and LB lines in an area of their
-// own.  At 814x257x193 the forward (inverse) transform takes 0.345 (0.203) ms, bound
+// own.  At 814x257x193 the forward (inverse) transform takes 0.327 (0.203) ms, bound
 // by the latency of its loads (HBM time 0.25 (0.125)); the unfolded products in
-// four waves took 0.42 (0.30).  511 points (7 x 73): 0.086 (0.060) ms per 12288
+// four waves took 0.42 (0.30).  511 points (7 x 73): 0.084 (0.058) ms per 12288
 // lines, on the vector units 0.15 (0.15).  FP32 (v_mfma_f32_16x16x4_f32, 814x257x193):
-// 0.218 (0.124) ms; unfolded split-BF16x3 products in four waves 0.25 (0.144).
+// 0.209 (0.124) ms; unfolded split-BF16x3 products in four waves 0.25 (0.144).
 // DIV: the line is the pseudo-pressure rhs (projection.f90:38-47) evaluated
 // on the fly from U, V, W (in = U, in2 = V, in3 = W, lines over cells
 // i = 1..N, j = 1..NM, k = 1..M) instead of being read from memory; with
