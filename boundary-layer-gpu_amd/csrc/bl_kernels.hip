@@ -3,8 +3,8 @@
 // Reference correspondence (0-based indices here, the reference is 1-based):
 //   k_rk_march      equations.f90:24-415 fused with time_integration.f90:351-458
 //   k_bc_*          boundary_conditions.f90:127-262
-//   k_divergence    projection.f90:34-49
-//   k_dct_*, k_zdft_*  the DCT-II/DFT stages of solve_poisson_gpu projection.f90:110-202
+//   k_dct_*, k_zdft_*  the DCT-II/DFT stages of solve_poisson_gpu projection.f90:110-202,
+//                   and in k_dct_fwd_m the divergence :34-49
 //   k_thomas        projection.f90:137-150
 //   k_project       projection.f90:355-386 with apply_periodic_z_pressure :293-303,
 //                   and the P record of the first sub-step :75-85
