@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "bl_internal.hpp"
+#include "bl_plan.hpp"
 
 namespace blgpu {
 
@@ -1007,6 +1008,7 @@ __global__ __launch_bounds__(256) void k_zdft_inv(int M, int C, long long plane,
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 constexpr int kLd = 4;  // loads per thread in flight in the line load phases
+constexpr int kDctShort = 4;  // most rows k1 <= N1/2 of a step A on the vector units
 
 __device__ __forceinline__ dbl4 mfma64(double a, double b, dbl4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -1059,12 +1061,6 @@ __device__ __forceinline__ T2 cmulc(T2 a, T2 b) {  // a * conj(b)
     return {a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y};
 }
 
-// row stride of the complex intermediate: odd, so that 16 lanes reading one
-// entry of 16 rows use different banks
-__host__ __device__ inline int dct_ld(int N2) { return N2 | 1; }
-// LDS elements of the line area (even: the complex area behind it is aligned)
-__host__ __device__ inline int dct_lines(int LB, int N) { return (LB * N + 1) / 2 * 2; }
-
 // the folded length-N2 DFT of the complex rows Bl (one per column): the four
 // real sums of row tile rt
 template <class T>
@@ -1114,11 +1110,21 @@ __device__ __forceinline__ DctSums<T> dct_sums(const DctArgs<T> &a, const typena
 // its inputs are read and the lines and the spectra share one LDS area (13.9 KB
 // at N = 812: the blocks' load, product and store phases overlap across ten
 // blocks per CU).  Otherwise four or eight waves, and LB lines in an area of their
-// own.  At 814x257x193 the forward (inverse) transform takes 0.327 (0.203) ms, bound
-// by the latency of its loads (HBM time 0.25 (0.125)); the unfolded products in
-// four waves took 0.42 (0.30).  511 points (7 x 73): 0.084 (0.058) ms per 12288
-// lines, on the vector units 0.15 (0.15).  FP32 (v_mfma_f32_16x16x4_f32, 814x257x193):
-// 0.209 (0.124) ms; unfolded split-BF16x3 products in four waves 0.25 (0.144).
+// own, by dct_plan.  At 814x257x193 the forward (inverse) transform takes 0.327
+// (0.203) ms, bound by the latency of its loads (HBM time 0.25 (0.125)); the
+// unfolded products in four waves took 0.42 (0.30).  511 points (7 x 73): 0.077
+// (0.050) ms per 12288 lines, on the vector units alone 0.15 (0.15).  FP32
+// (v_mfma_f32_16x16x4_f32, 814x257x193): 0.209 (0.124) ms; unfolded split-BF16x3
+// products in four waves 0.25 (0.144).
+// A first factor of 2 to 7 points (kDctShort rows k1) has no product in steps A
+// and A' but a column per thread on the vector units: of the 16 rows of a tile it
+// would use N1/2 + 1, and its many column tiles waited for their loads one after
+// the other.  Both directions, products -> vector units: 4 x 127 points, 20352
+// lines FP32 279 -> 204 us; 2 x 47, 2296 lines FP64 31 -> 24.  With dct_plan's
+// waves and lines FP32 4 x 251 points take 374 us there (955 before) and 2 x 251
+// 228 (468); the dense split-BF16 product, with factors to 2^-18 instead of 2^-24,
+// takes 502 and 209.  It is ahead for first factors of 1 and 2 with many lines only
+// (2 x 53 50 us against 55, 2 x 181 132 against 167), which keep the more exact product.
 // DIV: the line is the pseudo-pressure rhs (projection.f90:38-47) evaluated
 // on the fly from U, V, W (in = U, in2 = V, in3 = W, lines over cells
 // i = 1..N, j = 1..NM, k = 1..M) instead of being read from memory; with
@@ -1239,6 +1245,33 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? (sizeof(T) == 4 ? 6 : 5)
         for (int e = tid; e < LB * N; e += blockDim.x) {
             const int ln = e / N, n2 = e - ln * N;
             Bc[ln * ld + n2] = Mf<T>::make(v[e], 0);
+        }
+    } else if (K1 <= kDctShort) {  // a column per thread on the vector units
+        for (int e = tid; e < LB * N2; e += blockDim.x) {
+            const int ln = e / N2, n2 = e - ln * N2;
+            const T *vl = v + ln * N + n2;
+            T xs[kDctShort], xd[kDctShort];
+#pragma unroll
+            for (int n = 0; n < kDctShort; ++n) {
+                xs[n] = xd[n] = 0;
+                if (n < K1) {
+                    const T x = vl[N2 * n], y = vl[n == 0 ? 0 : N2 * (N1 - n)];
+                    xs[n] = n == 0 || 2 * n == N1 ? x : x + y;
+                    xd[n] = x - y;
+                }
+            }
+#pragma unroll
+            for (int k1 = 0; k1 < kDctShort; ++k1) {
+                if (k1 >= K1) continue;
+                T re = 0, im = 0;
+#pragma unroll
+                for (int n = 0; n < kDctShort; ++n) {
+                    const T2 w = a.t1[16 * n + k1];
+                    re = fma(w.x, xs[n], re);
+                    im = fma(w.y, xd[n], im);
+                }
+                Bc[(ln * K1 + k1) * ld + n2] = cmul(Mf<T>::make(re, -im), a.twA[k1 * N2 + n2]);
+            }
         }
     } else {
         for (int e = wave; e < CA * RT1; e += NW) {
@@ -1422,6 +1455,31 @@ __global__ __launch_bounds__(SMALL ? 128 : 512, SMALL ? (sizeof(T) == 4 ? 6 : 5)
         for (int e = tid; e < LB * N; e += blockDim.x) {
             const int ln = e / N, n = e - ln * N;
             o[ln * N + ((n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1)] = Cs[ln * ld + n].x * a.scale;
+        }
+    } else if (K1 <= kDctShort) {  // a column per thread, as in k_dct_fwd_m
+        for (int e = tid; e < LB * N2; e += blockDim.x) {
+            const int ln = e / N2, n2 = e - ln * N2;
+            const T2 *cl = Cs + ln * K1 * ld + n2;
+            T2 x[kDctShort];
+#pragma unroll
+            for (int k1 = 0; k1 < kDctShort; ++k1) x[k1] = k1 < K1 ? cl[k1 * ld] : Mf<T>::make(0, 0);
+            auto put = [&](int n1, T y) {
+                const int n = N2 * n1 + n2;
+                o[ln * N + ((n < (N + 1) / 2) ? 2 * n : 2 * (N - 1 - n) + 1)] = y * a.scale;
+            };
+#pragma unroll
+            for (int n1 = 0; n1 < kDctShort; ++n1) {
+                if (n1 >= K1) continue;
+                T p = 0, s = 0;
+#pragma unroll
+                for (int k1 = kDctShort - 1; k1 >= 0; --k1) {
+                    const T2 w = a.t1i[16 * k1 + n1];
+                    p = fma(w.x, x[k1].x, p);
+                    s = fma(w.y, x[k1].y, s);
+                }
+                put(n1, p - s);
+                if (n1 != 0 && 2 * n1 != N1) put(N1 - n1, p + s);
+            }
         }
     } else {
         for (int e = wave; e < CA * RT1; e += NW) {
@@ -2184,14 +2242,6 @@ void zdft_launch(Handle &h, int kid, bool forward, const double *in, double *out
     zdft_raw(h.stream, z, C, (long long)C, forward, in, out);
 }
 
-// lines per block of the x transform past the SMALL shapes: 16 columns of step
-// C (line, k1), as far as 80 KB of LDS (two blocks per CU) hold them; fewer lines
-// leave columns empty and read the tables more often (at N = 129, 3774 lines, 8,
-// 3 and 1 lines per block took 22, 25 and 40 us)
-size_t dct_line_bytes(int N, int N1, size_t es) {
-    return es * (N + 1 + 2 * (size_t)(N1 / 2 + 1) * dct_ld(N / N1));
-}
-
 template <class T>
 void dct_launch(Handle &h, int kid, DctArgs<T> a, bool forward, const T *in, T *out, const Fld3<T> *div = nullptr,
                 const BcPlanes<T> *bcp = nullptr, const IncSrc *incp = nullptr) {
@@ -2213,13 +2263,9 @@ void dct_launch(Handle &h, int kid, DctArgs<T> a, bool forward, const T *in, T *
     a.t1 = a.twC + K1 * a.N2;
     a.t1i = a.t1 + dct_frag(a.N1);
     a.t2 = a.t1i + dct_frag(a.N1);
-    const bool small = a.N1 <= 31 && a.N2 <= 31;
-    a.LB = small ? 2
-                 : std::max(1, std::min(std::max(2, (15 + K1) / K1),
-                                        (int)(81920 / dct_line_bytes(a.N, a.N1, sizeof(T)))));
-    // fewer lines where the blocks would not reach every compute unit (127 points,
-    // 1536 lines: 16 lines 14.9 and 11.8 us, 8 lines 12.6 and 10.5)
-    if (!small && (a.C + a.LB - 1) / a.LB < h.n_cu) a.LB = (a.LB + 1) / 2;
+    const bool small = dct_small(a.N, a.N1);
+    const DctPlan plan = dct_plan(a.N, a.N1, sizeof(T), a.C, h.n_cu);
+    a.LB = plan.lines;
     const size_t lines = sizeof(T) * dct_lines(a.LB, a.N), spec = sizeof(T2) * (size_t)a.LB * K1 * ld;
     // the inverse past the SMALL shapes: V (an area that also holds the lines) and C~
     const size_t lds = small ? std::max(lines, spec) : (forward ? lines + spec : std::max(lines, spec) + spec);
@@ -2227,11 +2273,7 @@ void dct_launch(Handle &h, int kid, DctArgs<T> a, bool forward, const T *in, T *
         last_error() = "x transform length too large for the LDS-resident DCT (N = " + std::to_string(a.N) + ")";
         throw ArgError();
     }
-    const dim3 grid((a.C + a.LB - 1) / a.LB);
-    // four waves per block, or eight where the blocks do not fill the chip (at 511
-    // points and 12288 lines four take 86 us and eight 103, at 129 points and
-    // 3774 lines 19 and 17)
-    const dim3 block(small ? 128 : ((int)grid.x < 4 * h.n_cu ? 512 : 256));
+    const dim3 grid((a.C + a.LB - 1) / a.LB), block(64 * plan.waves);
     auto fwd = [&](auto kern) {
         if (div)
             hipLaunchKernelGGL(kern, grid, block, lds, h.stream, a, d, h.m, bc, inc, div->u, div->v, div->w, out);

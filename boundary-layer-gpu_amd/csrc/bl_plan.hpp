@@ -1,0 +1,54 @@
+// How the passes are cut into blocks: host arithmetic on sizes and on what a
+// compute unit holds, free of the GPU runtime.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+
+namespace blgpu {
+
+// ---- x transform of N = N1 N2 points (k_dct_fwd_m, k_dct_inv_m) ----
+
+// row stride of the complex intermediate: odd, so that 16 lanes reading one
+// entry of 16 rows use different banks
+constexpr int dct_ld(int N2) { return N2 | 1; }
+// LDS elements of the line area (even: the complex area behind it is aligned)
+constexpr int dct_lines(int LB, int N) { return (LB * N + 1) / 2 * 2; }
+// LDS bytes of one line and its spectrum, elements of es bytes
+constexpr size_t dct_line_bytes(int N, int N1, size_t es) {
+    return es * (N + 1 + 2 * (size_t)(N1 / 2 + 1) * dct_ld(N / N1));
+}
+// both factors within one row tile and two column tiles: two lines in two waves
+constexpr bool dct_small(int N, int N1) { return N1 <= 31 && N / N1 <= 31; }
+
+struct DctPlan {
+    int lines, waves;  // per block
+};
+
+// Products of step C in lb lines: 16 columns of (line, k1) by 16 rows.
+constexpr int dct_products(int N, int N1, int lb) { return (lb * (N1 / 2 + 1) + 15) / 16 * ((N / N1 / 2 + 16) / 16); }
+
+// Past the small shapes a block has four waves, or eight for more than four
+// products, which would otherwise go through the same waves in two or more
+// rounds of dependent loads (2 x 251 points: four waves 288 us, eight 228), and
+// its lines fill 16 columns: rounded down or up, whichever takes fewer waves'
+// time per line (K1 = 3: five lines in one column tile, not six in two, the second
+// with two columns; 4 x 181 points FP32 322 -> 266 us for both directions, but with two
+// row tiles the second column tile costs no further round, and six lines stay:
+// 4 x 53 FP64 40 us against 49).  80 KB of LDS (two blocks per CU) bound the lines.
+// Fewer lines where the blocks would not reach every compute unit (127 points,
+// 1536 lines: 16 lines 14.9 and 11.8 us, 8 lines 12.6 and 10.5), and eight waves
+// where they do not fill the chip (129 points, 3774 lines: 19 and 17 us).
+inline DctPlan dct_plan(int N, int N1, size_t es, int nlines, int n_cu) {
+    if (dct_small(N, N1)) return {2, 2};
+    const int K1 = N1 / 2 + 1;
+    auto waves = [&](int lb) { return dct_products(N, N1, lb) > 4 ? 8 : 4; };
+    auto slots = [&](int lb) { return (dct_products(N, N1, lb) + waves(lb) - 1) / waves(lb) * waves(lb); };
+    const int up = std::max(2, (15 + K1) / K1), down = std::max(2, 16 / K1);
+    int lb = slots(down) * up < slots(up) * down ? down : up;
+    lb = std::max(1, std::min(lb, (int)(81920 / dct_line_bytes(N, N1, es))));
+    if ((nlines + lb - 1) / lb < n_cu) lb = (lb + 1) / 2;
+    return {lb, (nlines + lb - 1) / lb < 4 * n_cu ? 8 : waves(lb)};
+}
+
+}  // namespace blgpu

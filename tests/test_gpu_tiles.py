@@ -302,3 +302,21 @@ def test_march_streams(nx, scheme, les, precision):
         say("err", err)
         assert err < (1e-4 if precision else 1e-10)
     s.close()
+
+
+# first factors of 2 to 7 points go through the vector units, in blocks of four
+# waves (the last case: more than four blocks per CU) and of eight; the N2/2 + 1
+# rows of the second factor leave 1, 3, 5, .. 14 rows of a tile of 16.  Both
+# precisions, to the tolerances of the other lengths.
+SHORT_FACTORS = [(194, 5, 6), (94, 9, 7), (159, 6, 8), (164, 7, 9), (185, 6, 5), (258, 12, 9), (343, 9, 11),
+                 (502, 40, 34), (94, 97, 90)]
+
+
+@pytest.mark.parametrize("n,ny,nz", SHORT_FACTORS)
+def test_x_transform_short_factor(n, ny, nz):
+    test_x_transform_lengths(n, ny, nz)
+
+
+@pytest.mark.parametrize("n,ny,nz", SHORT_FACTORS)
+def test_x_transform_short_factor_mixed(n, ny, nz):
+    test_x_transform_lengths_mixed(n, ny, nz)

@@ -1,0 +1,83 @@
+"""The rules that cut the passes into blocks (csrc/bl_plan.hpp), compiled on
+their own with the host compiler and compared with a search over the choices
+that a rule has, over the sizes that the solver takes."""
+import os
+import subprocess
+
+import pytest
+
+from .blgpu_import import PKG
+
+MAIN = r"""
+#include <cstdio>
+#include <cstring>
+#include "bl_plan.hpp"
+using namespace blgpu;
+int main() {
+    char k[16];
+    int a, b, c, d, e;
+    while (std::scanf("%15s %d %d %d %d %d", k, &a, &b, &c, &d, &e) == 6) {
+        if (!std::strcmp(k, "dct")) {
+            const DctPlan p = dct_plan(a, b, (size_t)c, d, e);
+            std::printf("%d %d\n", p.lines, p.waves);
+        }
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    (d / "main.cpp").write_text(MAIN)
+    exe = str(d / "plan")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(PKG, "csrc"), str(d / "main.cpp"), "-o", exe],
+                   check=True)
+
+    def ask(rows):
+        text = "".join(" ".join(str(v) for v in r) + "\n" for r in rows)
+        out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout
+        return [tuple(int(v) for v in line.split()) for line in out.splitlines()]
+
+    return ask
+
+
+def factor(n):
+    n1 = max(a for a in range(1, int(n ** 0.5) + 1) if n % a == 0)
+    return n1, n // n1
+
+
+@pytest.mark.parametrize("es", [4, 8])
+def test_x_transform_plan(plan, es):
+    """Lengths with a factor past 31: where the blocks fill the chip, more than
+    four products of step C go to eight waves, and no number of lines up to a
+    full column tile (and that fits 80 KB) takes fewer wave slots per line."""
+    lengths = [n for n in range(32, 1300) if factor(n)[1] > 31 and factor(n)[1] <= 256]
+    for n, (lines, waves) in zip(lengths, plan([("dct", n, factor(n)[0], es, 40000, 256) for n in lengths])):
+        n1, n2 = factor(n)
+        k1 = n1 // 2 + 1
+        line = es * (n + 1 + 2 * k1 * (n2 | 1))
+
+        def products(lb):
+            return (lb * k1 + 15) // 16 * ((n2 // 2 + 16) // 16)
+
+        def slots(lb):
+            p = products(lb)
+            w = 8 if p > 4 else 4
+            return (p + w - 1) // w * w
+
+        assert lines == 1 or lines * line <= 81920
+        assert waves == (8 if products(lines) > 4 else 4), n
+        most = max(2, (15 + k1) // k1)
+        best = min(slots(lb) / lb for lb in range(1, most + 1) if lb == 1 or lb * line <= 81920)
+        assert slots(lines) / lines <= best * 1.0001, (n, lines)
+
+
+def test_x_transform_plan_small(plan):
+    """Two lines in two waves for two factors of up to 31; blocks of eight waves,
+    and of fewer lines, where a grid has too few lines for the chip."""
+    assert plan([("dct", 812, 28, 8, 49000, 256)]) == [(2, 2)]
+    assert plan([("dct", 961, 31, 4, 10, 256)]) == [(2, 2)]
+    full, = plan([("dct", 127, 1, 8, 40000, 256)])
+    few, = plan([("dct", 127, 1, 8, 1536, 256)])
+    assert few[0] == (full[0] + 1) // 2 and few[1] == 8 and full[1] == 4
