@@ -1008,7 +1008,6 @@ __global__ __launch_bounds__(256) void k_zdft_inv(int M, int C, long long plane,
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 constexpr int kLd = 4;  // loads per thread in flight in the line load phases
-constexpr int kDctShort = 4;  // most rows k1 <= N1/2 of a step A on the vector units
 
 __device__ __forceinline__ dbl4 mfma64(double a, double b, dbl4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);

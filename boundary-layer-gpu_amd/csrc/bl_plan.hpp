@@ -36,19 +36,29 @@ constexpr int dct_products(int N, int N1, int lb) { return (lb * (N1 / 2 + 1) + 
 // with two columns; 4 x 181 points FP32 322 -> 266 us for both directions, but with two
 // row tiles the second column tile costs no further round, and six lines stay:
 // 4 x 53 FP64 40 us against 49).  80 KB of LDS (two blocks per CU) bound the lines.
+// With many lines and step A on the matrix cores, as many more as four products
+// hold while four blocks fit a CU: one column tile is two products of two row
+// tiles, and two of the four waves idled (both directions, 25542 lines: 16 x 32 points
+// FP64 322 -> 275 us, FP32 191 -> 161; 14 x 41 358 -> 287 and 222 -> 170).
 // Fewer lines where the blocks would not reach every compute unit (127 points,
 // 1536 lines: 16 lines 14.9 and 11.8 us, 8 lines 12.6 and 10.5), and eight waves
-// where they do not fill the chip (129 points, 3774 lines: 19 and 17 us).
+// while all of them reside at once, 16 per CU in FP64 and 24 in FP32 by their
+// registers (129 points, 3774 lines: 19 and 17 us; but 16 x 32 FP64, 1170 lines, 585
+// blocks: 31 us with four waves, 42 with eight in two rounds).
+constexpr int kDctShort = 4;  // most rows k1 <= N1/2 of a step A on the vector units
 inline DctPlan dct_plan(int N, int N1, size_t es, int nlines, int n_cu) {
     if (dct_small(N, N1)) return {2, 2};
     const int K1 = N1 / 2 + 1;
+    const size_t line = dct_line_bytes(N, N1, es);
     auto waves = [&](int lb) { return dct_products(N, N1, lb) > 4 ? 8 : 4; };
     auto slots = [&](int lb) { return (dct_products(N, N1, lb) + waves(lb) - 1) / waves(lb) * waves(lb); };
     const int up = std::max(2, (15 + K1) / K1), down = std::max(2, 16 / K1);
     int lb = slots(down) * up < slots(up) * down ? down : up;
-    lb = std::max(1, std::min(lb, (int)(81920 / dct_line_bytes(N, N1, es))));
+    lb = std::max(1, std::min(lb, (int)(81920 / line)));
+    if (K1 > kDctShort)
+        while (dct_products(N, N1, lb + 1) <= 4 && (lb + 1) * line <= 40960 && nlines / (lb + 1) >= 8 * n_cu) ++lb;
     if ((nlines + lb - 1) / lb < n_cu) lb = (lb + 1) / 2;
-    return {lb, (nlines + lb - 1) / lb < 4 * n_cu ? 8 : waves(lb)};
+    return {lb, (nlines + lb - 1) / lb <= (es == 4 ? 3 : 2) * n_cu ? 8 : waves(lb)};
 }
 
 }  // namespace blgpu

@@ -320,3 +320,11 @@ def test_x_transform_short_factor(n, ny, nz):
 @pytest.mark.parametrize("n,ny,nz", SHORT_FACTORS)
 def test_x_transform_short_factor_mixed(n, ny, nz):
     test_x_transform_lengths_mixed(n, ny, nz)
+
+
+# with many lines a block takes as many as four products of the second factor
+# hold: three of 16 x 32 points and four of 14 x 41, with a part of a block left
+@pytest.mark.parametrize("n,ny,nz", [(512, 66, 99), (574, 70, 123)])
+def test_x_transform_more_lines(n, ny, nz):
+    test_x_transform_lengths(n, ny, nz)
+    test_x_transform_lengths_mixed(n, ny, nz)

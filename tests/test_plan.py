@@ -81,3 +81,26 @@ def test_x_transform_plan_small(plan):
     full, = plan([("dct", 127, 1, 8, 40000, 256)])
     few, = plan([("dct", 127, 1, 8, 1536, 256)])
     assert few[0] == (full[0] + 1) // 2 and few[1] == 8 and full[1] == 4
+
+
+@pytest.mark.parametrize("es", [4, 8])
+def test_x_transform_plan_waves(plan, es):
+    """Eight waves for four products or fewer only while all blocks reside at once
+    (16 waves per compute unit in FP64, 24 in FP32); with many lines and a first
+    factor past 7, no more lines that fit a quarter of the LDS fill the four waves'
+    products better (16 x 32 points: three lines in four products, not two)."""
+    lengths = [n for n in range(32, 1100) if factor(n)[1] > 31 and factor(n)[1] <= 256]
+    counts = [256, 432, 1170, 1536, 2360, 3774, 5568, 12288, 25542]
+    rows = [("dct", n, factor(n)[0], es, c, 256) for n in lengths for c in counts]
+    for (_, n, n1, _, c, _), (lines, waves) in zip(rows, plan(rows)):
+        n2, k1 = n // n1, n1 // 2 + 1
+        line = es * (n + 1 + 2 * k1 * (n2 | 1))
+
+        def products(lb):
+            return (lb * k1 + 15) // 16 * ((n2 // 2 + 16) // 16)
+
+        blocks = (c + lines - 1) // lines
+        if waves == 8 and products(lines) <= 4:
+            assert blocks * 8 <= 256 * (24 if es == 4 else 16), (n, c)
+        if c == 25542 and k1 > 4 and products(lines) <= 4:
+            assert products(lines + 1) > 4 or (lines + 1) * line > 40960 or c // (lines + 1) < 2048, (n, lines)
