@@ -75,13 +75,6 @@ __device__ __forceinline__ T get(const T *p) {
 // took 3 % longer).  128-wide FP32 tiles (fewer x-halo lines) measured
 // slower.
 // ------------------------------------------------------------------------
-template <class T>
-struct MarchTile {
-    static constexpr int TX = 64;                          // tile width (x)
-    static constexpr int RPT = sizeof(T) == 4 ? 3 : 2;    // rows per thread
-    static constexpr int TY = (256 / TX) * RPT, HX = TX + 2, HY = TY + 2, Plane = HX * HY;
-};
-
 // LES: the viscous terms use nu + nu_t (equations.f90:97-132, 231-270,
 // 367-404); nu_t is staged in a fourth LDS ring.
 template <int MODE, int FOUT, bool LES, bool NT, class T>
@@ -109,6 +102,8 @@ __global__ __launch_bounds__(256) void k_rk_march(
     // rdyg(j-1)): constant along the march, read from LDS with the velocities
     // instead of from global memory inside each equation's branch
     __shared__ T sMx[4][kTX], sMy[8][kTY];
+    static_assert(!LES || sizeof(sU) + sizeof(sV) + sizeof(sW) + sizeof(sN) + sizeof(sMx) + sizeof(sMy) ==
+                              march_lds<T>(LES), "the residency rule counts this");
     const int tid = threadIdx.x;
     const int tx = tid % kTX, ty = tid / kTX;
     const int nbx = (d.nxg - 1 + kTX - 1) / kTX, nby = (d.nyg - 2 + kTY - 1) / kTY;
@@ -2320,46 +2315,6 @@ const MetricsT<float> &metrics<float>(const Handle &h) {
 }
 
 
-template <class T>
-int march_tiles(const Dims &d) {
-    constexpr int kTX = MarchTile<T>::TX, kTY = MarchTile<T>::TY;
-    return (d.nxg - 1 + kTX - 1) / kTX * ((d.nyg - 2 + kTY - 1) / kTY);
-}
-
-// z-chunk length of the march.
-// While the launch fits in two rounds of resident blocks (three per compute
-// unit, `slots`), the chip is not filled by bytes but by plane steps in
-// sequence, and the chunk is the one with the fewest of them, rounds times
-// (chunk + 2): a block also loads the planes before and behind its chunk.  RK
-// stage, chunks of 16 or 24 planes -> this rule: 192x32x8 21 -> 9 us,
-// 129x49x34 LES FP32 54 -> 12, 257x97x64 LES FP32 76 -> 34, 131x75x53 36 -> 20,
-// 262x66x230 FP32 103 -> 52, 513x97x130 139 -> 109.
-// Larger launches are bound by HBM.  The tiles run in XCD-contiguous order
-// with the z chunk slowest, so with a multiple of 8 chunks each XCD holds
-// whole chunk layers and a tile's x and y neighbours (whose halos it shares)
-// sit in the same L2; the count is the multiple of 8 that gives chunks of
-// about 24 planes.  At 814x257x193 (8 chunks of 24 planes) this measured 1 %
-// (FP64) and 2.4 % (FP32) faster than 12 chunks of 16, and 3 % and 9 % faster
-// than the 28 planes that the first rule would take.  Below 128 planes, chunks
-// of up to 16 planes (the two re-read halo planes stay a small share).
-inline int march_chunk(int nz, int tiles, int slots) {
-    int best = nz;
-    long long cost = -1, nblk = 0;
-    for (int chunk = nz; chunk >= 1; --chunk) {
-        const long long blocks = (long long)tiles * ((nz + chunk - 1) / chunk);
-        const long long c = (blocks + slots - 1) / slots * (chunk + 2);
-        if (cost < 0 || c < cost) {
-            cost = c;
-            best = chunk;
-            nblk = blocks;
-        }
-    }
-    if (nblk <= 2LL * slots) return best;
-    const int nch = nz >= 8 * 16 ? 8 * std::max(1, (nz + 8 * 12) / (8 * 24))  // multiple of 8 nearest nz / 24
-                                 : (nz + 15) / 16;
-    return std::max(1, (nz + nch - 1) / nch);
-}
-
 // Whether a march accesses what it touches once (the old field and all results)
 // past the caches: where its nine arrays (the field, the old one or F1, the
 // result) exceed the 256 MB of the last-level cache.  RK stage and the x
@@ -2375,7 +2330,8 @@ template <int MODE, int FOUT, class T>
 void march(Handle &h, const Fld3<T> &cur, const Fld3<T> *old, const Fld3<T> *f1, Fld3<T> *nxt, Fld3<T> *fo,
            double c0, double c1, double dt, double g2 = 0.0) {
     const Dims &d = h.d;
-    const int tiles = march_tiles<T>(d), chunk = march_chunk(d.nzg - 2, tiles, 3 * h.n_cu);
+    const int tiles = march_tiles<T>(d.nxg, d.nyg);
+    const int chunk = march_chunk(d.nzg - 2, tiles, h.n_cu, march_resident<T>(h.les != 0));
     const dim3 grid(xcd_blocks(tiles * ((d.nzg - 2 + chunk - 1) / chunk))), block(256);
     const T *o[3] = {old ? old->u : nullptr, old ? old->v : nullptr, old ? old->w : nullptr};
     const T *f[3] = {f1 ? f1->u : nullptr, f1 ? f1->v : nullptr, f1 ? f1->w : nullptr};

@@ -61,4 +61,79 @@ inline DctPlan dct_plan(int N, int N1, size_t es, int nlines, int n_cu) {
     return {lb, (nlines + lb - 1) / lb <= (es == 4 ? 3 : 2) * n_cu ? 8 : waves(lb)};
 }
 
+// ---- marches in z ----
+
+// The chunk of nk planes with the fewest plane steps in sequence, rounds of the
+// resident blocks (`slots`) times (chunk + 2), since a block also loads the planes
+// before and behind its chunk; blocks: of the launch, `tiles` columns of chunks.
+// Of chunks with equally many, the longest, or the shortest while the launch has
+// no more than `most` blocks.
+struct ZChunk {
+    int planes;
+    long long blocks;
+};
+inline ZChunk fewest_plane_steps(int nk, int tiles, int slots, long long most = 0) {
+    ZChunk best{nk, 0};
+    long long cost = -1;
+    for (int chunk = nk; chunk >= 1; --chunk) {
+        const long long blocks = (long long)tiles * ((nk + chunk - 1) / chunk);
+        const long long c = (blocks + slots - 1) / slots * (chunk + 2);
+        if (cost < 0 || c < cost || (c == cost && blocks <= most)) {
+            cost = c;
+            best = {chunk, blocks};
+        }
+    }
+    return best;
+}
+
+// Tiles of the RK march (k_rk_march): 64 x 8 cells in FP64, 64 x 12 in FP32.
+template <class T>
+struct MarchTile {
+    static constexpr int TX = 64;                          // tile width (x)
+    static constexpr int RPT = sizeof(T) == 4 ? 3 : 2;    // rows per thread
+    static constexpr int TY = (256 / TX) * RPT, HX = TX + 2, HY = TY + 2, Plane = HX * HY;
+};
+template <class T>
+constexpr int march_tiles(int nxg, int nyg) {
+    return (nxg - 1 + MarchTile<T>::TX - 1) / MarchTile<T>::TX * ((nyg - 2 + MarchTile<T>::TY - 1) / MarchTile<T>::TY);
+}
+// LDS bytes of a block: two planes of U and V, three of W, with an eddy
+// viscosity three of nu_t, and the tile's metrics
+template <class T>
+constexpr size_t march_lds(bool les) {
+    return sizeof(T) * ((les ? 10 : 7) * MarchTile<T>::Plane + 4 * MarchTile<T>::TX + 8 * MarchTile<T>::TY);
+}
+// blocks that reside on a compute unit: three by the registers of the stages
+// (128 to 168 of them), two with an eddy viscosity in FP64 by its 54 KB of LDS
+template <class T>
+constexpr int march_resident(bool les) {
+    return std::min<int>(3, 163840 / march_lds<T>(les));
+}
+
+// z-chunk length of the RK march over nz planes.
+// While the launch is of up to six blocks per compute unit, the chip is not
+// filled by bytes but by plane steps in sequence, and the chunk is the one with
+// the fewest of them.  RK stage, chunks of 16 or 24 planes -> this rule:
+// 192x32x8 21 -> 9 us, 129x49x34 LES FP32 54 -> 12, 257x97x64 LES FP32 76 -> 34,
+// 131x75x53 36 -> 20, 262x66x230 FP32 103 -> 52, 513x97x130 139 -> 109.  FP64 LES,
+// of which two blocks reside, with three counted -> with two: 278x266x34 74 -> 58
+// us, 257x97x64 54 -> 42, 622x259x49 193 -> 158; short chunks of equal cost fill
+// the last round (390x244x57 FP64 LES: 28 planes 123 us, 8 planes 112).
+// Larger launches are bound by HBM.  The tiles run in XCD-contiguous order
+// with the z chunk slowest, so with a multiple of 8 chunks each XCD holds
+// whole chunk layers and a tile's x and y neighbours (whose halos it shares)
+// sit in the same L2; the count is the multiple of 8 that gives chunks of
+// about 24 planes.  At 814x257x193 (8 chunks of 24 planes) this measured 1 %
+// (FP64) and 2.4 % (FP32) faster than 12 chunks of 16, and 3 % and 9 % faster
+// than the 28 planes that the first rule would take.  Below 128 planes, chunks
+// of up to 16 planes (the two re-read halo planes stay a small share).
+inline int march_chunk(int nz, int tiles, int n_cu, int resident) {
+    const long long few = 6LL * n_cu;
+    const ZChunk c = fewest_plane_steps(nz, tiles, resident * n_cu, few);
+    if (c.blocks <= few) return c.planes;
+    const int nch = nz >= 8 * 16 ? 8 * std::max(1, (nz + 8 * 12) / (8 * 24))  // multiple of 8 nearest nz / 24
+                                 : (nz + 15) / 16;
+    return std::max(1, (nz + nch - 1) / nch);
+}
+
 }  // namespace blgpu

@@ -21,6 +21,11 @@ int main() {
             const DctPlan p = dct_plan(a, b, (size_t)c, d, e);
             std::printf("%d %d\n", p.lines, p.waves);
         }
+        if (!std::strcmp(k, "march")) {  // element size, eddy viscosity, nx, ny, nz; 256 compute units
+            const int res = a == 4 ? march_resident<float>(b) : march_resident<double>(b);
+            const int tiles = a == 4 ? march_tiles<float>(c + 1, d + 1) : march_tiles<double>(c + 1, d + 1);
+            std::printf("%d %d %d\n", march_chunk(e - 1, tiles, 256, res), tiles, res);
+        }
     }
 }
 """
@@ -104,3 +109,27 @@ def test_x_transform_plan_waves(plan, es):
             assert blocks * 8 <= 256 * (24 if es == 4 else 16), (n, c)
         if c == 25542 and k1 > 4 and products(lines) <= 4:
             assert products(lines + 1) > 4 or (lines + 1) * line > 40960 or c // (lines + 1) < 2048, (n, lines)
+
+
+def test_march_plan(plan):
+    """The z chunk of the RK march: no other chunk takes fewer plane steps in
+    sequence (rounds of the blocks that reside by their LDS, at most three, times
+    chunk + 2) while the launch is of up to six blocks per compute unit.  An FP64
+    block with an eddy viscosity holds ten planes of 66 x 10, so two reside, and
+    278x266x34 goes in one round."""
+    shapes = [(278, 266, 34), (161, 57, 42), (390, 244, 57), (292, 206, 196), (716, 261, 63), (24, 16, 8), (5, 4, 5)]
+    shapes += [(60 + 37 * i, 20 + 23 * i % 270, 8 + 41 * i % 230) for i in range(20)]
+    rows = [("march", es, les, *s) for s in shapes for es in (4, 8) for les in (0, 1)]
+    for (_, es, les, nx, ny, nz), (chunk, tiles, res) in zip(rows, plan(rows)):
+        plane = 66 * (4 * (3 if es == 4 else 2) + 2)
+        assert res == min(3, 163840 // (es * (plane * (10 if les else 7) + 4 * 64 + 8 * (plane // 66 - 2))))
+        assert res == (2 if es == 8 and les else 3)
+        nk = nz - 1
+        steps = {c: -(-tiles * -(-nk // c) // (256 * res)) * (c + 2) for c in range(1, nk + 1)}
+        blocks = tiles * -(-nk // chunk)
+        if blocks <= 6 * 256:
+            least = min(steps.values())
+            few = [c for c in steps if steps[c] == least and tiles * -(-nk // c) <= 6 * 256]
+            assert not few or chunk == min(few), (es, les, nx, ny, nz)
+        if (es, les, nx) == (8, 1, 278):
+            assert blocks <= 256 * res
