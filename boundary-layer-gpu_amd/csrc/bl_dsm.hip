@@ -36,6 +36,7 @@
 
 #include "../../include/blgpu.h"
 #include "bl_internal.hpp"
+#include "bl_plan.hpp"
 
 namespace blgpu {
 
@@ -269,9 +270,9 @@ __device__ __forceinline__ double filt_xy(PlanePtr<T> F, unsigned o, unsigned sx
 // (27 instead of 81 loads per cell).  The ghost and duplicated planes are
 // copies of centres 1, 2 and nzg-3, written with them.
 template <bool PX, class T>
-__global__ __launch_bounds__(256) void k_dsm_vfilter(Dims d, const T *__restrict__ U, const T *__restrict__ V,
-                                                     const T *__restrict__ W, double *__restrict__ Uf,
-                                                     double *__restrict__ Vf, double *__restrict__ Wf, int chunk) {
+__global__ __launch_bounds__(256, vfilter_resident<T>()) void k_dsm_vfilter(
+    Dims d, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W, double *__restrict__ Uf,
+    double *__restrict__ Vf, double *__restrict__ Wf, int chunk) {
     const int i = blockIdx.x * 64 + (threadIdx.x & 63);
     const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (i >= d.nxg || j >= d.nyg) return;
@@ -324,7 +325,8 @@ __global__ __launch_bounds__(256) void k_dsm_vfilter(Dims d, const T *__restrict
 // six |S| S_ij of the other buffer in y from LDS, in x between lanes and in z
 // through two running values per quantity in registers, and contract.  Nothing
 // but |S| and the two sums per column and chunk goes to memory.  Bound by
-// issue: FP64 arithmetic with two blocks (14 waves) per CU, 120 registers.
+// issue: FP64 arithmetic with two blocks (14 waves) per CU; 120 registers in FP32
+// fields, in FP64 fields all 128 and 60 bytes a lane spilled.
 // At 257x97x64 in FP32 fields the model's three passes take 0.022 + 0.064 +
 // 0.010 ms per stage.  With all steps in four waves, filters of 9 LDS reads and
 // plain loads, which waited one after the other, the middle one took 0.153;
@@ -572,28 +574,11 @@ void check() {
     }
 }
 
-// z chunk length of a marching pass over nk planes with `tiles` column tiles,
-// of which `slots` blocks are resident at a time: the one with the fewest plane
-// steps in sequence, rounds of blocks times (chunk + 2), since a chunk also
-// forms the plane before and the plane behind it.  At 257x97x64 (144 tiles, 512
-// slots) that is 9 planes, two full rounds, against 8 planes in 2.25 rounds.
-int dsm_chunk(int nk, int tiles, int slots) {
-    int best = nk;
-    long long cost = -1;
-    for (int chunk = nk; chunk >= 1; --chunk) {
-        const long long blocks = (long long)tiles * ((nk + chunk - 1) / chunk);
-        const long long c = (blocks + slots - 1) / slots * (chunk + 2);
-        if (cost < 0 || c < cost) {
-            cost = c;
-            best = chunk;
-        }
-    }
-    return best;
-}
-// resident blocks per compute unit, by their registers (and the LDS of k_dsm_stress)
-constexpr int kStressPerCU = 2, kVfilterPerCU = 4;
 int stress_tiles(const Dims &d) {
     return ((d.nxg - 2 + kDsX - 3) / (kDsX - 2)) * ((d.nyg - 2 + kDsY - 3) / (kDsY - 2));
+}
+int stress_chunk(const Handle &h, int nk) {
+    return fewest_plane_steps(nk, stress_tiles(h.d), kStressResident * h.n_cu).planes;
 }
 
 template <bool PX, class T>
@@ -607,13 +592,13 @@ void dsm_t(Handle &h, const Fld3<T> &f, T *nu_t) {
     const dim3 gcol((d.nxg + 63) / 64, (d.nyg + 3) / 4);
     {
         ProfScope ps(h, KID_DSM_VFILTER);
-        const int chunk = dsm_chunk(nk, gcol.x * gcol.y, kVfilterPerCU * h.n_cu);
+        const int chunk = fewest_plane_steps(nk, gcol.x * gcol.y, vfilter_resident<T>() * h.n_cu, 6 * h.n_cu).planes;
         hipLaunchKernelGGL((k_dsm_vfilter<PX, T>), dim3(gcol.x, gcol.y, (nk + chunk - 1) / chunk), block, 0, h.stream,
                            d, f.u, f.v, f.w, Uf, Vf, Wf, chunk);
         check();
     }
     const int tiles = stress_tiles(d);
-    const int chunk = dsm_chunk(nk, tiles, kStressPerCU * h.n_cu), nch = (nk + chunk - 1) / chunk;
+    const int chunk = stress_chunk(h, nk), nch = (nk + chunk - 1) / chunk;
     {
         ProfScope ps(h, KID_DSM_FILTER);
         hipLaunchKernelGGL((k_dsm_stress<PX, T>), dim3(tiles, nch), dim3(kDsX * kDsY + kDsOwn), 0, h.stream, d, h.m, f.u, f.v, f.w, Uf, Vf,
@@ -655,7 +640,7 @@ void eddy_t(Handle &h, const Fld3<T> &f, T *nu_t) {
 
 size_t dsm_doubles(const Handle &h) {
     const Dims &d = h.d;
-    const int nk = d.nzg - 3, chunk = dsm_chunk(nk, stress_tiles(d), kStressPerCU * h.n_cu);
+    const int nk = d.nzg - 3, chunk = stress_chunk(h, nk);
     return (size_t)d.sxy * ((size_t)D_END * d.nzg + 2 * (size_t)((nk + chunk - 1) / chunk));
 }
 

@@ -136,4 +136,17 @@ inline int march_chunk(int nz, int tiles, int n_cu, int resident) {
     return std::max(1, (nz + nch - 1) / nch);
 }
 
+// Blocks of the dynamic model's marching passes that reside on a compute unit:
+// k_dsm_vfilter has four waves of 122 registers in FP32 fields and of 170 in FP64
+// (two blocks; with four counted 130x100x32 took 23 us, now 19, 400x128x96 115 and
+// 121; 42 sizes 4 % less on average, the chunk among equal ones the shortest up to
+// six blocks); k_dsm_stress seven waves of up to 128 and 72 to 76 KB of LDS: at
+// 257x97x64 (144 tiles, 512 slots) it takes 9 planes, two full rounds, against 8
+// planes in 2.25 rounds.
+template <class T>
+constexpr int vfilter_resident() {
+    return sizeof(T) == 4 ? 4 : 2;
+}
+constexpr int kStressResident = 2;
+
 }  // namespace blgpu

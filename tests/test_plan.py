@@ -26,6 +26,8 @@ int main() {
             const int tiles = a == 4 ? march_tiles<float>(c + 1, d + 1) : march_tiles<double>(c + 1, d + 1);
             std::printf("%d %d %d\n", march_chunk(e - 1, tiles, 256, res), tiles, res);
         }
+        if (!std::strcmp(k, "steps")) std::printf("%d\n", fewest_plane_steps(a, b, c, d).planes);
+        if (!std::strcmp(k, "vfilter")) std::printf("%d\n", a == 4 ? vfilter_resident<float>() : vfilter_resident<double>());
     }
 }
 """
@@ -133,3 +135,18 @@ def test_march_plan(plan):
             assert not few or chunk == min(few), (es, les, nx, ny, nz)
         if (es, les, nx) == (8, 1, 278):
             assert blocks <= 256 * res
+
+
+def test_filter_plan(plan):
+    """The velocity filter of the dynamic model: blocks of four waves, of which a
+    compute unit holds four with up to 128 registers (FP32 fields) and two with up to
+    256 (FP64; the kernel's launch bounds are these figures), and the chunk of the
+    fewest plane steps among them, the shortest of equal ones up to a block count."""
+    assert plan([("vfilter", 4, 0, 0, 0, 0), ("vfilter", 8, 0, 0, 0, 0)]) == [(4,), (2,)]
+    rows = [("steps", nk, tiles, slots, most, 0) for nk in (3, 24, 62, 97) for tiles in (1, 18, 130, 192, 700)
+            for slots in (512, 1024) for most in (0, 1536)]
+    for (_, nk, tiles, slots, most, _), (chunk,) in zip(rows, plan(rows)):
+        steps = {c: -(-tiles * -(-nk // c) // slots) * (c + 2) for c in range(1, nk + 1)}
+        equal = [c for c in steps if steps[c] == min(steps.values())]
+        few = [c for c in equal if tiles * -(-nk // c) <= most]
+        assert chunk == (min(few) if few else max(equal))
