@@ -36,7 +36,6 @@
 
 #include "../../include/blgpu.h"
 #include "bl_internal.hpp"
-#include "bl_plan.hpp"
 
 namespace blgpu {
 

@@ -13,6 +13,8 @@
 #include <string>
 #include <vector>
 
+#include "bl_plan.hpp"
+
 namespace blgpu {
 
 struct Dims {
@@ -46,10 +48,6 @@ __device__ __forceinline__ int small_div(int a, float rb) { return (int)(((float
 // has xcd_blocks(T) blocks; a block whose tile is >= T returns at once.
 __host__ __device__ inline int xcd_blocks(int T) { return 8 * ((T + 7) / 8); }
 __host__ __device__ inline int xcd_tile(int b, int T) { return (b % 8) * ((T + 7) / 8) + b / 8; }
-
-// Partitioned Thomas solve: rows per segment (held in registers) and
-// segments per system, so systems up to NM = 256 rows take that kernel.
-constexpr int kThSeg = 32, kThMaxP = 8;
 
 // Block order of the Thomas sweeps (nkb kx blocks times M spectral rows, one
 // block id b each).  Rows q = 2k-1 and 2k (real and imaginary parts of z

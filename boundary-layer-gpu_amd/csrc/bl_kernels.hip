@@ -18,7 +18,6 @@
 #include <vector>
 
 #include "bl_internal.hpp"
-#include "bl_plan.hpp"
 
 namespace blgpu {
 
@@ -1722,9 +1721,10 @@ __device__ void solve00_block(const Solve00 &z, int NM);
 // L = 32 P: a[j] couples x(j-1), c[j] couples x(j+1), b[j] + kxx + kzz is
 // the diagonal.  The (0,0) system (kx = 0, q = 0, pinned first pivot) is
 // skipped (zero00 = 0) or zeroed (zero00 = 1); block 0 solves it (z) while
-// the other blocks run.  The other blocks (8 waves of more than 128 VGPRs each
-// reside on a CU) loop over the nq * ceil(N/64) tiles of 64 systems.
-// A tile's time is that of its loads plus that of its arithmetic (the 8 waves of
+// the other blocks run.  The other blocks, as many as reside (thomas_resident:
+// up to eight waves a CU, four with one segment), loop over the nq * ceil(N/64)
+// tiles of 64 systems.
+// A tile's time is that of its loads plus that of its arithmetic (the waves of
 // a CU go through both together).  The coefficients come from LDS, a row is a
 // scalar offset into a buffer and no row is masked: with scalar coefficient
 // loads and guarded rows 900 of the 2500 instructions were scalar register
@@ -1737,6 +1737,7 @@ __global__ __launch_bounds__(64 * kThMaxP) void k_thomas_seg(int N, int NM, int 
                                                              T *__restrict__ S, Solve00 z) {
     __shared__ double xs[6][kThMaxP][64];
     __shared__ double ca[kThSeg * kThMaxP], cb[kThSeg * kThMaxP], cc[kThSeg * kThMaxP];
+    static_assert(sizeof(xs) + 8 * sizeof(ca) == kThomasLds, "the residency rule counts this and solve00_block's rows");
     if (blockIdx.x == 0) {  // the (0,0) system, alongside the other blocks
         solve00_block<kThSeg * kThMaxP>(z, NM);
         return;
@@ -2537,11 +2538,11 @@ template <class T>
 bool launch_thomas_seg(Handle &h, T *S, int ldj, long long ldq, const Solve00 &z) {
     const Dims &d = h.d;
     if (h.th_p == 0) return false;
-    // the resident blocks (a CU has the registers of 8 waves), each looping over
-    // its tiles, one of them block 0 for the (0,0) system.  With one block per CU
-    // also where a block is 3 waves the solve took 39 us at 260x65x228 (FP32).
+    // the resident blocks, each looping over its tiles, one of them block 0 for the
+    // (0,0) system.  With one block per CU also where a block is 3 waves the solve
+    // took 39 us at 260x65x228 (FP32).
     const int ntiles = (d.N + 63) / 64 * d.M;
-    const int nblk = std::max(1, std::min(ntiles, std::max(2, h.n_cu) * (kThMaxP / h.th_p) - 1));
+    const int nblk = std::max(1, std::min(ntiles, std::max(2, h.n_cu) * thomas_resident(h.th_p) - 1));
     hipLaunchKernelGGL(k_thomas_seg<T>, dim3(1 + nblk), dim3(64 * h.th_p), 0, h.stream, d.N, d.NM, h.th_p, d.M,
                        ldj, ldq, (const double *)h.th_co, z.part ? 1 : 0, S, z);
     check_launch();

@@ -149,4 +149,18 @@ constexpr int vfilter_resident() {
 }
 constexpr int kStressResident = 2;
 
+// ---- partitioned Thomas solve (k_thomas_seg) ----
+
+// rows per segment (held in registers) and segments per system, so systems up to
+// NM = 256 rows take that kernel
+constexpr int kThSeg = 32, kThMaxP = 8;
+// LDS bytes of a block, whatever its segments: the interface values of up to eight,
+// the coefficients, and the rows of the (0,0) system for the block that solves it
+constexpr size_t kThomasLds = sizeof(double) * (6 * kThMaxP * 64 + (3 + 5) * kThSeg * kThMaxP);
+// Blocks of P waves that reside on a compute unit: eight waves by their registers
+// (more than 128), four blocks by their LDS.  A launch of more leaves blocks that
+// start with few tiles left: one segment, eight -> four blocks, 600x16x120 FP64 20.2
+// -> 17.8 us, 300x25x290 FP32 19.3 -> 17.5.
+constexpr int thomas_resident(int P) { return std::min<int>(kThMaxP / P, 163840 / kThomasLds); }
+
 }  // namespace blgpu

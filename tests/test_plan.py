@@ -26,6 +26,7 @@ int main() {
             const int tiles = a == 4 ? march_tiles<float>(c + 1, d + 1) : march_tiles<double>(c + 1, d + 1);
             std::printf("%d %d %d\n", march_chunk(e - 1, tiles, 256, res), tiles, res);
         }
+        if (!std::strcmp(k, "thomas")) std::printf("%d\n", thomas_resident(a));
         if (!std::strcmp(k, "steps")) std::printf("%d\n", fewest_plane_steps(a, b, c, d).planes);
         if (!std::strcmp(k, "vfilter")) std::printf("%d\n", a == 4 ? vfilter_resident<float>() : vfilter_resident<double>());
     }
@@ -150,3 +151,10 @@ def test_filter_plan(plan):
         equal = [c for c in steps if steps[c] == min(steps.values())]
         few = [c for c in equal if tiles * -(-nk // c) <= most]
         assert chunk == (min(few) if few else max(equal))
+
+
+def test_y_solve_plan(plan):
+    """Blocks of the y solve per compute unit: eight waves by their registers, and
+    each block, whatever its waves, has 40 KB of LDS, so four blocks at most."""
+    for p, (n,) in zip(range(1, 9), plan([("thomas", p, 0, 0, 0, 0) for p in range(1, 9)])):
+        assert n == min(8 // p, 163840 // 40960)
