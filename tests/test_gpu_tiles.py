@@ -328,3 +328,31 @@ def test_x_transform_short_factor_mixed(n, ny, nz):
 def test_x_transform_more_lines(n, ny, nz):
     test_x_transform_lengths(n, ny, nz)
     test_x_transform_lengths_mixed(n, ny, nz)
+
+
+# the same marches by what a step changes, each component against its own change.
+# With noise of 0.3 the eddy viscosity makes 0.15, 0.003 and 0.15 of the change of
+# U, V and W (FP32 grid; 0.29, 0.0035 and 0.21 FP64), so a march without it, or with
+# nu_t of another cell, is ten times past the bounds or more.  FP32: the z
+# transforms' 5e-5 (as for the recorded pressure above) of the pressure gradient,
+# whose norm is that of V's change at most, 2.7 times W's; the rounding of the RHS
+# (1e-5) and of what is stored (6 times 3e-8 of |U|, 11 times W's change) are far
+# below: 1.5e-4, and twice that.  FP64: 2e-11 of the pressure solution likewise,
+# 6e-11, and twice that.
+@pytest.mark.parametrize("nx,les,precision", [(130, 1, 0), (260, 0, 1), (260, 1, 1)])
+def test_march_streams_increment(nx, les, precision):
+    say("streaming march, increment", nx, les, precision)
+    case = cases.laminar_small(nx=nx, ny=130, nz=250, Lz=0.15, noise=0.3, seed=5, les=les, cfl=-1e-5)
+    o = case.oracle()
+    if precision:
+        o.set_fields(*[np.asfortranarray(a.astype(np.float32).astype(np.float64)) for a in o.fields()])
+    old = [a.copy() for a in o.fields()]
+    s = (mixed_solver(case, o) if precision else solver_for(case, o)[0])
+    o.compute_dt(), s.compute_dt()
+    o.step()
+    s.step()
+    for a, b, c in zip(s.fields(), o.fields(), old):
+        err = np.linalg.norm(a - b) / np.linalg.norm(b - c)
+        say("err", err)
+        assert err < (3e-4 if precision else 1.2e-10)
+    s.close()
