@@ -134,7 +134,7 @@ def test_statistics_block_edges(shape):
 
 
 # the z chunk of the stage march changes with the grid: one plane per block,
-# two, a remainder, and (nz = 193 with one tile row) the many-plane rule
+# two (with a remainder) and three
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("shape", [(70, 9, 5), (131, 20, 13), (66, 25, 101), (300, 60, 40)])
 def test_rhs_march_chunks(shape, precision):
@@ -356,3 +356,11 @@ def test_march_streams_increment(nx, les, precision):
         say("err", err)
         assert err < (3e-4 if precision else 1.2e-10)
     s.close()
+
+
+# large launches of fewer than 128 planes: 385 tiles by 12, 12 and 11 planes in FP64,
+# where no chunk keeps the launch to six blocks per compute unit at fewest plane steps;
+# the same grid in FP32 takes a short last chunk by the rule of the smaller launches
+@pytest.mark.parametrize("precision", [0, 1])
+def test_rhs_march_large_launch(precision):
+    test_rhs_march_chunks((642, 276, 36), precision)
