@@ -17,7 +17,10 @@
 //   Zf[q][m]: q = 0 -> 1, q = 2k-1 -> cos(2 pi k m / M), q = 2k -> -sin(2 pi k m / M)
 //   Zi[m][q]: q = 0 -> 1, q = 2k-1 -> 2 cos (cos at k = M/2), q = 2k -> -2 sin
 // Spectral work arrays: T1[m][j][kx] and S[q][j][kx], kx stride NP = N
-// rounded up to 32 (the padding stays zero).
+// rounded up to 32.  The padding kx >= N is undefined (T1 also stages field
+// transfers, so it may hold NaN patterns): the z transforms carry its columns along,
+// which are independent of the others, the y solves touch kx < N only, and a product
+// over kx masks k >= N.
 #include <hip/hip_runtime.h>
 
 #include <cmath>

@@ -364,3 +364,33 @@ def test_march_streams_increment(nx, les, precision):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_rhs_march_large_launch(precision):
     test_rhs_march_chunks((642, 276, 36), precision)
+
+
+# the spectral rows of the mixed path are padded to 32 values, and transfers pass
+# through the same array: uploads whose low words are FP32 NaN patterns leave NaN in
+# every other padding entry, and no solution entry may depend on it.  One length of each
+# path: two-factor and dense x, folded and dense z (past 96 rows), partitioned and
+# table y solve (past 256 rows).  To the bound of the mixed x transforms.
+@pytest.mark.parametrize("n,ny,nz", [(37, 7, 6), (251, 7, 6), (257, 6, 7), (37, 5, 202), (257, 5, 202), (37, 260, 6)])
+def test_mixed_padding_undefined(n, ny, nz):
+    say("mixed padding", n, ny, nz)
+    rng = np.random.default_rng(n)
+    nx = n + 2
+    x = 1.0 + 0.001 * np.arange(nx)
+    y = np.cumsum(np.r_[0, 0.002 + 0.0005 * rng.random(ny - 1)])
+    z = 0.0015 * np.arange(nz)
+    P = []
+    f = []
+    for sh in [(nx, ny + 1, nz + 1), (nx + 1, ny, nz + 1), (nx + 1, ny + 1, nz)]:
+        a = rng.standard_normal(sh)
+        a.view(np.uint32).reshape(-1, 2)[:, 0] = 0x7FC00001
+        f.append(np.asfortranarray(a))
+    for precision in (0, 1):
+        s = solver(x, y, z, precision=precision)
+        s.set_fields(*(f if precision else [np.asfortranarray(a.astype(np.float32).astype(np.float64)) for a in f]))
+        s.projection(1, 1e-4)
+        P.append(s.download(3)[1:n + 1, 1:ny, 1:nz - 1])
+        s.close()
+    err = np.linalg.norm(P[1] - P[0]) / np.linalg.norm(P[0])
+    say("err", err)
+    assert err < 5e-5
