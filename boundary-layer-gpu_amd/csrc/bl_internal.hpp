@@ -267,13 +267,15 @@ struct IncLine {
     __device__ __forceinline__ double at(int n) const { return div(load(n), n); }
 };
 
-// Kernel classes timed by the optional HIP-event profiler.
+// Kernel classes timed by the optional HIP-event profiler.  Their ids and names are
+// part of the interface (the bits of bl_profile_select), so a class stays where its
+// launches have become part of another's.
 enum KernelId {
     KID_RK_STAGE = 0,
-    KID_BC_INOUT,
-    KID_BC_PERIODIC,
-    KID_BC_TOPWALL,
-    KID_BC_MASSFLUX,
+    KID_BC_INOUT,     // the boundary values of the stages (k_bc_planes)
+    KID_BC_PERIODIC,  // no launch of its own: part of the next
+    KID_BC_TOPWALL,   // every boundary and ghost entry: in- and outflow, periodic planes, top and wall (k_bc_apply)
+    KID_BC_MASSFLUX,  // the shift of the outflow (k_bc_shift)
     KID_DIVERGENCE,
     KID_XFORM_X_FWD,
     KID_XFORM_Z_FWD,

@@ -306,7 +306,10 @@ int bl_profile_select(bl_handle *h, unsigned long long mask);
 /* Accumulated milliseconds and launch counts per kernel class id 0..n-1
  * since profiling was enabled. */
 int bl_profile_read(bl_handle *h, double *ms, long long *launches, int n);
-/* Number of kernel classes and the name of class id. */
+/* Number of kernel classes and the name of class id.  Ids and names do not
+ * change; a class whose launches are part of another's counts none: bc_topwall
+ * is the gather of every boundary and ghost entry, bc_periodic's among them, and
+ * divergence is part of xform_x_fwd where the x transform forms it. */
 int bl_profile_count(void);
 const char *bl_profile_name(int id);
 
