@@ -459,15 +459,11 @@ void build(Handle &h, const bl_config *c) {
             return std::pair<double, double>((double)cosl(ang), (double)sinl(ang));
         };
         const int k1n = n1 / 2 + 1;
-        if (!(n1 <= 32 && k1n <= 16 && n2 <= 32) && h.precision == BL_PREC_FP64) {
-            // lengths whose two lines and their spectra do not fit 64 KB of LDS are refused
-            const size_t lds = sizeof(double2) * (2 * (size_t)N + 2 * (size_t)k1n * n2 + n1 + n2);
-            if (lds > 65536) {
-                last_error() = "bl_create: the x transform of nx - 2 = " + std::to_string(N) + " points (" +
-                               std::to_string(n1) + " x " + std::to_string(n2) +
-                               ") does not fit the LDS-resident DCT; choose nx - 2 with a divisor near its square root";
-                throw ArgError();
-            }
+        if (h.precision == BL_PREC_FP64 && !dct_takes_fp64(N, n1)) {
+            last_error() = "bl_create: the x transform of nx - 2 = " + std::to_string(N) + " points (" +
+                           std::to_string(n1) + " x " + std::to_string(n2) +
+                           ") does not fit the LDS-resident DCT; choose nx - 2 with a divisor near its square root";
+            throw ArgError();
         }
         std::vector<double> tab;
         auto push = [&](std::pair<double, double> w) {

@@ -366,7 +366,7 @@ struct Handle {
     // mixed precision: BF16 hi/lo transform matrices, FP64 (0,0) mode
     int NP;                         // kx stride of the FP32 spectral arrays (N rounded up to 32)
     int kpx, kpz;                   // GEMM depths N and M rounded up to 32
-    bool mx_two = false;            // x transform as two short FP32 DFTs (dct_fits_mixed), else a dense GEMM
+    bool mx_two = false;            // x transform as two short FP32 DFTs (dct_takes_mixed), else a dense GEMM
     unsigned short *mx_tab;         // one allocation for the eight matrices below
     unsigned short *zmf = nullptr;  // folded z transform fragments (k_zdft_mx), M/2 + 1 <= 96
     int zmf_rt = 0;
@@ -531,9 +531,8 @@ void snapshot_free(Handle &h);
 // ---- mixed precision (bl_mixed.hip) ----
 void build_mixed(Handle &h);
 // the mixed path's x transforms as two short FP32 DFTs (bl_kernels.hip), for
-// lengths N = N1 N2 that they take: divergence, its FP64 line sums (p00[j][m]) and
+// lengths N = N1 N2 that they take (dct_takes_mixed): divergence, its FP64 line sums (p00[j][m]) and
 // the forward transform into rows of stride NP; the inverse plus add[j]
-bool dct_fits_mixed(int N, int N1);
 void launch_xfwd_mixed(Handle &h, const Fld3<float> &f, float *T1, const BcPlanes<float> *bc, const IncSrc *inc);
 void launch_xinv_mixed(Handle &h, const float *T1, const double *add, float *phi);
 void launch_poisson_mixed(Handle &h, float *phi, const Fld3<float> &f, const BcPlanes<float> *bc = nullptr,

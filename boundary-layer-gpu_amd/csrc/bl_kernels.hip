@@ -2505,12 +2505,6 @@ void launch_poisson(Handle &h, double *phi, const Field3 *div, const BcPlanes<do
     dct_launch(h, KID_XFORM_X_INV, da, false, (const double *)h.T1, phi);
 }
 
-bool dct_fits_mixed(int N, int N1) {
-    const int N2 = N / N1, K1 = N1 / 2 + 1;
-    // small_div's range, and one line in LDS (forward and inverse)
-    return N2 <= 256 && K1 <= 128 && K1 * N2 < 16384 && 2 * dct_line_bytes(N, N1, sizeof(float)) <= 163840;
-}
-
 void launch_xfwd_mixed(Handle &h, const Fld3<float> &f, float *T1, const BcPlanes<float> *bc, const IncSrc *inc) {
     const Dims &d = h.d;
     DctArgs<float> a{};

@@ -671,7 +671,7 @@ void build_mixed(Handle &h) {
     h.dct_n1 = 1;
     for (int a = 1; (long long)a * a <= N; ++a)
         if (N % a == 0) h.dct_n1 = a;
-    h.mx_two = dct_fits_mixed(N, h.dct_n1);
+    h.mx_two = dct_takes_mixed(N, h.dct_n1);
     if (!h.mx_two) {
         split_matrix(N, N, rpx, h.kpx, [&](int k, int n) { return 2.0L * cosx(k, n); }, t[0], t[1]);
         split_matrix(N, N, rpx, h.kpx,

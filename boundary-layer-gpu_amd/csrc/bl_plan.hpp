@@ -18,6 +18,24 @@ constexpr int dct_lines(int LB, int N) { return (LB * N + 1) / 2 * 2; }
 constexpr size_t dct_line_bytes(int N, int N1, size_t es) {
     return es * (N + 1 + 2 * (size_t)(N1 / 2 + 1) * dct_ld(N / N1));
 }
+// What the kernels hold of N = N1 N2 points: an entry of a line's spectrum and a row
+// k1 <= N1/2 in the range of small_div, one line of either direction in 160 KB.
+constexpr bool dct_holds(int N, int N1, size_t es) {
+    return N1 / 2 + 1 <= 128 && (N1 / 2 + 1) * (N / N1) < 16384 && 2 * dct_line_bytes(N, N1, es) <= 163840;
+}
+// FP64 lengths that bl_create takes: both factors up to 32, or 16-byte values of two
+// lines, their spectra and both factors' roots in 64 KB (primes up to 811).  That is
+// narrower than dct_holds, and kept: which lengths are refused is part of the interface.
+constexpr bool dct_takes_fp64(int N, int N1) {
+    const int K1 = N1 / 2 + 1, N2 = N / N1;
+    return (N1 <= 31 && N2 <= 32) || 16 * (2 * (size_t)N + 2 * (size_t)K1 * N2 + N1 + N2) <= 65536;
+}
+// FP32 lengths that go through these kernels, the others through the dense
+// split-BF16 product.  A long factor is a matrix product of its own here: at 1 x 251
+// points, 25542 lines, both directions take 131 us against 101 for the dense product
+// with its divergence pass, but in FP32 factors, not in 2^-18; longer ones would be
+// further behind.
+constexpr bool dct_takes_mixed(int N, int N1) { return N / N1 <= 256 && dct_holds(N, N1, 4); }
 // both factors within one row tile and two column tiles: two lines in two waves
 constexpr bool dct_small(int N, int N1) { return N1 <= 31 && N / N1 <= 31; }
 

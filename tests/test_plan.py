@@ -26,6 +26,8 @@ int main() {
             const int tiles = a == 4 ? march_tiles<float>(c + 1, d + 1) : march_tiles<double>(c + 1, d + 1);
             std::printf("%d %d %d\n", march_chunk(e - 1, tiles, 256, res), tiles, res);
         }
+        if (!std::strcmp(k, "takes"))
+            std::printf("%d %d %d %d\n", dct_takes_fp64(a, b), dct_takes_mixed(a, b), dct_holds(a, b, 8), dct_holds(a, b, 4));
         if (!std::strcmp(k, "thomas")) std::printf("%d\n", thomas_resident(a));
         if (!std::strcmp(k, "steps")) std::printf("%d\n", fewest_plane_steps(a, b, c, d).planes);
         if (!std::strcmp(k, "vfilter")) std::printf("%d\n", a == 4 ? vfilter_resident<float>() : vfilter_resident<double>());
@@ -158,3 +160,22 @@ def test_y_solve_plan(plan):
     each block, whatever its waves, has 40 KB of LDS, so four blocks at most."""
     for p, (n,) in zip(range(1, 9), plan([("thomas", p, 0, 0, 0, 0) for p in range(1, 9)])):
         assert n == min(8 // p, 163840 // 40960)
+
+
+def test_x_transform_lengths_taken(plan):
+    """FP64 takes the lengths that it always took (two 16-byte lines, their spectra and
+    the roots of both factors in 64 KB, or factors of up to 32), mixed precision factors
+    of up to 256 on the same kernels; and every length taken is one that the kernels
+    hold: the small division's range and one line of either direction in 160 KB."""
+    lengths = list(range(3, 5000))
+    for n, (fp64, mixed, holds64, holds32) in zip(lengths, plan([("takes", n, factor(n)[0], 0, 0, 0) for n in lengths])):
+        n1, n2 = factor(n)
+        k1 = n1 // 2 + 1
+        assert fp64 == ((n1 <= 32 and k1 <= 16 and n2 <= 32) or 16 * (2 * n + 2 * k1 * n2 + n1 + n2) <= 65536)
+        spec = 2 * k1 * (n2 | 1)
+        for es, holds in ((8, holds64), (4, holds32)):
+            if holds:
+                assert k1 <= 128 and k1 * n2 < 16384 and es * (max(n + 1, spec) + spec) <= 163840, n
+        assert not fp64 or holds64
+        assert not mixed or holds32
+        assert mixed == (n2 <= 256 and holds32)
